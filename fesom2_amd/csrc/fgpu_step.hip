@@ -32,6 +32,21 @@
 
 #define NG 8    // edges per gather batch in K_B and K_C
 
+// A value at a wave-uniform address that the running kernel does not write: a
+// mesh record, the processing order or a tracer's scheme. Read through the
+// constant address space it is one scalar load. As an ordinary load the
+// compiler has to assume that the field stores of the tracer loop may change
+// it, and issues one vector load per value, tracer and wave: 17 of K_A's 27
+// vector loads per tracer were such broadcasts of the edge record (K_A at
+// 127 thousand nodes, 47 layers, 2 tracers: 669 -> 544 us; with two levels per
+// lane at 40 thousand nodes, 70 layers, 10 tracers: 1490 -> 1266 us).
+#define CONST_AS __attribute__((address_space(4)))
+template <typename T>
+__device__ __forceinline__ T ldc(const T *p)
+{
+    return *(const CONST_AS T *)(unsigned long long)p;
+}
+
 __device__ __forceinline__ double dmx(double a, double b) { return a > b ? a : b; }
 __device__ __forceinline__ double dmn(double a, double b) { return a < b ? a : b; }
 
@@ -143,7 +158,7 @@ __global__ void __launch_bounds__(LB) kG_node(DevMesh m, DevTracers t, const int
 {
     const int jn = xcd_column(m.N2);
     if (jn >= m.N2) return;
-    const int n = m.node_ord[jn];
+    const int n = ldc(m.node_ord + jn);
     const int k0 = kneed[n], nzmax = m.nlevn[n];
     if (k0 > nzmax - 1) return;
     const int L = m.L;
@@ -164,7 +179,7 @@ __global__ void __launch_bounds__(LB) kG_node(DevMesh m, DevTracers t, const int
     const bool act = (k >= k0 && k <= nzmax - 1);
     const int trb = blockIdx.y * tpb, tre = min(t.ntr, trb + tpb);
     for (int tr = trb; tr < tre; ++tr) {
-        if (t.hor[tr] == HOR_UPW1) continue;   // node means feed MFCT and MUSCL
+        if (ldc(t.hor + tr) == HOR_UPW1) continue;   // node means feed MFCT and MUSCL
         const double *T = t.T + t.sN * tr;
         double tvol = 0.0, tx = 0.0, ty = 0.0;
         for (int i = 0; i < num; ++i) {
@@ -199,12 +214,12 @@ __global__ void __launch_bounds__(LB) __attribute__((amdgpu_waves_per_eu(6, 8)))
 {
     const int je = xcd_column(m.E2);
     if (je >= m.E2) return;
-    const int e = m.edge_ord[je];
+    const int e = ldc(m.edge_ord + je);
     const int k = threadIdx.x + 1;
     const int L = m.L;
     const int *ri = m.erec_i + (size_t)e * ERI;
     const double *rd = m.erec_d + (size_t)e * ERD;
-    const int nl1 = ri[ER_NL1], nu1 = ri[ER_NU1], nl2 = ri[ER_NL2], nu2 = ri[ER_NU2];
+    const int nl1 = ldc(ri + ER_NL1), nu1 = ldc(ri + ER_NU1), nl2 = ldc(ri + ER_NL2), nu2 = ldc(ri + ER_NU2);
     const int nl12 = min(nl1, nl2), nu12 = max(nu1, nu2);
     bool in[5];
     in[0] = (k >= nu1 && k <= nu12 - 1);
@@ -213,9 +228,9 @@ __global__ void __launch_bounds__(LB) __attribute__((amdgpu_waves_per_eu(6, 8)))
     in[3] = (k >= nl12 + 1 && k <= nl1);
     in[4] = (k >= nl12 + 1 && k <= nl2);
     if (!(in[0] || in[1] || in[2] || in[3] || in[4])) return;
-    const int n1 = ri[ER_N1], n2 = ri[ER_N2], el1 = ri[ER_EL1], el2 = ri[ER_EL2];
-    const double dX1 = rd[ER_DX1], dY1 = rd[ER_DY1], dX2 = rd[ER_DX2], dY2 = rd[ER_DY2];
-    const double a = rd[ER_A], edx = rd[ER_EDX], edy = rd[ER_EDY];
+    const int n1 = ldc(ri + ER_N1), n2 = ldc(ri + ER_N2), el1 = ldc(ri + ER_EL1), el2 = ldc(ri + ER_EL2);
+    const double dX1 = ldc(rd + ER_DX1), dY1 = ldc(rd + ER_DY1), dX2 = ldc(rd + ER_DX2), dY2 = ldc(rd + ER_DY2);
+    const double a = ldc(rd + ER_A), edx = ldc(rd + ER_EDX), edy = ldc(rd + ER_EDY);
     const size_t q1 = (size_t)el1 * L + k - 1;
     const double u1 = d.uv[2 * q1], v1 = d.uv[2 * q1 + 1], h1 = m.helem[q1];
     double u2 = 0.0, v2 = 0.0, h2 = 0.0;
@@ -234,9 +249,9 @@ __global__ void __launch_bounds__(LB) __attribute__((amdgpu_waves_per_eu(6, 8)))
     // gradient rule of fill_up_dn_grad at this level (oce_muscl_adv.F90:375-520);
     // writes in the reference's order, a later write wins
     bool shared = false, mean1 = false, mean2 = false;
-    const int u1l = ri[ER_U1], u2l = ri[ER_U2], nl1n = ri[ER_NL1N], nl2n = ri[ER_NL2N];
-    if (ri[ER_RULE]) {
-        const int nzmin = ri[ER_NZMIN], nzmax = ri[ER_NZMAX];
+    const int u1l = ldc(ri + ER_U1), u2l = ldc(ri + ER_U2), nl1n = ldc(ri + ER_NL1N), nl2n = ldc(ri + ER_NL2N);
+    if (ldc(ri + ER_RULE)) {
+        const int nzmin = ldc(ri + ER_NZMIN), nzmax = ldc(ri + ER_NZMAX);
         mean1 = (k >= u1l && k <= nzmin - 1);
         mean2 = (k >= u2l && k <= nzmin - 1);
         if (k >= nzmin && k <= nzmax - 1) { shared = true; mean1 = false; mean2 = false; }
@@ -246,8 +261,8 @@ __global__ void __launch_bounds__(LB) __attribute__((amdgpu_waves_per_eu(6, 8)))
         mean1 = (k >= u1l && k <= nl1n - 1);
         mean2 = (k >= u2l && k <= nl2n - 1);
     }
-    const int ua0 = ri[ER_UA0], ua1 = ri[ER_UA1], ua2 = ri[ER_UA2];
-    const int da0 = ri[ER_DA0], da1 = ri[ER_DA1], da2 = ri[ER_DA2];
+    const int ua0 = ldc(ri + ER_UA0), ua1 = ldc(ri + ER_UA1), ua2 = ldc(ri + ER_UA2);
+    const int da0 = ldc(ri + ER_DA0), da1 = ldc(ri + ER_DA1), da2 = ldc(ri + ER_DA2);
     const size_t o1 = (size_t)n1 * L + k - 1, o2 = (size_t)n2 * L + k - 1;
     const size_t ei = (size_t)e * L + k - 1;
     const size_t kk = (size_t)k - 1;
@@ -255,7 +270,7 @@ __global__ void __launch_bounds__(LB) __attribute__((amdgpu_waves_per_eu(6, 8)))
     for (int tr = trb; tr < tre; ++tr) {
         const double *T = t.T + t.sN * tr;
         const double *Told = t.Told + t.sOld * tr;
-        const int abo = t.abo[tr], lim = t.lim[tr], hor = t.hor[tr];
+        const int abo = ldc(t.abo + tr), lim = ldc(t.lim + tr), hor = ldc(t.hor + tr);
         double flo = 0.0;
         const double T1 = T[o1], T2 = T[o2];
         if (lim == LIM_FCT) {
@@ -273,15 +288,15 @@ __global__ void __launch_bounds__(LB) __attribute__((amdgpu_waves_per_eu(6, 8)))
         }
         double f = flo;
         if (hor != HOR_UPW1) {   // MFCT, MUSCL
-            const double no = t.ph[tr];
+            const double no = ldc(t.ph + tr);
             double g[4] = {0.0, 0.0, 0.0, 0.0};
             if (shared) {
                 const double u0 = T[(size_t)ua0 * L + kk], u1_ = T[(size_t)ua1 * L + kk], u2_ = T[(size_t)ua2 * L + kk];
                 const double w0 = T[(size_t)da0 * L + kk], w1 = T[(size_t)da1 * L + kk], w2 = T[(size_t)da2 * L + kk];
-                g[0] = rd[ER_GU0] * u0 + rd[ER_GU1] * u1_ + rd[ER_GU2] * u2_;
-                g[2] = rd[ER_GU3] * u0 + rd[ER_GU4] * u1_ + rd[ER_GU5] * u2_;
-                g[1] = rd[ER_GD0] * w0 + rd[ER_GD1] * w1 + rd[ER_GD2] * w2;
-                g[3] = rd[ER_GD3] * w0 + rd[ER_GD4] * w1 + rd[ER_GD5] * w2;
+                g[0] = ldc(rd + ER_GU0) * u0 + ldc(rd + ER_GU1) * u1_ + ldc(rd + ER_GU2) * u2_;
+                g[2] = ldc(rd + ER_GU3) * u0 + ldc(rd + ER_GU4) * u1_ + ldc(rd + ER_GU5) * u2_;
+                g[1] = ldc(rd + ER_GD0) * w0 + ldc(rd + ER_GD1) * w1 + ldc(rd + ER_GD2) * w2;
+                g[3] = ldc(rd + ER_GD3) * w0 + ldc(rd + ER_GD4) * w1 + ldc(rd + ER_GD5) * w2;
             } else {
                 const double *gm = t.gmean + t.sG * tr;
                 if (mean1) { g[0] = gm[2 * o1]; g[2] = gm[2 * o1 + 1]; }
@@ -289,7 +304,7 @@ __global__ void __launch_bounds__(LB) __attribute__((amdgpu_waves_per_eu(6, 8)))
             }
             double Tmean2, Tmean1;
             if (hor == HOR_MUSCL) {   // reconstruction only down to nboundary_lay (oce_adv_tra_hor.F90:356-367)
-                const double c1 = k <= ri[ER_NBL1] ? 1.0 : 0.0, c2 = k <= ri[ER_NBL2] ? 1.0 : 0.0;
+                const double c1 = k <= ldc(ri + ER_NBL1) ? 1.0 : 0.0, c2 = k <= ldc(ri + ER_NBL2) ? 1.0 : 0.0;
                 Tmean2 = A2 - (2.0 * (A2 - A1) + edx * a * g[1] + edy * FGPU_R_EARTH * g[3]) / 6.0 * c2;
                 Tmean1 = A1 + (2.0 * (A2 - A1) + edx * a * g[0] + edy * FGPU_R_EARTH * g[2]) / 6.0 * c1;
             } else {
@@ -337,12 +352,12 @@ __global__ void __launch_bounds__(64) kA2_edge(DevMesh m, DevDyn d, DevTracers t
 {
     const int je = xcd_column(m.E2);
     if (je >= m.E2) return;
-    const int e = m.edge_ord[je];
+    const int e = ldc(m.edge_ord + je);
     const int kb = 2 * (int)threadIdx.x + 1;   // this lane's levels: kb, kb + 1
     const int L = m.L;
     const int *ri = m.erec_i + (size_t)e * ERI;
     const double *rd = m.erec_d + (size_t)e * ERD;
-    const int nl1 = ri[ER_NL1], nu1 = ri[ER_NU1], nl2 = ri[ER_NL2], nu2 = ri[ER_NU2];
+    const int nl1 = ldc(ri + ER_NL1), nu1 = ldc(ri + ER_NU1), nl2 = ldc(ri + ER_NL2), nu2 = ldc(ri + ER_NU2);
     const int nl12 = min(nl1, nl2), nu12 = max(nu1, nu2);
     bool act[2], need2[2];
     int s1[2], s2[2];
@@ -361,9 +376,9 @@ __global__ void __launch_bounds__(64) kA2_edge(DevMesh m, DevDyn d, DevTracers t
         s2[s] = i1 ? 1 : (i4 ? 4 : -1);
     }
     if (!act[0] && !act[1]) return;
-    const int n1 = ri[ER_N1], n2 = ri[ER_N2], el1 = ri[ER_EL1], el2 = ri[ER_EL2];
-    const double dX1 = rd[ER_DX1], dY1 = rd[ER_DY1], dX2 = rd[ER_DX2], dY2 = rd[ER_DY2];
-    const double a = rd[ER_A], edx = rd[ER_EDX], edy = rd[ER_EDY];
+    const int n1 = ldc(ri + ER_N1), n2 = ldc(ri + ER_N2), el1 = ldc(ri + ER_EL1), el2 = ldc(ri + ER_EL2);
+    const double dX1 = ldc(rd + ER_DX1), dY1 = ldc(rd + ER_DY1), dX2 = ldc(rd + ER_DX2), dY2 = ldc(rd + ER_DY2);
+    const double a = ldc(rd + ER_A), edx = ldc(rd + ER_EDX), edy = ldc(rd + ER_EDY);
     double vf1[2], vf2[2];
     {
         const size_t q1 = (size_t)el1 * L + kb - 1;
@@ -384,13 +399,13 @@ __global__ void __launch_bounds__(64) kA2_edge(DevMesh m, DevDyn d, DevTracers t
     }
     // gradient rule of fill_up_dn_grad per level (oce_muscl_adv.F90:375-520)
     bool shared[2], mean1[2], mean2[2];
-    const int u1l = ri[ER_U1], u2l = ri[ER_U2], nl1n = ri[ER_NL1N], nl2n = ri[ER_NL2N];
+    const int u1l = ldc(ri + ER_U1), u2l = ldc(ri + ER_U2), nl1n = ldc(ri + ER_NL1N), nl2n = ldc(ri + ER_NL2N);
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
         const int k = kb + s;
         shared[s] = false;
-        if (ri[ER_RULE]) {
-            const int nzmin = ri[ER_NZMIN], nzmax = ri[ER_NZMAX];
+        if (ldc(ri + ER_RULE)) {
+            const int nzmin = ldc(ri + ER_NZMIN), nzmax = ldc(ri + ER_NZMAX);
             mean1[s] = (k >= u1l && k <= nzmin - 1);
             mean2[s] = (k >= u2l && k <= nzmin - 1);
             if (k >= nzmin && k <= nzmax - 1) { shared[s] = true; mean1[s] = false; mean2[s] = false; }
@@ -404,8 +419,8 @@ __global__ void __launch_bounds__(64) kA2_edge(DevMesh m, DevDyn d, DevTracers t
     const bool any_sh = (act[0] && shared[0]) || (act[1] && shared[1]);
     const bool any_m1 = (act[0] && !shared[0] && mean1[0]) || (act[1] && !shared[1] && mean1[1]);
     const bool any_m2 = (act[0] && !shared[0] && mean2[0]) || (act[1] && !shared[1] && mean2[1]);
-    const int ua0 = ri[ER_UA0], ua1 = ri[ER_UA1], ua2 = ri[ER_UA2];
-    const int da0 = ri[ER_DA0], da1 = ri[ER_DA1], da2 = ri[ER_DA2];
+    const int ua0 = ldc(ri + ER_UA0), ua1 = ldc(ri + ER_UA1), ua2 = ldc(ri + ER_UA2);
+    const int da0 = ldc(ri + ER_DA0), da1 = ldc(ri + ER_DA1), da2 = ldc(ri + ER_DA2);
     const size_t o1 = (size_t)n1 * L + kb - 1, o2 = (size_t)n2 * L + kb - 1;
     const size_t ei = (size_t)e * L + kb - 1;
     const size_t kk = (size_t)kb - 1;
@@ -413,7 +428,7 @@ __global__ void __launch_bounds__(64) kA2_edge(DevMesh m, DevDyn d, DevTracers t
     for (int tr = trb; tr < tre; ++tr) {
         const double *T = t.T + t.sN * tr;
         const double *Told = t.Told + t.sOld * tr;
-        const int abo = t.abo[tr], lim = t.lim[tr], hor = t.hor[tr];
+        const int abo = ldc(t.abo + tr), lim = ldc(t.lim + tr), hor = ldc(t.hor + tr);
         const double2 t1 = ld2(T + o1), t2 = ld2(T + o2);
         const double T1[2] = {t1.x, t1.y}, T2[2] = {t2.x, t2.y};
         double flo[2] = {0.0, 0.0};
@@ -444,7 +459,7 @@ __global__ void __launch_bounds__(64) kA2_edge(DevMesh m, DevDyn d, DevTracers t
         }
         double f[2] = {flo[0], flo[1]};
         if (hor != HOR_UPW1) {   // MFCT, MUSCL
-            const double no = t.ph[tr];
+            const double no = ldc(t.ph + tr);
             double2 ux0, ux1, ux2, wx0, wx1, wx2;
             if (any_sh) {
                 ux0 = ld2(T + (size_t)ua0 * L + kk);
@@ -464,10 +479,10 @@ __global__ void __launch_bounds__(64) kA2_edge(DevMesh m, DevDyn d, DevTracers t
                 if (shared[s]) {
                     const double u0 = s ? ux0.y : ux0.x, u1_ = s ? ux1.y : ux1.x, u2_ = s ? ux2.y : ux2.x;
                     const double w0 = s ? wx0.y : wx0.x, w1 = s ? wx1.y : wx1.x, w2 = s ? wx2.y : wx2.x;
-                    g[0] = rd[ER_GU0] * u0 + rd[ER_GU1] * u1_ + rd[ER_GU2] * u2_;
-                    g[2] = rd[ER_GU3] * u0 + rd[ER_GU4] * u1_ + rd[ER_GU5] * u2_;
-                    g[1] = rd[ER_GD0] * w0 + rd[ER_GD1] * w1 + rd[ER_GD2] * w2;
-                    g[3] = rd[ER_GD3] * w0 + rd[ER_GD4] * w1 + rd[ER_GD5] * w2;
+                    g[0] = ldc(rd + ER_GU0) * u0 + ldc(rd + ER_GU1) * u1_ + ldc(rd + ER_GU2) * u2_;
+                    g[2] = ldc(rd + ER_GU3) * u0 + ldc(rd + ER_GU4) * u1_ + ldc(rd + ER_GU5) * u2_;
+                    g[1] = ldc(rd + ER_GD0) * w0 + ldc(rd + ER_GD1) * w1 + ldc(rd + ER_GD2) * w2;
+                    g[3] = ldc(rd + ER_GD3) * w0 + ldc(rd + ER_GD4) * w1 + ldc(rd + ER_GD5) * w2;
                 } else {
                     if (mean1[s]) { const double2 q = s ? m1b : m1a; g[0] = q.x; g[2] = q.y; }
                     if (mean2[s]) { const double2 q = s ? m2b : m2a; g[1] = q.x; g[3] = q.y; }
@@ -475,7 +490,7 @@ __global__ void __launch_bounds__(64) kA2_edge(DevMesh m, DevDyn d, DevTracers t
                 double Tmean2, Tmean1;
                 if (hor == HOR_MUSCL) {   // reconstruction only down to nboundary_lay (oce_adv_tra_hor.F90:356-367)
                     const int k = kb + s;
-                    const double c1 = k <= ri[ER_NBL1] ? 1.0 : 0.0, c2 = k <= ri[ER_NBL2] ? 1.0 : 0.0;
+                    const double c1 = k <= ldc(ri + ER_NBL1) ? 1.0 : 0.0, c2 = k <= ldc(ri + ER_NBL2) ? 1.0 : 0.0;
                     Tmean2 = A2[s] - (2.0 * (A2[s] - A1[s]) + edx * a * g[1] + edy * FGPU_R_EARTH * g[3]) / 6.0 * c2;
                     Tmean1 = A1[s] + (2.0 * (A2[s] - A1[s]) + edx * a * g[0] + edy * FGPU_R_EARTH * g[2]) / 6.0 * c1;
                 } else {
@@ -550,7 +565,7 @@ __global__ void __launch_bounds__(LB) kB_node(DevMesh m, DevDyn d, DevTracers t,
 {
     const int j = xcd_column(m.N2);
     if (j >= m.N2) return;
-    const int n = m.node_ord[j];
+    const int n = ldc(m.node_ord + j);
     __shared__ double sT[LB + 2], sA[LB + 2], sW[LB + 2], sWe[LB + 2], sAr[LB + 2], sZ[LB + 2], sZb[LB + 2];
     __shared__ double sLo[LB + 2], sHn[XV ? LB + 2 : 1], sHo[XV ? LB + 2 : 1];
     constexpr int NW = WS ? LB + 2 : 1;
@@ -608,8 +623,8 @@ __global__ void __launch_bounds__(LB) kB_node(DevMesh m, DevDyn d, DevTracers t,
     for (int tr = trb; tr < tre; ++tr) {
         const double *T = t.T + t.sN * tr;
         const double *Told = t.Told + t.sOld * tr;
-        const int abo = t.abo[tr], lim = t.lim[tr], ver = t.ver[tr];
-        const double pv = t.pv[tr];
+        const int abo = ldc(t.abo + tr), lim = ldc(t.lim + tr), ver = ldc(t.ver + tr);
+        const double pv = ldc(t.pv + tr);
         __syncthreads();
         if (k <= L) {
             sT[tid] = T[ci];
@@ -716,7 +731,7 @@ __global__ void __launch_bounds__(64) kB2_node(DevMesh m, DevDyn d, DevTracers t
 {
     const int jc = xcd_column(m.N2);
     if (jc >= m.N2) return;
-    const int n = m.node_ord[jc];
+    const int n = ldc(m.node_ord + jc);
     __shared__ double sT[130], sA[130], sW[130], sWe[130], sAr[130], sZ[130], sZb[130], sLo[130];
     const int kb = 2 * (int)threadIdx.x + 1;   // this lane's levels and interfaces: kb, kb + 1
     const int L = m.L, NL = m.NL;
@@ -753,8 +768,8 @@ __global__ void __launch_bounds__(64) kB2_node(DevMesh m, DevDyn d, DevTracers t
     for (int tr = trb; tr < tre; ++tr) {
         const double *T = t.T + t.sN * tr;
         const double *Told = t.Told + t.sOld * tr;
-        const int abo = t.abo[tr], lim = t.lim[tr], ver = t.ver[tr];
-        const double pv = t.pv[tr];
+        const int abo = ldc(t.abo + tr), lim = ldc(t.lim + tr), ver = ldc(t.ver + tr);
+        const double pv = ldc(t.pv + tr);
         __syncthreads();
         if (kb <= L) {   // T and T^AB (oce_tracer_mod.F90:44-59) of both levels
             const double2 tv = ld2(T + ci);
@@ -845,7 +860,7 @@ __global__ void __launch_bounds__(LB) kC_node(DevMesh m, DevTracers t, double dt
 {
     const int j = xcd_column(m.N2);
     if (j >= m.N2) return;
-    const int n = m.node_ord[j];
+    const int n = ldc(m.node_ord + j);
     __shared__ double sMx[LB + 2], sMn[LB + 2];
     const int tid = threadIdx.x, k = tid + 1;
     const int L = m.L, NL = m.NL;
@@ -862,7 +877,7 @@ __global__ void __launch_bounds__(LB) kC_node(DevMesh m, DevTracers t, double dt
     const bool padded = k < pr.x || k >= pr.y;   // an element around n lacks level k
     const int trb = blockIdx.y * tpb, tre = min(t.ntr, trb + tpb);
     for (int tr = trb; tr < tre; ++tr) {
-        if (t.lim[tr] != LIM_FCT) continue;   // uniform over the block
+        if (ldc(t.lim + tr) != LIM_FCT) continue;   // uniform over the block
         const double *T = t.T + t.sN * tr;
         const double *LO = t.fct_lo + t.sN * tr;
         const double *ah = t.a_h + t.sE * tr;
@@ -955,7 +970,7 @@ __global__ void __launch_bounds__(64) kCf_node(DevMesh m, DevTracers t, double d
     __shared__ double sMx[TPF][RS], sMn[TPF][RS];
     const int jn = xcd_column(m.N2);
     if (jn >= m.N2) return;
-    const int n = m.node_ord[jn];
+    const int n = ldc(m.node_ord + jn);
     const int lane = threadIdx.x;
     const int L = m.L, NL = m.NL;
     const int nzmin = m.ulevn[n], nzmax = m.nlevn[n];
@@ -975,7 +990,7 @@ __global__ void __launch_bounds__(64) kCf_node(DevMesh m, DevTracers t, double d
         const bool on = i < items;
         const int tri = on ? (int)(((float)i + 0.5f) * inw) : 0;
         const int tr = trb + tri, k = nzmin + (on ? i - tri * nw : 0);
-        const bool act = on && t.lim[tr] == LIM_FCT;
+        const bool act = on && ldc(t.lim + tr) == LIM_FCT;
         const size_t ci = (size_t)n * L + k - 1;
         const double *T = t.T + t.sN * tr;
         const double *LO = t.fct_lo + t.sN * tr;
@@ -1047,7 +1062,7 @@ __global__ void __launch_bounds__(64) kCf_node(DevMesh m, DevTracers t, double d
         const bool on = i < items;
         const int tri = on ? (int)(((float)i + 0.5f) * inw) : 0;
         const int tr = trb + tri, k = nzmin + (on ? i - tri * nw : 0);
-        if (!(on && t.lim[tr] == LIM_FCT)) continue;
+        if (!(on && ldc(t.lim + tr) == LIM_FCT)) continue;
         const size_t ci = (size_t)n * L + k - 1;
         const double hn = m.hnode_new[ci], av_ = m.areasvol[(size_t)n * NL + k - 1];
         const double lo = lo_[c], vmax = sMx[tri][k - 1], vmin = sMn[tri][k - 1];
@@ -1191,8 +1206,8 @@ __global__ void __launch_bounds__(LB * CPB) __attribute__((amdgpu_waves_per_eu(6
             const int tr = t0 + c;
             double *T = t.T + t.sN * tr;
             double *Told = t.Told + t.sOld * tr;
-            const int abo = t.abo[tr];
-            const bool fct = t.lim[tr] == LIM_FCT;
+            const int abo = ldc(t.abo + tr);
+            const bool fct = ldc(t.lim + tr) == LIM_FCT;
             const double *av = t.a_v + t.sNI * tr + (size_t)n * NL;
             __syncthreads();
             if (fct && k <= L) {
@@ -1295,7 +1310,7 @@ __global__ void __launch_bounds__(LB * CPB) __attribute__((amdgpu_waves_per_eu(6
                 }
             }
             if (act) {
-                if (DX && !t.ivd[tr]) del = del + t.ve[t.sN * tr + ci];
+                if (DX && !ldc(t.ivd + tr)) del = del + t.ve[t.sN * tr + ci];
                 if (DX && d.redi) del = del + t.vr[t.sN * tr + ci];
                 del = del + Tk * (hh - hn);
                 sTsA[w][c][tid] = Tk + del / hn;
@@ -1312,17 +1327,17 @@ __global__ void __launch_bounds__(LB * CPB) __attribute__((amdgpu_waves_per_eu(6
         // right-hand sides (oce_ale_tracer.F90:1206-1229, 1377-1383), all tracers of the chunk
         for (int c = 0; c < nch; ++c) {
             const int tr = t0 + c;
-            if (!t.ivd[tr] || !act) continue;
+            if (!ldc(t.ivd + tr) || !act) continue;
             const double dz = hn;
             const double *ts = sTsA[w][c];
-            const bool wim = WS && t.lim[tr] != LIM_FCT;
+            const bool wim = WS && ldc(t.lim + tr) != LIM_FCT;
             const double *ra = wim ? swaA[w] : sa, *rb = wim ? swbA[w] : sb, *rc = wim ? swcA[w] : sc;
             double r;
             if (k == nzmin) r = -(rb[tid] - dz) * ts[tid] - rc[tid] * ts[tid + 1];
             else if (k <= nzmax - 2) r = -ra[tid] * ts[tid - 1] - (rb[tid] - dz) * ts[tid] - rc[tid] * ts[tid + 1];
             else r = -ra[tid] * ts[tid - 1] - (rb[tid] - dz) * ts[tid];
-            if (bc_every_layer(t.id[tr], d)) r = r + bc_surface_dev(t.id[tr], dt, d, m.N2, L, n, k, ts[tid]);
-            else if (k == nzmin) r = r + bc_surface_dev(t.id[tr], dt, d, m.N2, L, n, nzmin, ts[tid]);
+            if (bc_every_layer(ldc(t.id + tr), d)) r = r + bc_surface_dev(ldc(t.id + tr), dt, d, m.N2, L, n, k, ts[tid]);
+            else if (k == nzmin) r = r + bc_surface_dev(ldc(t.id + tr), dt, d, m.N2, L, n, nzmin, ts[tid]);
             stpA[w][c][tid] = r;
         }
         __syncthreads();
@@ -1332,8 +1347,8 @@ __global__ void __launch_bounds__(LB * CPB) __attribute__((amdgpu_waves_per_eu(6
         if (threadIdx.x < CPB * nch) {
             const int wc = threadIdx.x / nch, c = threadIdx.x % nch;
             const int z0 = sNz[wc][0], z1 = sNz[wc][1];
-            if (z1 - 1 >= z0 && t.ivd[t0 + c]) {
-                const bool wim = WS && t.lim[t0 + c] != LIM_FCT;
+            if (z1 - 1 >= z0 && ldc(t.ivd + t0 + c)) {
+                const bool wim = WS && ldc(t.lim + t0 + c) != LIM_FCT;
                 const double *a_ = wim ? swaA[wc] : saA[wc], *b_ = wim ? swbA[wc] : sbA[wc], *c_ = wim ? swcA[wc] : scA[wc];
                 double *tp_ = stpA[wc][c], *ts = sTsA[wc][c];
                 double *cp_ = c == 0 ? sRpA[wc] : (c == 1 ? sRmA[wc] : scpX[wc][c >= 2 ? c - 2 : 0]);
@@ -1543,7 +1558,7 @@ kDp_node(DevMesh m, DevDyn d, DevTracers t, double dt, int clamp_tracer, int tpb
         if (lane < nw * nch) {
             const int wc = wlo + lane / nch, c = lane % nch;
             const int z0 = sNz[wc][0], z1 = sNz[wc][1];
-            if (z1 - 1 >= z0 && t.ivd[t0 + c]) {
+            if (z1 - 1 >= z0 && ldc(t.ivd + t0 + c)) {
                 const double *a_ = saA[wc], *b_ = sbA[wc], *c_ = scA[wc];
                 double *tp_ = stpA[bf][wc][c], *ts = sTsA[bf][wc][c], *cp_ = scpA[wc];
                 double tp = tp_[z0 - 1] / b_[z0 - 1];
@@ -1607,8 +1622,8 @@ kDp_node(DevMesh m, DevDyn d, DevTracers t, double dt, int clamp_tracer, int tpb
                 const int tr = t0 + c;
                 double *T = t.T + t.sN * tr;
                 double *Told = t.Told + t.sOld * tr;
-                const int abo = t.abo[tr];
-                const bool fct = t.lim[tr] == LIM_FCT;
+                const int abo = ldc(t.abo + tr);
+                const bool fct = ldc(t.lim + tr) == LIM_FCT;
                 const double *av = t.a_v + t.sNI * tr + (size_t)n * NL;
                 double rp_[S], rm_[S], rpu_[S], rmu_[S], avk_[S], avd_[S];
                 if constexpr (SH) {
@@ -1726,7 +1741,7 @@ kDp_node(DevMesh m, DevDyn d, DevTracers t, double dt, int clamp_tracer, int tpb
             // right-hand sides (oce_ale_tracer.F90:1206-1229, 1377-1383)
             for (int c = 0; c < nch; ++c) {
                 const int tr = t0 + c;
-                if (!t.ivd[tr]) continue;
+                if (!ldc(t.ivd + tr)) continue;
                 const double *ts = sTsA[bf][w][c];
 #pragma unroll
                 for (int s = 0; s < S; ++s) {
@@ -1737,15 +1752,15 @@ kDp_node(DevMesh m, DevDyn d, DevTracers t, double dt, int clamp_tracer, int tpb
                     if (k == nzmin) r = -(sb[i] - dz) * ts[i] - sc[i] * ts[i + 1];
                     else if (k <= nzmax - 2) r = -sa[i] * ts[i - 1] - (sb[i] - dz) * ts[i] - sc[i] * ts[i + 1];
                     else r = -sa[i] * ts[i - 1] - (sb[i] - dz) * ts[i];
-                    if (bc_every_layer(t.id[tr], d)) r = r + bc_surface_dev(t.id[tr], dt, d, m.N2, L, n, k, ts[i]);
-                    else if (k == nzmin) r = r + bc_surface_dev(t.id[tr], dt, d, m.N2, L, n, nzmin, ts[i]);
+                    if (bc_every_layer(ldc(t.id + tr), d)) r = r + bc_surface_dev(ldc(t.id + tr), dt, d, m.N2, L, n, k, ts[i]);
+                    else if (k == nzmin) r = r + bc_surface_dev(ldc(t.id + tr), dt, d, m.N2, L, n, nzmin, ts[i]);
                     stpA[bf][w][c][i] = r;
                 }
             }
             if (!SW) {   // this wave sweeps and stores its own column
                 wave_sync();
                 sweep_store(p, w, 1);
-                for (int c = 0; c < nch && !piv_ok; ++c) piv_ok = t.ivd[t0 + c] != 0;
+                for (int c = 0; c < nch && !piv_ok; ++c) piv_ok = ldc(t.ivd + t0 + c) != 0;
             }
         } else if (sweeper && p >= 1) {
             sweep_store(p - 1, 0, CPB);
