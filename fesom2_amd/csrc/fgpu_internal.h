@@ -148,14 +148,12 @@ struct ProfEntry {
     int launches = 0;
 };
 
-// variants of the fused step's last kernel (same results bit for bit)
-#define KD_LOCKSTEP 0    // kD_node: the block's waves in lock-step, sweeps on the first wave's lanes
-#define KD_SWEEPWAVE 1   // kDp_node<..., true>: one wave per column plus a sweep wave per block
-#define KD_WAVELOCAL 2   // kDp_node<..., false>: one wave per column, which sweeps its own column
-// kDp_node's LDS rows for columns of 65..KDP_SHORT_NL interfaces (70-layer
-// meshes): KDP_SHORT_NL + 2 doubles instead of 130, so that more blocks fit per
-// CU, and 3 or 4 columns per block
-#define KDP_SHORT_NL 72
+// last-kernel settings of fgpu_set_step_shape, kept as fgpu_step_variant
+// reports them; the step's kernels no longer differ by them
+#define KD_LOCKSTEP 0
+#define KD_SWEEPWAVE 1
+#define KD_WAVELOCAL 2
+#define KDP_SHORT_NL 72   // columns to this many interfaces take three or four per block in fgpu_step_shape's report
 
 struct fgpu_context {
     int device = 0;
@@ -184,13 +182,13 @@ struct fgpu_context {
     bool graph_valid = false;
     bool fused = true;        // batched step: fused kernels (false: one kernel per reference stage)
     int step_tpb = 4096;      // tracers per block of the fused step kernels (clamped to the tracer count)
-    int step_tch = 2;         // tracers per Thomas chunk of the fused step's last kernel (2 or 4)
-    int step_cpb = 1;         // columns per block of the fused step's last kernel (1, 4 or 8; 64-lane columns)
+    int step_tch = 2;         // fgpu_set_step_shape's Thomas chunk and columns per block, reported by
+    int step_cpb = 1;         // fgpu_step_shape
     int step_order = 1;       // processing order of the fused step's columns: 1 Hilbert, 0 index (FGPU_STEP_ORDER)
     int step_kcf = 0;         // K_C over (tracer, level) items with this many tracers per block (1, 2, 4); 0: kC_node
     int step_ka2 = 0;         // 1: K_A with two adjacent levels per lane (kA2_edge), for an even number of layers
     int step_kb2 = 0;         // 1: K_B likewise (kB2_node), without the W split and CDIFF/PPM tracers
-    int step_kdp = 0;         // last kernel of the plain step: KD_LOCKSTEP (kD_node), KD_SWEEPWAVE or KD_WAVELOCAL (kDp_node)
+    int step_kdp = 0;         // fgpu_set_step_shape's last-kernel variant, reported by fgpu_step_variant
     int stage_slots = 0;      // tr_xy/aux slots allocated for the per-stage kernels (0: none yet)
     // profiling
     bool prof = false;

@@ -34,7 +34,9 @@ extern "C" int fgpu_version(void) { return 1; }
 
 int fgpu_alloc(fgpu_context *c, void **p, size_t bytes, bool tracer_scope)
 {
-    if (bytes == 0) bytes = 8;
+    // the fused step reads rows of levels two or three at a time, so a row's last
+    // read may run up to 16 bytes past its end (the values are not used)
+    bytes += 64;
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess)
         return fgpu_fail(FGPU_ERR_NOMEM, std::string("hipMalloc(") + std::to_string(bytes) +

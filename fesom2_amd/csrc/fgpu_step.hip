@@ -1,4 +1,4 @@
-// Fused, batched tracer step for gfx950: five launches per step for all tracers.
+// Fused, batched tracer step for gfx950: six launches per step for all tracers.
 //
 //   K_G  node pass   area-weighted mean element gradient of T^n at the levels
 //                    where an edge needs it (fill_up_dn_grad's non-shared levels)
@@ -7,11 +7,12 @@
 //                    evaluated on the fly
 //   K_B  node pass   LO solution and antidiffusive vertical flux (QR4C/UPW1)
 //   K_C  node pass   FCT bounds over the 1-ring (edge gather), P+/P-, R+/R-
-//   K_D  node pass   limited vertical and horizontal fluxes, flux2dtracer, T*,
-//                    implicit vertical diffusion (Thomas), salinity clamp,
+//   K_L  node pass   limited vertical and horizontal fluxes, flux2dtracer, T*,
 //                    valuesold rotation
+//   K_V  column pass implicit vertical diffusion (Thomas), salinity clamp
+//   K_D  K_L and K_V in one, for the W split and the explicit diffusion terms
 //
-// K_B..K_D are separated by the three global dependencies of FCT (LO of the
+// K_B..K_L are separated by the three global dependencies of FCT (LO of the
 // neighbours, R+/R- of the neighbours, limited edge fluxes). One block owns one
 // column (an edge or a node) and every tracer; lanes run over levels, so a
 // column's topology and geometry are wave-uniform and its field accesses are
@@ -1084,19 +1085,18 @@ __global__ void __launch_bounds__(64) kCf_node(DevMesh m, DevTracers t, double d
 // ------------------------------------------------------------------------------
 // K_D: limited fluxes, flux2dtracer, T*, implicit vertical diffusion
 // ------------------------------------------------------------------------------
-// TCH: tracers per Thomas chunk; CPB: columns per block (one column per LB
-// lanes). The Thomas sweeps of all CPB x TCH (column, tracer) pairs of a block
-// run in one wave, one lane per pair, while the other waves wait: a serial
-// sweep then costs one wave's issue slots for CPB columns instead of one per
-// column. Both are launch-shape choices; the arithmetic is the same for all.
+// For the steps whose last stage carries extra terms; the plain step runs K_L
+// and K_V. The Thomas sweeps of a chunk of TCH tracers run on the first wave's
+// lanes, one per tracer.
 // XF bit 0 (use_wsplit): the non-FCT tracers' implicit diffusion also takes
 // the implicit part w_i of the split W (second set of rows). XF bit 1: the
 // explicit diffusion increments (Ki, Redi, i_vert_diff off) and the Redi K33
 // terms are compiled in. Both are launched only when in use.
-template <int LB, int TCH, int CPB, int XF>
-__global__ void __launch_bounds__(LB * CPB) __attribute__((amdgpu_waves_per_eu(6))) kD_node(DevMesh m, DevDyn d, DevTracers t, double dt, int clamp_tracer,
+template <int LB, int XF>
+__global__ void __launch_bounds__(LB) __attribute__((amdgpu_waves_per_eu(6))) kD_node(DevMesh m, DevDyn d, DevTracers t, double dt, int clamp_tracer,
                                                     int tpb)
 {
+    constexpr int TCH = 2, CPB = 1;
     const int w = threadIdx.x / LB;
     const int j0 = xcd_column(m.N2) * CPB + w;
     const bool valid = j0 < m.N2;
@@ -1388,386 +1388,459 @@ __global__ void __launch_bounds__(LB * CPB) __attribute__((amdgpu_waves_per_eu(6
 }
 
 // ------------------------------------------------------------------------------
-// K_D with one wave per column (plain step: no W split, no explicit diffusion)
+// Column waves: one wave per node column (or edge), NV adjacent levels per lane
+// and GT tracers per wave, 64 / GT lanes each. Rows are read and written NV
+// levels at a time.
 // ------------------------------------------------------------------------------
-// One wave per node column, S levels per lane (level k = lane + 1 + 64 s), so
-// every exchange between levels of a column stays inside one wave and needs
-// no workgroup barrier. The tracers of the block are taken in chunks of TCH.
-// SW: CPB column waves plus one sweep wave per block. In phase p the column
-//     waves compute the limited fluxes, T* and the tridiagonal right-hand
-//     sides of chunk p into one of two LDS buffers, while the sweep wave runs
-//     the Thomas sweeps of chunk p-1 (one lane per (column, tracer) pair) from
-//     the other buffer and stores that chunk's T^{n+1}; the serial sweeps
-//     overlap the level-parallel work of the next chunk.
-// !SW: CPB independent column waves, each of which sweeps and stores its own
-//     column after each chunk.
-// Same arithmetic as kD_node, so the results are bit-identical to it. Which of
-// the three is fastest depends on the workload (the autotuner picks): at
-// 1.3 M columns of up to 70 levels and 10 tracers the sweep wave gives
-// 63.5 ms per launch against 66.8 ms lock-step; at 127 k columns of up to
-// 47 levels and 2 tracers (one chunk, nothing to overlap) the lock-step
-// kernel is fastest (0.76 ms, against 0.84 ms wave-local).
+// two adjacent levels of a row: 16 bytes at any 8-byte boundary
+typedef double lv2 __attribute__((ext_vector_type(2), aligned(8)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x8 __attribute__((ext_vector_type(8)));
 
-
-// A column's values one level up and one level down the wave: lane j, slot s
-// holds level j + 1 + 64 s (the lane below, or across the slot boundary)
-template <int S>
-__device__ __forceinline__ void level_up(const double (&x)[S], double (&y)[S], int lane)
+// row values at p + off (bytes, 32 bits: the row base is wave-uniform)
+template <int NV>
+__device__ __forceinline__ void row_load(const double *p, unsigned off, double (&x)[NV])
 {
-    y[0] = __shfl_up(x[0], 1);   // lane 0 gets its own value (level 0 does not exist)
-    if constexpr (S == 2) {
-        const double last0 = __shfl(x[0], 63);
-        const double u1 = __shfl_up(x[1], 1);
-        y[1] = lane == 0 ? last0 : u1;
-    }
-}
-template <int S>
-__device__ __forceinline__ void level_down(const double (&x)[S], double (&y)[S], int lane)
-{
-    const double d0 = __shfl_down(x[0], 1);
-    if constexpr (S == 2) {
-        const double first1 = __shfl(x[1], 0);
-        y[0] = lane == 63 ? first1 : d0;
-        y[1] = __shfl_down(x[1], 1);
-    } else {
-        y[0] = d0;
-    }
-}
-
-// A one-wave block of short rows is held to 96 VGPRs (5 waves per SIMD; it
-// spills 40 bytes per lane): 54.1 -> 52.8 ms at 1.3 M columns of 70 levels
-template <int S, int TCH, int CPB, bool SW, int RS = 64 * S + 2, bool SH = false>
-__global__ void __launch_bounds__(64 * (CPB + (SW ? 1 : 0)))
-__attribute__((amdgpu_waves_per_eu((!SW && CPB == 1 && S == 2 && RS <= KDP_SHORT_NL + 2) ? 5 : 1, 8)))
-kDp_node(DevMesh m, DevDyn d, DevTracers t, double dt, int clamp_tracer, int tpb)
-{
-    // RS: LDS row of at least NL + 2 doubles (index k - 1 of levels and
-    // interfaces 1..NL, plus a guard); every LDS access is within k <= NL
-    constexpr int NB = SW ? 2 : 1;   // chunk buffers
-    // SH: R+- and the limited vertical fluxes, read one level away only, move
-    // between lanes by shuffles instead of LDS rows
-    __shared__ double sRpA[SH ? 1 : CPB][SH ? 1 : RS], sRmA[SH ? 1 : CPB][SH ? 1 : RS], sAvA[SH ? 1 : CPB][SH ? 1 : RS];
-    __shared__ double saA[CPB][RS], sbA[CPB][RS], scA[CPB][RS], scpA[CPB][RS];
-    __shared__ double sTsA[NB][CPB][TCH][RS], stpA[NB][CPB][TCH][RS];
-    __shared__ int sNz[CPB][2];
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const bool sweeper = SW && w == CPB;
-    const int L = m.L, NL = m.NL;
-    const int col0 = xcd_column(m.N2) * CPB;
-    const int trb = blockIdx.y * tpb, tre = min(t.ntr, trb + tpb);
-    const int nchunk = (tre - trb + TCH - 1) / TCH;
-
-    // ---- column waves: geometry and the tracer-independent tridiagonal rows
-    const int wc_ = sweeper ? 0 : w;
-    const int j0 = col0 + wc_;
-    const bool valid = !sweeper && j0 < m.N2;
-    const int n = m.node_ord[j0 < m.N2 ? j0 : m.N2 - 1];
-    const int nzmin = valid ? m.ulevn[n] : 1, nzmax = valid ? m.nlevn[n] : 0;
-    double *sRp = sRpA[SH ? 0 : wc_], *sRm = sRmA[SH ? 0 : wc_], *sAv = sAvA[SH ? 0 : wc_];
-    double *sZ = SH ? sTsA[0][wc_][0] : sAvA[wc_];   // a row that is dead before the first chunk
-    double *sa = saA[wc_], *sb = sbA[wc_], *sc = scA[wc_];
-    int kk_[S];
-    bool act_[S];
-    size_t ci_[S];
-    double hn_[S], hh_[S], av_[S], arv_[S];
+    const char *a = (const char *)p + off;
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-        const int k = lane + 1 + 64 * s;
-        kk_[s] = k;
-        act_[s] = k >= nzmin && k <= nzmax - 1;
-        ci_[s] = (size_t)n * L + (k <= L ? k - 1 : L - 1);
-        hn_[s] = 1.0; hh_[s] = 0.0; av_[s] = 1.0; arv_[s] = 0.0;
-        if (act_[s]) {
-            hn_[s] = m.hnode_new[ci_[s]];
-            hh_[s] = m.hnode[ci_[s]];
-            av_[s] = m.areasvol[(size_t)n * NL + k - 1];
-            arv_[s] = m.area[(size_t)n * NL + k - 1];
+    for (int s = 0; s + 1 < NV; s += 2) {
+        const lv2 v = *(const lv2 *)(a + 8 * s);
+        x[s] = v.x;
+        x[s + 1] = v.y;
+    }
+    if constexpr (NV % 2 == 1) x[NV - 1] = *(const double *)(a + 8 * (NV - 1));
+}
+
+template <int NV>
+__device__ __forceinline__ void row_store(double *p, unsigned off, const double (&x)[NV], const bool (&on)[NV])
+{
+    char *a = (char *)p + off;
+#pragma unroll
+    for (int s = 0; s + 1 < NV; s += 2) {
+        if (on[s] && on[s + 1]) {
+            lv2 v;
+            v.x = x[s];
+            v.y = x[s + 1];
+            *(lv2 *)(a + 8 * s) = v;
+        } else if (on[s]) {
+            *(double *)(a + 8 * s) = x[s];
+        } else if (on[s + 1]) {
+            *(double *)(a + 8 * s + 8) = x[s + 1];
         }
     }
-    NodeEdges E;
-    if (!sweeper) {
-        E = load_node_edges(m, n);
-        if (lane == 0) { sNz[w][0] = nzmin; sNz[w][1] = nzmax; }
+    if constexpr (NV % 2 == 1)
+        if (on[NV - 1]) *(double *)(a + 8 * (NV - 1)) = x[NV - 1];
+}
+
+// value of the next lower / higher lane of the wave (the end lanes keep their own)
+__device__ __forceinline__ double lane_below(double x)
+{
+    const long long b = __double_as_longlong(x);
+    const int lo = (int)(b & 0xffffffffLL), hi = (int)(b >> 32);
+    const int l = __builtin_amdgcn_update_dpp(lo, lo, 0x138, 0xf, 0xf, false);   // wave_shr:1
+    const int h = __builtin_amdgcn_update_dpp(hi, hi, 0x138, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)h << 32) | (unsigned int)l);
+}
+__device__ __forceinline__ double lane_above(double x)
+{
+    const long long b = __double_as_longlong(x);
+    const int lo = (int)(b & 0xffffffffLL), hi = (int)(b >> 32);
+    const int l = __builtin_amdgcn_update_dpp(lo, lo, 0x130, 0xf, 0xf, false);   // wave_shl:1
+    const int h = __builtin_amdgcn_update_dpp(hi, hi, 0x130, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)h << 32) | (unsigned int)l);
+}
+
+// a column's values one level up (k - 1) and one level down (k + 1)
+template <int NV>
+__device__ __forceinline__ void col_up(const double (&x)[NV], double (&y)[NV])
+{
+    y[0] = lane_below(x[NV - 1]);
 #pragma unroll
-        for (int s = 0; s < S; ++s)
-            if (act_[s]) sZ[kk_[s] - 1] = m.zn_vd[ci_[s]];
-        wave_sync();
+    for (int s = 1; s < NV; ++s) y[s] = x[s - 1];
+}
+template <int NV>
+__device__ __forceinline__ void col_down(const double (&x)[NV], double (&y)[NV])
+{
+    y[NV - 1] = lane_above(x[0]);
+#pragma unroll
+    for (int s = 0; s + 1 < NV; ++s) y[s] = x[s + 1];
+}
+
+// a / b, correctly rounded, for a divisor used many times: y = 1 / b rounded
+// once. Two Newton steps on the quotient with exact fma residuals; the second
+// starts from a faithful quotient, which with the rounded reciprocal gives the
+// correctly rounded one (Markstein, IBM J. Res. Dev. 34, 1990). That needs the
+// residuals clear of underflow: numerators outside 1e-200..1e200 (zeros,
+// infinities and NaN among them) and divisors outside 1e-60..1e60 (y_ok false)
+// take the division itself.
+struct Recip {
+    double b, y;
+    bool ok;
+};
+__device__ __forceinline__ Recip recip(double b)
+{
+    const double ab = fabs(b);
+    return {b, 1.0 / b, ab > 1e-60 && ab < 1e60};
+}
+__device__ __forceinline__ double div_by(double a, const Recip &r)
+{
+    const double q0 = a * r.y;
+    const double q1 = fma(fma(-r.b, q0, a), r.y, q0);
+    double q = fma(fma(-r.b, q1, a), r.y, q1);
+    const double aa = fabs(a);
+    if (!(r.ok && aa > 1e-200 && aa < 1e200)) {
+        q = q0;
+        if (!(r.ok && a == 0.0)) q = a / r.b;
+    }
+    return q;
+}
+
+// ------------------------------------------------------------------------------
+// K_L: limited fluxes, flux2dtracer and T* (oce_adv_tra_fct.F90:425-497,
+// oce_adv_tra_driver.F90:494-646, oce_ale_tracer.F90:595-626); T* replaces T,
+// T^n goes to valuesold. The implicit vertical diffusion follows in K_V.
+// Bound by the gathers of the neighbours' R+- and of the edge fluxes and, next,
+// by FP64 issue. The sweeps are a kernel of their own because inside the
+// column's wave they kept 2 to 10 of 64 lanes busy for most of its
+// instructions: 126,858 nodes, 47 layers, 2 tracers: one kernel 757 us, K_L
+// 356 us + K_V 159 us; 40 thousand nodes, 70 layers, 10 tracers: 1364 us,
+// 743 + 328 us. The divisions by areasvol and hnode_new, one per edge and
+// level, use a reciprocal formed once per column (div_by).
+// ------------------------------------------------------------------------------
+template <int NV, int GT>
+__global__ void __launch_bounds__(256) kL_node(DevMesh m, DevTracers t, double dt, int tpb)
+{
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int jc = xcd_column(m.N2) * 4 + w;
+    if (jc >= m.N2) return;
+    const int n = ldc(m.node_ord + jc);
+    const i32x4 nr = ldc((const i32x4 *)m.node_rec + n);
+    const int p0 = nr.x, deg = nr.y, nzmin = nr.z, nzmax = nr.w;
+    constexpr int LP = 64 / GT;
+    const int g = lane / LP, kb = (lane % LP) * NV + 1;
+    const int L = m.L, NL = m.NL;
+    const size_t nL = (size_t)n * L, nNL = (size_t)n * NL;
+    bool wet[NV];
+    Recip av[NV], hn[NV];
+    double hh[NV];
+    {
+        double a[NV], b[NV], c[NV];
+#pragma unroll
+        for (int s = 0; s < NV; ++s) {
+            wet[s] = kb + s >= nzmin && kb + s <= nzmax - 1;
+            a[s] = b[s] = c[s] = 1.0;
+        }
+        bool some = false;
+#pragma unroll
+        for (int s = 0; s < NV; ++s) some = some || wet[s];
+        if (some) {
+            const unsigned off = 8u * (unsigned)(kb - 1);
+            row_load<NV>(m.hnode_new + nL, off, a);
+            row_load<NV>(m.hnode + nL, off, b);
+            row_load<NV>(m.areasvol + nNL, off, c);
+        }
+#pragma unroll
+        for (int s = 0; s < NV; ++s) {
+            hn[s] = recip(a[s]);
+            hh[s] = b[s];
+            av[s] = recip(c[s]);
+        }
+    }
+    const int trb = blockIdx.y * tpb, tre = min(t.ntr, trb + tpb);
+    for (int tb = trb; tb < tre; tb += GT) {
+        const bool fct = ldc(t.lim + tb) == LIM_FCT;
+        const int abo = ldc(t.abo + tb);
+        const bool tr_on = GT == 1 || tb + g < tre;
+        const unsigned oN = 8u * ((unsigned)(kb - 1) + (unsigned)g * (unsigned)t.sN);
+        const unsigned oNI = 8u * ((unsigned)(kb - 1) + (unsigned)g * (unsigned)t.sNI);
+        const unsigned oE = 8u * ((unsigned)(kb - 1) + (unsigned)g * (unsigned)t.sE);
+        double *T = t.T + t.sN * tb + nL;
+        const double *rpT = t.rp + t.sN * tb, *rmT = t.rm + t.sN * tb, *ah = t.a_h + t.sE * tb;
+        bool act[NV], any = false, anyi = false;
+        double rp[NV], rm[NV], Tk[NV], lo[NV], f[NV], h[NV];
+#pragma unroll
+        for (int s = 0; s < NV; ++s) {
+            act[s] = wet[s] && tr_on;
+            any = any || act[s];
+            anyi = anyi || (tr_on && kb + s >= nzmin && kb + s <= nzmax);
+            rp[s] = rm[s] = 1.0;
+            Tk[s] = lo[s] = f[s] = h[s] = 0.0;
+        }
+        if (any) {
+            row_load<NV>(T, oN, Tk);
+            if (fct) {
+                row_load<NV>(rpT + nL, oN, rp);
+                row_load<NV>(rmT + nL, oN, rm);
+                row_load<NV>(t.fct_lo + t.sN * tb + nL, oN, lo);
+            }
+        }
+        if (anyi) row_load<NV>(t.a_v + t.sNI * tb + nNL, oNI, f);
+        // limited vertical antidiffusive flux at interface k (oce_adv_tra_fct.F90:425-456)
+        double v[NV];
+        {
+            double rpu[NV], rmu[NV], fd[NV];
+            if (fct) {
+                col_up<NV>(rp, rpu);
+                col_up<NV>(rm, rmu);
+#pragma unroll
+                for (int s = 0; s < NV; ++s) {
+                    const int k = kb + s;
+                    const double flux = f[s];
+                    const bool pos = flux >= 0.0;
+                    // above the interface R- (R+) of the layer, below it R+ (R-); none above the top one
+                    const double below = pos ? rp[s] : rm[s], above = pos ? rmu[s] : rpu[s];
+                    double ae = k == nzmin ? 1.0 : dmn(1.0, above);
+                    ae = dmn(ae, below);
+                    if (k <= nzmax - 1) f[s] = ae * flux;
+                }
+            }
+            col_down<NV>(f, fd);
+#pragma unroll
+            for (int s = 0; s < NV; ++s) {
+                v[s] = 0.0;
+                if (fct) v[s] = v[s] - Tk[s] * hh[s] + lo[s] * hn[s].b;
+                v[s] = v[s] + div_by((f[s] - fd[s]) * dt, av[s]);
+            }
+        }
+        // the edges' limited antidiffusive fluxes, in ascending order; three edges' loads at a time
+        constexpr int NB = NV == 3 ? 2 : 3;
+        for (int u0 = 0; u0 < deg; u0 += NB) {
+            double fl[NB][NV], rpo[NB][NV], rmo[NB][NV];
+            i32x8 rec[NB];
+#pragma unroll
+            for (int u = 0; u < NB; ++u) {
+                if (u0 + u >= deg) break;
+                rec[u] = ldc((const i32x8 *)m.ne_rec + p0 + u0 + u);
+            }
+#pragma unroll
+            for (int u = 0; u < NB; ++u) {
+                if (u0 + u >= deg) break;
+                const int q = rec[u][0], mo = rec[u][1], a0 = rec[u][2], a1 = rec[u][3];
+                if (any && kb + NV - 1 >= a0 && kb <= a1) {
+                    row_load<NV>(ah + (size_t)(q >> 1) * L, oE, fl[u]);
+                    if (fct) {
+                        row_load<NV>(rpT + (size_t)mo * L, oN, rpo[u]);
+                        row_load<NV>(rmT + (size_t)mo * L, oN, rmo[u]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < NB; ++u) {
+                if (u0 + u >= deg) break;
+                const int side = rec[u][0] & 1, a0 = rec[u][2], a1 = rec[u][3];
+#pragma unroll
+                for (int s = 0; s < NV; ++s) {
+                    const int k = kb + s;
+                    if (!(act[s] && k >= a0 && k <= a1)) continue;
+                    double x = fl[u][s];
+                    if (fct) {
+                        // node 1 takes R+ of an inflow, node 2 R- of the same flux, and the other way round
+                        const bool up = (x >= 0.0) != (side != 0);
+                        const double own = up ? rp[s] : rm[s], oth = up ? rmo[u][s] : rpo[u][s];
+                        x = (side ? dmn(dmn(1.0, oth), own) : dmn(dmn(1.0, own), oth)) * x;
+                    }
+                    const double c = div_by(x * dt, av[s]);
+                    h[s] = side ? h[s] - c : h[s] + c;
+                }
+            }
+        }
+        if (any) {
+            double ts[NV];
+#pragma unroll
+            for (int s = 0; s < NV; ++s) {
+                double del = 0.0 + h[s] + v[s];
+                del = del + Tk[s] * (hh[s] - hn[s].b);
+                ts[s] = Tk[s] + div_by(del, hn[s]);
+            }
+            row_store<NV>(T, oN, ts, act);
+            // valuesold rotation (oce_tracer_mod.F90:94-123)
+            double *Told = t.Told + t.sOld * (size_t)(GT == 1 ? tb : tb + g);
+            if (abo == 2) {
+                row_store<NV>(Told + nL, 8u * (unsigned)(kb - 1), Tk, act);
+            } else {
+#pragma unroll
+                for (int s = 0; s < NV; ++s) {
+                    if (!act[s]) continue;
+                    double *o = Told + 2 * (nL + kb - 1 + s);
+                    o[1] = o[0];
+                    o[0] = Tk[s];
+                }
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------
+// K_V: implicit vertical diffusion of T* in place (diff_ver_part_impl_ale,
+// oce_ale_tracer.F90:907-1435) and the salinity clamp. Bound by the latency of
+// a block: three dependent loads, the rows, and two serial passes over the
+// levels (about 200 cycles a level for the two dependent divisions).
+// ------------------------------------------------------------------------------
+// A block of eight waves takes NC columns x TB tracers, NC x TB <= 64 rows. Each
+// wave forms the tridiagonal rows and right-hand sides of its columns with
+// lanes over the levels and leaves them in LDS; one wave sweeps with one lane
+// per row, and the waves add the result to T*. LDS rows have an odd length, so
+// that the lanes of the sweep, each on its own row, use different banks.
+#define KV_NW 8   // waves of a block
+#define KV_TP 2   // tracers whose rows are loaded together
+template <int NV>
+__global__ void __launch_bounds__(64 * KV_NW) __attribute__((amdgpu_waves_per_eu(8)))
+kV_cols(DevMesh m, DevDyn d, DevTracers t, double dt, int clamp_tracer, int NC, int TB)
+{
+    extern __shared__ double lds[];
+    const int L = m.L, NL = m.NL, RS = L | 1;
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int col0 = xcd_unit() * NC;
+    if (col0 >= m.N2) return;
+    const int ncol = min(NC, m.N2 - col0);
+    const int trb = blockIdx.y * TB, ntb = min(TB, t.ntr - trb);
+    double *sa = lds, *sb = sa + (size_t)NC * RS, *sc = sb + (size_t)NC * RS, *sr = sc + (size_t)NC * RS;
+    // the block's columns, one per lane
+    const int nl_ = m.node_ord[col0 + min(lane, ncol - 1)];
+    const int z0l = m.ulevn[nl_], z1l = m.nlevn[nl_];
+    const int kb = lane * NV + 1;
+    const unsigned off = 8u * (unsigned)(kb - 1);
+    for (int c = w; c < ncol; c += KV_NW) {
+        const int n = rl(nl_, c), nzmin = rl(z0l, c), nzmax = rl(z1l, c);
+        const size_t nL = (size_t)n * L, nNL = (size_t)n * NL;
+        double hn[NV], av[NV], zk[NV], kv[NV], ar[NV], zu[NV], zd[NV], kvd[NV], ard[NV], a_[NV], c_[NV], bd_[NV];
+        double ts[KV_TP][NV];
+#pragma unroll
+        for (int s = 0; s < NV; ++s) hn[s] = av[s] = zk[s] = kv[s] = ar[s] = 1.0;
+        const bool layer = kb <= nzmax - 1;
+        if (kb <= nzmax) {   // interfaces to nzmax
+            row_load<NV>(d.Kv + nNL, off, kv);
+            row_load<NV>(m.area + nNL, off, ar);
+            row_load<NV>(m.areasvol + nNL, off, av);
+        }
+        if (layer) {
+            row_load<NV>(m.hnode_new + nL, off, hn);
+            row_load<NV>(m.zn_vd + nL, off, zk);
+#pragma unroll
+            for (int j = 0; j < KV_TP; ++j)
+                if (j < ntb) row_load<NV>(t.T + t.sN * (trb + j) + nL, off, ts[j]);
+        }
+        col_up<NV>(zk, zu);
+        col_down<NV>(zk, zd);
+        col_down<NV>(kv, kvd);
+        col_down<NV>(ar, ard);
         // tridiagonal coefficients (oce_ale_tracer.F90:1098-1175)
 #pragma unroll
-        for (int s = 0; s < S; ++s) {
-            if (!act_[s]) continue;
-            const int k = kk_[s];
-            const double *kv = d.Kv + (size_t)n * NL;
+        for (int s = 0; s < NV; ++s) {
+            const int k = kb + s;
+            a_[s] = c_[s] = bd_[s] = 0.0;
+            if (k < nzmin || k > nzmax - 1) continue;
             const double zinv = 1.0 * dt;
-            double a = 0.0, b, c;
-            if (k == nzmin) {
-                const double zinv2 = 1.0 / (sZ[k - 1] - sZ[k]);
-                c = -(kv[k]) * zinv2 * zinv * m.area[(size_t)n * NL + k] / av_[s];
-                b = -c + hn_[s];
-            } else if (k <= nzmax - 2) {
-                const double zinv1 = 1.0 / (sZ[k - 2] - sZ[k - 1]);
-                const double zinv2 = 1.0 / (sZ[k - 1] - sZ[k]);
-                a = -(kv[k - 1]) * zinv1 * zinv * (arv_[s] / av_[s]);
-                c = -(kv[k]) * zinv2 * zinv * m.area[(size_t)n * NL + k] / av_[s];
-                b = -a - c + hn_[s];
-            } else {
-                const double zinv1 = 1.0 / (sZ[k - 2] - sZ[k - 1]);
-                a = -(kv[k - 1]) * zinv1 * zinv * (arv_[s] / av_[s]);
-                c = 0.0;
-                b = -a + hn_[s];
+            double a = 0.0, b, cc = 0.0;
+            if (k > nzmin) {
+                const double zinv1 = 1.0 / (zu[s] - zk[s]);
+                a = -(kv[s]) * zinv1 * zinv * (ar[s] / av[s]);
             }
-            sa[k - 1] = a;
-            sb[k - 1] = b;
-            sc[k - 1] = c;
+            if (k <= nzmax - 2) {
+                const double zinv2 = 1.0 / (zk[s] - zd[s]);
+                cc = -(kvd[s]) * zinv2 * zinv * ard[s] / av[s];
+            }
+            if (k == nzmin) b = -cc + hn[s];
+            else if (k <= nzmax - 2) b = -a - cc + hn[s];
+            else b = -a + hn[s];
+            sa[c * RS + k - 1] = a;
+            sb[c * RS + k - 1] = b;
+            sc[c * RS + k - 1] = cc;
+            a_[s] = a;
+            c_[s] = cc;
+            bd_[s] = b - hn[s];
+        }
+        // right-hand sides (oce_ale_tracer.F90:1206-1229, 1377-1383)
+        for (int j0 = 0; j0 < ntb; j0 += KV_TP) {
+            if (j0 > 0 && layer) {
+#pragma unroll
+                for (int j = 0; j < KV_TP; ++j)
+                    if (j0 + j < ntb) row_load<NV>(t.T + t.sN * (trb + j0 + j) + nL, off, ts[j]);
+            }
+#pragma unroll
+            for (int j = 0; j < KV_TP; ++j) {
+                if (j0 + j >= ntb) break;
+                const int id = ldc(t.id + trb + j0 + j);
+                double tu[NV], td[NV];
+                col_up<NV>(ts[j], tu);
+                col_down<NV>(ts[j], td);
+#pragma unroll
+                for (int s = 0; s < NV; ++s) {
+                    const int k = kb + s;
+                    if (k < nzmin || k > nzmax - 1) continue;
+                    double r;
+                    if (k == nzmin) r = -bd_[s] * ts[j][s] - c_[s] * td[s];
+                    else if (k <= nzmax - 2) r = -a_[s] * tu[s] - bd_[s] * ts[j][s] - c_[s] * td[s];
+                    else r = -a_[s] * tu[s] - bd_[s] * ts[j][s];
+                    if (bc_every_layer(id, d)) r = r + bc_surface_dev(id, dt, d, m.N2, L, n, k, ts[j][s]);
+                    else if (k == nzmin) r = r + bc_surface_dev(id, dt, d, m.N2, L, n, nzmin, ts[j][s]);
+                    sr[(c * TB + j0 + j) * RS + k - 1] = r;
+                }
+            }
         }
     }
-    if (SW) __syncthreads();
-
-    // The forward-elimination pivots of the columns (oce_ale_tracer.F90:1406-1414):
-    // m = b - c'a and c' = c / m depend on the column only. With the sweep
-    // wave, its first CPB lanes compute the c' rows while the column waves
-    // work on the first chunk; every sweep then forms m again from b, a and
-    // the c' above (the same two operations) and divides once per level.
-    auto pivots = [&]() {
-        if (lane < CPB) {
-            const int wc = lane, z0 = sNz[wc][0], z1 = sNz[wc][1];
-            if (z1 - 1 >= z0) {
-                const double *a_ = saA[wc], *b_ = sbA[wc], *c_ = scA[wc];
-                double *cp_ = scpA[wc];
-                double cp = c_[z0 - 1] / b_[z0 - 1];
-                cp_[z0 - 1] = cp;
-                for (int nz = z0 + 1; nz <= z1 - 1; ++nz) {
-                    const double mm = b_[nz - 1] - cp * a_[nz - 1];
-                    cp = c_[nz - 1] / mm;
-                    cp_[nz - 1] = cp;
-                }
-            }
+    __syncthreads();
+    // Thomas sweeps (oce_ale_tracer.F90:1406-1430), one lane per row; the lanes
+    // of a column all compute its pivots. c' replaces c.
+    if (w == 0 && lane < ncol * ntb) {
+        const int c = lane / ntb, j = lane % ntb;
+        const int z0 = __shfl(z0l, c), z1 = __shfl(z1l, c);
+        const double *pa = sa + c * RS - 1, *pb = sb + c * RS - 1;
+        double *pc = sc + c * RS - 1, *pr = sr + (c * TB + j) * RS - 1;
+        double cp = pc[z0] / pb[z0], tp = pr[z0] / pb[z0];
+        pc[z0] = cp;
+        pr[z0] = tp;
+        double an = pa[z0 + 1], bn = pb[z0 + 1], cn = pc[z0 + 1], rn = pr[z0 + 1];
+        for (int nz = z0 + 1; nz <= z1 - 1; ++nz) {
+            const int nx = min(nz + 1, z1 - 1);   // the next level's rows, loaded ahead
+            const double a1 = pa[nx], b1 = pb[nx], c1 = pc[nx], r1 = pr[nx];
+            const double mm = bn - cp * an;
+            cp = cn / mm;
+            tp = (rn - tp * an) / mm;
+            pc[nz] = cp;
+            pr[nz] = tp;
+            an = a1; bn = b1; cn = c1; rn = r1;
         }
-    };
-
-    // Without the sweep wave, the first sweep of a column writes its c' row
-    // (every lane of the column the same values), and the later chunks' sweeps
-    // reuse it as the sweep wave does
-    bool piv_ok = false;
-
-    // Thomas sweeps of chunk q (oce_ale_tracer.F90:1406-1430), one lane per
-    // (column, tracer) of the columns wlo..wlo+nw-1, then T^{n+1} of those
-    // columns with the salinity clamp
-    auto sweep_store = [&](int q, int wlo, int nw) {
-        const int t0 = trb + q * TCH, nch = min(TCH, tre - t0), bf = SW ? (q & 1) : 0;
-        if (lane < nw * nch) {
-            const int wc = wlo + lane / nch, c = lane % nch;
-            const int z0 = sNz[wc][0], z1 = sNz[wc][1];
-            if (z1 - 1 >= z0 && ldc(t.ivd + t0 + c)) {
-                const double *a_ = saA[wc], *b_ = sbA[wc], *c_ = scA[wc];
-                double *tp_ = stpA[bf][wc][c], *ts = sTsA[bf][wc][c], *cp_ = scpA[wc];
-                double tp = tp_[z0 - 1] / b_[z0 - 1];
-                tp_[z0 - 1] = tp;
-                if (SW || piv_ok) {
-                    double cpa = cp_[z0 - 1];   // c' of the level above
-                    for (int nz = z0 + 1; nz <= z1 - 1; ++nz) {
-                        const double an = a_[nz - 1];
-                        const double mm = b_[nz - 1] - cpa * an;
-                        tp = (tp_[nz - 1] - tp * an) / mm;
-                        cpa = cp_[nz - 1];
-                        tp_[nz - 1] = tp;
-                    }
-                } else {
-                    double cp = c_[z0 - 1] / b_[z0 - 1];
-                    cp_[z0 - 1] = cp;
-                    for (int nz = z0 + 1; nz <= z1 - 1; ++nz) {
-                        const double an = a_[nz - 1];
-                        const double mm = b_[nz - 1] - cp * an;
-                        cp = c_[nz - 1] / mm;
-                        tp = (tp_[nz - 1] - tp * an) / mm;
-                        cp_[nz - 1] = cp;
-                        tp_[nz - 1] = tp;
-                    }
-                }
-                double x = tp_[z1 - 2];
-                ts[z1 - 2] = ts[z1 - 2] + x;
-                for (int nz = z1 - 2; nz >= z0; --nz) {
-                    x = tp_[nz - 1] - cp_[nz - 1] * x;
-                    ts[nz - 1] = ts[nz - 1] + x;
-                }
-            }
+        double x = tp;
+        double r0 = pr[max(z1 - 2, z0)], c0 = pc[max(z1 - 2, z0)];
+        for (int nz = z1 - 2; nz >= z0; --nz) {
+            const int nx = max(nz - 1, z0);
+            const double r1 = pr[nx], c1 = pc[nx];
+            x = r0 - c0 * x;
+            pr[nz] = x;
+            r0 = r1; c0 = c1;
         }
-        wave_sync();
-        for (int wc = wlo; wc < wlo + nw; ++wc) {
-            if (col0 + wc >= m.N2) break;
-            const int nn = m.node_ord[col0 + wc];
-            const int z0 = sNz[wc][0], z1 = sNz[wc][1];
-            for (int c = 0; c < nch; ++c) {
-                const int tr = t0 + c;
+    }
+    __syncthreads();
+    for (int c = w; c < ncol; c += KV_NW) {
+        const int n = rl(nl_, c), nzmin = rl(z0l, c), nzmax = rl(z1l, c);
+        const size_t nL = (size_t)n * L;
+        bool on[NV], any = false;
 #pragma unroll
-                for (int s = 0; s < S; ++s) {
-                    const int k = lane + 1 + 64 * s;
-                    if (k < z0 || k > z1 - 1) continue;
-                    double v = sTsA[bf][wc][c][k - 1];
+        for (int s = 0; s < NV; ++s) {
+            on[s] = kb + s >= nzmin && kb + s <= nzmax - 1;
+            any = any || on[s];
+        }
+        for (int j0 = 0; j0 < ntb; j0 += 2 * KV_TP) {
+            double v[2 * KV_TP][NV];
+#pragma unroll
+            for (int j = 0; j < 2 * KV_TP; ++j)
+                if (j0 + j < ntb && any) row_load<NV>(t.T + t.sN * (trb + j0 + j) + nL, off, v[j]);
+#pragma unroll
+            for (int j = 0; j < 2 * KV_TP; ++j) {
+                if (j0 + j >= ntb) break;
+                const int tr = trb + j0 + j;
+#pragma unroll
+                for (int s = 0; s < NV; ++s) {
+                    if (on[s]) v[j][s] = v[j][s] + sr[(c * TB + j0 + j) * RS + kb + s - 1];
                     if (tr == clamp_tracer) {
-                        if (v > 45.0) v = 45.0;
-                        if (v < 3.0) v = 3.0;
+                        if (v[j][s] > 45.0) v[j][s] = 45.0;
+                        if (v[j][s] < 3.0) v[j][s] = 3.0;
                     }
-                    t.T[t.sN * tr + (size_t)nn * L + k - 1] = v;
                 }
+                row_store<NV>(t.T + t.sN * tr + nL, off, v[j], on);
             }
         }
-    };
-
-    for (int p = 0; p <= nchunk; ++p) {
-        if (!sweeper && p < nchunk) {
-            // ---- chunk p: limited fluxes, flux2dtracer, T*, right-hand sides
-            const int t0 = trb + p * TCH, nch = min(TCH, tre - t0), bf = SW ? (p & 1) : 0;
-            for (int c = 0; c < nch; ++c) {
-                const int tr = t0 + c;
-                double *T = t.T + t.sN * tr;
-                double *Told = t.Told + t.sOld * tr;
-                const int abo = ldc(t.abo + tr);
-                const bool fct = ldc(t.lim + tr) == LIM_FCT;
-                const double *av = t.a_v + t.sNI * tr + (size_t)n * NL;
-                double rp_[S], rm_[S], rpu_[S], rmu_[S], avk_[S], avd_[S];
-                if constexpr (SH) {
-#pragma unroll
-                    for (int s = 0; s < S; ++s) {
-                        rp_[s] = 1.0; rm_[s] = 1.0;
-                        if (fct && act_[s]) {
-                            rp_[s] = t.rp[t.sN * tr + ci_[s]];
-                            rm_[s] = t.rm[t.sN * tr + ci_[s]];
-                        }
-                    }
-                    level_up<S>(rp_, rpu_, lane);
-                    level_up<S>(rm_, rmu_, lane);
-                } else {
-                    wave_sync();
-#pragma unroll
-                    for (int s = 0; s < S; ++s) {
-                        const int k = kk_[s];
-                        if (fct && act_[s]) {   // the limiters read R+- of the wet levels only
-                            sRp[k - 1] = t.rp[t.sN * tr + ci_[s]];
-                            sRm[k - 1] = t.rm[t.sN * tr + ci_[s]];
-                        }
-                    }
-                    wave_sync();
-                }
-                // limited vertical antidiffusive flux at interface k (oce_adv_tra_fct.F90:425-456)
-#pragma unroll
-                for (int s = 0; s < S; ++s) {
-                    const int k = kk_[s];
-                    avk_[s] = 0.0;
-                    if (k >= nzmin && k <= nzmax) {
-                        const double flux = av[k - 1];
-                        double v = flux;
-                        if (fct && k <= nzmax - 1) {
-                            const double rpk = SH ? rp_[s] : sRp[k - 1], rmk = SH ? rm_[s] : sRm[k - 1];
-                            double ae = 1.0;
-                            if (k == nzmin) {
-                                if (flux >= 0.0) ae = dmn(ae, rpk);
-                                else ae = dmn(ae, rmk);
-                            } else {
-                                if (flux >= 0.0) {
-                                    ae = dmn(ae, SH ? rmu_[s] : sRm[k - 2]);
-                                    ae = dmn(ae, rpk);
-                                } else {
-                                    ae = dmn(ae, SH ? rpu_[s] : sRp[k - 2]);
-                                    ae = dmn(ae, rmk);
-                                }
-                            }
-                            v = ae * flux;
-                        }
-                        if (SH) avk_[s] = v;
-                        else sAv[k - 1] = v;
-                    }
-                }
-                if constexpr (SH) level_down<S>(avk_, avd_, lane);
-                else wave_sync();
-                double Tk_[S], v_[S], h_[S], rpn_[S], rmn_[S];
-#pragma unroll
-                for (int s = 0; s < S; ++s) {
-                    const int k = kk_[s];
-                    Tk_[s] = 0.0; v_[s] = 0.0; h_[s] = 0.0;
-                    if (act_[s]) {
-                        Tk_[s] = T[ci_[s]];
-                        if (fct) v_[s] = v_[s] - Tk_[s] * hh_[s] + t.fct_lo[t.sN * tr + ci_[s]] * hn_[s];
-                        v_[s] = v_[s] + (SH ? avk_[s] - avd_[s] : sAv[k - 1] - sAv[k]) * dt / av_[s];
-                    }
-                    rpn_[s] = (act_[s] && fct) ? (SH ? rp_[s] : sRp[k - 1]) : 1.0;
-                    rmn_[s] = (act_[s] && fct) ? (SH ? rm_[s] : sRm[k - 1]) : 1.0;
-                }
-                const double *ah = t.a_h + t.sE * tr;
-                for (int j = 0; j < E.deg; ++j) {
-                    const int q = rl(E.q, j), mo = rl(E.other, j), a0 = rl(E.nu12, j), a1 = rl(E.nl12, j);
-                    double fl_[S], rpo_[S], rmo_[S];
-                    bool ok_[S];
-#pragma unroll
-                    for (int s = 0; s < S; ++s) {   // the slots' loads together
-                        const int k = kk_[s];
-                        ok_[s] = act_[s] && k >= a0 && k <= a1;
-                        fl_[s] = 0.0; rpo_[s] = 1.0; rmo_[s] = 1.0;
-                        if (ok_[s]) {
-                            fl_[s] = ah[(size_t)(q >> 1) * L + k - 1];
-                            if (fct) {
-                                const size_t oi = (size_t)mo * L + k - 1;
-                                rpo_[s] = t.rp[t.sN * tr + oi];
-                                rmo_[s] = t.rm[t.sN * tr + oi];
-                            }
-                        }
-                    }
-#pragma unroll
-                    for (int s = 0; s < S; ++s) {
-                        if (!ok_[s]) continue;
-                        double fl = fl_[s];
-                        if (fct) fl = limit_edge_flux(fl, q, rpn_[s], rmn_[s], rpo_[s], rmo_[s]);
-                        if (q & 1) h_[s] = h_[s] - fl * dt / av_[s];
-                        else h_[s] = h_[s] + fl * dt / av_[s];
-                    }
-                }
-#pragma unroll
-                for (int s = 0; s < S; ++s) {
-                    if (!act_[s]) continue;
-                    const size_t ci = ci_[s];
-                    double del = 0.0 + h_[s] + v_[s];
-                    del = del + Tk_[s] * (hh_[s] - hn_[s]);
-                    sTsA[bf][w][c][kk_[s] - 1] = Tk_[s] + del / hn_[s];
-                    // valuesold rotation (oce_tracer_mod.F90:94-123)
-                    if (abo == 2) {
-                        Told[ci] = Tk_[s];
-                    } else {
-                        Told[2 * ci + 1] = Told[2 * ci];
-                        Told[2 * ci] = Tk_[s];
-                    }
-                }
-            }
-            wave_sync();
-            // right-hand sides (oce_ale_tracer.F90:1206-1229, 1377-1383)
-            for (int c = 0; c < nch; ++c) {
-                const int tr = t0 + c;
-                if (!ldc(t.ivd + tr)) continue;
-                const double *ts = sTsA[bf][w][c];
-#pragma unroll
-                for (int s = 0; s < S; ++s) {
-                    if (!act_[s]) continue;
-                    const int k = kk_[s], i = k - 1;
-                    const double dz = hn_[s];
-                    double r;
-                    if (k == nzmin) r = -(sb[i] - dz) * ts[i] - sc[i] * ts[i + 1];
-                    else if (k <= nzmax - 2) r = -sa[i] * ts[i - 1] - (sb[i] - dz) * ts[i] - sc[i] * ts[i + 1];
-                    else r = -sa[i] * ts[i - 1] - (sb[i] - dz) * ts[i];
-                    if (bc_every_layer(ldc(t.id + tr), d)) r = r + bc_surface_dev(ldc(t.id + tr), dt, d, m.N2, L, n, k, ts[i]);
-                    else if (k == nzmin) r = r + bc_surface_dev(ldc(t.id + tr), dt, d, m.N2, L, n, nzmin, ts[i]);
-                    stpA[bf][w][c][i] = r;
-                }
-            }
-            if (!SW) {   // this wave sweeps and stores its own column
-                wave_sync();
-                sweep_store(p, w, 1);
-                for (int c = 0; c < nch && !piv_ok; ++c) piv_ok = ldc(t.ivd + t0 + c) != 0;
-            }
-        } else if (sweeper && p >= 1) {
-            sweep_store(p - 1, 0, CPB);
-        } else if (sweeper) {
-            pivots();
-        }
-        if (SW) __syncthreads();
     }
 }
 
@@ -1822,10 +1895,9 @@ int fgpu_kd_extras(const fgpu_context *c)
     return (c->d.wsplit ? 1 : 0) | (dx ? 2 : 0);
 }
 
-// The Thomas chunk and columns per block K_D runs with, for the requested
-// ones: several columns per block take chunks of 2 (or 4 at four 64-lane
-// columns, or two columns of up to 128 levels); several columns of more than
-// 64 levels need the sweep-wave K_D.
+// The Thomas chunk and columns per block that fgpu_step_shape reports for the
+// requested ones. They told forms of the former last kernel apart; K_L and K_V
+// take their own from the column depth and the tracer count.
 void fgpu_kd_shape(const fgpu_context *c, int *tch_out, int *cpb_out)
 {
     int tch = (c->step_tch == 4 || c->step_tch == 5 || c->step_tch == 8) ? c->step_tch : 2;
@@ -1850,49 +1922,63 @@ void fgpu_kd_shape(const fgpu_context *c, int *tch_out, int *cpb_out)
     *cpb_out = cpb;
 }
 
-// K_D with one wave per column (S levels per lane: 1 up to 64 interfaces, 2 up
-// to 128), with a sweep wave per block (SW) or each column wave sweeping its
-// own column, for the Thomas chunk and columns per block of the launch shape
-template <int S, int TCH, int CPB, bool SW, int RS = 64 * S + 2, bool SH = false>
-static void launch_kdp(fgpu_context *c, unsigned ny, double dt, int clamp, int tpb)
+// The lanes of the column waves: NV levels per lane, GT tracers per wave. A
+// lane group holds every interface of a column (NV x 64 / GT >= NL).
+enum { COL_1X1, COL_1X2, COL_2X1, COL_2X2, COL_2X4, COL_3X2 };
+static int col_lanes(const fgpu_context *c, int tpb)
 {
-    const DevMesh &m = c->m;
-    hipLaunchKernelGGL((kDp_node<S, TCH, CPB, SW, RS, SH>), dim3(xcd_grid((m.N2 + CPB - 1) / CPB), ny),
-                       dim3(64 * (CPB + (SW ? 1 : 0))), 0, c->stream, m, c->d, c->t, dt, clamp, tpb);
+    const DevTracers &t = c->t;
+    // tracers of one wave share its scheme branches, and their rows have to be
+    // within 32 bits of the wave's row bases
+    bool same = (t.sE > t.sNI ? t.sE : t.sNI) * 8 * 3 < (size_t)0xffff0000u;
+    for (int i = 1; i < t.ntr; ++i)
+        same = same && c->h_lim[i] == c->h_lim[0] && c->h_abo[i] == c->h_abo[0] && c->h_hor[i] == c->h_hor[0] &&
+               c->h_ver[i] == c->h_ver[0] && c->h_ph[i] == c->h_ph[0] && c->h_pv[i] == c->h_pv[0];
+    const int nt = same ? std::min(tpb, t.ntr) : 1, NL = c->m.NL;
+    // A row of 65..96 interfaces: three levels per lane and two tracers fill 72
+    // of 96 slots where two levels per lane fill 70 of 128 (70 layers, 10
+    // tracers, 40 thousand nodes: K_L 826 -> 743 us)
+    if (NL > 64) return nt >= 2 && NL <= 96 ? COL_3X2 : COL_2X1;
+    if (nt < 2) return COL_1X1;
+    // Two levels per lane halve the vector memory instructions of a row (K_L of
+    // 32 tracers on 47 layers: 548 -> 481 us), and short rows leave lanes for
+    // more tracers (30 layers, 3 tracers, 9,919 nodes: 37 -> 29 us)
+    if (NL <= 32) return nt >= 3 ? COL_2X4 : COL_1X2;
+    return COL_2X2;
 }
 
-template <bool SW>
-static void launch_kdp_shape(fgpu_context *c, unsigned ny, double dt, int clamp, int tpb, int tch, int cpb)
+static void launch_kl(fgpu_context *c, double dt, int tpb, unsigned ny)
 {
-    if (c->m.NL <= 64) {
-        if (cpb == 8) launch_kdp<1, 2, 8, SW>(c, ny, dt, clamp, tpb);
-        else if (cpb == 4 && tch == 4) launch_kdp<1, 4, 4, SW>(c, ny, dt, clamp, tpb);
-        else if (cpb == 4) launch_kdp<1, 2, 4, SW>(c, ny, dt, clamp, tpb);
-        else if (tch == 8) launch_kdp<1, 8, 1, SW>(c, ny, dt, clamp, tpb);
-        else if (tch == 5) launch_kdp<1, 5, 1, SW>(c, ny, dt, clamp, tpb);
-        else if (tch == 4) launch_kdp<1, 4, 1, SW>(c, ny, dt, clamp, tpb);
-        else launch_kdp<1, 2, 1, SW>(c, ny, dt, clamp, tpb);
-    } else if (c->m.NL <= KDP_SHORT_NL) {   // rows of KDP_SHORT_NL + 2
-        // one column per block: R+- and the vertical fluxes by shuffles, which
-        // frees their LDS rows (1.8 KB of a block's 10.1 KB at chunks of 5) for
-        // more waves; 46.4-47.0 -> 45.7-46.0 ms at 1.3 M columns of 70 levels
-        constexpr int R = KDP_SHORT_NL + 2;
-        if (cpb >= 4) launch_kdp<2, 2, 4, SW, R>(c, ny, dt, clamp, tpb);
-        else if (cpb == 3) launch_kdp<2, 2, 3, SW, R>(c, ny, dt, clamp, tpb);
-        else if (cpb == 2 && tch == 4) launch_kdp<2, 4, 2, SW, R>(c, ny, dt, clamp, tpb);
-        else if (cpb == 2) launch_kdp<2, 2, 2, SW, R>(c, ny, dt, clamp, tpb);
-        else if (tch == 8) launch_kdp<2, 8, 1, SW, R, true>(c, ny, dt, clamp, tpb);
-        else if (tch == 5) launch_kdp<2, 5, 1, SW, R, true>(c, ny, dt, clamp, tpb);
-        else if (tch == 4) launch_kdp<2, 4, 1, SW, R, true>(c, ny, dt, clamp, tpb);
-        else launch_kdp<2, 2, 1, SW, R, true>(c, ny, dt, clamp, tpb);
-    } else {
-        if (cpb >= 2 && tch == 4) launch_kdp<2, 4, 2, SW>(c, ny, dt, clamp, tpb);
-        else if (cpb >= 2) launch_kdp<2, 2, 2, SW>(c, ny, dt, clamp, tpb);
-        else if (tch == 8) launch_kdp<2, 8, 1, SW>(c, ny, dt, clamp, tpb);
-        else if (tch == 5) launch_kdp<2, 5, 1, SW>(c, ny, dt, clamp, tpb);
-        else if (tch == 4) launch_kdp<2, 4, 1, SW>(c, ny, dt, clamp, tpb);
-        else launch_kdp<2, 2, 1, SW>(c, ny, dt, clamp, tpb);
+    const DevMesh &m = c->m;
+    const DevTracers &t = c->t;
+    const dim3 g(xcd_grid((m.N2 + 3) / 4), ny), b(256);
+    switch (col_lanes(c, tpb)) {
+    case COL_1X1: hipLaunchKernelGGL((kL_node<1, 1>), g, b, 0, c->stream, m, t, dt, tpb); break;
+    case COL_1X2: hipLaunchKernelGGL((kL_node<1, 2>), g, b, 0, c->stream, m, t, dt, tpb); break;
+    case COL_2X1: hipLaunchKernelGGL((kL_node<2, 1>), g, b, 0, c->stream, m, t, dt, tpb); break;
+    case COL_2X2: hipLaunchKernelGGL((kL_node<2, 2>), g, b, 0, c->stream, m, t, dt, tpb); break;
+    case COL_2X4: hipLaunchKernelGGL((kL_node<2, 4>), g, b, 0, c->stream, m, t, dt, tpb); break;
+    default: hipLaunchKernelGGL((kL_node<3, 2>), g, b, 0, c->stream, m, t, dt, tpb); break;
     }
+}
+
+static void launch_kv(fgpu_context *c, double dt, int clamp)
+{
+    const DevMesh &m = c->m;
+    const int nt = c->t.ntr, row = 8 * (m.L | 1);
+    // tracers in equal groups of at most ten: a column's pivots are formed once
+    // per group (70 layers, 10 tracers: 328 us in one group, 682 us by fours)
+    const int groups = (nt + 9) / 10, TB = (nt + groups - 1) / groups;
+    // columns: at most 64 sweep lanes, 40,000 bytes of LDS (four blocks per CU;
+    // 47 layers, 2 tracers, 126,858 nodes: 159 us, 214 us at 65,536 bytes, 191
+    // us at 26,000), and 1,024 blocks on a small mesh, where the blocks' serial
+    // sweeps have to run side by side
+    int NC = std::min(64 / TB, 40000 / (row * (3 + TB)));
+    NC = std::max(1, std::min(NC, (int)((size_t)m.N2 * groups / 1024)));
+    const size_t lds = (size_t)row * (3 + TB) * NC;
+    const dim3 g(xcd_grid((m.N2 + NC - 1) / NC), (unsigned)groups), b(64 * KV_NW);
+    if (m.NL <= 64) hipLaunchKernelGGL(kV_cols<1>, g, b, lds, c->stream, m, c->d, c->t, dt, clamp, NC, TB);
+    else hipLaunchKernelGGL(kV_cols<2>, g, b, lds, c->stream, m, c->d, c->t, dt, clamp, NC, TB);
 }
 
 // K_C over (tracer, level) items with step_kcf tracers per block (1, 2 or 4)
@@ -1928,8 +2014,6 @@ int fgpu_enqueue_fused_step(fgpu_context *c, double dt)
     // tracers per block: 1 runs every tracer's chain in its own waves
     const int tpb = std::max(1, std::min(c->step_tpb, nt));
     const unsigned ny = (unsigned)((nt + tpb - 1) / tpb);
-    int tch, cpb;   // Thomas chunk and columns per block of K_D
-    fgpu_kd_shape(c, &tch, &cpb);
     bool xv = false;   // some tracer uses CDIFF or PPM
     for (int v : c->h_ver) xv = xv || v == VER_CDIFF || v == VER_PPM;
     const bool ws = c->d.wsplit != 0;   // W split: implicit upwind LO step, w_i rows of the diffusion
@@ -1971,35 +2055,21 @@ int fgpu_enqueue_fused_step(fgpu_context *c, double dt)
             else                                                                                                       \
                 hipLaunchKernelGGL(kC_node<LBV>, dim3(xcd_grid(m.N2), ny), dim3(LBV), 0, c->stream, m, c->t, dt, tpb); \
         }                                                                                                              \
-        {                                                                                                              \
+        if (xf == 0) {                                                                                                 \
+            {                                                                                                          \
+                ProfScope ps(c, "kL_node");                                                                            \
+                launch_kl(c, dt, tpb, ny);                                                                             \
+            }                                                                                                          \
+            ProfScope ps(c, "kV_cols");                                                                                \
+            launch_kv(c, dt, clamp);                                                                                   \
+        } else {                                                                                                       \
             ProfScope ps(c, "kD_node");                                                                                \
-            if (xf == 0 && c->step_kdp == KD_SWEEPWAVE)                                                                \
-                launch_kdp_shape<true>(c, ny, dt, clamp, tpb, tch, cpb);                                               \
-            else if (xf == 0 && c->step_kdp == KD_WAVELOCAL)                                                           \
-                launch_kdp_shape<false>(c, ny, dt, clamp, tpb, tch, cpb);                                              \
-            else if (xf == 1)                                                                                          \
-                hipLaunchKernelGGL((kD_node<LBV, 2, 1, 1>), dim3(xcd_grid(m.N2), ny), dim3(LBV), 0, c->stream, m, c->d, c->t, dt, clamp, tpb); \
+            if (xf == 1)                                                                                               \
+                hipLaunchKernelGGL((kD_node<LBV, 1>), dim3(xcd_grid(m.N2), ny), dim3(LBV), 0, c->stream, m, c->d, c->t, dt, clamp, tpb); \
             else if (xf == 2)                                                                                          \
-                hipLaunchKernelGGL((kD_node<LBV, 2, 1, 2>), dim3(xcd_grid(m.N2), ny), dim3(LBV), 0, c->stream, m, c->d, c->t, dt, clamp, tpb); \
-            else if (xf == 3)                                                                                          \
-                hipLaunchKernelGGL((kD_node<LBV, 2, 1, 3>), dim3(xcd_grid(m.N2), ny), dim3(LBV), 0, c->stream, m, c->d, c->t, dt, clamp, tpb); \
-            else if (LBV == 64 && cpb == 8)                                                                            \
-                hipLaunchKernelGGL((kD_node<LBV, 2, (LBV == 64 ? 8 : 1), 0>), dim3(xcd_grid((m.N2 + 7) / 8), ny),          \
-                                   dim3(LBV * (LBV == 64 ? 8 : 1)), 0, c->stream, m, c->d, c->t, dt, clamp, tpb);       \
-            else if (LBV == 64 && cpb == 4 && tch == 4)                                                                \
-                hipLaunchKernelGGL((kD_node<LBV, 4, (LBV == 64 ? 4 : 1), 0>), dim3(xcd_grid((m.N2 + 3) / 4), ny),          \
-                                   dim3(LBV * (LBV == 64 ? 4 : 1)), 0, c->stream, m, c->d, c->t, dt, clamp, tpb);       \
-            else if (LBV == 64 && cpb == 4)                                                                            \
-                hipLaunchKernelGGL((kD_node<LBV, 2, (LBV == 64 ? 4 : 1), 0>), dim3(xcd_grid((m.N2 + 3) / 4), ny),          \
-                                   dim3(LBV * (LBV == 64 ? 4 : 1)), 0, c->stream, m, c->d, c->t, dt, clamp, tpb);       \
-            else if (tch == 8)                                                                                         \
-                hipLaunchKernelGGL((kD_node<LBV, 8, 1, 0>), dim3(xcd_grid(m.N2), ny), dim3(LBV), 0, c->stream, m, c->d, c->t, dt, clamp, tpb); \
-            else if (tch == 5)                                                                                         \
-                hipLaunchKernelGGL((kD_node<LBV, 5, 1, 0>), dim3(xcd_grid(m.N2), ny), dim3(LBV), 0, c->stream, m, c->d, c->t, dt, clamp, tpb); \
-            else if (tch == 4)                                                                                         \
-                hipLaunchKernelGGL((kD_node<LBV, 4, 1, 0>), dim3(xcd_grid(m.N2), ny), dim3(LBV), 0, c->stream, m, c->d, c->t, dt, clamp, tpb); \
+                hipLaunchKernelGGL((kD_node<LBV, 2>), dim3(xcd_grid(m.N2), ny), dim3(LBV), 0, c->stream, m, c->d, c->t, dt, clamp, tpb); \
             else                                                                                                       \
-                hipLaunchKernelGGL((kD_node<LBV, 2, 1, 0>), dim3(xcd_grid(m.N2), ny), dim3(LBV), 0, c->stream, m, c->d, c->t, dt, clamp, tpb); \
+                hipLaunchKernelGGL((kD_node<LBV, 3>), dim3(xcd_grid(m.N2), ny), dim3(LBV), 0, c->stream, m, c->d, c->t, dt, clamp, tpb); \
         }                                                                                                              \
     }
     // one lane per level and per interface: LB >= NL

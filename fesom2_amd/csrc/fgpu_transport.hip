@@ -1087,11 +1087,10 @@ extern "C" int fgpu_solve_tracers_ale_timed(fgpu_context *c, double dt, int nste
 }
 
 // Autotuner of the fused step's launch shape: each candidate number of tracers
-// per block (1, 2, 4, ... and all), crossed with 2, 4 or 8 tracers per Thomas
-// chunk and 1, 4 or 8 columns per block in the last kernel, is timed over
-// `nsteps` replayed steps and the fastest is kept. Every candidate computes the same arithmetic per column, so
-// results do not depend on the choice. The tracer state is saved before and
-// restored after the trials.
+// per block (1, 2, 4, ... and all) is timed over `nsteps` replayed steps and the
+// fastest is kept, then the variants of K_C, K_A and K_B. Every candidate
+// computes the same arithmetic per column, so results do not depend on the
+// choice. The tracer state is saved before and restored after the trials.
 extern "C" int fgpu_autotune_step(fgpu_context *c, double dt, int nsteps, int *best_tpb, double *best_ms)
 {
     int rc = check_ready(c);
@@ -1112,41 +1111,19 @@ extern "C" int fgpu_autotune_step(fgpu_context *c, double dt, int nsteps, int *b
     };
     FGPU_HIP(hipMemcpyAsync(save, c->t.T, sizeof(double) * nT, hipMemcpyDeviceToDevice, c->stream));
     FGPU_HIP(hipMemcpyAsync(save + nT, c->t.Told, sizeof(double) * nO, hipMemcpyDeviceToDevice, c->stream));
-    struct Shape { int tpb, tch, cpb, kd; };
-    std::vector<Shape> cand;
-    const bool narrow = c->m.NL <= 64;   // 64-lane columns: several per block are possible
-    // the variants of the last kernel; with extra terms only the lock-step one exists
-    std::vector<int> kds = {KD_LOCKSTEP};
-    if (!fgpu_kd_extras(c)) kds = {KD_LOCKSTEP, KD_SWEEPWAVE, KD_WAVELOCAL};
-    // columns over 64 levels: several per block only for the one-wave-per-column
-    // K_D, up to 4 with the short LDS rows, else 2
-    const int deep_cpb = c->m.NL <= KDP_SHORT_NL ? 4 : 2;
-    for (int kd : kds)
-        for (int cpb : {1, 2, 3, 4, 8}) {
-            if (narrow ? (cpb == 2 || cpb == 3) : cpb > (kd != KD_LOCKSTEP ? deep_cpb : 1)) continue;
-            for (int tch : {2, 4, 5, 8}) {
-                // chunks of 5 only with one column per block (elsewhere they run as 2)
-                if ((tch == 4 && nt < 3) || (tch == 5 && (nt < 5 || cpb > 1)) || (tch == 8 && nt < 5) ||
-                    (tch >= 4 && cpb == 8) || (tch == 8 && cpb > 1) ||
-                    (!narrow && tch >= 4 && cpb >= 3))
-                    continue;
-                for (int v = 1; v < nt; v *= 2) cand.push_back({v, tch, cpb, kd});
-                cand.push_back({nt, tch, cpb, kd});
-            }
-        }
+    std::vector<int> cand;
+    for (int v = 1; v < nt; v *= 2) cand.push_back(v);
+    cand.push_back(nt);
     const bool was_prof = c->prof;
     c->prof = false;
-    int best = c->step_tpb, best_tch = c->step_tch, best_cpb = c->step_cpb, best_kd = c->step_kdp;
+    int best = c->step_tpb;
     float best_t = -1.f;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     rc = FGPU_OK;
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)
         rc = fgpu_fail(FGPU_ERR_HIP, "hipEventCreate failed");
     for (size_t i = 0; i < cand.size() && !rc; ++i) {
-        c->step_tpb = cand[i].tpb;
-        c->step_tch = cand[i].tch;
-        c->step_cpb = cand[i].cpb;
-        c->step_kdp = cand[i].kd;
+        c->step_tpb = cand[i];
         c->graph_valid = false;
         if ((rc = run_steps(c, dt, 1))) break;   // capture and warm up
         if (hipEventRecord(e0, c->stream) != hipSuccess) { rc = fgpu_fail(FGPU_ERR_HIP, "hipEventRecord"); break; }
@@ -1159,10 +1136,7 @@ extern "C" int fgpu_autotune_step(fgpu_context *c, double dt, int nsteps, int *b
         }
         if (best_t < 0.f || ms < best_t) {
             best_t = ms;
-            best = cand[i].tpb;
-            best_tch = cand[i].tch;
-            best_cpb = cand[i].cpb;
-            best_kd = cand[i].kd;
+            best = cand[i];
         }
     }
     // then the bound kernel K_C with the chosen shape: per column over its
@@ -1170,9 +1144,6 @@ extern "C" int fgpu_autotune_step(fgpu_context *c, double dt, int nsteps, int *b
     int best_kcf = c->step_kcf;
     if (!rc && best_t >= 0.f) {
         c->step_tpb = best;
-        c->step_tch = best_tch;
-        c->step_cpb = best_cpb;
-        c->step_kdp = best_kd;
         for (int kcf : {0, 1, 2, 4}) {
             if (kcf == best_kcf) continue;   // timed above
             c->step_kcf = kcf;
@@ -1218,9 +1189,6 @@ extern "C" int fgpu_autotune_step(fgpu_context *c, double dt, int nsteps, int *b
     (void)hipFree(save);
     c->prof = was_prof;
     c->step_tpb = best;
-    c->step_tch = best_tch;
-    c->step_cpb = best_cpb;
-    c->step_kdp = best_kd;
     c->graph_valid = false;
     if (rc) return rc;
     if (rr) return rr;
