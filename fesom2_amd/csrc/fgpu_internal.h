@@ -58,7 +58,8 @@ struct DevMesh {
     const double *Z3d;                    // N2*L
     const double *zbar_n_bot;             // N2
     const double *zbar_e_bot, *zbar_e_srf;  // F2
-    // packed per-edge records of the fused edge pass (one scalar batch per edge)
+    // packed per-edge records of the fused edge pass (one scalar batch per
+    // edge), in processing order
     const int *erec_i;       // E2*ERI
     const double *erec_d;    // E2*ERD
     const double *zn_vd;     // N2*L: Z levels rebuilt from hnode_new for the implicit diffusion
@@ -67,12 +68,15 @@ struct DevMesh {
     // nodes / edges; results do not depend on it): along a Hilbert curve over
     // the coordinates, so that the columns running at once on one XCD are
     // spatial neighbours and share their neighbour gathers in its L2
+    const int *col_rec;      // 8 per column in processing order: node, offset into col_ne, degree, ulevels_nod2D,
+                             // nlevels_nod2D, 0, 0, 0
+    const int *col_ne;       // ne_rec in processing order of the columns, its first two ints q, other node
     const int *node_ord;     // N2
     const int *edge_ord;     // E2
 };
 // erec_i fields
 enum { ER_N1, ER_N2, ER_EL1, ER_EL2, ER_NL1, ER_NU1, ER_NL2, ER_NU2, ER_UA0, ER_UA1, ER_UA2, ER_DA0, ER_DA1,
-       ER_DA2, ER_RULE, ER_NZMIN, ER_NZMAX, ER_U1, ER_U2, ER_NL1N, ER_NL2N, ER_NBL1, ER_NBL2, ER_I_PAD3, ERI };
+       ER_DA2, ER_RULE, ER_NZMIN, ER_NZMAX, ER_U1, ER_U2, ER_NL1N, ER_NL2N, ER_NBL1, ER_NBL2, ER_E, ERI };
 // erec_d fields
 enum { ER_DX1, ER_DY1, ER_DX2, ER_DY2, ER_A, ER_EDX, ER_EDY, ER_GU0, ER_GU1, ER_GU2, ER_GU3, ER_GU4, ER_GU5,
        ER_GD0, ER_GD1, ER_GD2, ER_GD3, ER_GD4, ER_GD5, ER_D_PAD, ERD };
@@ -125,7 +129,9 @@ struct DevTracers {
     size_t sN, sNI, sE, sF2, sOld, sG;             // strides: N2*L, N2*NL, E2*L, F2*L*2, N2*L*(AB_order-1), N2*L*2
     size_t sStg;              // tracer stride of tr_xy/aux: F2*L*2 with a slot per tracer, 0 with one shared slot
     double *T, *Told;
-    double *lo_h, *a_h;       // E2*L
+    double *a_h;              // E2*L
+    double *vf;               // E2*L, all tracers': volume flux through an edge per level
+    double *lo_h;             // E2*L, per-stage kernels
     double *fct_lo;           // N2*L
     double *a_v;              // N2*NL
     double *rp, *rm;          // N2*L
@@ -165,6 +171,7 @@ struct fgpu_context {
     DevTracers t{};
     int N2 = 0, F2 = 0, E2 = 0, nl = 0, kmax = 0;
     double cyclic_length = 0.0;
+    bool edge_gap = false;             // some edge's elements share no level and leave a gap between their ranges
     std::vector<void *> allocs;        // everything hipMalloc'ed by the context
     std::vector<void *> tracer_allocs; // released on fgpu_tracers_init
     // tracer configuration (host mirror)
@@ -185,6 +192,7 @@ struct fgpu_context {
     int step_tch = 2;         // fgpu_set_step_shape's Thomas chunk and columns per block, reported by
     int step_cpb = 1;         // fgpu_step_shape
     int step_order = 1;       // processing order of the fused step's columns: 1 Hilbert, 0 index (FGPU_STEP_ORDER)
+    bool step_wide = false;   // 64-bit row offsets in the fused step whatever the field size (FGPU_STEP_ROWS=wide)
     int step_kcf = 0;         // K_C over (tracer, level) items with this many tracers per block (1, 2, 4); 0: kC_node
     int step_ka2 = 0;         // 1: K_A with two adjacent levels per lane (kA2_edge), for an even number of layers
     int step_kb2 = 0;         // 1: K_B likewise (kB2_node), without the W split and CDIFF/PPM tracers

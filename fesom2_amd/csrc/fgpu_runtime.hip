@@ -154,6 +154,7 @@ extern "C" int fgpu_create(fgpu_context **out, int device)
     if (const char *tv = std::getenv("FGPU_STEP_TCH")) c->step_tch = std::atoi(tv);
     if (const char *pv = std::getenv("FGPU_STEP_CPB")) c->step_cpb = std::atoi(pv);
     if (const char *ov = std::getenv("FGPU_STEP_ORDER")) c->step_order = std::string(ov) != "index";
+    if (const char *wv = std::getenv("FGPU_STEP_ROWS")) c->step_wide = std::string(wv) == "wide";
     if (const char *fv = std::getenv("FGPU_STEP_KC")) c->step_kcf = std::atoi(fv);
     if (const char *av = std::getenv("FGPU_STEP_KA")) c->step_ka2 = std::atoi(av) == 2;
     if (const char *bv = std::getenv("FGPU_STEP_KB")) c->step_kb2 = std::atoi(bv) == 2;
@@ -202,8 +203,8 @@ int fgpu_ensure_staged(fgpu_context *c, int slots)
     int rc;
     if (!t.TAB) {
         struct A { double **p; size_t n; } arrs[] = {
-            {&t.TAB, t.sN * (size_t)t.ntr}, {&t.dttf_h, t.sN}, {&t.dttf_v, t.sN}, {&t.dbg_av, t.sNI},
-            {&t.dbg_grad, t.sE * 4}};
+            {&t.TAB, t.sN * (size_t)t.ntr}, {&t.lo_h, t.sE * (size_t)t.ntr}, {&t.dttf_h, t.sN}, {&t.dttf_v, t.sN},
+            {&t.dbg_av, t.sNI}, {&t.dbg_grad, t.sE * 4}};
         for (auto &a : arrs) {
             if ((rc = fgpu_alloc(c, (void **)a.p, a.n * sizeof(double), true))) return rc;
             FGPU_HIP(hipMemset(*a.p, 0, a.n * sizeof(double)));
@@ -404,6 +405,7 @@ extern "C" int fgpu_mesh_init(fgpu_context *c, int nod2D, int elem2D, int edge2D
         if (nu2 > 0) nu12 = std::min(nu1, nu2);
         erange[2 * e] = nu12;
         erange[2 * e + 1] = nl12;
+        if (el2 >= 0 && std::min(nl1, nl2) + 1 < std::max(nu1, nu2)) c->edge_gap = true;
         int n1 = ed[2 * e], n2 = ed[2 * e + 1];
         if (nl12 > nlevels_nod2D[n1] - 1 || nl12 > nlevels_nod2D[n2] - 1)
             return fgpu_fail(FGPU_ERR_ARG, "edge deeper than one of its nodes");
@@ -505,6 +507,7 @@ extern "C" int fgpu_mesh_init(fgpu_context *c, int nod2D, int elem2D, int edge2D
         UP(p_i, nrec.data(), nrec.size()); m.node_rec = p_i;
     }
     UP(p_i, kneed.data(), kneed.size()); c->d_kneed = p_i;
+    std::vector<int> eo;   // the edges in processing order
     {
         // processing order of the fused step's column blocks: nodes by the
         // Hilbert index of their coordinates, edges by that of their midpoints
@@ -521,8 +524,26 @@ extern "C" int fgpu_mesh_init(fgpu_context *c, int nod2D, int elem2D, int edge2D
         }
         const bool hil = c->step_order != 0;
         const std::vector<int> no = hil ? hilbert_order(nx, ny) : identity_order(N2);
-        const std::vector<int> eo = hil ? hilbert_order(ex, ey) : identity_order(E2);
+        eo = hil ? hilbert_order(ex, ey) : identity_order(E2);
         UP(p_i, no.data(), no.size()); m.node_ord = p_i;
+        std::vector<int> crec(8 * (size_t)N2, 0), cne;
+        cne.reserve(8 * ne_idx.size());
+        for (int i = 0; i < N2; ++i) {
+            const int n = no[i];
+            int *r = crec.data() + 8 * (size_t)i;
+            r[0] = n;
+            r[1] = (int)(cne.size() / 8);
+            r[2] = ne_ptr[n + 1] - ne_ptr[n];
+            r[3] = ulevels_nod2D[n];
+            r[4] = nlevels_nod2D[n];
+            for (int p = ne_ptr[n]; p < ne_ptr[n + 1]; ++p) {
+                const int q = ne_idx[p], e = q >> 1;
+                cne.insert(cne.end(), {q, ed[2 * e + (1 - (q & 1))], erange[2 * e], erange[2 * e + 1], einfo[4 * e],
+                                       einfo[4 * e + 1], einfo[4 * e + 2], einfo[4 * e + 3]});
+            }
+        }
+        UP(p_i, crec.data(), crec.size()); m.col_rec = p_i;
+        UP(p_i, cne.data(), cne.size()); m.col_ne = p_i;
         UP(p_i, eo.data(), eo.size()); m.edge_ord = p_i;
     }
     // nboundary_lay of MUSCL (muscl_adv_init, oce_muscl_adv.F90:91-157): nl-1,
@@ -563,9 +584,11 @@ extern "C" int fgpu_mesh_init(fgpu_context *c, int nod2D, int elem2D, int edge2D
         // packed edge records (mesh arrays and the fill_up_dn_grad level rule)
         std::vector<int> ri((size_t)E2 * ERI, 0);
         std::vector<double> rd((size_t)E2 * ERD, 0.0);
-        for (int e = 0; e < E2; ++e) {
-            int *r = ri.data() + (size_t)e * ERI;
-            double *q = rd.data() + (size_t)e * ERD;
+        for (int i = 0; i < E2; ++i) {   // in processing order
+            const int e = eo[i];
+            int *r = ri.data() + (size_t)i * ERI;
+            double *q = rd.data() + (size_t)i * ERD;
+            r[ER_E] = e;
             const int n1 = ed[2 * e], n2 = ed[2 * e + 1], el1 = et[2 * e], el2 = et[2 * e + 1];
             r[ER_N1] = n1; r[ER_N2] = n2; r[ER_EL1] = el1; r[ER_EL2] = el2;
             for (int j = 0; j < 4; ++j) r[ER_NL1 + j] = einfo[4 * e + j];
@@ -796,14 +819,14 @@ extern "C" int fgpu_tracers_init(fgpu_context *c, int num_tracers)
     t.sOld = N2 * L;   // AB2; grows to 2*N2*L when a tracer is configured with AB_order 3
     t.sG = N2 * L * 2;
     t.sStg = 0;
-    t.TAB = t.tr_xy = t.aux = t.dttf_h = t.dttf_v = t.dbg_av = t.dbg_grad = nullptr;
+    int rc;
+    t.lo_h = t.TAB = t.tr_xy = t.aux = t.dttf_h = t.dttf_v = t.dbg_av = t.dbg_grad = nullptr;
     t.hd = t.ve = t.vr = nullptr;
     c->stage_slots = 0;
-    int rc;
     // the fused batched step needs only these; the per-stage buffers come with
     // the first per-tracer call (fgpu_ensure_staged)
     struct A { double **p; size_t n; } arrs[] = {
-        {&t.T, t.sN * nt}, {&t.Told, t.sOld * nt}, {&t.lo_h, t.sE * nt}, {&t.a_h, t.sE * nt},
+        {&t.T, t.sN * nt}, {&t.Told, t.sOld * nt}, {&t.a_h, t.sE * nt}, {&t.vf, t.sE},
         {&t.fct_lo, t.sN * nt}, {&t.a_v, t.sNI * nt}, {&t.rp, t.sN * nt}, {&t.rm, t.sN * nt},
         {&t.gmean, t.sG * nt}};
     for (auto &a : arrs) {

@@ -13,14 +13,12 @@
 //   K_D  K_L and K_V in one, for the W split and the explicit diffusion terms
 //
 // K_B..K_L are separated by the three global dependencies of FCT (LO of the
-// neighbours, R+/R- of the neighbours, limited edge fluxes). One block owns one
-// column (an edge or a node) and every tracer; lanes run over levels, so a
-// column's topology and geometry are wave-uniform and its field accesses are
-// contiguous column segments. The node kernels load the metadata of a node's
-// edges (or elements) once, one edge per lane, and hand it to the gather loops
-// with v_readlane, so the per-tracer loops carry no dependent scalar loads.
-// Blocks are mapped to columns XCD by XCD (workgroups are dispatched to the
-// XCDs round-robin), so neighbouring columns share an L2.
+// neighbours, R+/R- of the neighbours, limited edge fluxes). One wave owns one
+// column (an edge or a node) and every tracer of its block; lanes run over
+// levels, so a column's topology and geometry are wave-uniform and its field
+// accesses are contiguous column segments. Blocks are mapped to columns XCD by
+// XCD (workgroups are dispatched to the XCDs round-robin), so neighbouring
+// columns share an L2.
 //
 // Arithmetic is the same sequence of operations as the per-function kernels
 // and the reference (no FMA contraction); edge->node sums run over the node's
@@ -156,9 +154,7 @@ __device__ __forceinline__ NodeEdges load_node_edges(const DevMesh &m, int n)
 // ------------------------------------------------------------------------------
 // One wave per node. The range is a handful of levels at the bottom of most
 // columns, so the lanes take (tracer, level) pairs, as many tracers at a time
-// as fit, instead of one tracer's levels: at 40 thousand nodes, 70 layers and
-// 10 tracers 7 % of the lanes were active, and it took 357 us instead of 71; at
-// 12 thousand nodes, 47 layers and 32 tracers 268 instead of 105.
+// as fit, instead of one tracer's levels.
 __global__ void __launch_bounds__(64) kG_node(DevMesh m, DevTracers t, const int *kneed, int tpb)
 {
     const int jn = xcd_column(m.N2);
@@ -214,311 +210,350 @@ __global__ void __launch_bounds__(64) kG_node(DevMesh m, DevTracers t, const int
 }
 
 // ------------------------------------------------------------------------------
+// Column waves: one wave per node column (or edge), NV adjacent levels per lane
+// and GT tracers per wave, 64 / GT lanes each.
+//
+// These kernels are bound by instruction issue: a SIMD issues one instruction
+// every four cycles whatever its kind, and with 64-bit row addresses formed in
+// scalar registers and branches around masked lanes the scalar instructions
+// outnumbered the vector ones. So the rows' byte offsets are formed once per
+// column in vector registers (the tracers of a block only change the scalar
+// base), loads are not masked (lanes without a wet level read a valid row
+// entry), and the level ranges of the edges are lane masks that select results.
+// One wave per block: with four, a block's slots stay taken until its slowest
+// wave is done (70 layers, 10 tracers: K_L 3 % slower).
+// ------------------------------------------------------------------------------
+// two adjacent levels of a row: 16 bytes at any 8-byte boundary
+typedef double lv2 __attribute__((ext_vector_type(2), aligned(8)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x8 __attribute__((ext_vector_type(8)));
+
+// row values at byte offset off from a wave-uniform base
+template <int NV, typename OFF>
+__device__ __forceinline__ void row_load(const double *p, OFF off, double (&x)[NV])
+{
+    const char *a = (const char *)p + off;
+#pragma unroll
+    for (int s = 0; s + 1 < NV; s += 2) {
+        const lv2 v = *(const lv2 *)(a + 8 * s);
+        x[s] = v.x;
+        x[s + 1] = v.y;
+    }
+    if constexpr (NV % 2 == 1) x[NV - 1] = *(const double *)(a + 8 * (NV - 1));
+}
+
+template <int NV, typename OFF>
+__device__ __forceinline__ void row_store(double *p, OFF off, const double (&x)[NV], const bool (&on)[NV])
+{
+    char *a = (char *)p + off;
+#pragma unroll
+    for (int s = 0; s + 1 < NV; s += 2) {
+        if (on[s] && on[s + 1]) {
+            lv2 v;
+            v.x = x[s];
+            v.y = x[s + 1];
+            *(lv2 *)(a + 8 * s) = v;
+        } else if (on[s]) {
+            *(double *)(a + 8 * s) = x[s];
+        } else if (on[s + 1]) {
+            *(double *)(a + 8 * s + 8) = x[s + 1];
+        }
+    }
+    if constexpr (NV % 2 == 1)
+        if (on[NV - 1]) *(double *)(a + 8 * (NV - 1)) = x[NV - 1];
+}
+
+// value of the next lower / higher lane of the wave (the end lanes keep their own)
+__device__ __forceinline__ double lane_below(double x)
+{
+    const long long b = __double_as_longlong(x);
+    const int lo = (int)(b & 0xffffffffLL), hi = (int)(b >> 32);
+    const int l = __builtin_amdgcn_update_dpp(lo, lo, 0x138, 0xf, 0xf, false);   // wave_shr:1
+    const int h = __builtin_amdgcn_update_dpp(hi, hi, 0x138, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)h << 32) | (unsigned int)l);
+}
+__device__ __forceinline__ double lane_above(double x)
+{
+    const long long b = __double_as_longlong(x);
+    const int lo = (int)(b & 0xffffffffLL), hi = (int)(b >> 32);
+    const int l = __builtin_amdgcn_update_dpp(lo, lo, 0x130, 0xf, 0xf, false);   // wave_shl:1
+    const int h = __builtin_amdgcn_update_dpp(hi, hi, 0x130, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)h << 32) | (unsigned int)l);
+}
+
+// a column's values one level up (k - 1) and one level down (k + 1)
+template <int NV>
+__device__ __forceinline__ void col_up(const double (&x)[NV], double (&y)[NV])
+{
+    y[0] = lane_below(x[NV - 1]);
+#pragma unroll
+    for (int s = 1; s < NV; ++s) y[s] = x[s - 1];
+}
+template <int NV>
+__device__ __forceinline__ void col_down(const double (&x)[NV], double (&y)[NV])
+{
+    y[NV - 1] = lane_above(x[0]);
+#pragma unroll
+    for (int s = 0; s + 1 < NV; ++s) y[s] = x[s + 1];
+}
+
+// a / 3 and a / 6 with the constant's reciprocal in two parts, zh + zl: one
+// rounding of a zh + (a zl). A quotient by 3 (or 6) is never nearer to a
+// rounding boundary than a sixth of its last place and the two-part product is
+// within 2^-104 of it, so this is the correctly rounded quotient wherever a zl
+// does not underflow. The caller sends smaller numerators to the division.
+#define TINY_NUM 1e-280
+__device__ __forceinline__ double third(double a) { return fma(a, 0x1.5555555555555p-2, a * 0x1.5555555555555p-56); }
+__device__ __forceinline__ double sixth(double a) { return fma(a, 0x1.5555555555555p-3, a * 0x1.5555555555555p-57); }
+__device__ __forceinline__ bool tiny(double a) { return fabs(a) < TINY_NUM && a != 0.0; }
+
+// the column of a wave and its edges: byte offsets of the other nodes' rows and
+// of the edge rows, first level and level count - 1 of the edge. Lanes outside
+// an edge's levels, and the missing edges of the last batch, read rows that
+// exist: the column's own and the first edge's.
+#define CE 8   // edges kept in registers; a node's further ones are read in place
+template <typename OFF, int NV, int GT>
+struct Column {
+    int n, deg, p0, nzmin, nzmax;
+    int g, kb, kc;       // tracer of the wave, first level of the lane, the same within the row
+    bool wet[NV];
+    OFF own, ownI;       // offsets of the lane in layer and interface rows of one tracer's field
+    OFF on[CE], oe[CE];
+    int a0[CE], len[CE], side[CE];
+};
+
+// x, or -x on the edge's second node (sgn: bit 63)
+__device__ __forceinline__ double signed_by(double x, long long sgn)
+{
+    return __longlong_as_double(__double_as_longlong(x) ^ sgn);
+}
+
+// level kb + s is one of the edge's levels
+__device__ __forceinline__ bool edge_has(int kb, int s, int a0, int len) { return (unsigned)(kb + s - a0) <= (unsigned)len; }
+
+template <typename OFF, int NV, int GT>
+__device__ __forceinline__ void edge_offsets(const DevMesh &m, const DevTracers &t, const Column<OFF, NV, GT> &c, int u,
+                                             OFF &on, OFF &oe, int &a0, int &len, int &side)
+{
+    const i32x8 r = ldc((const i32x8 *)m.col_ne + c.p0 + u);
+    const OFF lev = 8 * (OFF)(c.kc - 1);
+    side = r[0] & 1;
+    a0 = r[2];
+    len = r[3] - r[2];
+    bool some = false;
+#pragma unroll
+    for (int s = 0; s < NV; ++s) some = some || edge_has(c.kb, s, a0, len);
+    on = some ? lev + 8 * (OFF)c.g * (OFF)t.sN + 8 * (OFF)r[1] * (OFF)m.L : c.own;
+    oe = lev + 8 * (OFF)c.g * (OFF)t.sE + 8 * (OFF)(r[0] >> 1) * (OFF)m.L;
+}
+
+template <bool LANES_OFF, typename OFF, int NV, int GT>
+__device__ __forceinline__ bool load_column(const DevMesh &m, const DevTracers &t, Column<OFF, NV, GT> &c)
+{
+    const int lane = threadIdx.x;
+    const int jc = xcd_column(m.N2);
+    if (jc >= m.N2) return false;
+    const i32x8 r = ldc((const i32x8 *)m.col_rec + jc);
+    c.n = r[0];
+    c.p0 = r[1];
+    c.deg = r[2];
+    c.nzmin = r[3];
+    c.nzmax = r[4];
+    constexpr int LP = 64 / GT;
+    c.g = lane / LP;
+    c.kb = (lane % LP) * NV + 1;
+    // LANES_OFF: the lanes without a level or interface of the column are off
+    // throughout; a lane exchange only leaves the column's ends to them, which
+    // have rules of their own
+    if (LANES_OFF && (c.kb > c.nzmax || c.kb + NV - 1 < c.nzmin)) return false;
+    c.kc = c.kb <= m.L ? c.kb : 1;
+#pragma unroll
+    for (int s = 0; s < NV; ++s) c.wet[s] = c.kb + s >= c.nzmin && c.kb + s <= c.nzmax - 1;
+    c.own = 8 * ((OFF)(c.kc - 1) + (OFF)c.g * (OFF)t.sN + (OFF)c.n * (OFF)m.L);
+    c.ownI = 8 * ((OFF)((LANES_OFF || c.kb <= m.NL ? c.kb : 1) - 1) + (OFF)c.g * (OFF)t.sNI + (OFF)c.n * (OFF)m.NL);
+#pragma unroll
+    for (int u = 0; u < CE; ++u) {
+        c.on[u] = c.own;
+        c.oe[u] = c.oe[0];
+        c.a0[u] = 0x40000000;
+        c.len[u] = 0;
+        c.side[u] = 0;
+        if (u < c.deg) edge_offsets<OFF, NV, GT>(m, t, c, u, c.on[u], c.oe[u], c.a0[u], c.len[u], c.side[u]);
+    }
+    return true;
+}
+
+// ------------------------------------------------------------------------------
 // K_A: edge pass
 // ------------------------------------------------------------------------------
-template <int LB>
-__global__ void __launch_bounds__(LB) __attribute__((amdgpu_waves_per_eu(6, 8))) kA_edge(DevMesh m, DevDyn d, DevTracers t, int tpb)
+// Per tracer it gathers T and the old level at the edge's nodes and T at the
+// nodes of the upwind and downwind triangles. Bound by the vector memory
+// pipeline (ten row loads and a store per tracer) and the latency of a wave's
+// dependent loads. The volume fluxes are stored once for all tracers instead of
+// a LO flux per tracer. 126,858 nodes, 47 layers, 2 tracers: 544 -> 473 us; 12
+// thousand nodes, 32 tracers: 689 -> 430; 40 thousand nodes, 70 layers, 10
+// tracers: 1067 -> 730.
+template <typename OFF, int NV, int GT>
+__global__ void __launch_bounds__(64) kA_edge(DevMesh m, DevDyn d, DevTracers t, int tpb)
 {
+    const int lane = threadIdx.x;
     const int je = xcd_column(m.E2);
     if (je >= m.E2) return;
-    const int e = ldc(m.edge_ord + je);
-    const int k = threadIdx.x + 1;
+    constexpr int LP = 64 / GT;
+    const int g = lane / LP, kb = (lane % LP) * NV + 1;
     const int L = m.L;
-    const int *ri = m.erec_i + (size_t)e * ERI;
-    const double *rd = m.erec_d + (size_t)e * ERD;
+    const int *ri = m.erec_i + (size_t)je * ERI;
+    const double *rd = m.erec_d + (size_t)je * ERD;
     const int nl1 = ldc(ri + ER_NL1), nu1 = ldc(ri + ER_NU1), nl2 = ldc(ri + ER_NL2), nu2 = ldc(ri + ER_NU2);
-    const int nl12 = min(nl1, nl2), nu12 = max(nu1, nu2);
-    bool in[5];
-    in[0] = (k >= nu1 && k <= nu12 - 1);
-    in[1] = (nu2 > 0 && k >= nu2 && k <= nu12 - 1);
-    in[2] = (k >= nu12 && k <= nl12);
-    in[3] = (k >= nl12 + 1 && k <= nl1);
-    in[4] = (k >= nl12 + 1 && k <= nl2);
-    if (!(in[0] || in[1] || in[2] || in[3] || in[4])) return;
-    const int n1 = ldc(ri + ER_N1), n2 = ldc(ri + ER_N2), el1 = ldc(ri + ER_EL1), el2 = ldc(ri + ER_EL2);
-    const double dX1 = ldc(rd + ER_DX1), dY1 = ldc(rd + ER_DY1), dX2 = ldc(rd + ER_DX2), dY2 = ldc(rd + ER_DY2);
-    const double a = ldc(rd + ER_A), edx = ldc(rd + ER_EDX), edy = ldc(rd + ER_EDY);
-    const size_t q1 = (size_t)el1 * L + k - 1;
-    const double u1 = d.uv[2 * q1], v1 = d.uv[2 * q1 + 1], h1 = m.helem[q1];
-    double u2 = 0.0, v2 = 0.0, h2 = 0.0;
-    if (el2 >= 0 && (in[1] || in[2] || in[4])) {
-        const size_t q2 = (size_t)el2 * L + k - 1;
-        u2 = d.uv[2 * q2];
-        v2 = d.uv[2 * q2 + 1];
-        h2 = m.helem[q2];
-    }
-    // at most two segments meet at one level, in this order: A then B, or C, or
-    // D then E (A..E as in oce_adv_tra_hor.F90:166-249)
-    const int s1 = in[0] ? 0 : (in[2] ? 2 : (in[3] ? 3 : -1));
-    const int s2 = in[1] ? 1 : (in[4] ? 4 : -1);
-    const double vf1 = s1 >= 0 ? seg_vflux(s1, u1, v1, u2, v2, h1, h2, dX1, dY1, dX2, dY2) : 0.0;
-    const double vf2 = s2 >= 0 ? seg_vflux(s2, u1, v1, u2, v2, h1, h2, dX1, dY1, dX2, dY2) : 0.0;
-    // gradient rule of fill_up_dn_grad at this level (oce_muscl_adv.F90:375-520);
-    // writes in the reference's order, a later write wins
-    bool shared = false, mean1 = false, mean2 = false;
-    const int u1l = ldc(ri + ER_U1), u2l = ldc(ri + ER_U2), nl1n = ldc(ri + ER_NL1N), nl2n = ldc(ri + ER_NL2N);
-    if (ldc(ri + ER_RULE)) {
-        const int nzmin = ldc(ri + ER_NZMIN), nzmax = ldc(ri + ER_NZMAX);
-        mean1 = (k >= u1l && k <= nzmin - 1);
-        mean2 = (k >= u2l && k <= nzmin - 1);
-        if (k >= nzmin && k <= nzmax - 1) { shared = true; mean1 = false; mean2 = false; }
-        if (k >= nzmax && k <= nl1n - 1) { mean1 = true; shared = false; }
-        if (k >= nzmax && k <= nl2n - 1) { mean2 = true; shared = false; }
-    } else {
-        mean1 = (k >= u1l && k <= nl1n - 1);
-        mean2 = (k >= u2l && k <= nl2n - 1);
-    }
-    const int ua0 = ldc(ri + ER_UA0), ua1 = ldc(ri + ER_UA1), ua2 = ldc(ri + ER_UA2);
-    const int da0 = ldc(ri + ER_DA0), da1 = ldc(ri + ER_DA1), da2 = ldc(ri + ER_DA2);
-    const size_t o1 = (size_t)n1 * L + k - 1, o2 = (size_t)n2 * L + k - 1;
-    const size_t ei = (size_t)e * L + k - 1;
-    const size_t kk = (size_t)k - 1;
-    const int trb = blockIdx.y * tpb, tre = min(t.ntr, trb + tpb);
-    for (int tr = trb; tr < tre; ++tr) {
-        const double *T = t.T + t.sN * tr;
-        const double *Told = t.Told + t.sOld * tr;
-        const int abo = ldc(t.abo + tr), lim = ldc(t.lim + tr), hor = ldc(t.hor + tr);
-        double flo = 0.0;
-        const double T1 = T[o1], T2 = T[o2];
-        if (lim == LIM_FCT) {
-            if (s1 >= 0) flo = upw1_h(T1, T2, vf1, flo);
-            if (s2 >= 0) flo = upw1_h(T1, T2, vf2, flo);
-            t.lo_h[t.sE * tr + ei] = flo;
-        }
-        double A1, A2;
-        if (abo == 2) {
-            A1 = -(0.5 + FGPU_EPS_AB) * Told[o1] + (1.5 + FGPU_EPS_AB) * T1;
-            A2 = -(0.5 + FGPU_EPS_AB) * Told[o2] + (1.5 + FGPU_EPS_AB) * T2;
-        } else {
-            A1 = t_ab(abo, T, Told, o1);
-            A2 = t_ab(abo, T, Told, o2);
-        }
-        double f = flo;
-        if (hor != HOR_UPW1) {   // MFCT, MUSCL
-            const double no = ldc(t.ph + tr);
-            double g[4] = {0.0, 0.0, 0.0, 0.0};
-            if (shared) {
-                const double u0 = T[(size_t)ua0 * L + kk], u1_ = T[(size_t)ua1 * L + kk], u2_ = T[(size_t)ua2 * L + kk];
-                const double w0 = T[(size_t)da0 * L + kk], w1 = T[(size_t)da1 * L + kk], w2 = T[(size_t)da2 * L + kk];
-                g[0] = ldc(rd + ER_GU0) * u0 + ldc(rd + ER_GU1) * u1_ + ldc(rd + ER_GU2) * u2_;
-                g[2] = ldc(rd + ER_GU3) * u0 + ldc(rd + ER_GU4) * u1_ + ldc(rd + ER_GU5) * u2_;
-                g[1] = ldc(rd + ER_GD0) * w0 + ldc(rd + ER_GD1) * w1 + ldc(rd + ER_GD2) * w2;
-                g[3] = ldc(rd + ER_GD3) * w0 + ldc(rd + ER_GD4) * w1 + ldc(rd + ER_GD5) * w2;
-            } else {
-                const double *gm = t.gmean + t.sG * tr;
-                if (mean1) { g[0] = gm[2 * o1]; g[2] = gm[2 * o1 + 1]; }
-                if (mean2) { g[1] = gm[2 * o2]; g[3] = gm[2 * o2 + 1]; }
-            }
-            double Tmean2, Tmean1;
-            if (hor == HOR_MUSCL) {   // reconstruction only down to nboundary_lay (oce_adv_tra_hor.F90:356-367)
-                const double c1 = k <= ldc(ri + ER_NBL1) ? 1.0 : 0.0, c2 = k <= ldc(ri + ER_NBL2) ? 1.0 : 0.0;
-                Tmean2 = A2 - (2.0 * (A2 - A1) + edx * a * g[1] + edy * FGPU_R_EARTH * g[3]) / 6.0 * c2;
-                Tmean1 = A1 + (2.0 * (A2 - A1) + edx * a * g[0] + edy * FGPU_R_EARTH * g[2]) / 6.0 * c1;
-            } else {
-                Tmean2 = A2 - (2.0 * (A2 - A1) + edx * a * g[1] + edy * FGPU_R_EARTH * g[3]) / 6.0;
-                Tmean1 = A1 + (2.0 * (A2 - A1) + edx * a * g[0] + edy * FGPU_R_EARTH * g[2]) / 6.0;
-            }
-            for (int sg = 0; sg < 2; ++sg) {
-                if ((sg == 0 ? s1 : s2) < 0) continue;
-                const double vflux = sg == 0 ? vf1 : vf2;
-                const double cHO = (vflux + fabs(vflux)) * Tmean1 + (vflux - fabs(vflux)) * Tmean2;
-                f = -0.5 * (1.0 - no) * cHO - vflux * no * 0.5 * (Tmean1 + Tmean2) - f;
-            }
-        } else {
-            if (s1 >= 0) f = upw1_h(A1, A2, vf1, f);
-            if (s2 >= 0) f = upw1_h(A1, A2, vf2, f);
-        }
-        t.a_h[t.sE * tr + ei] = f;
-    }
-}
-
-__device__ __forceinline__ double2 ld2(const double *p) { return *(const double2 *)p; }
-
-// store levels k (x) and k + 1 (y) of a row, those with their flag set: both
-// with one 16-byte store, one of them with an 8-byte store
-__device__ __forceinline__ void st2(double *p, double x, double y, bool a0, bool a1)
-{
-    if (a0 && a1) {
-        *(double2 *)p = make_double2(x, y);
-    } else if (a0) {
-        p[0] = x;
-    } else if (a1) {
-        p[1] = y;
-    }
-}
-
-// ------------------------------------------------------------------------------
-// K_A with two adjacent levels per lane: lane j takes levels 2j+1 and 2j+2, so
-// one wave covers an edge of up to 128 levels, and each per-level row is read
-// and written with 16-byte accesses (an even number of layers keeps every row
-// 16-byte aligned). A 16-byte load per lane costs the vector memory pipeline
-// what an 8-byte one does, so this halves its work against kA_edge<128>. Each
-// level's arithmetic is kA_edge's, in the same order.
-// ------------------------------------------------------------------------------
-__global__ void __launch_bounds__(64) kA2_edge(DevMesh m, DevDyn d, DevTracers t, int tpb)
-{
-    const int je = xcd_column(m.E2);
-    if (je >= m.E2) return;
-    const int e = ldc(m.edge_ord + je);
-    const int kb = 2 * (int)threadIdx.x + 1;   // this lane's levels: kb, kb + 1
-    const int L = m.L;
-    const int *ri = m.erec_i + (size_t)e * ERI;
-    const double *rd = m.erec_d + (size_t)e * ERD;
-    const int nl1 = ldc(ri + ER_NL1), nu1 = ldc(ri + ER_NU1), nl2 = ldc(ri + ER_NL2), nu2 = ldc(ri + ER_NU2);
-    const int nl12 = min(nl1, nl2), nu12 = max(nu1, nu2);
-    bool act[2], need2[2];
-    int s1[2], s2[2];
+    if (kb + NV - 1 < min(nu1, nu2 > 0 ? nu2 : nu1) || kb > max(nl1, nl2)) return;
+    const int e = ldc(ri + ER_E), el1 = ldc(ri + ER_EL1), el2 = ldc(ri + ER_EL2);
+    const OFF lev = 8 * (OFF)(kb - 1);
+    const OFF gN = lev + 8 * (OFF)g * (OFF)t.sN, gO = lev + 8 * (OFF)g * (OFF)t.sOld;
+    // byte offsets of the rows of the edge's nodes and of its upwind and downwind triangle's nodes
+    const OFF o1 = 8 * (OFF)ldc(ri + ER_N1) * (OFF)L, o2 = 8 * (OFF)ldc(ri + ER_N2) * (OFF)L;
+    OFF ou[3], ow[3];
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        const int k = kb + s;
-        const bool i0 = (k >= nu1 && k <= nu12 - 1);
-        const bool i1 = (nu2 > 0 && k >= nu2 && k <= nu12 - 1);
-        const bool i2 = (k >= nu12 && k <= nl12);
-        const bool i3 = (k >= nl12 + 1 && k <= nl1);
-        const bool i4 = (k >= nl12 + 1 && k <= nl2);
-        act[s] = i0 || i1 || i2 || i3 || i4;
-        need2[s] = i1 || i2 || i4;
-        // at most two segments meet at one level: A then B, or C, or D then E
-        s1[s] = i0 ? 0 : (i2 ? 2 : (i3 ? 3 : -1));
-        s2[s] = i1 ? 1 : (i4 ? 4 : -1);
+    for (int j = 0; j < 3; ++j) {
+        ou[j] = gN + 8 * (OFF)ldc(ri + ER_UA0 + j) * (OFF)L;
+        ow[j] = gN + 8 * (OFF)ldc(ri + ER_DA0 + j) * (OFF)L;
     }
-    if (!act[0] && !act[1]) return;
-    const int n1 = ldc(ri + ER_N1), n2 = ldc(ri + ER_N2), el1 = ldc(ri + ER_EL1), el2 = ldc(ri + ER_EL2);
-    const double dX1 = ldc(rd + ER_DX1), dY1 = ldc(rd + ER_DY1), dX2 = ldc(rd + ER_DX2), dY2 = ldc(rd + ER_DY2);
-    const double a = ldc(rd + ER_A), edx = ldc(rd + ER_EDX), edy = ldc(rd + ER_EDY);
-    double vf1[2], vf2[2];
+    // volume flux per level: the elements with that level add up
+    double vf[NV];
+    bool act[NV], mean[NV], any_mean = false;
     {
-        const size_t q1 = (size_t)el1 * L + kb - 1;
-        const double2 uva = ld2(d.uv + 2 * q1), uvb = ld2(d.uv + 2 * q1 + 2), hh1 = ld2(m.helem + q1);
-        const double u1[2] = {uva.x, uvb.x}, v1[2] = {uva.y, uvb.y}, h1[2] = {hh1.x, hh1.y};
-        double u2[2] = {0.0, 0.0}, v2[2] = {0.0, 0.0}, h2[2] = {0.0, 0.0};
-        if (el2 >= 0 && ((act[0] && need2[0]) || (act[1] && need2[1]))) {
-            const size_t q2 = (size_t)el2 * L + kb - 1;
-            const double2 wa = ld2(d.uv + 2 * q2), wb = ld2(d.uv + 2 * q2 + 2), hh2 = ld2(m.helem + q2);
-            if (need2[0]) { u2[0] = wa.x; v2[0] = wa.y; h2[0] = hh2.x; }
-            if (need2[1]) { u2[1] = wb.x; v2[1] = wb.y; h2[1] = hh2.y; }
-        }
+        const double dX1 = ldc(rd + ER_DX1), dY1 = ldc(rd + ER_DY1), dX2 = ldc(rd + ER_DX2), dY2 = ldc(rd + ER_DY2);
+        double uv1[2 * NV], h1[NV], uv2[2 * NV], h2[NV];
+        const size_t q1 = (size_t)el1 * L, q2 = (size_t)(el2 >= 0 ? el2 : el1) * L;
+        row_load<2 * NV>(d.uv + 2 * q1, 16u * (unsigned)(kb - 1), uv1);
+        row_load<NV>(m.helem + q1, 8u * (unsigned)(kb - 1), h1);
+        row_load<2 * NV>(d.uv + 2 * q2, 16u * (unsigned)(kb - 1), uv2);
+        row_load<NV>(m.helem + q2, 8u * (unsigned)(kb - 1), h2);
+        const int s0 = ldc(ri + ER_NZMIN), s1 = ldc(ri + ER_NZMAX);
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            vf1[s] = s1[s] >= 0 ? seg_vflux(s1[s], u1[s], v1[s], u2[s], v2[s], h1[s], h2[s], dX1, dY1, dX2, dY2) : 0.0;
-            vf2[s] = s2[s] >= 0 ? seg_vflux(s2[s], u1[s], v1[s], u2[s], v2[s], h1[s], h2[s], dX1, dY1, dX2, dY2) : 0.0;
+        for (int s = 0; s < NV; ++s) {
+            const int k = kb + s;
+            const bool in1 = k >= nu1 && k <= nl1, in2 = nu2 > 0 && k >= nu2 && k <= nl2;
+            const double f1 = (-uv1[2 * s + 1] * dX1 + uv1[2 * s] * dY1) * h1[s];
+            const double f2 = (uv2[2 * s + 1] * dX2 - uv2[2 * s] * dY2) * h2[s];
+            vf[s] = in1 ? (in2 ? f1 + f2 : f1) : f2;
+            act[s] = in1 || in2;
+            // fill_up_dn_grad (oce_muscl_adv.F90:375-520): the triangles' gradients at the levels their
+            // nodes share (an empty range without both triangles), else the node means
+            mean[s] = act[s] && !(k >= s0 && k <= s1 - 1);
+            any_mean = any_mean || mean[s];
         }
     }
-    // gradient rule of fill_up_dn_grad per level (oce_muscl_adv.F90:375-520)
-    bool shared[2], mean1[2], mean2[2];
-    const int u1l = ldc(ri + ER_U1), u2l = ldc(ri + ER_U2), nl1n = ldc(ri + ER_NL1N), nl2n = ldc(ri + ER_NL2N);
+    double vp[NV], vm[NV];
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        const int k = kb + s;
-        shared[s] = false;
-        if (ldc(ri + ER_RULE)) {
-            const int nzmin = ldc(ri + ER_NZMIN), nzmax = ldc(ri + ER_NZMAX);
-            mean1[s] = (k >= u1l && k <= nzmin - 1);
-            mean2[s] = (k >= u2l && k <= nzmin - 1);
-            if (k >= nzmin && k <= nzmax - 1) { shared[s] = true; mean1[s] = false; mean2[s] = false; }
-            if (k >= nzmax && k <= nl1n - 1) { mean1[s] = true; shared[s] = false; }
-            if (k >= nzmax && k <= nl2n - 1) { mean2[s] = true; shared[s] = false; }
-        } else {
-            mean1[s] = (k >= u1l && k <= nl1n - 1);
-            mean2[s] = (k >= u2l && k <= nl2n - 1);
-        }
+    for (int s = 0; s < NV; ++s) {
+        vp[s] = vf[s] + fabs(vf[s]);
+        vm[s] = vf[s] - fabs(vf[s]);
     }
-    const bool any_sh = (act[0] && shared[0]) || (act[1] && shared[1]);
-    const bool any_m1 = (act[0] && !shared[0] && mean1[0]) || (act[1] && !shared[1] && mean1[1]);
-    const bool any_m2 = (act[0] && !shared[0] && mean2[0]) || (act[1] && !shared[1] && mean2[1]);
-    const int ua0 = ldc(ri + ER_UA0), ua1 = ldc(ri + ER_UA1), ua2 = ldc(ri + ER_UA2);
-    const int da0 = ldc(ri + ER_DA0), da1 = ldc(ri + ER_DA1), da2 = ldc(ri + ER_DA2);
-    const size_t o1 = (size_t)n1 * L + kb - 1, o2 = (size_t)n2 * L + kb - 1;
-    const size_t ei = (size_t)e * L + kb - 1;
-    const size_t kk = (size_t)kb - 1;
+    const double edxa = ldc(rd + ER_EDX) * ldc(rd + ER_A), edyr = ldc(rd + ER_EDY) * FGPU_R_EARTH;
+    const OFF oE = lev + 8 * (OFF)g * (OFF)t.sE;
     const int trb = blockIdx.y * tpb, tre = min(t.ntr, trb + tpb);
-    for (int tr = trb; tr < tre; ++tr) {
-        const double *T = t.T + t.sN * tr;
-        const double *Told = t.Told + t.sOld * tr;
-        const int abo = ldc(t.abo + tr), lim = ldc(t.lim + tr), hor = ldc(t.hor + tr);
-        const double2 t1 = ld2(T + o1), t2 = ld2(T + o2);
-        const double T1[2] = {t1.x, t1.y}, T2[2] = {t2.x, t2.y};
-        double flo[2] = {0.0, 0.0};
+    if (trb == 0 && g == 0) row_store<NV>(t.vf + (size_t)e * L, lev, vf, act);   // K_B forms the LO fluxes again from it
+    for (int tb = trb; tb < tre; tb += GT) {
+        if (GT > 1 && tb + g >= tre) return;   // the last group's missing tracers
+        const double *T = t.T + t.sN * tb, *Told = t.Told + t.sOld * tb;
+        const int abo = ldc(t.abo + tb), lim = ldc(t.lim + tb), hor = ldc(t.hor + tb);
+        double T1[NV], T2[NV], A1[NV], A2[NV], ux[3][NV], wx[3][NV];
+        row_load<NV>(T, gN + o1, T1);
+        row_load<NV>(T, gN + o2, T2);
+        if (abo == 2) {
+            row_load<NV>(Told, gO + o1, A1);
+            row_load<NV>(Told, gO + o2, A2);
+        }
+        if (hor != HOR_UPW1) {
+#pragma unroll
+            for (int j = 0; j < 3; ++j) row_load<NV>(T, ou[j], ux[j]);
+#pragma unroll
+            for (int j = 0; j < 3; ++j) row_load<NV>(T, ow[j], wx[j]);
+        }
+        if (abo == 2) {   // T^AB (oce_tracer_mod.F90:44-59)
+#pragma unroll
+            for (int s = 0; s < NV; ++s) {
+                A1[s] = -(0.5 + FGPU_EPS_AB) * A1[s] + (1.5 + FGPU_EPS_AB) * T1[s];
+                A2[s] = -(0.5 + FGPU_EPS_AB) * A2[s] + (1.5 + FGPU_EPS_AB) * T2[s];
+            }
+        } else {
+            double q1[2 * NV], q2[2 * NV];
+            row_load<2 * NV>(Told, lev + gO + 2 * o1, q1);
+            row_load<2 * NV>(Told, lev + gO + 2 * o2, q2);
+#pragma unroll
+            for (int s = 0; s < NV; ++s) {
+                A1[s] = (5.0 * q1[2 * s + 1] - 16.0 * q1[2 * s] + 23.0 * T1[s]) / 12.0;
+                A2[s] = (5.0 * q2[2 * s + 1] - 16.0 * q2[2 * s] + 23.0 * T2[s]) / 12.0;
+            }
+        }
+        double f[NV];
         if (lim == LIM_FCT) {
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                if (s1[s] >= 0) flo[s] = upw1_h(T1[s], T2[s], vf1[s], flo[s]);
-                if (s2[s] >= 0) flo[s] = upw1_h(T1[s], T2[s], vf2[s], flo[s]);
-            }
-            st2(t.lo_h + t.sE * tr + ei, flo[0], flo[1], act[0], act[1]);
-        }
-        double A1[2], A2[2];   // T^AB (oce_tracer_mod.F90:44-59)
-        if (abo == 2) {
-            const double2 p1 = ld2(Told + o1), p2 = ld2(Told + o2);
-            const double O1[2] = {p1.x, p1.y}, O2[2] = {p2.x, p2.y};
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                A1[s] = -(0.5 + FGPU_EPS_AB) * O1[s] + (1.5 + FGPU_EPS_AB) * T1[s];
-                A2[s] = -(0.5 + FGPU_EPS_AB) * O2[s] + (1.5 + FGPU_EPS_AB) * T2[s];
-            }
+            for (int s = 0; s < NV; ++s) f[s] = -0.5 * (T1[s] * vp[s] + T2[s] * vm[s]) - 0.0;
         } else {
-            const double2 p1a = ld2(Told + 2 * o1), p1b = ld2(Told + 2 * o1 + 2);
-            const double2 p2a = ld2(Told + 2 * o2), p2b = ld2(Told + 2 * o2 + 2);
-            A1[0] = (5.0 * p1a.y - 16.0 * p1a.x + 23.0 * T1[0]) / 12.0;
-            A1[1] = (5.0 * p1b.y - 16.0 * p1b.x + 23.0 * T1[1]) / 12.0;
-            A2[0] = (5.0 * p2a.y - 16.0 * p2a.x + 23.0 * T2[0]) / 12.0;
-            A2[1] = (5.0 * p2b.y - 16.0 * p2b.x + 23.0 * T2[1]) / 12.0;
+#pragma unroll
+            for (int s = 0; s < NV; ++s) f[s] = 0.0;
         }
-        double f[2] = {flo[0], flo[1]};
         if (hor != HOR_UPW1) {   // MFCT, MUSCL
-            const double no = ldc(t.ph + tr);
-            double2 ux0, ux1, ux2, wx0, wx1, wx2;
-            if (any_sh) {
-                ux0 = ld2(T + (size_t)ua0 * L + kk);
-                ux1 = ld2(T + (size_t)ua1 * L + kk);
-                ux2 = ld2(T + (size_t)ua2 * L + kk);
-                wx0 = ld2(T + (size_t)da0 * L + kk);
-                wx1 = ld2(T + (size_t)da1 * L + kk);
-                wx2 = ld2(T + (size_t)da2 * L + kk);
-            }
-            const double *gm = t.gmean + t.sG * tr;
-            double2 m1a, m1b, m2a, m2b;
-            if (any_m1) { m1a = ld2(gm + 2 * o1); m1b = ld2(gm + 2 * o1 + 2); }
-            if (any_m2) { m2a = ld2(gm + 2 * o2); m2b = ld2(gm + 2 * o2 + 2); }
+            const double no = ldc(t.ph + tb);
+            double gr[4][NV];
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                double g[4] = {0.0, 0.0, 0.0, 0.0};
-                if (shared[s]) {
-                    const double u0 = s ? ux0.y : ux0.x, u1_ = s ? ux1.y : ux1.x, u2_ = s ? ux2.y : ux2.x;
-                    const double w0 = s ? wx0.y : wx0.x, w1 = s ? wx1.y : wx1.x, w2 = s ? wx2.y : wx2.x;
-                    g[0] = ldc(rd + ER_GU0) * u0 + ldc(rd + ER_GU1) * u1_ + ldc(rd + ER_GU2) * u2_;
-                    g[2] = ldc(rd + ER_GU3) * u0 + ldc(rd + ER_GU4) * u1_ + ldc(rd + ER_GU5) * u2_;
-                    g[1] = ldc(rd + ER_GD0) * w0 + ldc(rd + ER_GD1) * w1 + ldc(rd + ER_GD2) * w2;
-                    g[3] = ldc(rd + ER_GD3) * w0 + ldc(rd + ER_GD4) * w1 + ldc(rd + ER_GD5) * w2;
-                } else {
-                    if (mean1[s]) { const double2 q = s ? m1b : m1a; g[0] = q.x; g[2] = q.y; }
-                    if (mean2[s]) { const double2 q = s ? m2b : m2a; g[1] = q.x; g[3] = q.y; }
+            for (int s = 0; s < NV; ++s) {
+                gr[0][s] = ldc(rd + ER_GU0) * ux[0][s] + ldc(rd + ER_GU1) * ux[1][s] + ldc(rd + ER_GU2) * ux[2][s];
+                gr[2][s] = ldc(rd + ER_GU3) * ux[0][s] + ldc(rd + ER_GU4) * ux[1][s] + ldc(rd + ER_GU5) * ux[2][s];
+                gr[1][s] = ldc(rd + ER_GD0) * wx[0][s] + ldc(rd + ER_GD1) * wx[1][s] + ldc(rd + ER_GD2) * wx[2][s];
+                gr[3][s] = ldc(rd + ER_GD3) * wx[0][s] + ldc(rd + ER_GD4) * wx[1][s] + ldc(rd + ER_GD5) * wx[2][s];
+            }
+            if (any_mean) {
+                const double *gm = t.gmean + t.sG * tb;
+                const OFF oG = 2 * lev + 8 * (OFF)g * (OFF)t.sG;
+                double m1[2 * NV], m2[2 * NV];
+                row_load<2 * NV>(gm, oG + 2 * o1, m1);
+                row_load<2 * NV>(gm, oG + 2 * o2, m2);
+#pragma unroll
+                for (int s = 0; s < NV; ++s) {
+                    gr[0][s] = mean[s] ? m1[2 * s] : gr[0][s];
+                    gr[2][s] = mean[s] ? m1[2 * s + 1] : gr[2][s];
+                    gr[1][s] = mean[s] ? m2[2 * s] : gr[1][s];
+                    gr[3][s] = mean[s] ? m2[2 * s + 1] : gr[3][s];
                 }
-                double Tmean2, Tmean1;
-                if (hor == HOR_MUSCL) {   // reconstruction only down to nboundary_lay (oce_adv_tra_hor.F90:356-367)
-                    const int k = kb + s;
-                    const double c1 = k <= ldc(ri + ER_NBL1) ? 1.0 : 0.0, c2 = k <= ldc(ri + ER_NBL2) ? 1.0 : 0.0;
-                    Tmean2 = A2[s] - (2.0 * (A2[s] - A1[s]) + edx * a * g[1] + edy * FGPU_R_EARTH * g[3]) / 6.0 * c2;
-                    Tmean1 = A1[s] + (2.0 * (A2[s] - A1[s]) + edx * a * g[0] + edy * FGPU_R_EARTH * g[2]) / 6.0 * c1;
-                } else {
-                    Tmean2 = A2[s] - (2.0 * (A2[s] - A1[s]) + edx * a * g[1] + edy * FGPU_R_EARTH * g[3]) / 6.0;
-                    Tmean1 = A1[s] + (2.0 * (A2[s] - A1[s]) + edx * a * g[0] + edy * FGPU_R_EARTH * g[2]) / 6.0;
+            }
+            double x1[NV], x2[NV], c1[NV], c2[NV];
+            bool small = false;
+#pragma unroll
+            for (int s = 0; s < NV; ++s) {
+                const double dA = 2.0 * (A2[s] - A1[s]);
+                x2[s] = dA + edxa * gr[1][s] + edyr * gr[3][s];
+                x1[s] = dA + edxa * gr[0][s] + edyr * gr[2][s];
+                c2[s] = sixth(x2[s]);
+                c1[s] = sixth(x1[s]);
+                small = small || tiny(x1[s]) || tiny(x2[s]);
+            }
+            if (__any(small)) {
+#pragma unroll
+                for (int s = 0; s < NV; ++s) {
+                    c2[s] = x2[s] / 6.0;
+                    c1[s] = x1[s] / 6.0;
                 }
-                for (int sg = 0; sg < 2; ++sg) {
-                    if ((sg == 0 ? s1[s] : s2[s]) < 0) continue;
-                    const double vflux = sg == 0 ? vf1[s] : vf2[s];
-                    const double cHO = (vflux + fabs(vflux)) * Tmean1 + (vflux - fabs(vflux)) * Tmean2;
-                    f[s] = -0.5 * (1.0 - no) * cHO - vflux * no * 0.5 * (Tmean1 + Tmean2) - f[s];
+            }
+            if (hor == HOR_MUSCL) {   // reconstruction only down to nboundary_lay (oce_adv_tra_hor.F90:356-367)
+#pragma unroll
+                for (int s = 0; s < NV; ++s) {
+                    c1[s] = c1[s] * (kb + s <= ldc(ri + ER_NBL1) ? 1.0 : 0.0);
+                    c2[s] = c2[s] * (kb + s <= ldc(ri + ER_NBL2) ? 1.0 : 0.0);
                 }
+            }
+#pragma unroll
+            for (int s = 0; s < NV; ++s) {
+                const double Tmean2 = A2[s] - c2[s], Tmean1 = A1[s] + c1[s];
+                const double cHO = vp[s] * Tmean1 + vm[s] * Tmean2;
+                f[s] = -0.5 * (1.0 - no) * cHO - vf[s] * no * 0.5 * (Tmean1 + Tmean2) - f[s];
             }
         } else {
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                if (s1[s] >= 0) f[s] = upw1_h(A1[s], A2[s], vf1[s], f[s]);
-                if (s2[s] >= 0) f[s] = upw1_h(A1[s], A2[s], vf2[s], f[s]);
-            }
+            for (int s = 0; s < NV; ++s) f[s] = -0.5 * (A1[s] * vp[s] + A2[s] * vm[s]) - f[s];
         }
-        st2(t.a_h + t.sE * tr + ei, f[0], f[1], act[0], act[1]);
+        row_store<NV>(t.a_h + t.sE * tb + (size_t)e * L, oE, f, act);
     }
 }
 
@@ -562,19 +597,18 @@ __device__ __forceinline__ double col_qr4c(int j, int nzmin, int nzmax, const do
 // ------------------------------------------------------------------------------
 // K_B: LO solution and antidiffusive vertical flux per node column
 // ------------------------------------------------------------------------------
-// XV: the CDIFF and PPM vertical schemes are compiled in (launched only when a
-// tracer uses one; their registers and LDS would slow the QR4C/UPW1 version).
+// For steps with a CDIFF or PPM tracer or the W split; the others run kB_cols.
 // WS: use_wsplit, the LO solution of FCT tracers takes the implicit upwind
 // advection with w_i (adv_tra_vert_impl, oce_adv_tra_ver.F90:90-240) and the
 // HO scheme is handed the upwind flux with the full W.
-template <int LB, bool XV, bool WS>
+template <int LB, bool WS>
 __global__ void __launch_bounds__(LB) kB_node(DevMesh m, DevDyn d, DevTracers t, double dt, int tpb)
 {
     const int j = xcd_column(m.N2);
     if (j >= m.N2) return;
     const int n = ldc(m.node_ord + j);
     __shared__ double sT[LB + 2], sA[LB + 2], sW[LB + 2], sWe[LB + 2], sAr[LB + 2], sZ[LB + 2], sZb[LB + 2];
-    __shared__ double sLo[LB + 2], sHn[XV ? LB + 2 : 1], sHo[XV ? LB + 2 : 1];
+    __shared__ double sLo[LB + 2], sHn[LB + 2], sHo[LB + 2];
     constexpr int NW = WS ? LB + 2 : 1;
     __shared__ double sIa[NW], sIb[NW], sIc[NW], sIcp[NW], sIf[NW], sIr[NW];
     const int tid = threadIdx.x, k = tid + 1;
@@ -591,10 +625,8 @@ __global__ void __launch_bounds__(LB) kB_node(DevMesh m, DevDyn d, DevTracers t,
     }
     if (k <= L) {
         sZ[tid] = m.Z3d[ci];
-        if (XV) {   // PPM: thicknesses of the neighbouring layers
-            sHn[tid] = m.hnode_new[ci];
-            sHo[tid] = m.hnode[ci];
-        }
+        sHn[tid] = m.hnode_new[ci];   // PPM: thicknesses of the neighbouring layers
+        sHo[tid] = m.hnode[ci];
     }
     double hn = 1.0, hh = 0.0, av_ = 1.0;
     if (act) {
@@ -651,19 +683,19 @@ __global__ void __launch_bounds__(LB) kB_node(DevMesh m, DevDyn d, DevTracers t,
             const double fk = (WS && lim == LIM_FCT) ? col_upw1(k, nzmin, nzmax, sT, sW, sAr, 0.0) : lk;
             double ho;
             if (ver == VER_QR4C) ho = col_qr4c(k, nzmin, nzmax, sA, W, sAr, sZ, sZb, pv, fk);
-            else if (XV && ver == VER_CDIFF) ho = ver_cdiff(k, nzmin, nzmax, sA, W, sAr, fk);
-            else if (XV && ver == VER_PPM) ho = ver_ppm(k, nzmin, nzmax, sA, W, sAr, sHn, sHo, dt, fk);
+            else if (ver == VER_CDIFF) ho = ver_cdiff(k, nzmin, nzmax, sA, W, sAr, fk);
+            else if (ver == VER_PPM) ho = ver_ppm(k, nzmin, nzmax, sA, W, sAr, sHn, sHo, dt, fk);
             else ho = col_upw1(k, nzmin, nzmax, sA, W, sAr, fk);
             av[k - 1] = ho;
         }
         if (lim == LIM_FCT) {
-            const double *lo_h = t.lo_h + t.sE * tr;
             double acc = 0.0;
-            // edges in batches of NG: the batch's loads are issued together
-            // (clamped to valid addresses), then added in ascending edge order
+            // the edges' LO fluxes from the volume fluxes, in batches of NG: the
+            // batch's loads are issued together (clamped to valid addresses),
+            // then the fluxes added in ascending edge order
             const int kk = min(k, L) - 1;
             for (int j0 = 0; j0 < E.deg; j0 += NG) {
-                double fl_[NG];
+                double v_[NG], tm_[NG];
                 int q_[NG];
                 bool ok_[NG];
 #pragma unroll
@@ -673,11 +705,16 @@ __global__ void __launch_bounds__(LB) kB_node(DevMesh m, DevDyn d, DevTracers t,
                     const int q = rl(E.q, j), a0 = rl(E.nu12, j), a1 = rl(E.nl12, j);
                     ok_[u] = real && act && k >= a0 && k <= a1;
                     q_[u] = q;
-                    fl_[u] = lo_h[(size_t)(q >> 1) * L + kk];
+                    v_[u] = t.vf[(size_t)(q >> 1) * L + kk];
+                    tm_[u] = T[(size_t)rl(E.other, j) * L + kk];
                 }
 #pragma unroll
-                for (int u = 0; u < NG; ++u)
-                    if (ok_[u]) acc = (q_[u] & 1) ? acc - fl_[u] : acc + fl_[u];
+                for (int u = 0; u < NG; ++u) {
+                    if (!ok_[u]) continue;
+                    const double t1 = (q_[u] & 1) ? tm_[u] : sT[tid], t2 = (q_[u] & 1) ? sT[tid] : tm_[u];
+                    const double fl = upw1_h(t1, t2, v_[u], 0.0);
+                    acc = (q_[u] & 1) ? acc - fl : acc + fl;
+                }
             }
             if (!WS) {
                 if (act) {
@@ -724,133 +761,180 @@ __global__ void __launch_bounds__(LB) kB_node(DevMesh m, DevDyn d, DevTracers t,
     }
 }
 
+
 // ------------------------------------------------------------------------------
-// K_B with two adjacent levels per lane: lane j takes levels and interfaces
-// 2j+1 and 2j+2, so one wave covers a column of up to 128 levels, and the
-// per-level rows (T, valuesold, Z, the thicknesses, the edges' LO fluxes and
-// fct_LO) move with 16-byte accesses (an even number of layers keeps those
-// rows 16-byte aligned). The interface rows (w, area, zbar, A_v) keep 8-byte
-// accesses: with an odd interface count every other column's row starts
-// 8 bytes off. Each level's arithmetic is kB_node's, in the same order. For
-// the step without the W split and without CDIFF or PPM tracers.
+// K_B: LO solution and antidiffusive vertical flux per node column
 // ------------------------------------------------------------------------------
-__global__ void __launch_bounds__(64) kB2_node(DevMesh m, DevDyn d, DevTracers t, double dt, int tpb)
+// The edges' LO fluxes are formed again from the volume fluxes and the T of the
+// neighbours, whose rows a node's edges share, where a stored LO flux is a row
+// per edge and tracer, three times as many. Levels exchange values by wave
+// shifts. 12 thousand nodes, 47 layers, 32 tracers: 350 -> 270 us; 40 thousand
+// nodes, 70 layers, 10 tracers: 551 -> 520; 126,858 nodes, 47 layers, 2 tracers:
+// 287 -> 298, against K_A's gain.
+template <typename OFF, int NV, int GT>
+__global__ void __launch_bounds__(64) kB_cols(DevMesh m, DevDyn d, DevTracers t, double dt, int tpb)
 {
-    const int jc = xcd_column(m.N2);
-    if (jc >= m.N2) return;
-    const int n = ldc(m.node_ord + jc);
-    __shared__ double sT[130], sA[130], sW[130], sWe[130], sAr[130], sZ[130], sZb[130], sLo[130];
-    const int kb = 2 * (int)threadIdx.x + 1;   // this lane's levels and interfaces: kb, kb + 1
-    const int L = m.L, NL = m.NL;
-    const int nzmin = m.ulevn[n], nzmax = m.nlevn[n];
-    bool act[2];
+    Column<OFF, NV, GT> c;
+    if (!load_column<(NV > 1), OFF, NV, GT>(m, t, c)) return;
+    const int nzmin = c.nzmin, nzmax = c.nzmax;
+    const int L = m.L;
+    bool first[NV], inner[NV], deep[NV], last[NV], face[NV];
+    double W[NV], We[NV], ar[NV], hn[NV], hh[NV], av[NV], dz[NV], d1[NV], d2[NV];
+    constexpr int NB = NV == 1 ? 8 : 3;   // edges whose loads are issued together
+    constexpr bool VREG = NV == 1;        // the edges' volume fluxes stay in registers over the tracers
+    double vf[VREG ? CE : NB][NV];
+    {
+        const size_t nL = (size_t)c.n * L, nNL = (size_t)c.n * m.NL;
+        const unsigned oL = 8u * (unsigned)(c.kc - 1), oI = 8u * (unsigned)((c.kb <= m.NL ? c.kb : 1) - 1);
+        double z[NV], zu[NV], zb[NV];
+        row_load<NV>(d.w + nNL, oI, W);
+        row_load<NV>(d.w_e + nNL, oI, We);
+        row_load<NV>(m.area + nNL, oI, ar);
+        row_load<NV>(m.zbar3d + nNL, oI, zb);
+        row_load<NV>(m.areasvol + nNL, oI, av);
+        row_load<NV>(m.hnode_new + nL, oL, hn);
+        row_load<NV>(m.hnode + nL, oL, hh);
+        row_load<NV>(m.Z3d + nL, oL, z);
+        if constexpr (VREG) {
 #pragma unroll
-    for (int s = 0; s < 2; ++s) act[s] = kb + s >= nzmin && kb + s <= nzmax - 1;
-    const size_t ci = (size_t)n * L + kb - 1;   // even
-    const NodeEdges E = load_node_edges(m, n);
+            for (int u = 0; u < CE; ++u)
+                if (u < c.deg) row_load<NV>(t.vf, c.oe[u] - 8 * (OFF)c.g * (OFF)t.sE, vf[u]);
+        }
+        col_up<NV>(z, zu);
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        const int k = kb + s;
-        if (k <= NL) {
-            const size_t ii = (size_t)n * NL + k - 1;
-            sW[k - 1] = d.w[ii];
-            sWe[k - 1] = d.w_e[ii];
-            sAr[k - 1] = m.area[ii];
-            sZb[k - 1] = m.zbar3d[ii];
+        for (int s = 0; s < NV; ++s) {
+            const int k = c.kb + s;
+            first[s] = k == nzmin;
+            last[s] = k == nzmax;
+            inner[s] = k >= nzmin + 1 && k <= nzmax - 1;
+            deep[s] = k >= nzmin + 2 && k <= nzmax - 2;
+            face[s] = k >= nzmin && k <= nzmax;
+            dz[s] = zu[s] - z[s];
+            d1[s] = zb[s] - z[s];
+            d2[s] = zb[s] - zu[s];
         }
     }
-    if (kb <= L) {
-        const double2 z = ld2(m.Z3d + ci);
-        sZ[kb - 1] = z.x;
-        sZ[kb] = z.y;
-    }
-    double hn[2] = {1.0, 1.0}, hh[2] = {0.0, 0.0}, av_[2] = {1.0, 1.0};
-    if (act[0] || act[1]) {
-        const double2 a = ld2(m.hnode_new + ci), b = ld2(m.hnode + ci);
-        if (act[0]) { hn[0] = a.x; hh[0] = b.x; av_[0] = m.areasvol[(size_t)n * NL + kb - 1]; }
-        if (act[1]) { hn[1] = a.y; hh[1] = b.y; av_[1] = m.areasvol[(size_t)n * NL + kb]; }
-    }
-    const size_t kk = (size_t)min(kb, L - 1) - 1;   // even; the row's last pair for lanes past L
     const int trb = blockIdx.y * tpb, tre = min(t.ntr, trb + tpb);
-    for (int tr = trb; tr < tre; ++tr) {
-        const double *T = t.T + t.sN * tr;
-        const double *Told = t.Told + t.sOld * tr;
-        const int abo = ldc(t.abo + tr), lim = ldc(t.lim + tr), ver = ldc(t.ver + tr);
-        const double pv = ldc(t.pv + tr);
-        __syncthreads();
-        if (kb <= L) {   // T and T^AB (oce_tracer_mod.F90:44-59) of both levels
-            const double2 tv = ld2(T + ci);
-            sT[kb - 1] = tv.x;
-            sT[kb] = tv.y;
-            if (abo == 2) {
-                const double2 o = ld2(Told + ci);
-                sA[kb - 1] = -(0.5 + FGPU_EPS_AB) * o.x + (1.5 + FGPU_EPS_AB) * tv.x;
-                sA[kb] = -(0.5 + FGPU_EPS_AB) * o.y + (1.5 + FGPU_EPS_AB) * tv.y;
-            } else {
-                const double2 oa = ld2(Told + 2 * ci), ob = ld2(Told + 2 * ci + 2);
-                sA[kb - 1] = (5.0 * oa.y - 16.0 * oa.x + 23.0 * tv.x) / 12.0;
-                sA[kb] = (5.0 * ob.y - 16.0 * ob.x + 23.0 * tv.y) / 12.0;
-            }
+    for (int tb = trb; tb < tre; tb += GT) {
+        if (GT > 1 && tb + c.g >= tre) return;   // the last group's missing tracers
+        const int abo = ldc(t.abo + tb), lim = ldc(t.lim + tb), ver = ldc(t.ver + tb);
+        const double pv = ldc(t.pv + tb);
+        const bool fct = lim == LIM_FCT;
+        const double *T = t.T + t.sN * tb, *Told = t.Told + t.sOld * tb;
+        double Tk[NV], A[NV], Tu[NV], Au[NV], tm[NB][NV];
+        row_load<NV>(T, c.own, Tk);
+        const OFF oO = 8 * ((OFF)(c.kc - 1) + (OFF)c.g * (OFF)t.sOld);
+        if (abo == 2) row_load<NV>(Told + (size_t)c.n * L, oO, A);
+        if (abo == 2) {   // T^AB (oce_tracer_mod.F90:44-59)
+#pragma unroll
+            for (int s = 0; s < NV; ++s) A[s] = -(0.5 + FGPU_EPS_AB) * A[s] + (1.5 + FGPU_EPS_AB) * Tk[s];
+        } else {
+            double p[2 * NV];
+            row_load<2 * NV>(Told + 2 * (size_t)c.n * L, oO + 8 * (OFF)(c.kc - 1), p);
+#pragma unroll
+            for (int s = 0; s < NV; ++s) A[s] = (5.0 * p[2 * s + 1] - 16.0 * p[2 * s] + 23.0 * Tk[s]) / 12.0;
         }
-        __syncthreads();
-        double *av = t.a_v + t.sNI * tr + (size_t)n * NL;
-        const double *W = (lim == LIM_FCT) ? sW : sWe;
-        double lk[2] = {0.0, 0.0};
-        if (lim == LIM_FCT) {
+        col_up<NV>(Tk, Tu);
+        col_up<NV>(A, Au);
+        // LO flux at interface k: upwind with w_e
+        double lk[NV], f[NV];
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                const int k = kb + s;
-                if (k >= nzmin && k <= nzmax) lk[s] = col_upw1(k, nzmin, nzmax, sT, sWe, sAr, 0.0);
-                sLo[k - 1] = lk[s];
-            }
+        for (int s = 0; s < NV; ++s) {
+            const double a = -We[s] * Tk[s] * ar[s];
+            const double b = -0.5 * (Tk[s] * (We[s] + fabs(We[s])) + Tu[s] * (We[s] - fabs(We[s]))) * ar[s];
+            lk[s] = fct ? (first[s] ? a : (inner[s] ? b : 0.0)) : 0.0;
         }
-        __syncthreads();
+        // HO flux minus the LO one (oce_adv_tra_ver.F90:332-434, 244-328)
+        if (ver == VER_QR4C) {
+            double qc[NV], qu[NV], qd[NV], x1[NV], x2[NV], y1[NV], y2[NV];
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            const int k = kb + s;
-            if (k >= nzmin && k <= nzmax) {
-                double ho;
-                if (ver == VER_QR4C) ho = col_qr4c(k, nzmin, nzmax, sA, W, sAr, sZ, sZb, pv, lk[s]);
-                else ho = col_upw1(k, nzmin, nzmax, sA, W, sAr, lk[s]);
-                av[k - 1] = ho;
+            for (int s = 0; s < NV; ++s) qc[s] = (Au[s] - A[s]) / dz[s];   // the slope over interface k
+            col_down<NV>(qc, qu);
+            col_up<NV>(qc, qd);
+            bool small = false;
+#pragma unroll
+            for (int s = 0; s < NV; ++s) {
+                x1[s] = (2 * qc[s] + qu[s]) * d1[s];
+                x2[s] = (2 * qc[s] + qd[s]) * d2[s];
+                y1[s] = third(x1[s]);
+                y2[s] = third(x2[s]);
+                small = small || (deep[s] && (tiny(x1[s]) || tiny(x2[s])));
             }
-        }
-        if (lim == LIM_FCT) {
-            const double *lo_h = t.lo_h + t.sE * tr;
-            double acc[2] = {0.0, 0.0};
-            // edges in batches of NG: the batch's loads are issued together,
-            // then added in ascending edge order
-            for (int j0 = 0; j0 < E.deg; j0 += NG) {
-                double2 fl_[NG];
-                int q_[NG], a0_[NG], a1_[NG];
-                bool real_[NG];
+            if (__any(small)) {
 #pragma unroll
-                for (int u = 0; u < NG; ++u) {
-                    real_[u] = j0 + u < E.deg;
-                    const int j = real_[u] ? j0 + u : 0;
-                    q_[u] = rl(E.q, j);
-                    a0_[u] = rl(E.nu12, j);
-                    a1_[u] = rl(E.nl12, j);
-                    fl_[u] = ld2(lo_h + (size_t)(q_[u] >> 1) * L + kk);
-                }
-#pragma unroll
-                for (int u = 0; u < NG; ++u) {
-#pragma unroll
-                    for (int s = 0; s < 2; ++s) {
-                        const int k = kb + s;
-                        if (real_[u] && act[s] && k >= a0_[u] && k <= a1_[u]) {
-                            const double fl = s ? fl_[u].y : fl_[u].x;
-                            acc[s] = (q_[u] & 1) ? acc[s] - fl : acc[s] + fl;
-                        }
-                    }
+                for (int s = 0; s < NV; ++s) {
+                    y1[s] = x1[s] / 3.0;
+                    y2[s] = x2[s] / 3.0;
                 }
             }
-            double o[2] = {0.0, 0.0};
 #pragma unroll
-            for (int s = 0; s < 2; ++s)
-                if (act[s]) o[s] = (sT[kb - 1 + s] * hh[s] + (acc[s] + (lk[s] - sLo[kb + s])) * dt / av_[s]) / hn[s];
-            st2(t.fct_lo + t.sN * tr + ci, o[0], o[1], act[0], act[1]);
+            for (int s = 0; s < NV; ++s) {
+                const double ww = fct ? W[s] : We[s];
+                const double Tmean1 = A[s] + y1[s], Tmean2 = Au[s] + y2[s];
+                const double Tmean = (ww + fabs(ww)) * Tmean1 + (ww - fabs(ww)) * Tmean2;
+                const double ho = (-0.5 * (1.0 - pv) * Tmean - pv * (0.5 * (Tmean1 + Tmean2)) * ww) * ar[s];
+                const double top = -A[s] * ww * ar[s];
+                const double near = -0.5 * (Au[s] + A[s]) * ww * ar[s];   // next to the surface and the bottom
+                f[s] = (first[s] ? top : (deep[s] ? ho : (last[s] ? 0.0 : near))) - lk[s];
+                if (nzmax - nzmin == 2 && inner[s]) f[s] = near - f[s];   // both rows at once
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < NV; ++s) {
+                const double ww = fct ? W[s] : We[s];
+                const double a = -ww * A[s] * ar[s];
+                const double b = -0.5 * (A[s] * (ww + fabs(ww)) + Au[s] * (ww - fabs(ww))) * ar[s];
+                f[s] = (first[s] ? a : (inner[s] ? b : 0.0)) - lk[s];
+            }
         }
+        row_store<NV>(t.a_v + t.sNI * tb, c.ownI, f, face);
+        if (!fct) continue;
+        // the edges' LO fluxes, formed again from the volume fluxes, in ascending order
+        double acc[NV];
+#pragma unroll
+        for (int s = 0; s < NV; ++s) acc[s] = 0.0;
+        int kb = c.kb;
+        if constexpr (NV > 1) asm volatile("" : "+v"(kb));   // the level masks are formed in place: they would not fit the scalar registers
+        auto add = [&](int side, const double (&v)[NV], const double (&to)[NV], int a0, int len)
+            __attribute__((always_inline)) {
+            // side 0: acc + -0.5 (Tk (v + |v|) + to (v - |v|)); side 1: acc - -0.5 (to (v + |v|) + Tk (v - |v|))
+            const long long sgn = (long long)side << 63;
+            const double half = side ? 0.5 : -0.5;
+#pragma unroll
+            for (int s = 0; s < NV; ++s) {
+                const double a = signed_by(fabs(v[s]), sgn);
+                const double x = acc[s] + half * (Tk[s] * (v[s] + a) + to[s] * (v[s] - a));
+                acc[s] = edge_has(kb, s, a0, len) ? x : acc[s];
+            }
+        };
+#pragma unroll
+        for (int u0 = 0; u0 < CE; u0 += NB) {
+            if (u0 < c.deg) {
+#pragma unroll
+                for (int u = 0; u < NB; ++u) {
+                    if (u0 + u >= CE || u0 + u >= c.deg) break;
+                    row_load<NV>(T, c.on[u0 + u], tm[u]);
+                    if constexpr (!VREG) row_load<NV>(t.vf, c.oe[u0 + u] - 8 * (OFF)c.g * (OFF)t.sE, vf[u]);
+                }
+#pragma unroll
+                for (int u = 0; u < NB; ++u)
+                    if (u0 + u < CE && u0 + u < c.deg) add(c.side[u0 + u], vf[VREG ? u0 + u : u], tm[u], c.a0[u0 + u], c.len[u0 + u]);
+            }
+        }
+        for (int u = CE; u < c.deg; ++u) {
+            OFF on, oe;
+            int a0, len, side;
+            edge_offsets<OFF, NV, GT>(m, t, c, u, on, oe, a0, len, side);
+            double v[NV], to[NV];
+            row_load<NV>(t.vf, oe - 8 * (OFF)c.g * (OFF)t.sE, v);
+            row_load<NV>(T, on, to);
+            add(side, v, to, a0, len);
+        }
+        double ld[NV], o[NV];
+        col_down<NV>(lk, ld);
+#pragma unroll
+        for (int s = 0; s < NV; ++s) o[s] = (Tk[s] * hh[s] + (acc[s] + (lk[s] - ld[s])) * dt / av[s]) / hn[s];
+        row_store<NV>(t.fct_lo + t.sN * tb, c.own, o, c.wet);
     }
 }
 
@@ -862,229 +946,110 @@ __global__ void __launch_bounds__(64) kB2_node(DevMesh m, DevDyn d, DevTracers t
 // together with the padding -1e3 (max) / +1e3 (min) of every element around
 // the node that lacks the level (oce_adv_tra_fct.F90:148-178).
 // ------------------------------------------------------------------------------
-template <int LB>
-__global__ void __launch_bounds__(LB) kC_node(DevMesh m, DevTracers t, double dt, int tpb)
+// 126,858 nodes, 47 layers, 2 tracers: 344 -> 295 us; 12 thousand nodes, 32
+// tracers: 520 -> 395; 40 thousand nodes, 70 layers, 10 tracers: 744 -> 610.
+template <typename OFF, int NV, int GT>
+__global__ void __launch_bounds__(64) kC_cols(DevMesh m, DevTracers t, double dt, int tpb)
 {
-    const int j = xcd_column(m.N2);
-    if (j >= m.N2) return;
-    const int n = ldc(m.node_ord + j);
-    __shared__ double sMx[LB + 2], sMn[LB + 2];
-    const int tid = threadIdx.x, k = tid + 1;
-    const int L = m.L, NL = m.NL;
-    const int nzmin = m.ulevn[n], nzmax = m.nlevn[n];
-    const bool act = (k >= nzmin && k <= nzmax - 1);
-    const size_t ci = (size_t)n * L + k - 1;
-    const NodeEdges E = load_node_edges(m, n);
-    double hn = 1.0, av_ = 1.0;
-    if (act) {
-        hn = m.hnode_new[ci];
-        av_ = m.areasvol[(size_t)n * NL + k - 1];
+    Column<OFF, NV, GT> c;
+    if (!load_column<true, OFF, NV, GT>(m, t, c)) return;
+    const int L = m.L;
+    const int pad0 = ldc(m.fct_pad + 2 * (size_t)c.n), pad1 = ldc(m.fct_pad + 2 * (size_t)c.n + 1);
+    double av[NV], hn[NV];
+    row_load<NV>(m.areasvol + (size_t)c.n * m.NL, 8u * (unsigned)(c.kc - 1), av);
+    row_load<NV>(m.hnode_new + (size_t)c.n * L, 8u * (unsigned)(c.kc - 1), hn);
+    bool padded[NV], alone[NV];
+#pragma unroll
+    for (int s = 0; s < NV; ++s) {
+        const int k = c.kb + s;
+        padded[s] = k < pad0 || k >= pad1;   // an element around n lacks level k
+        alone[s] = k == c.nzmax - 1 || k == c.nzmin;
     }
-    const int2 pr = *(const int2 *)(m.fct_pad + 2 * (size_t)n);
-    const bool padded = k < pr.x || k >= pr.y;   // an element around n lacks level k
     const int trb = blockIdx.y * tpb, tre = min(t.ntr, trb + tpb);
-    for (int tr = trb; tr < tre; ++tr) {
-        if (ldc(t.lim + tr) != LIM_FCT) continue;   // uniform over the block
-        const double *T = t.T + t.sN * tr;
-        const double *LO = t.fct_lo + t.sN * tr;
-        const double *ah = t.a_h + t.sE * tr;
-        double vmax = -1e3, vmin = 1e3, lo = 0.0, p = 0.0, q = 0.0;
-        if (act) {
-            lo = LO[ci];
-            const double tk = T[ci];
-            vmax = dmx(lo, tk);
-            vmin = dmn(lo, tk);
-            if (padded) {
-                vmax = dmx(vmax, -1e3);
-                vmin = dmn(vmin, 1e3);
-            }
-            const double *av = t.a_v + t.sNI * tr + (size_t)n * NL;
-            p = p + (dmx(0.0, av[k - 1]) + dmx(0.0, -av[k]));
-            q = q + (dmn(0.0, av[k - 1]) + dmn(0.0, -av[k]));
-        }
-        const int kk = min(k, L) - 1;
-        for (int j0 = 0; j0 < E.deg; j0 += NG) {
-            double lm_[NG], tm_[NG], fl_[NG];
-            int qq_[NG];
-            bool has_[NG], in_[NG];
+    for (int tb = trb; tb < tre; tb += GT) {
+        if (GT > 1 && tb + c.g >= tre) return;   // the last group's missing tracers
+        if (ldc(t.lim + tb) != LIM_FCT) continue;
+        const double *T = t.T + t.sN * tb, *LO = t.fct_lo + t.sN * tb, *ah = t.a_h + t.sE * tb;
+        double lo[NV], tk[NV], f[NV], fd[NV], vmax[NV], vmin[NV], p[NV], q[NV];
+        row_load<NV>(LO, c.own, lo);
+        row_load<NV>(T, c.own, tk);
+        row_load<NV>(t.a_v + t.sNI * tb, c.ownI, f);
+        constexpr int NB = NV == 1 || GT == 1 ? 3 : 4;   // edges whose loads are issued together
+        double lm[NB][NV], tm[NB][NV], fl[NB][NV];
+        auto load = [&](int u0) __attribute__((always_inline)) {
 #pragma unroll
-            for (int u = 0; u < NG; ++u) {
-                const bool real = j0 + u < E.deg;
-                const int j = real ? j0 + u : 0;
-                const int qq = rl(E.q, j), mo = rl(E.other, j);
-                const int a0 = rl(E.nu12, j), a1 = rl(E.nl12, j);
-                const int b_nu1 = rl(E.nu1, j), b_nl1 = rl(E.nl1, j), b_nu2 = rl(E.nu2, j), b_nl2 = rl(E.nl2, j);
-                has_[u] = real && act && ((k >= b_nu1 && k <= b_nl1) || (b_nu2 > 0 && k >= b_nu2 && k <= b_nl2));
-                in_[u] = real && act && k >= a0 && k <= a1;
-                qq_[u] = qq;
-                const size_t mi = (size_t)mo * L + kk;
-                lm_[u] = LO[mi];
-                tm_[u] = T[mi];
-                fl_[u] = ah[(size_t)(qq >> 1) * L + kk];
+            for (int u = 0; u < NB; ++u) {
+                if (u0 + u >= CE || u0 + u >= c.deg) break;
+                row_load<NV>(LO, c.on[u0 + u], lm[u]);
+                row_load<NV>(T, c.on[u0 + u], tm[u]);
+                row_load<NV>(ah, c.oe[u0 + u], fl[u]);
             }
+        };
+        int kb = c.kb;
+        if constexpr (NV > 1) asm volatile("" : "+v"(kb));   // see K_B
+        auto add = [&](int side, const double (&a)[NV], const double (&b)[NV], const double (&x)[NV], int a0, int len)
+            __attribute__((always_inline)) {
+            const long long sgn = (long long)side << 63;
 #pragma unroll
-            for (int u = 0; u < NG; ++u) {
-                if (has_[u]) {
-                    vmax = dmx(vmax, dmx(lm_[u], tm_[u]));
-                    vmin = dmn(vmin, dmn(lm_[u], tm_[u]));
+            for (int s = 0; s < NV; ++s) {
+                const bool has = edge_has(kb, s, a0, len);
+                if constexpr (NV == 1) {   // outside the edge's levels a and b are the column's own values
+                    vmax[s] = dmx(vmax[s], dmx(a[s], b[s]));
+                    vmin[s] = dmn(vmin[s], dmn(a[s], b[s]));
+                } else {
+                    const double hi = dmx(vmax[s], dmx(a[s], b[s])), lw = dmn(vmin[s], dmn(a[s], b[s]));
+                    vmax[s] = has ? hi : vmax[s];
+                    vmin[s] = has ? lw : vmin[s];
                 }
-                if (in_[u]) {
-                    const double fl = fl_[u];
-                    if (qq_[u] & 1) {
-                        p = p + dmx(0.0, -fl);
-                        q = q + dmn(0.0, -fl);
-                    } else {
-                        p = p + dmx(0.0, fl);
-                        q = q + dmn(0.0, fl);
-                    }
-                }
+                const double y = has ? signed_by(x[s], sgn) : 0.0;
+                p[s] = p[s] + dmx(0.0, y);
+                q[s] = q[s] + dmn(0.0, y);
             }
-        }
-        __syncthreads();
-        sMx[tid] = vmax;
-        sMn[tid] = vmin;
-        __syncthreads();
-        if (act) {
-            double bmax, bmin;
-            if (k == nzmax - 1 || k == nzmin) {
-                bmax = vmax - lo;
-                bmin = vmin - lo;
-            } else {
-                bmax = dmx(dmx(sMx[tid - 1], vmax), sMx[tid + 1]) - lo;
-                bmin = dmn(dmn(sMn[tid - 1], vmin), sMn[tid + 1]) - lo;
-            }
-            double flux = p * dt / av_ / hn + 1e-16;
-            t.rp[t.sN * tr + ci] = dmn(1.0, bmax / flux);
-            flux = q * dt / av_ / hn - 1e-16;
-            t.rm[t.sN * tr + ci] = dmn(1.0, bmin / flux);
-        }
-    }
-}
-
-// ------------------------------------------------------------------------------
-// K_C over (tracer, level) items: one wave per node column and TPF tracers;
-// lane j of chunk c takes item i = 64 c + j, tracer trb + i / nw and level
-// nzmin + i % nw of the column's nw wet layers, so a wave instruction covers
-// 64 wet (tracer, level) pairs instead of one tracer's column padded to the
-// lane count. Same arithmetic per (tracer, level) as kC_node, neighbours added
-// in the same order, so the results are bit-identical to it. NCH bounds the
-// chunks: TPF x (levels of the deepest column) / 64, rounded up.
-// ------------------------------------------------------------------------------
-template <int TPF, int NCH>
-__global__ void __launch_bounds__(64) kCf_node(DevMesh m, DevTracers t, double dt)
-{
-    constexpr int RS = 130;   // LDS row per tracer: levels 1..128 (index k - 1) and a guard
-    __shared__ double sMx[TPF][RS], sMn[TPF][RS];
-    const int jn = xcd_column(m.N2);
-    if (jn >= m.N2) return;
-    const int n = ldc(m.node_ord + jn);
-    const int lane = threadIdx.x;
-    const int L = m.L, NL = m.NL;
-    const int nzmin = m.ulevn[n], nzmax = m.nlevn[n];
-    const int nw = nzmax - nzmin;   // wet layers nzmin..nzmax-1
-    if (nw < 1) return;
-    const NodeEdges E = load_node_edges(m, n);
-    const int2 pr = *(const int2 *)(m.fct_pad + 2 * (size_t)n);
-    const int trb = blockIdx.y * TPF, tre = min(t.ntr, trb + TPF);
-    const int items = (tre - trb) * nw;
-    const float inw = 1.0f / (float)nw;
-    double lo_[NCH], p_[NCH], q_[NCH];
+        };
+        load(0);
+        col_down<NV>(f, fd);
 #pragma unroll
-    for (int c = 0; c < NCH; ++c) {
-        lo_[c] = 0.0; p_[c] = 0.0; q_[c] = 0.0;
-        const int i = 64 * c + lane;
-        if (64 * c >= items) break;   // uniform
-        const bool on = i < items;
-        const int tri = on ? (int)(((float)i + 0.5f) * inw) : 0;
-        const int tr = trb + tri, k = nzmin + (on ? i - tri * nw : 0);
-        const bool act = on && ldc(t.lim + tr) == LIM_FCT;
-        const size_t ci = (size_t)n * L + k - 1;
-        const double *T = t.T + t.sN * tr;
-        const double *LO = t.fct_lo + t.sN * tr;
-        const double *ah = t.a_h + t.sE * tr;
-        double vmax = -1e3, vmin = 1e3, lo = 0.0, p = 0.0, q = 0.0;
-        if (act) {
-            lo = LO[ci];
-            const double tk = T[ci];
-            vmax = dmx(lo, tk);
-            vmin = dmn(lo, tk);
-            if (k < pr.x || k >= pr.y) {   // an element around n lacks level k
-                vmax = dmx(vmax, -1e3);
-                vmin = dmn(vmin, 1e3);
-            }
-            const double *av = t.a_v + t.sNI * tr + (size_t)n * NL;
-            p = p + (dmx(0.0, av[k - 1]) + dmx(0.0, -av[k]));
-            q = q + (dmn(0.0, av[k - 1]) + dmn(0.0, -av[k]));
+        for (int s = 0; s < NV; ++s) {
+            vmax[s] = dmx(lo[s], tk[s]);
+            vmin[s] = dmn(lo[s], tk[s]);
+            vmax[s] = padded[s] ? dmx(vmax[s], -1e3) : vmax[s];
+            vmin[s] = padded[s] ? dmn(vmin[s], 1e3) : vmin[s];
+            p[s] = 0.0 + (dmx(0.0, f[s]) + dmx(0.0, -fd[s]));
+            q[s] = 0.0 + (dmn(0.0, f[s]) + dmn(0.0, -fd[s]));
         }
-        for (int j0 = 0; j0 < E.deg; j0 += NG) {
-            double lm_[NG], tm_[NG], fl_[NG];
-            int qq_[NG];
-            bool has_[NG], in_[NG];
 #pragma unroll
-            for (int u = 0; u < NG; ++u) {
-                const bool real = j0 + u < E.deg;
-                const int j = real ? j0 + u : 0;
-                const int qq = rl(E.q, j), mo = rl(E.other, j);
-                const int a0 = rl(E.nu12, j), a1 = rl(E.nl12, j);
-                const int b_nu1 = rl(E.nu1, j), b_nl1 = rl(E.nl1, j), b_nu2 = rl(E.nu2, j), b_nl2 = rl(E.nl2, j);
-                has_[u] = real && act && ((k >= b_nu1 && k <= b_nl1) || (b_nu2 > 0 && k >= b_nu2 && k <= b_nl2));
-                in_[u] = real && act && k >= a0 && k <= a1;
-                qq_[u] = qq;
-                const size_t mi = (size_t)mo * L + k - 1;
-                lm_[u] = LO[mi];
-                tm_[u] = T[mi];
-                fl_[u] = ah[(size_t)(qq >> 1) * L + k - 1];
-            }
+        for (int u0 = 0; u0 < CE; u0 += NB) {
+            if (u0 < c.deg) {
+                if (u0 > 0) load(u0);
 #pragma unroll
-            for (int u = 0; u < NG; ++u) {
-                if (has_[u]) {
-                    vmax = dmx(vmax, dmx(lm_[u], tm_[u]));
-                    vmin = dmn(vmin, dmn(lm_[u], tm_[u]));
-                }
-                if (in_[u]) {
-                    const double fl = fl_[u];
-                    if (qq_[u] & 1) {
-                        p = p + dmx(0.0, -fl);
-                        q = q + dmn(0.0, -fl);
-                    } else {
-                        p = p + dmx(0.0, fl);
-                        q = q + dmn(0.0, fl);
-                    }
-                }
+                for (int u = 0; u < NB; ++u)
+                    if (u0 + u < CE && u0 + u < c.deg) add(c.side[u0 + u], lm[u], tm[u], fl[u], c.a0[u0 + u], c.len[u0 + u]);
             }
         }
-        if (on) {
-            sMx[tri][k - 1] = vmax;
-            sMn[tri][k - 1] = vmin;
+        for (int u = CE; u < c.deg; ++u) {
+            OFF on, oe;
+            int a0, len, side;
+            edge_offsets<OFF, NV, GT>(m, t, c, u, on, oe, a0, len, side);
+            double a[NV], b[NV], x[NV];
+            row_load<NV>(LO, on, a);
+            row_load<NV>(T, on, b);
+            row_load<NV>(ah, oe, x);
+            add(side, a, b, x, a0, len);
         }
-        lo_[c] = lo;
-        p_[c] = p;
-        q_[c] = q;
-    }
-    wave_sync();
+        double mxu[NV], mxd[NV], mnu[NV], mnd[NV], rp[NV], rm[NV];
+        col_up<NV>(vmax, mxu);
+        col_down<NV>(vmax, mxd);
+        col_up<NV>(vmin, mnu);
+        col_down<NV>(vmin, mnd);
 #pragma unroll
-    for (int c = 0; c < NCH; ++c) {
-        const int i = 64 * c + lane;
-        if (64 * c >= items) break;
-        const bool on = i < items;
-        const int tri = on ? (int)(((float)i + 0.5f) * inw) : 0;
-        const int tr = trb + tri, k = nzmin + (on ? i - tri * nw : 0);
-        if (!(on && ldc(t.lim + tr) == LIM_FCT)) continue;
-        const size_t ci = (size_t)n * L + k - 1;
-        const double hn = m.hnode_new[ci], av_ = m.areasvol[(size_t)n * NL + k - 1];
-        const double lo = lo_[c], vmax = sMx[tri][k - 1], vmin = sMn[tri][k - 1];
-        double bmax, bmin;
-        if (k == nzmax - 1 || k == nzmin) {
-            bmax = vmax - lo;
-            bmin = vmin - lo;
-        } else {
-            bmax = dmx(dmx(sMx[tri][k - 2], vmax), sMx[tri][k]) - lo;
-            bmin = dmn(dmn(sMn[tri][k - 2], vmin), sMn[tri][k]) - lo;
+        for (int s = 0; s < NV; ++s) {
+            const double hi = dmx(dmx(mxu[s], vmax[s]), mxd[s]), lw = dmn(dmn(mnu[s], vmin[s]), mnd[s]);
+            const double bmax = (alone[s] ? vmax[s] : hi) - lo[s], bmin = (alone[s] ? vmin[s] : lw) - lo[s];
+            rp[s] = dmn(1.0, bmax / (p[s] * dt / av[s] / hn[s] + 1e-16));
+            rm[s] = dmn(1.0, bmin / (q[s] * dt / av[s] / hn[s] - 1e-16));
         }
-        double flux = p_[c] * dt / av_ / hn + 1e-16;
-        t.rp[t.sN * tr + ci] = dmn(1.0, bmax / flux);
-        flux = q_[c] * dt / av_ / hn - 1e-16;
-        t.rm[t.sN * tr + ci] = dmn(1.0, bmin / flux);
+        row_store<NV>(t.rp + t.sN * tb, c.own, rp, c.wet);
+        row_store<NV>(t.rm + t.sN * tb, c.own, rm, c.wet);
     }
 }
 
@@ -1394,195 +1359,83 @@ __global__ void __launch_bounds__(LB) __attribute__((amdgpu_waves_per_eu(6))) kD
 }
 
 // ------------------------------------------------------------------------------
-// Column waves: one wave per node column (or edge), NV adjacent levels per lane
-// and GT tracers per wave, 64 / GT lanes each. Rows are read and written NV
-// levels at a time.
-// ------------------------------------------------------------------------------
-// two adjacent levels of a row: 16 bytes at any 8-byte boundary
-typedef double lv2 __attribute__((ext_vector_type(2), aligned(8)));
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-typedef int i32x8 __attribute__((ext_vector_type(8)));
-
-// row values at p + off (bytes, 32 bits: the row base is wave-uniform)
-template <int NV>
-__device__ __forceinline__ void row_load(const double *p, unsigned off, double (&x)[NV])
-{
-    const char *a = (const char *)p + off;
-#pragma unroll
-    for (int s = 0; s + 1 < NV; s += 2) {
-        const lv2 v = *(const lv2 *)(a + 8 * s);
-        x[s] = v.x;
-        x[s + 1] = v.y;
-    }
-    if constexpr (NV % 2 == 1) x[NV - 1] = *(const double *)(a + 8 * (NV - 1));
-}
-
-template <int NV>
-__device__ __forceinline__ void row_store(double *p, unsigned off, const double (&x)[NV], const bool (&on)[NV])
-{
-    char *a = (char *)p + off;
-#pragma unroll
-    for (int s = 0; s + 1 < NV; s += 2) {
-        if (on[s] && on[s + 1]) {
-            lv2 v;
-            v.x = x[s];
-            v.y = x[s + 1];
-            *(lv2 *)(a + 8 * s) = v;
-        } else if (on[s]) {
-            *(double *)(a + 8 * s) = x[s];
-        } else if (on[s + 1]) {
-            *(double *)(a + 8 * s + 8) = x[s + 1];
-        }
-    }
-    if constexpr (NV % 2 == 1)
-        if (on[NV - 1]) *(double *)(a + 8 * (NV - 1)) = x[NV - 1];
-}
-
-// value of the next lower / higher lane of the wave (the end lanes keep their own)
-__device__ __forceinline__ double lane_below(double x)
-{
-    const long long b = __double_as_longlong(x);
-    const int lo = (int)(b & 0xffffffffLL), hi = (int)(b >> 32);
-    const int l = __builtin_amdgcn_update_dpp(lo, lo, 0x138, 0xf, 0xf, false);   // wave_shr:1
-    const int h = __builtin_amdgcn_update_dpp(hi, hi, 0x138, 0xf, 0xf, false);
-    return __longlong_as_double(((long long)h << 32) | (unsigned int)l);
-}
-__device__ __forceinline__ double lane_above(double x)
-{
-    const long long b = __double_as_longlong(x);
-    const int lo = (int)(b & 0xffffffffLL), hi = (int)(b >> 32);
-    const int l = __builtin_amdgcn_update_dpp(lo, lo, 0x130, 0xf, 0xf, false);   // wave_shl:1
-    const int h = __builtin_amdgcn_update_dpp(hi, hi, 0x130, 0xf, 0xf, false);
-    return __longlong_as_double(((long long)h << 32) | (unsigned int)l);
-}
-
-// a column's values one level up (k - 1) and one level down (k + 1)
-template <int NV>
-__device__ __forceinline__ void col_up(const double (&x)[NV], double (&y)[NV])
-{
-    y[0] = lane_below(x[NV - 1]);
-#pragma unroll
-    for (int s = 1; s < NV; ++s) y[s] = x[s - 1];
-}
-template <int NV>
-__device__ __forceinline__ void col_down(const double (&x)[NV], double (&y)[NV])
-{
-    y[NV - 1] = lane_above(x[0]);
-#pragma unroll
-    for (int s = 0; s + 1 < NV; ++s) y[s] = x[s + 1];
-}
-
-// a / b, correctly rounded, for a divisor used many times: y = 1 / b rounded
-// once. Two Newton steps on the quotient with exact fma residuals; the second
-// starts from a faithful quotient, which with the rounded reciprocal gives the
-// correctly rounded one (Markstein, IBM J. Res. Dev. 34, 1990). That needs the
-// residuals clear of underflow: numerators outside 1e-200..1e200 (zeros,
-// infinities and NaN among them) and divisors outside 1e-60..1e60 (y_ok false)
-// take the division itself.
-struct Recip {
-    double b, y;
-    bool ok;
-};
-__device__ __forceinline__ Recip recip(double b)
-{
-    const double ab = fabs(b);
-    return {b, 1.0 / b, ab > 1e-60 && ab < 1e60};
-}
-__device__ __forceinline__ double div_by(double a, const Recip &r)
-{
-    const double q0 = a * r.y;
-    const double q1 = fma(fma(-r.b, q0, a), r.y, q0);
-    double q = fma(fma(-r.b, q1, a), r.y, q1);
-    const double aa = fabs(a);
-    if (!(r.ok && aa > 1e-200 && aa < 1e200)) {
-        q = q0;
-        if (!(r.ok && a == 0.0)) q = a / r.b;
-    }
-    return q;
-}
-
-// ------------------------------------------------------------------------------
 // K_L: limited fluxes, flux2dtracer and T* (oce_adv_tra_fct.F90:425-497,
 // oce_adv_tra_driver.F90:494-646, oce_ale_tracer.F90:595-626); T* replaces T,
-// T^n goes to valuesold. The implicit vertical diffusion follows in K_V.
-// Bound by the gathers of the neighbours' R+- and of the edge fluxes and, next,
-// by FP64 issue. The sweeps are a kernel of their own because inside the
-// column's wave they kept 2 to 10 of 64 lanes busy for most of its
-// instructions: 126,858 nodes, 47 layers, 2 tracers: one kernel 757 us, K_L
-// 356 us + K_V 159 us; 40 thousand nodes, 70 layers, 10 tracers: 1364 us,
-// 743 + 328 us. The divisions by areasvol and hnode_new, one per edge and
-// level, use a reciprocal formed once per column (div_by).
+// T^n goes to valuesold. The implicit vertical diffusion follows in K_V: inside
+// the column's wave its sweeps kept 2 to 10 of 64 lanes busy for most of the
+// kernel's instructions. One kernel for both took 757 us at 126,858 nodes, 47
+// layers, 2 tracers (K_L 349 us, K_V 159), 1179 us at 12 thousand nodes, 32
+// tracers (439, 151) and 1364 us at 40 thousand nodes, 70 layers, 10 tracers
+// (700, 328).
 // ------------------------------------------------------------------------------
-template <int NV, int GT>
-__global__ void __launch_bounds__(256) kL_node(DevMesh m, DevTracers t, double dt, int tpb)
+template <typename OFF, int NV, int GT>
+__global__ void __launch_bounds__(64) kL_node(DevMesh m, DevTracers t, double dt, int tpb)
 {
-    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
-    const int jc = xcd_column(m.N2) * 4 + w;
-    if (jc >= m.N2) return;
-    const int n = ldc(m.node_ord + jc);
-    const i32x4 nr = ldc((const i32x4 *)m.node_rec + n);
-    const int p0 = nr.x, deg = nr.y, nzmin = nr.z, nzmax = nr.w;
-    constexpr int LP = 64 / GT;
-    const int g = lane / LP, kb = (lane % LP) * NV + 1;
-    const int L = m.L, NL = m.NL;
-    const size_t nL = (size_t)n * L, nNL = (size_t)n * NL;
-    bool wet[NV];
-    Recip av[NV], hn[NV];
-    double hh[NV];
-    {
-        double a[NV], b[NV], c[NV];
+    Column<OFF, NV, GT> c;
+    if (!load_column<true, OFF, NV, GT>(m, t, c)) return;
+    const int L = m.L;
+    double av[NV], hn[NV], hh[NV];
+    row_load<NV>(m.areasvol + (size_t)c.n * m.NL, 8u * (unsigned)(c.kc - 1), av);
+    row_load<NV>(m.hnode_new + (size_t)c.n * L, 8u * (unsigned)(c.kc - 1), hn);
+    row_load<NV>(m.hnode + (size_t)c.n * L, 8u * (unsigned)(c.kc - 1), hh);
+    bool first[NV], lim_[NV];
 #pragma unroll
-        for (int s = 0; s < NV; ++s) {
-            wet[s] = kb + s >= nzmin && kb + s <= nzmax - 1;
-            a[s] = b[s] = c[s] = 1.0;
-        }
-        bool some = false;
-#pragma unroll
-        for (int s = 0; s < NV; ++s) some = some || wet[s];
-        if (some) {
-            const unsigned off = 8u * (unsigned)(kb - 1);
-            row_load<NV>(m.hnode_new + nL, off, a);
-            row_load<NV>(m.hnode + nL, off, b);
-            row_load<NV>(m.areasvol + nNL, off, c);
-        }
-#pragma unroll
-        for (int s = 0; s < NV; ++s) {
-            hn[s] = recip(a[s]);
-            hh[s] = b[s];
-            av[s] = recip(c[s]);
-        }
+    for (int s = 0; s < NV; ++s) {
+        first[s] = c.kb + s == c.nzmin;
+        lim_[s] = c.kb + s <= c.nzmax - 1;
     }
     const int trb = blockIdx.y * tpb, tre = min(t.ntr, trb + tpb);
     for (int tb = trb; tb < tre; tb += GT) {
+        if (GT > 1 && tb + c.g >= tre) return;   // the last group's missing tracers
         const bool fct = ldc(t.lim + tb) == LIM_FCT;
         const int abo = ldc(t.abo + tb);
-        const bool tr_on = GT == 1 || tb + g < tre;
-        const unsigned oN = 8u * ((unsigned)(kb - 1) + (unsigned)g * (unsigned)t.sN);
-        const unsigned oNI = 8u * ((unsigned)(kb - 1) + (unsigned)g * (unsigned)t.sNI);
-        const unsigned oE = 8u * ((unsigned)(kb - 1) + (unsigned)g * (unsigned)t.sE);
-        double *T = t.T + t.sN * tb + nL;
+        double *T = t.T + t.sN * tb;
         const double *rpT = t.rp + t.sN * tb, *rmT = t.rm + t.sN * tb, *ah = t.a_h + t.sE * tb;
-        bool act[NV], any = false, anyi = false;
-        double rp[NV], rm[NV], Tk[NV], lo[NV], f[NV], h[NV];
+        double rp[NV], rm[NV], Tk[NV], lo[NV], f[NV], h[NV], v[NV];
 #pragma unroll
-        for (int s = 0; s < NV; ++s) {
-            act[s] = wet[s] && tr_on;
-            any = any || act[s];
-            anyi = anyi || (tr_on && kb + s >= nzmin && kb + s <= nzmax);
-            rp[s] = rm[s] = 1.0;
-            Tk[s] = lo[s] = f[s] = h[s] = 0.0;
+        for (int s = 0; s < NV; ++s) rp[s] = rm[s] = lo[s] = 1.0;
+        constexpr int NB = NV == 1 ? 4 : (NV == 2 ? 2 : 3);   // edges whose loads are issued together
+        double fl[NB][NV], rpo[NB][NV], rmo[NB][NV];
+        int kb = c.kb;
+        if constexpr (NV > 1) asm volatile("" : "+v"(kb));   // see K_B
+        row_load<NV>(t.a_v + t.sNI * tb, c.ownI, f);
+        row_load<NV>(T, c.own, Tk);
+        if (fct) {
+            row_load<NV>(rpT, c.own, rp);
+            row_load<NV>(rmT, c.own, rm);
+            row_load<NV>(t.fct_lo + t.sN * tb, c.own, lo);
         }
-        if (any) {
-            row_load<NV>(T, oN, Tk);
-            if (fct) {
-                row_load<NV>(rpT + nL, oN, rp);
-                row_load<NV>(rmT + nL, oN, rm);
-                row_load<NV>(t.fct_lo + t.sN * tb + nL, oN, lo);
+        auto load = [&](int u0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < NB; ++u) {
+                if (u0 + u >= CE || u0 + u >= c.deg) break;
+                row_load<NV>(ah, c.oe[u0 + u], fl[u]);
+                if (fct) {
+                    row_load<NV>(rpT, c.on[u0 + u], rpo[u]);
+                    row_load<NV>(rmT, c.on[u0 + u], rmo[u]);
+                }
             }
-        }
-        if (anyi) row_load<NV>(t.a_v + t.sNI * tb + nNL, oNI, f);
+        };
+        // node 1 takes R+ of an inflow, node 2 R- of the same flux, and the other way round
+        auto add = [&](int side, const double (&x)[NV], const double (&po)[NV], const double (&mo)[NV], int a0, int len)
+            __attribute__((always_inline)) {
+            const long long sgn = (long long)side << 63;
+#pragma unroll
+            for (int s = 0; s < NV; ++s) {
+                double y = x[s];
+                if (fct) {
+                    const bool plus = (x[s] >= 0.0) != (side != 0);
+                    const double own = plus ? rp[s] : rm[s], oth = plus ? mo[s] : po[s];
+                    // min(min(1, R of node 1), R of node 2), R <= 1
+                    const bool mine = side ? !(oth < own) : own < oth;
+                    y = (mine ? own : oth) * y;
+                }
+                const double hs = h[s] + signed_by(y * dt / av[s], sgn);
+                h[s] = edge_has(kb, s, a0, len) ? hs : h[s];
+            }
+        };
+        load(0);
         // limited vertical antidiffusive flux at interface k (oce_adv_tra_fct.F90:425-456)
-        double v[NV];
         {
             double rpu[NV], rmu[NV], fd[NV];
             if (fct) {
@@ -1590,87 +1443,63 @@ __global__ void __launch_bounds__(256) kL_node(DevMesh m, DevTracers t, double d
                 col_up<NV>(rm, rmu);
 #pragma unroll
                 for (int s = 0; s < NV; ++s) {
-                    const int k = kb + s;
                     const double flux = f[s];
                     const bool pos = flux >= 0.0;
                     // above the interface R- (R+) of the layer, below it R+ (R-); none above the top one
                     const double below = pos ? rp[s] : rm[s], above = pos ? rmu[s] : rpu[s];
-                    double ae = k == nzmin ? 1.0 : dmn(1.0, above);
+                    double ae = first[s] ? 1.0 : dmn(1.0, above);
                     ae = dmn(ae, below);
-                    if (k <= nzmax - 1) f[s] = ae * flux;
+                    f[s] = lim_[s] ? ae * flux : flux;
                 }
             }
             col_down<NV>(f, fd);
 #pragma unroll
             for (int s = 0; s < NV; ++s) {
+                h[s] = 0.0;
                 v[s] = 0.0;
-                if (fct) v[s] = v[s] - Tk[s] * hh[s] + lo[s] * hn[s].b;
-                v[s] = v[s] + div_by((f[s] - fd[s]) * dt, av[s]);
+                if (fct) v[s] = v[s] - Tk[s] * hh[s] + lo[s] * hn[s];
+                v[s] = v[s] + (f[s] - fd[s]) * dt / av[s];
             }
         }
-        // the edges' limited antidiffusive fluxes, in ascending order; three edges' loads at a time
-        constexpr int NB = NV == 3 ? 2 : 3;
-        for (int u0 = 0; u0 < deg; u0 += NB) {
-            double fl[NB][NV], rpo[NB][NV], rmo[NB][NV];
-            i32x8 rec[NB];
 #pragma unroll
-            for (int u = 0; u < NB; ++u) {
-                if (u0 + u >= deg) break;
-                rec[u] = ldc((const i32x8 *)m.ne_rec + p0 + u0 + u);
-            }
+        for (int u0 = 0; u0 < CE; u0 += NB) {
+            if (u0 < c.deg) {
+                if (u0 > 0) load(u0);
 #pragma unroll
-            for (int u = 0; u < NB; ++u) {
-                if (u0 + u >= deg) break;
-                const int q = rec[u][0], mo = rec[u][1], a0 = rec[u][2], a1 = rec[u][3];
-                if (any && kb + NV - 1 >= a0 && kb <= a1) {
-                    row_load<NV>(ah + (size_t)(q >> 1) * L, oE, fl[u]);
-                    if (fct) {
-                        row_load<NV>(rpT + (size_t)mo * L, oN, rpo[u]);
-                        row_load<NV>(rmT + (size_t)mo * L, oN, rmo[u]);
-                    }
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < NB; ++u) {
-                if (u0 + u >= deg) break;
-                const int side = rec[u][0] & 1, a0 = rec[u][2], a1 = rec[u][3];
-#pragma unroll
-                for (int s = 0; s < NV; ++s) {
-                    const int k = kb + s;
-                    if (!(act[s] && k >= a0 && k <= a1)) continue;
-                    double x = fl[u][s];
-                    if (fct) {
-                        // node 1 takes R+ of an inflow, node 2 R- of the same flux, and the other way round
-                        const bool up = (x >= 0.0) != (side != 0);
-                        const double own = up ? rp[s] : rm[s], oth = up ? rmo[u][s] : rpo[u][s];
-                        x = (side ? dmn(dmn(1.0, oth), own) : dmn(dmn(1.0, own), oth)) * x;
-                    }
-                    const double c = div_by(x * dt, av[s]);
-                    h[s] = side ? h[s] - c : h[s] + c;
-                }
+                for (int u = 0; u < NB; ++u)
+                    if (u0 + u < CE && u0 + u < c.deg) add(c.side[u0 + u], fl[u], rpo[u], rmo[u], c.a0[u0 + u], c.len[u0 + u]);
             }
         }
-        if (any) {
-            double ts[NV];
+        for (int u = CE; u < c.deg; ++u) {
+            OFF on, oe;
+            int a0, len, side;
+            edge_offsets<OFF, NV, GT>(m, t, c, u, on, oe, a0, len, side);
+            double x[NV], po[NV], mo[NV];
+            row_load<NV>(ah, oe, x);
+            if (fct) {
+                row_load<NV>(rpT, on, po);
+                row_load<NV>(rmT, on, mo);
+            }
+            add(side, x, po, mo, a0, len);
+        }
+        double ts[NV];
+#pragma unroll
+        for (int s = 0; s < NV; ++s) {
+            double del = 0.0 + h[s] + v[s];
+            del = del + Tk[s] * (hh[s] - hn[s]);
+            ts[s] = Tk[s] + del / hn[s];
+        }
+        row_store<NV>(T, c.own, ts, c.wet);
+        // valuesold rotation (oce_tracer_mod.F90:94-123)
+        double *Told = t.Told + t.sOld * (size_t)(GT == 1 ? tb : tb + c.g) + (size_t)(abo - 1) * ((size_t)c.n * L + c.kc - 1);
+        if (abo == 2) {
+            row_store<NV>(Told, 0u, Tk, c.wet);
+        } else {
 #pragma unroll
             for (int s = 0; s < NV; ++s) {
-                double del = 0.0 + h[s] + v[s];
-                del = del + Tk[s] * (hh[s] - hn[s].b);
-                ts[s] = Tk[s] + div_by(del, hn[s]);
-            }
-            row_store<NV>(T, oN, ts, act);
-            // valuesold rotation (oce_tracer_mod.F90:94-123)
-            double *Told = t.Told + t.sOld * (size_t)(GT == 1 ? tb : tb + g);
-            if (abo == 2) {
-                row_store<NV>(Told + nL, 8u * (unsigned)(kb - 1), Tk, act);
-            } else {
-#pragma unroll
-                for (int s = 0; s < NV; ++s) {
-                    if (!act[s]) continue;
-                    double *o = Told + 2 * (nL + kb - 1 + s);
-                    o[1] = o[0];
-                    o[0] = Tk[s];
-                }
+                if (!c.wet[s]) continue;
+                Told[2 * s + 1] = Told[2 * s];
+                Told[2 * s] = Tk[s];
             }
         }
     }
@@ -1928,45 +1757,42 @@ void fgpu_kd_shape(const fgpu_context *c, int *tch_out, int *cpb_out)
     *cpb_out = cpb;
 }
 
-// The lanes of the column waves: NV levels per lane, GT tracers per wave. A
-// lane group holds every interface of a column (NV x 64 / GT >= NL).
-enum { COL_1X1, COL_1X2, COL_2X1, COL_2X2, COL_2X4, COL_3X2 };
-static int col_lanes(const fgpu_context *c, int tpb)
+// The lanes of the column waves: NV levels per lane and GT tracers per wave, so
+// that a lane group holds every interface of a column (NV x 64 / GT >= NL). Two
+// tracers share a wave where they share its scheme branches and both rows lie
+// within a 32-bit offset of the wave's base. The lines between the mappings were
+// measured per kernel, in us, at 47 layers with 2 tracers (126,858 nodes) and 32
+// tracers (12 thousand), and at 70 layers with 10 tracers (40 thousand):
+//   K_A  <1,1> 473, 567; <2,2> 502, 430 | <2,1> 728, <3,2> 744
+//   K_B  <1,1> 298, 270; <2,2> 349, 297 | <2,1> 591, <3,2> 520
+//   K_C  <1,1> 295, 459; <2,2> 330, 395 | <2,1> 610, <3,2> 638
+//   K_L  <1,1> 362, 494; <2,2> 349, 439 | <2,1> 732, <3,2> 686
+// Two levels per lane halve a row's vector memory instructions, two tracers per
+// wave form the offsets once for both; against that stand the registers (fewer
+// waves per SIMD) and what a second tracer's lanes repeat of the first one's
+// tracer-independent work. Rows of up to 32 interfaces leave half a wave free,
+// which a second tracer takes at no cost.
+struct ColLanes {
+    bool pair;    // tracers two to a wave
+    bool wide;    // row offsets need 64 bits
+};
+static ColLanes col_lanes(const fgpu_context *c, int tpb)
 {
     const DevTracers &t = c->t;
-    // tracers of one wave share its scheme branches, and their rows have to be
-    // within 32 bits of the wave's row bases
-    bool same = (t.sE > t.sNI ? t.sE : t.sNI) * 8 * 3 < (size_t)0xffff0000u;
+    const size_t field = 8 * std::max(std::max(t.sE, t.sNI), std::max(t.sOld, t.sG)) + 4096;
+    bool same = true;
     for (int i = 1; i < t.ntr; ++i)
         same = same && c->h_lim[i] == c->h_lim[0] && c->h_abo[i] == c->h_abo[0] && c->h_hor[i] == c->h_hor[0] &&
                c->h_ver[i] == c->h_ver[0] && c->h_ph[i] == c->h_ph[0] && c->h_pv[i] == c->h_pv[0];
-    const int nt = same ? std::min(tpb, t.ntr) : 1, NL = c->m.NL;
-    // A row of 65..96 interfaces: three levels per lane and two tracers fill 72
-    // of 96 slots where two levels per lane fill 70 of 128 (70 layers, 10
-    // tracers, 40 thousand nodes: K_L 826 -> 743 us)
-    if (NL > 64) return nt >= 2 && NL <= 96 ? COL_3X2 : COL_2X1;
-    if (nt < 2) return COL_1X1;
-    // Two levels per lane halve the vector memory instructions of a row (K_L of
-    // 32 tracers on 47 layers: 548 -> 481 us), and short rows leave lanes for
-    // more tracers (30 layers, 3 tracers, 9,919 nodes: 37 -> 29 us)
-    if (NL <= 32) return nt >= 3 ? COL_2X4 : COL_1X2;
-    return COL_2X2;
+    const size_t reach = c->step_wide ? 0 : 0xffffffffu;
+    return {same && std::min(tpb, t.ntr) >= 2 && 2 * field < (size_t)0xffffffffu, field >= reach};
 }
 
-static void launch_kl(fgpu_context *c, double dt, int tpb, unsigned ny)
-{
-    const DevMesh &m = c->m;
-    const DevTracers &t = c->t;
-    const dim3 g(xcd_grid((m.N2 + 3) / 4), ny), b(256);
-    switch (col_lanes(c, tpb)) {
-    case COL_1X1: hipLaunchKernelGGL((kL_node<1, 1>), g, b, 0, c->stream, m, t, dt, tpb); break;
-    case COL_1X2: hipLaunchKernelGGL((kL_node<1, 2>), g, b, 0, c->stream, m, t, dt, tpb); break;
-    case COL_2X1: hipLaunchKernelGGL((kL_node<2, 1>), g, b, 0, c->stream, m, t, dt, tpb); break;
-    case COL_2X2: hipLaunchKernelGGL((kL_node<2, 2>), g, b, 0, c->stream, m, t, dt, tpb); break;
-    case COL_2X4: hipLaunchKernelGGL((kL_node<2, 4>), g, b, 0, c->stream, m, t, dt, tpb); break;
-    default: hipLaunchKernelGGL((kL_node<3, 2>), g, b, 0, c->stream, m, t, dt, tpb); break;
-    }
-}
+#define COL_LAUNCH(kern, NV, GT, grid, ...)                                                                          \
+    do {                                                                                                             \
+        if (wide) hipLaunchKernelGGL((kern<size_t, NV, GT>), grid, dim3(64), 0, c->stream, __VA_ARGS__);             \
+        else hipLaunchKernelGGL((kern<unsigned, NV, GT>), grid, dim3(64), 0, c->stream, __VA_ARGS__);                \
+    } while (0)
 
 static void launch_kv(fgpu_context *c, double dt, int clamp)
 {
@@ -1987,28 +1813,19 @@ static void launch_kv(fgpu_context *c, double dt, int clamp)
     else hipLaunchKernelGGL(kV_cols<2>, g, b, lds, c->stream, m, c->d, c->t, dt, clamp, NC, TB);
 }
 
-// K_C over (tracer, level) items with step_kcf tracers per block (1, 2 or 4)
-template <int TPF, int NCH>
-static void launch_kcf_t(fgpu_context *c, double dt)
+// one block of LB lanes per node column: K_B and K_D of the steps with extra schemes or terms
+template <int LB>
+static void launch_kb_node(fgpu_context *c, const dim3 &g, double dt, int tpb)
 {
-    const DevMesh &m = c->m;
-    const unsigned ny = (unsigned)((c->t.ntr + TPF - 1) / TPF);
-    hipLaunchKernelGGL((kCf_node<TPF, NCH>), dim3(xcd_grid(m.N2), ny), dim3(64), 0, c->stream, m, c->t, dt);
+    if (c->d.wsplit) hipLaunchKernelGGL((kB_node<LB, true>), g, dim3(LB), 0, c->stream, c->m, c->d, c->t, dt, tpb);
+    else hipLaunchKernelGGL((kB_node<LB, false>), g, dim3(LB), 0, c->stream, c->m, c->d, c->t, dt, tpb);
 }
-
-static void launch_kcf(fgpu_context *c, double dt)
+template <int LB>
+static void launch_kd_node(fgpu_context *c, const dim3 &g, int xf, double dt, int clamp, int tpb)
 {
-    const bool narrow = c->m.NL <= 64;
-    if (c->step_kcf >= 4) {
-        if (narrow) launch_kcf_t<4, 4>(c, dt);
-        else launch_kcf_t<4, 8>(c, dt);
-    } else if (c->step_kcf >= 2) {
-        if (narrow) launch_kcf_t<2, 2>(c, dt);
-        else launch_kcf_t<2, 4>(c, dt);
-    } else {
-        if (narrow) launch_kcf_t<1, 1>(c, dt);
-        else launch_kcf_t<1, 2>(c, dt);
-    }
+    if (xf == 1) hipLaunchKernelGGL((kD_node<LB, 1>), g, dim3(LB), 0, c->stream, c->m, c->d, c->t, dt, clamp, tpb);
+    else if (xf == 2) hipLaunchKernelGGL((kD_node<LB, 2>), g, dim3(LB), 0, c->stream, c->m, c->d, c->t, dt, clamp, tpb);
+    else hipLaunchKernelGGL((kD_node<LB, 3>), g, dim3(LB), 0, c->stream, c->m, c->d, c->t, dt, clamp, tpb);
 }
 
 int fgpu_enqueue_fused_step(fgpu_context *c, double dt)
@@ -2020,68 +1837,60 @@ int fgpu_enqueue_fused_step(fgpu_context *c, double dt)
     // tracers per block: 1 runs every tracer's chain in its own waves
     const int tpb = std::max(1, std::min(c->step_tpb, nt));
     const unsigned ny = (unsigned)((nt + tpb - 1) / tpb);
-    bool xv = false;   // some tracer uses CDIFF or PPM
-    for (int v : c->h_ver) xv = xv || v == VER_CDIFF || v == VER_PPM;
-    const bool ws = c->d.wsplit != 0;   // W split: implicit upwind LO step, w_i rows of the diffusion
+    bool extra = c->d.wsplit != 0;   // the W split (implicit upwind LO step) or a CDIFF or PPM tracer
+    for (int v : c->h_ver) extra = extra || v == VER_CDIFF || v == VER_PPM;
     const int xf = fgpu_kd_extras(c);
-    const bool ka2 = c->step_ka2 && m.L % 2 == 0;   // two levels per lane: 16-byte aligned rows only
-    const bool kb2 = c->step_kb2 && m.L % 2 == 0 && !ws && !xv;
     {   // explicit diffusion terms from T^n (no-op without Ki, Redi or explicit vertical diffusion)
         int rc = fgpu_launch_diff(c, 0, nt, dt);
         if (rc) return rc;
     }
-#define LAUNCH5(LBV)                                                                                                   \
-    {                                                                                                                  \
-        {                                                                                                              \
-            ProfScope ps(c, "kG_node");                                                                                \
-            hipLaunchKernelGGL(kG_node, dim3(xcd_grid(m.N2), ny), dim3(64), 0, c->stream, m, c->t, c->d_kneed, tpb);            \
-        }                                                                                                              \
-        {                                                                                                              \
-            ProfScope ps(c, "kA_edge");                                                                                \
-            if (ka2)                                                                                                   \
-                hipLaunchKernelGGL(kA2_edge, dim3(xcd_grid(m.E2), ny), dim3(64), 0, c->stream, m, c->d, c->t, tpb);    \
-            else                                                                                                       \
-                hipLaunchKernelGGL(kA_edge<LBV>, dim3(xcd_grid(m.E2), ny), dim3(LBV), 0, c->stream, m, c->d, c->t, tpb); \
-        }                                                                                                              \
-        {                                                                                                              \
-            ProfScope ps(c, "kB_node");                                                                                \
-            if (kb2)                                                                                                   \
-                hipLaunchKernelGGL(kB2_node, dim3(xcd_grid(m.N2), ny), dim3(64), 0, c->stream, m, c->d, c->t, dt, tpb); \
-            else if (ws)                                                                                               \
-                hipLaunchKernelGGL((kB_node<LBV, true, true>), dim3(xcd_grid(m.N2), ny), dim3(LBV), 0, c->stream, m, c->d, c->t, dt, tpb); \
-            else if (xv)                                                                                               \
-                hipLaunchKernelGGL((kB_node<LBV, true, false>), dim3(xcd_grid(m.N2), ny), dim3(LBV), 0, c->stream, m, c->d, c->t, dt, tpb); \
-            else                                                                                                       \
-                hipLaunchKernelGGL((kB_node<LBV, false, false>), dim3(xcd_grid(m.N2), ny), dim3(LBV), 0, c->stream, m, c->d, c->t, dt, tpb); \
-        }                                                                                                              \
-        {                                                                                                              \
-            ProfScope ps(c, "kC_node");                                                                                \
-            if (c->step_kcf > 0)                                                                                       \
-                launch_kcf(c, dt);                                                                                     \
-            else                                                                                                       \
-                hipLaunchKernelGGL(kC_node<LBV>, dim3(xcd_grid(m.N2), ny), dim3(LBV), 0, c->stream, m, c->t, dt, tpb); \
-        }                                                                                                              \
-        if (xf == 0) {                                                                                                 \
-            {                                                                                                          \
-                ProfScope ps(c, "kL_node");                                                                            \
-                launch_kl(c, dt, tpb, ny);                                                                             \
-            }                                                                                                          \
-            ProfScope ps(c, "kV_cols");                                                                                \
-            launch_kv(c, dt, clamp);                                                                                   \
-        } else {                                                                                                       \
-            ProfScope ps(c, "kD_node");                                                                                \
-            if (xf == 1)                                                                                               \
-                hipLaunchKernelGGL((kD_node<LBV, 1>), dim3(xcd_grid(m.N2), ny), dim3(LBV), 0, c->stream, m, c->d, c->t, dt, clamp, tpb); \
-            else if (xf == 2)                                                                                          \
-                hipLaunchKernelGGL((kD_node<LBV, 2>), dim3(xcd_grid(m.N2), ny), dim3(LBV), 0, c->stream, m, c->d, c->t, dt, clamp, tpb); \
-            else                                                                                                       \
-                hipLaunchKernelGGL((kD_node<LBV, 3>), dim3(xcd_grid(m.N2), ny), dim3(LBV), 0, c->stream, m, c->d, c->t, dt, clamp, tpb); \
-        }                                                                                                              \
+    const bool narrow = m.NL <= 64, slim = m.NL <= 32;
+    const dim3 nodes(xcd_grid(m.N2), ny), edges(xcd_grid(m.E2), ny);
+    const ColLanes cl = col_lanes(c, tpb);
+    const bool pair = cl.pair, wide = cl.wide, many = pair && std::min(tpb, nt) >= 4;
+    {
+        ProfScope ps(c, "kG_node");
+        hipLaunchKernelGGL(kG_node, nodes, dim3(64), 0, c->stream, m, c->t, c->d_kneed, tpb);
     }
-    // one lane per level and per interface: LB >= NL
-    if (m.NL <= 64) LAUNCH5(64)
-    else LAUNCH5(128)
-#undef LAUNCH5
+    {
+        ProfScope ps(c, "kA_edge");
+        if (!narrow) COL_LAUNCH(kA_edge, 2, 1, edges, m, c->d, c->t, tpb);
+        else if (slim && pair) COL_LAUNCH(kA_edge, 1, 2, edges, m, c->d, c->t, tpb);
+        else if (many) COL_LAUNCH(kA_edge, 2, 2, edges, m, c->d, c->t, tpb);
+        else COL_LAUNCH(kA_edge, 1, 1, edges, m, c->d, c->t, tpb);
+    }
+    {
+        ProfScope ps(c, "kB_node");
+        if (extra && narrow) launch_kb_node<64>(c, nodes, dt, tpb);
+        else if (extra) launch_kb_node<128>(c, nodes, dt, tpb);
+        else if (pair && m.NL > 64 && m.NL <= 96) COL_LAUNCH(kB_cols, 3, 2, nodes, m, c->d, c->t, dt, tpb);
+        else if (!narrow) COL_LAUNCH(kB_cols, 2, 1, nodes, m, c->d, c->t, dt, tpb);
+        else if (slim && pair) COL_LAUNCH(kB_cols, 1, 2, nodes, m, c->d, c->t, dt, tpb);
+        else COL_LAUNCH(kB_cols, 1, 1, nodes, m, c->d, c->t, dt, tpb);
+    }
+    {
+        ProfScope ps(c, "kC_node");
+        if (!narrow) COL_LAUNCH(kC_cols, 2, 1, nodes, m, c->t, dt, tpb);
+        else if (slim && pair) COL_LAUNCH(kC_cols, 1, 2, nodes, m, c->t, dt, tpb);
+        else if (many) COL_LAUNCH(kC_cols, 2, 2, nodes, m, c->t, dt, tpb);
+        else COL_LAUNCH(kC_cols, 1, 1, nodes, m, c->t, dt, tpb);
+    }
+    if (xf == 0) {
+        {
+            ProfScope ps(c, "kL_node");
+            if (pair && m.NL > 64 && m.NL <= 96) COL_LAUNCH(kL_node, 3, 2, nodes, m, c->t, dt, tpb);
+            else if (!narrow) COL_LAUNCH(kL_node, 2, 1, nodes, m, c->t, dt, tpb);
+            else if (slim && pair) COL_LAUNCH(kL_node, 1, 2, nodes, m, c->t, dt, tpb);
+            else if (pair) COL_LAUNCH(kL_node, 2, 2, nodes, m, c->t, dt, tpb);
+            else COL_LAUNCH(kL_node, 1, 1, nodes, m, c->t, dt, tpb);
+        }
+        ProfScope ps(c, "kV_cols");
+        launch_kv(c, dt, clamp);
+    } else {
+        ProfScope ps(c, "kD_node");
+        if (narrow) launch_kd_node<64>(c, nodes, xf, dt, clamp, tpb);
+        else launch_kd_node<128>(c, nodes, xf, dt, clamp, tpb);
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fgpu_fail(FGPU_ERR_HIP, std::string("fused step launch: ") + hipGetErrorString(e));
     return FGPU_OK;

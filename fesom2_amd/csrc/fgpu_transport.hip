@@ -1003,10 +1003,16 @@ extern "C" int fgpu_diff_ver_part_impl_ale(fgpu_context *c, double dt, int tr_nu
     return FGPU_OK;
 }
 
+// The fused step takes a level of an edge as belonging to its first element,
+// its second or both. Where the elements' level ranges leave a gap between
+// them, the reference's segments reach into it (oce_adv_tra_hor.F90:166-249)
+// and two of them meet: such a mesh steps through the per-stage kernels.
+static bool step_fused(const fgpu_context *c) { return c->fused && !c->edge_gap; }
+
 // one batched step of every tracer, enqueued on the context stream
 static int enqueue_step(fgpu_context *c, double dt)
 {
-    if (c->fused) return fgpu_enqueue_fused_step(c, dt);
+    if (step_fused(c)) return fgpu_enqueue_fused_step(c, dt);
     const int nt = c->t.ntr;
     int rc;
     if ((rc = launch_init_ab(c, 0, nt))) return rc;
@@ -1028,7 +1034,7 @@ static int check_step(fgpu_context *c)
 static int run_steps(fgpu_context *c, double dt, int nsteps)
 {
     int rc;
-    if (!c->fused && (rc = fgpu_ensure_staged(c, c->t.ntr))) return rc;
+    if (!step_fused(c) && (rc = fgpu_ensure_staged(c, c->t.ntr))) return rc;
     if ((rc = fgpu_ensure_diff(c))) return rc;   // before any capture
     if (c->prof) {
         for (int s = 0; s < nsteps; ++s)
@@ -1088,9 +1094,9 @@ extern "C" int fgpu_solve_tracers_ale_timed(fgpu_context *c, double dt, int nste
 
 // Autotuner of the fused step's launch shape: each candidate number of tracers
 // per block (1, 2, 4, ... and all) is timed over `nsteps` replayed steps and the
-// fastest is kept, then the variants of K_C, K_A and K_B. Every candidate
-// computes the same arithmetic per column, so results do not depend on the
-// choice. The tracer state is saved before and restored after the trials.
+// fastest is kept. Every candidate computes the same arithmetic per column, so
+// results do not depend on the choice. The tracer state is saved before and
+// restored after the trials.
 extern "C" int fgpu_autotune_step(fgpu_context *c, double dt, int nsteps, int *best_tpb, double *best_ms)
 {
     int rc = check_ready(c);
@@ -1138,50 +1144,6 @@ extern "C" int fgpu_autotune_step(fgpu_context *c, double dt, int nsteps, int *b
             best_t = ms;
             best = cand[i];
         }
-    }
-    // then the bound kernel K_C with the chosen shape: per column over its
-    // levels (0) or over (tracer, level) items with 1, 2 or 4 tracers per block
-    int best_kcf = c->step_kcf;
-    if (!rc && best_t >= 0.f) {
-        c->step_tpb = best;
-        for (int kcf : {0, 1, 2, 4}) {
-            if (kcf == best_kcf) continue;   // timed above
-            c->step_kcf = kcf;
-            c->graph_valid = false;
-            if ((rc = run_steps(c, dt, 1))) break;
-            if (hipEventRecord(e0, c->stream) != hipSuccess) { rc = fgpu_fail(FGPU_ERR_HIP, "hipEventRecord"); break; }
-            if ((rc = run_steps(c, dt, nsteps))) break;
-            float ms = 0.f;
-            if (hipEventRecord(e1, c->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
-                hipEventElapsedTime(&ms, e0, e1) != hipSuccess) {
-                rc = fgpu_fail(FGPU_ERR_HIP, "timing the autotuner trial failed");
-                break;
-            }
-            if (ms < best_t) {
-                best_t = ms;
-                best_kcf = kcf;
-            }
-        }
-    }
-    c->step_kcf = best_kcf;
-    // then K_A and K_B with two levels per lane, where the rows allow it: each
-    // flag flipped once, kept if faster
-    for (int *flag : {&c->step_ka2, &c->step_kb2}) {
-        if (rc || best_t < 0.f || c->m.L % 2 != 0) break;
-        const int tried = *flag;
-        *flag = !tried;
-        c->graph_valid = false;
-        float ms = 0.f;
-        if ((rc = run_steps(c, dt, 1))) break;
-        if (hipEventRecord(e0, c->stream) != hipSuccess) { rc = fgpu_fail(FGPU_ERR_HIP, "hipEventRecord"); break; }
-        if ((rc = run_steps(c, dt, nsteps))) break;
-        if (hipEventRecord(e1, c->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
-            hipEventElapsedTime(&ms, e0, e1) != hipSuccess) {
-            rc = fgpu_fail(FGPU_ERR_HIP, "timing the autotuner trial failed");
-            break;
-        }
-        if (ms < best_t) best_t = ms;
-        else *flag = tried;
     }
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);

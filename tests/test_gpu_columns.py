@@ -1,9 +1,14 @@
 """The column waves of the fused step (levels per lane and tracers per wave
 chosen from the column depth and the tracer count) against the oracle, bit for
-bit, at the depths where a lane group is just full or just too short: 32, 33,
-64, 65, 96, 97 and 128 interfaces, with even and odd tracer counts, one tracer
+bit: at the depths where a lane group is just full or just too short (32, 33,
+64, 65, 96, 97 and 128 interfaces), with even and odd tracer counts, one tracer
 group or several in the vertical solve, and tracers of different schemes, which
-keep a wave each."""
+keep a wave each; with 64-bit row offsets; around a node with more edges than
+the waves keep in registers; for tracers whose values reach the smallest
+doubles; and on a mesh with a level gap across an edge, which steps through the
+per-stage kernels."""
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -21,18 +26,13 @@ def _case(layers, ntr):
     return mesh, mg.build_state(mesh, seed=layers, ntr=ntr, dt=600.0, dx=20e3, kv_range=(1e-5, 1e-2))
 
 
-@pytest.mark.parametrize("layers,ntr,schemes", [
-    (4, 1, None), (31, 2, None), (31, 5, None), (31, 4, MIXED), (32, 3, None), (47, 11, None), (63, 2, None),
-    (63, 4, MIXED), (64, 3, None), (95, 3, None), (95, 4, MIXED), (96, 2, None), (127, 1, None), (127, 21, None)])
-def test_column_waves_bitwise(layers, ntr, schemes):
+def _check(mesh, st, schemes=None):
     from fesom2_amd import gpu
     from oracle.oracle import Oracle
-    mesh, st = _case(layers, ntr)
-    print(f"[gpu] {layers} layers, {ntr} tracers, 2 steps", flush=True)
     ctx = gpu.context_for(mesh, st, schemes=schemes)
     try:
         ctx.solve_tracers_ale(st.dt, 2)
-        out = [ctx.tracer_download(i + 1) for i in range(ntr)]
+        out = [ctx.tracer_download(i + 1) for i in range(st.ntr)]
     finally:
         ctx.close()
     v, vo = st.values.copy(), st.valuesold.copy()
@@ -44,3 +44,65 @@ def test_column_waves_bitwise(layers, ntr, schemes):
     for i, (gv, gvo) in enumerate(out):
         np.testing.assert_array_equal(gv[w], v[i][w], err_msg=f"tracer {i + 1}")
         np.testing.assert_array_equal(gvo[w], vo[i][w], err_msg=f"tracer {i + 1} valuesold")
+
+
+@pytest.mark.parametrize("layers,ntr,schemes", [
+    (4, 1, None), (31, 2, None), (31, 5, None), (31, 4, MIXED), (32, 3, None), (47, 11, None), (63, 2, None),
+    (63, 4, MIXED), (64, 3, None), (95, 3, None), (95, 4, MIXED), (96, 2, None), (127, 1, None), (127, 21, None)])
+def test_column_waves_bitwise(layers, ntr, schemes):
+    mesh, st = _case(layers, ntr)
+    print(f"[gpu] {layers} layers, {ntr} tracers, 2 steps", flush=True)
+    _check(mesh, st, schemes)
+
+
+@pytest.mark.parametrize("layers,ntr,schemes", [(24, 3, None), (47, 2, MIXED[:2]), (70, 3, None), (100, 1, None)])
+def test_wide_row_offsets(monkeypatch, layers, ntr, schemes):
+    monkeypatch.setenv("FGPU_STEP_ROWS", "wide")
+    mesh, st = _case(layers, ntr)
+    print(f"[gpu] 64-bit row offsets, {layers} layers, {ntr} tracers", flush=True)
+    _check(mesh, st, schemes)
+
+
+@pytest.mark.parametrize("layers,ntr", [(12, 2), (40, 1), (40, 5), (70, 2)])
+def test_node_of_many_edges(layers, ntr):
+    """A hub with 15 spokes inside two rings."""
+    m, r = 15, 3e-3
+    ang = 2 * np.pi * np.arange(m) / m
+    ring = np.stack([np.cos(ang), np.sin(ang)], 1)
+    coord = np.concatenate([[[0.0, 0.0]], r * ring, 2.2 * r * ring]) + [1.0, 0.1]
+    i, j = np.arange(m), (np.arange(m) + 1) % m
+    elem = np.concatenate([np.stack([0 * i, 1 + i, 1 + j], 1), np.stack([1 + i, 1 + m + i, 1 + j], 1),
+                           np.stack([1 + j, 1 + m + i, 1 + m + j], 1)])
+    depth = -(3000.0 + 1500.0 * np.sin(3.0 * np.arange(len(coord))))
+    mesh = mg.assemble_mesh(coord, elem, L=2 * np.pi, cartesian=False, zbar=-np.linspace(0.0, 4500.0, layers + 1),
+                            depth=depth, min_layers=4, max_layers=layers)
+    st = mg.build_state(mesh, seed=1, ntr=ntr, dt=300.0, kv_range=(1e-5, 1e-2))
+    assert np.bincount(mesh.edges.ravel()).max() == m
+    print(f"[gpu] hub of {m} edges, {layers} layers, {ntr} tracers", flush=True)
+    _check(mesh, st)
+
+
+@pytest.mark.parametrize("layers,ntr", [(24, 2), (47, 4), (70, 2)])
+def test_tiny_values(layers, ntr):
+    """Values from 1e-250 down through the subnormal numbers to zero beside one of order one."""
+    mesh, st = _case(layers, ntr)
+    rng = np.random.default_rng(3)
+    v = st.values.copy()
+    v[-1] = np.where(v[-1] != 0.0, 10.0 ** -rng.uniform(250.0, 330.0, v[-1].shape), 0.0)
+    v[-1][: mesh.nod2D // 4] = 1.0
+    st = dataclasses.replace(st, values=v, valuesold=v.copy(), ids=np.array([301] * ntr, np.int32))
+    print(f"[gpu] tiny values, {layers} layers, {ntr} tracers", flush=True)
+    _check(mesh, st)
+
+
+def test_level_gap_across_an_edge():
+    mesh, st = _case(24, 2)
+    e = int(np.flatnonzero((mesh.edge_tri >= 0).all(1) & (mesh.nlevels[mesh.edge_tri].min(1) > 12))[50])
+    a, b = mesh.edge_tri[e]
+    nl, ul = mesh.nlevels.copy(), mesh.ulevels.copy()
+    nl[a], ul[b] = 4, 8
+    nmin, umax = mesh.nlevels_nod2D_min.copy(), mesh.ulevels_nod2D_max.copy()
+    nmin[mesh.elem2D_nodes[a]], umax[mesh.elem2D_nodes[b]] = 4, 8
+    gap = dataclasses.replace(mesh, nlevels=nl, ulevels=ul, nlevels_nod2D_min=nmin, ulevels_nod2D_max=umax)
+    print("[gpu] level gap", flush=True)
+    _check(gap, st)
