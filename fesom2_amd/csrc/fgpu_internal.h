@@ -25,6 +25,39 @@ __device__ __forceinline__ int xcd_unit()
 }
 static inline unsigned xcd_grid(int units) { return (unsigned)((units + NXCD - 1) / NXCD * NXCD); }
 
+// A value at a wave-uniform address that the running kernel does not write: a
+// mesh record, the processing order or a tracer's scheme. Read through the
+// constant address space it is one scalar load. As an ordinary load the
+// compiler has to assume that the field stores of the tracer loop may change
+// it, and issues one vector load per value, tracer and wave: 17 of K_A's 27
+// vector loads per tracer were such broadcasts of the edge record (K_A at
+// 127 thousand nodes, 47 layers, 2 tracers: 669 -> 544 us; with two levels per
+// lane at 40 thousand nodes, 70 layers, 10 tracers: 1490 -> 1266 us).
+#define CONST_AS __attribute__((address_space(4)))
+template <typename T>
+__device__ __forceinline__ T ldc(const T *p)
+{
+    return *(const CONST_AS T *)(unsigned long long)p;
+}
+
+// value of the next lower / higher lane of the wave (the end lanes keep their own)
+__device__ __forceinline__ double lane_below(double x)
+{
+    const long long b = __double_as_longlong(x);
+    const int lo = (int)(b & 0xffffffffLL), hi = (int)(b >> 32);
+    const int l = __builtin_amdgcn_update_dpp(lo, lo, 0x138, 0xf, 0xf, false);   // wave_shr:1
+    const int h = __builtin_amdgcn_update_dpp(hi, hi, 0x138, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)h << 32) | (unsigned int)l);
+}
+__device__ __forceinline__ double lane_above(double x)
+{
+    const long long b = __double_as_longlong(x);
+    const int lo = (int)(b & 0xffffffffLL), hi = (int)(b >> 32);
+    const int l = __builtin_amdgcn_update_dpp(lo, lo, 0x130, 0xf, 0xf, false);   // wave_shl:1
+    const int h = __builtin_amdgcn_update_dpp(hi, hi, 0x130, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)h << 32) | (unsigned int)l);
+}
+
 // tracer scheme codes
 enum { HOR_MFCT = 0, HOR_UPW1 = 1, HOR_MUSCL = 2 };
 enum { VER_QR4C = 0, VER_UPW1 = 1, VER_CDIFF = 2, VER_PPM = 3 };
@@ -146,6 +179,7 @@ struct DevTracers {
     double *hd;               // E2*L: edge flux c of diff_part_hor_redi (node 1 adds 0+c, node 2 adds 0-c)
     double *ve;               // N2*L: diff_ver_part_expl_ale increment (i_vert_diff off)
     double *vr;               // N2*L: diff_ver_part_redi_expl increment
+    double *zbh;              // N2*NL: interface depths rebuilt from hnode, of diff_ver_part_redi_expl
 };
 
 struct ProfEntry {

@@ -821,7 +821,7 @@ extern "C" int fgpu_tracers_init(fgpu_context *c, int num_tracers)
     t.sStg = 0;
     int rc;
     t.lo_h = t.TAB = t.tr_xy = t.aux = t.dttf_h = t.dttf_v = t.dbg_av = t.dbg_grad = nullptr;
-    t.hd = t.ve = t.vr = nullptr;
+    t.hd = t.ve = t.vr = t.zbh = nullptr;
     c->stage_slots = 0;
     // the fused batched step needs only these; the per-stage buffers come with
     // the first per-tracer call (fgpu_ensure_staged)

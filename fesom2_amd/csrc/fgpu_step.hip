@@ -31,21 +31,6 @@
 
 #define NG 8    // edges per gather batch in K_B and K_C
 
-// A value at a wave-uniform address that the running kernel does not write: a
-// mesh record, the processing order or a tracer's scheme. Read through the
-// constant address space it is one scalar load. As an ordinary load the
-// compiler has to assume that the field stores of the tracer loop may change
-// it, and issues one vector load per value, tracer and wave: 17 of K_A's 27
-// vector loads per tracer were such broadcasts of the edge record (K_A at
-// 127 thousand nodes, 47 layers, 2 tracers: 669 -> 544 us; with two levels per
-// lane at 40 thousand nodes, 70 layers, 10 tracers: 1490 -> 1266 us).
-#define CONST_AS __attribute__((address_space(4)))
-template <typename T>
-__device__ __forceinline__ T ldc(const T *p)
-{
-    return *(const CONST_AS T *)(unsigned long long)p;
-}
-
 __device__ __forceinline__ double dmx(double a, double b) { return a > b ? a : b; }
 __device__ __forceinline__ double dmn(double a, double b) { return a < b ? a : b; }
 
@@ -261,24 +246,6 @@ __device__ __forceinline__ void row_store(double *p, OFF off, const double (&x)[
     }
     if constexpr (NV % 2 == 1)
         if (on[NV - 1]) *(double *)(a + 8 * (NV - 1)) = x[NV - 1];
-}
-
-// value of the next lower / higher lane of the wave (the end lanes keep their own)
-__device__ __forceinline__ double lane_below(double x)
-{
-    const long long b = __double_as_longlong(x);
-    const int lo = (int)(b & 0xffffffffLL), hi = (int)(b >> 32);
-    const int l = __builtin_amdgcn_update_dpp(lo, lo, 0x138, 0xf, 0xf, false);   // wave_shr:1
-    const int h = __builtin_amdgcn_update_dpp(hi, hi, 0x138, 0xf, 0xf, false);
-    return __longlong_as_double(((long long)h << 32) | (unsigned int)l);
-}
-__device__ __forceinline__ double lane_above(double x)
-{
-    const long long b = __double_as_longlong(x);
-    const int lo = (int)(b & 0xffffffffLL), hi = (int)(b >> 32);
-    const int l = __builtin_amdgcn_update_dpp(lo, lo, 0x130, 0xf, 0xf, false);   // wave_shl:1
-    const int h = __builtin_amdgcn_update_dpp(hi, hi, 0x130, 0xf, 0xf, false);
-    return __longlong_as_double(((long long)h << 32) | (unsigned int)l);
 }
 
 // a column's values one level up (k - 1) and one level down (k + 1)

@@ -106,3 +106,21 @@ def test_level_gap_across_an_edge():
     gap = dataclasses.replace(mesh, nlevels=nl, ulevels=ul, nlevels_nod2D_min=nmin, ulevels_nod2D_max=umax)
     print("[gpu] level gap", flush=True)
     _check(gap, st)
+
+
+@pytest.mark.parametrize("path", ["fused", "staged"])
+@pytest.mark.parametrize("layers,ntr,redi", [(7, 9, True), (8, 3, True), (31, 3, True), (32, 2, False), (63, 3, True),
+                                             (64, 2, True), (70, 2, False), (127, 2, True)])
+def test_explicit_diffusion_waves(monkeypatch, path, layers, ntr, redi):
+    """The explicit diffusion terms where a lane group just holds a column, or
+    takes it in two or three passes."""
+    mesh, st = _case(layers, ntr)
+    rng = np.random.default_rng(layers)
+    Ki = rng.uniform(20.0, 400.0, (mesh.nod2D, layers))
+    S = rng.normal(0.0, 0.01, (mesh.nod2D, layers, 3)) if redi else None
+    st = dataclasses.replace(st, Ki=Ki, slope_tapered=S, redi=redi)
+    schemes = [dict(i_vert_diff=i % 2 == 1) for i in range(ntr)]
+    if path == "staged":
+        monkeypatch.setenv("FGPU_STEP", "staged")
+    print(f"[gpu] explicit diffusion, {layers} layers, {ntr} tracers, {path}", flush=True)
+    _check(mesh, st, schemes)
