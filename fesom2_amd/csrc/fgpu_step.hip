@@ -10,7 +10,6 @@
 //   K_L  node pass   limited vertical and horizontal fluxes, flux2dtracer, T*,
 //                    valuesold rotation
 //   K_V  column pass implicit vertical diffusion (Thomas), salinity clamp
-//   K_D  K_L and K_V in one, for the W split and the explicit diffusion terms
 //
 // K_B..K_L are separated by the three global dependencies of FCT (LO of the
 // neighbours, R+/R- of the neighbours, limited edge fluxes). One wave owns one
@@ -28,8 +27,6 @@
 
 #include "fgpu_internal.h"
 #include "fgpu_vert.h"
-
-#define NG 8    // edges per gather batch in K_B and K_C
 
 __device__ __forceinline__ double dmx(double a, double b) { return a > b ? a : b; }
 __device__ __forceinline__ double dmn(double a, double b) { return a < b ? a : b; }
@@ -59,78 +56,6 @@ __device__ __forceinline__ int xcd_column(int ncol)
 {
     const int per = (int)(gridDim.x / NXCD);
     return (int)(blockIdx.x % NXCD) * per + (int)(blockIdx.x / NXCD);
-}
-
-__device__ __forceinline__ double upw1_h(double t1, double t2, double vflux, double fin)
-{
-    return -0.5 * (t1 * (vflux + fabs(vflux)) + t2 * (vflux - fabs(vflux))) - fin;
-}
-
-// T^AB from values and valuesold (oce_tracer_mod.F90:44-59)
-__device__ __forceinline__ double t_ab(int abo, const double *T, const double *Told, size_t i)
-{
-    if (abo == 2) return -(0.5 + FGPU_EPS_AB) * Told[i] + (1.5 + FGPU_EPS_AB) * T[i];
-    const double a = 5.0 * Told[2 * i + 1] - 16.0 * Told[2 * i] + 23.0 * T[i];
-    return a / 12.0;
-}
-
-__device__ __forceinline__ double seg_vflux(int seg, double u1, double v1, double u2, double v2, double h1,
-                                            double h2, double dX1, double dY1, double dX2, double dY2)
-{
-    if (seg == 0 || seg == 3) return (-v1 * dX1 + u1 * dY1) * h1;
-    if (seg == 1 || seg == 4) return (v2 * dX2 - u2 * dY2) * h2;
-    return (-v1 * dX1 + u1 * dY1) * h1 + (v2 * dX2 - u2 * dY2) * h2;
-}
-
-// limited antidiffusive edge flux as seen from a node (b3 horizontal,
-// oce_adv_tra_fct.F90:483-497): R of this node (rpn, rmn) and of the edge's
-// other node (rpo, rmo); q = 2e + side, side 1 when this node is the edge's
-// second node
-__device__ __forceinline__ double limit_edge_flux(double fl, int q, double rpn, double rmn, double rpo, double rmo)
-{
-    const double rp1 = (q & 1) ? rpo : rpn, rm1 = (q & 1) ? rmo : rmn;
-    const double rp2 = (q & 1) ? rpn : rpo, rm2 = (q & 1) ? rmn : rmo;
-    double ae = 1.0;
-    if (fl >= 0.0) {
-        ae = dmn(ae, rp1);
-        ae = dmn(ae, rm2);
-    } else {
-        ae = dmn(ae, rm1);
-        ae = dmn(ae, rp2);
-    }
-    return ae * fl;
-}
-
-// metadata of a node's edges, one edge per lane (lane < deg)
-struct NodeEdges {
-    int deg;
-    int q;          // 2*e + side
-    int other;      // the edge's other node
-    int nu12, nl12; // edge scatter range (max/min rule)
-    int nu1, nl1, nu2, nl2;
-};
-
-__device__ __forceinline__ NodeEdges load_node_edges(const DevMesh &m, int n)
-{
-    NodeEdges E;
-    const int4 nr = *(const int4 *)(m.node_rec + 4 * (size_t)n);
-    const int p0 = nr.x;
-    E.deg = nr.y;
-    const int j = threadIdx.x & 63;
-    E.q = 0; E.other = 0; E.nu12 = 1; E.nl12 = 0; E.nu1 = 1; E.nl1 = 0; E.nu2 = 0; E.nl2 = 0;
-    if (j < E.deg) {
-        const int4 a = *(const int4 *)(m.ne_rec + 8 * (size_t)(p0 + j));
-        const int4 b = *(const int4 *)(m.ne_rec + 8 * (size_t)(p0 + j) + 4);
-        E.q = a.x;
-        E.other = a.y;
-        E.nu12 = a.z;
-        E.nl12 = a.w;
-        E.nl1 = b.x;
-        E.nu1 = b.y;
-        E.nl2 = b.z;
-        E.nu2 = b.w;
-    }
-    return E;
 }
 
 // ------------------------------------------------------------------------------
@@ -525,211 +450,6 @@ __global__ void __launch_bounds__(64) kA_edge(DevMesh m, DevDyn d, DevTracers t,
 }
 
 // ------------------------------------------------------------------------------
-// column helpers on LDS copies (index = level - 1)
-// ------------------------------------------------------------------------------
-__device__ __forceinline__ double col_upw1(int j, int nzmin, int nzmax, const double *T, const double *W,
-                                           const double *ar, double f)
-{
-    if (j == nzmin) f = -W[j - 1] * T[j - 1] * ar[j - 1] - f;
-    if (j == nzmax) f = 0.0 - f;
-    if (j >= nzmin + 1 && j <= nzmax - 1) {
-        const double w = W[j - 1];
-        f = -0.5 * (T[j - 1] * (w + fabs(w)) + T[j - 2] * (w - fabs(w))) * ar[j - 1] - f;
-    }
-    return f;
-}
-
-__device__ __forceinline__ double col_qr4c(int j, int nzmin, int nzmax, const double *T, const double *W,
-                                           const double *ar, const double *Zn, const double *zb, double num_ord,
-                                           double f)
-{
-    if (j == nzmin) f = -T[j - 1] * W[j - 1] * ar[j - 1] - f;
-    if (j == nzmin + 1) f = -0.5 * (T[j - 2] + T[j - 1]) * W[j - 1] * ar[j - 1] - f;
-    if (j == nzmax - 1) f = -0.5 * (T[j - 2] + T[j - 1]) * W[j - 1] * ar[j - 1] - f;
-    if (j == nzmax) f = 0.0 - f;
-    if (j >= nzmin + 2 && j <= nzmax - 2) {
-        const int nz = j;
-        const double qc = (T[nz - 2] - T[nz - 1]) / (Zn[nz - 2] - Zn[nz - 1]);
-        const double qu = (T[nz - 1] - T[nz]) / (Zn[nz - 1] - Zn[nz]);
-        const double qd = (T[nz - 3] - T[nz - 2]) / (Zn[nz - 3] - Zn[nz - 2]);
-        const double Tmean1 = T[nz - 1] + (2 * qc + qu) * (zb[nz - 1] - Zn[nz - 1]) / 3.0;
-        const double Tmean2 = T[nz - 2] + (2 * qc + qd) * (zb[nz - 1] - Zn[nz - 2]) / 3.0;
-        const double ww = W[nz - 1];
-        const double Tmean = (ww + fabs(ww)) * Tmean1 + (ww - fabs(ww)) * Tmean2;
-        f = (-0.5 * (1.0 - num_ord) * Tmean - num_ord * (0.5 * (Tmean1 + Tmean2)) * ww) * ar[nz - 1] - f;
-    }
-    return f;
-}
-
-// ------------------------------------------------------------------------------
-// K_B: LO solution and antidiffusive vertical flux per node column
-// ------------------------------------------------------------------------------
-// For steps with a CDIFF or PPM tracer or the W split; the others run kB_cols.
-// WS: use_wsplit, the LO solution of FCT tracers takes the implicit upwind
-// advection with w_i (adv_tra_vert_impl, oce_adv_tra_ver.F90:90-240) and the
-// HO scheme is handed the upwind flux with the full W.
-template <int LB, bool WS>
-__global__ void __launch_bounds__(LB) kB_node(DevMesh m, DevDyn d, DevTracers t, double dt, int tpb)
-{
-    const int j = xcd_column(m.N2);
-    if (j >= m.N2) return;
-    const int n = ldc(m.node_ord + j);
-    __shared__ double sT[LB + 2], sA[LB + 2], sW[LB + 2], sWe[LB + 2], sAr[LB + 2], sZ[LB + 2], sZb[LB + 2];
-    __shared__ double sLo[LB + 2], sHn[LB + 2], sHo[LB + 2];
-    constexpr int NW = WS ? LB + 2 : 1;
-    __shared__ double sIa[NW], sIb[NW], sIc[NW], sIcp[NW], sIf[NW], sIr[NW];
-    const int tid = threadIdx.x, k = tid + 1;
-    const int L = m.L, NL = m.NL;
-    const int nzmin = m.ulevn[n], nzmax = m.nlevn[n];
-    const bool act = (k >= nzmin && k <= nzmax - 1);
-    const size_t ci = (size_t)n * L + k - 1;
-    const NodeEdges E = load_node_edges(m, n);
-    if (k <= NL) {
-        sW[tid] = d.w[(size_t)n * NL + tid];
-        sWe[tid] = d.w_e[(size_t)n * NL + tid];
-        sAr[tid] = m.area[(size_t)n * NL + tid];
-        sZb[tid] = m.zbar3d[(size_t)n * NL + tid];
-    }
-    if (k <= L) {
-        sZ[tid] = m.Z3d[ci];
-        sHn[tid] = m.hnode_new[ci];   // PPM: thicknesses of the neighbouring layers
-        sHo[tid] = m.hnode[ci];
-    }
-    double hn = 1.0, hh = 0.0, av_ = 1.0;
-    if (act) {
-        hn = m.hnode_new[ci];
-        hh = m.hnode[ci];
-        av_ = m.areasvol[(size_t)n * NL + k - 1];
-    }
-    if (WS) __syncthreads();   // sAr
-    if (WS && act) {   // tridiagonal rows of the implicit upwind step (tracer independent)
-        const double *wi = d.w_i + (size_t)n * NL;
-        const double zinv = 1.0 * dt;
-        double v_adv = zinv * sAr[k - 1] / av_;
-        double a, b, c;
-        if (k == nzmin) {
-            a = 0.0;
-            b = hn + wi[k - 1] * v_adv;
-        } else {
-            a = dmn(0.0, wi[k - 1]) * v_adv;
-            b = hn + dmx(0.0, wi[k - 1]) * v_adv;
-        }
-        if (k <= nzmax - 2) {
-            v_adv = zinv * sAr[k] / av_;
-            b = b - dmn(0.0, wi[k]) * v_adv;
-            c = -dmx(0.0, wi[k]) * v_adv;
-        } else {
-            c = 0.0;
-        }
-        sIa[tid] = a;
-        sIb[tid] = b;
-        sIc[tid] = c;
-    }
-    const int trb = blockIdx.y * tpb, tre = min(t.ntr, trb + tpb);
-    for (int tr = trb; tr < tre; ++tr) {
-        const double *T = t.T + t.sN * tr;
-        const double *Told = t.Told + t.sOld * tr;
-        const int abo = ldc(t.abo + tr), lim = ldc(t.lim + tr), ver = ldc(t.ver + tr);
-        const double pv = ldc(t.pv + tr);
-        __syncthreads();
-        if (k <= L) {
-            sT[tid] = T[ci];
-            sA[tid] = t_ab(abo, T, Told, ci);
-        }
-        __syncthreads();
-        double *av = t.a_v + t.sNI * tr + (size_t)n * NL;
-        const double *W = (lim == LIM_FCT) ? sW : sWe;
-        double lk = 0.0;
-        if (lim == LIM_FCT) {
-            if (k >= nzmin && k <= nzmax) lk = col_upw1(k, nzmin, nzmax, sT, sWe, sAr, 0.0);
-            sLo[tid] = lk;
-        }
-        __syncthreads();
-        if (k >= nzmin && k <= nzmax) {
-            // LO flux subtracted from the HO one: upwind with the full W under the split
-            const double fk = (WS && lim == LIM_FCT) ? col_upw1(k, nzmin, nzmax, sT, sW, sAr, 0.0) : lk;
-            double ho;
-            if (ver == VER_QR4C) ho = col_qr4c(k, nzmin, nzmax, sA, W, sAr, sZ, sZb, pv, fk);
-            else if (ver == VER_CDIFF) ho = ver_cdiff(k, nzmin, nzmax, sA, W, sAr, fk);
-            else if (ver == VER_PPM) ho = ver_ppm(k, nzmin, nzmax, sA, W, sAr, sHn, sHo, dt, fk);
-            else ho = col_upw1(k, nzmin, nzmax, sA, W, sAr, fk);
-            av[k - 1] = ho;
-        }
-        if (lim == LIM_FCT) {
-            double acc = 0.0;
-            // the edges' LO fluxes from the volume fluxes, in batches of NG: the
-            // batch's loads are issued together (clamped to valid addresses),
-            // then the fluxes added in ascending edge order
-            const int kk = min(k, L) - 1;
-            for (int j0 = 0; j0 < E.deg; j0 += NG) {
-                double v_[NG], tm_[NG];
-                int q_[NG];
-                bool ok_[NG];
-#pragma unroll
-                for (int u = 0; u < NG; ++u) {
-                    const bool real = j0 + u < E.deg;
-                    const int j = real ? j0 + u : 0;
-                    const int q = rl(E.q, j), a0 = rl(E.nu12, j), a1 = rl(E.nl12, j);
-                    ok_[u] = real && act && k >= a0 && k <= a1;
-                    q_[u] = q;
-                    v_[u] = t.vf[(size_t)(q >> 1) * L + kk];
-                    tm_[u] = T[(size_t)rl(E.other, j) * L + kk];
-                }
-#pragma unroll
-                for (int u = 0; u < NG; ++u) {
-                    if (!ok_[u]) continue;
-                    const double t1 = (q_[u] & 1) ? tm_[u] : sT[tid], t2 = (q_[u] & 1) ? sT[tid] : tm_[u];
-                    const double fl = upw1_h(t1, t2, v_[u], 0.0);
-                    acc = (q_[u] & 1) ? acc - fl : acc + fl;
-                }
-            }
-            if (!WS) {
-                if (act) {
-                    const double lk1 = sLo[tid + 1];
-                    t.fct_lo[t.sN * tr + ci] = (sT[tid] * hh + (acc + (lk - lk1)) * dt / av_) / hn;
-                }
-            } else {
-                if (act) {
-                    const double lk1 = sLo[tid + 1];
-                    sIf[tid] = (sT[tid] * hh + (acc + (lk - lk1)) * dt / av_) / hn;
-                }
-                __syncthreads();
-                if (act) {   // right-hand side of the implicit step
-                    double r;
-                    if (k == nzmin) r = -(sIb[tid] - hn) * sIf[tid] - sIc[tid] * sIf[tid + 1];
-                    else if (k <= nzmax - 2) r = -sIa[tid] * sIf[tid - 1] - (sIb[tid] - hn) * sIf[tid] - sIc[tid] * sIf[tid + 1];
-                    else r = -sIa[tid] * sIf[tid - 1] - (sIb[tid] - hn) * sIf[tid];
-                    sIr[tid] = r;
-                }
-                __syncthreads();
-                if (tid == 0) {   // Thomas sweeps of the column, one lane
-                    double cp = sIc[nzmin - 1] / sIb[nzmin - 1];
-                    double tp = sIr[nzmin - 1] / sIb[nzmin - 1];
-                    sIcp[nzmin - 1] = cp;
-                    sIr[nzmin - 1] = tp;
-                    for (int nz = nzmin + 1; nz <= nzmax - 1; ++nz) {
-                        const double an = sIa[nz - 1];
-                        const double mm = sIb[nz - 1] - cp * an;
-                        cp = sIc[nz - 1] / mm;
-                        tp = (sIr[nz - 1] - tp * an) / mm;
-                        sIcp[nz - 1] = cp;
-                        sIr[nz - 1] = tp;
-                    }
-                    double x = tp;
-                    for (int nz = nzmax - 2; nz >= nzmin; --nz) {
-                        x = sIr[nz - 1] - sIcp[nz - 1] * x;
-                        sIr[nz - 1] = x;
-                    }
-                }
-                __syncthreads();
-                if (act) t.fct_lo[t.sN * tr + ci] = sIf[tid] + sIr[tid];
-            }
-        }
-    }
-}
-
-
-// ------------------------------------------------------------------------------
 // K_B: LO solution and antidiffusive vertical flux per node column
 // ------------------------------------------------------------------------------
 // The edges' LO fluxes are formed again from the volume fluxes and the T of the
@@ -738,11 +458,20 @@ __global__ void __launch_bounds__(LB) kB_node(DevMesh m, DevDyn d, DevTracers t,
 // shifts. 12 thousand nodes, 47 layers, 32 tracers: 350 -> 270 us; 40 thousand
 // nodes, 70 layers, 10 tracers: 551 -> 520; 126,858 nodes, 47 layers, 2 tracers:
 // 287 -> 298, against K_A's gain.
-template <typename OFF, int NV, int GT>
+// EXTRA compiles in the CDIFF and PPM tracers and the W split (use_wsplit), where
+// the HO scheme is handed the upwind flux with the full W and the LO solution of
+// FCT tracers takes the implicit upwind advection with w_i afterwards (K_V on
+// it). PPM reads up to four layers around an interface, from LDS. 20 thousand
+// nodes, 47 layers, 4 tracers, W split: 140 us and 45 for the implicit step, 367
+// with a block per column, its sweeps on one lane.
+template <typename OFF, int NV, int GT, bool EXTRA>
 __global__ void __launch_bounds__(64) kB_cols(DevMesh m, DevDyn d, DevTracers t, double dt, int tpb)
 {
     Column<OFF, NV, GT> c;
     if (!load_column<(NV > 1), OFF, NV, GT>(m, t, c)) return;
+    static_assert(!EXTRA || GT == 1, "one column's rows in LDS");
+    __shared__ double sT[EXTRA ? 64 * NV : 1], sHn[EXTRA ? 64 * NV : 1], sHo[EXTRA ? 64 * NV : 1];
+    __shared__ double sW[EXTRA ? 64 * NV : 1], sWe[EXTRA ? 64 * NV : 1], sAr[EXTRA ? 64 * NV : 1];
     const int nzmin = c.nzmin, nzmax = c.nzmax;
     const int L = m.L;
     bool first[NV], inner[NV], deep[NV], last[NV], face[NV];
@@ -779,6 +508,14 @@ __global__ void __launch_bounds__(64) kB_cols(DevMesh m, DevDyn d, DevTracers t,
             dz[s] = zu[s] - z[s];
             d1[s] = zb[s] - z[s];
             d2[s] = zb[s] - zu[s];
+            if constexpr (EXTRA) {
+                const int i = c.kb + s - 1;
+                sHn[i] = hn[s];
+                sHo[i] = hh[s];
+                sW[i] = W[s];
+                sWe[i] = We[s];
+                sAr[i] = ar[s];
+            }
         }
     }
     const int trb = blockIdx.y * tpb, tre = min(t.ntr, trb + tpb);
@@ -804,12 +541,18 @@ __global__ void __launch_bounds__(64) kB_cols(DevMesh m, DevDyn d, DevTracers t,
         col_up<NV>(Tk, Tu);
         col_up<NV>(A, Au);
         // LO flux at interface k: upwind with w_e
-        double lk[NV], f[NV];
+        double lk[NV], f[NV], lw[NV];   // lw: with the full W, what the HO flux has taken off
 #pragma unroll
         for (int s = 0; s < NV; ++s) {
             const double a = -We[s] * Tk[s] * ar[s];
             const double b = -0.5 * (Tk[s] * (We[s] + fabs(We[s])) + Tu[s] * (We[s] - fabs(We[s]))) * ar[s];
             lk[s] = fct ? (first[s] ? a : (inner[s] ? b : 0.0)) : 0.0;
+            lw[s] = lk[s];
+            if (EXTRA && d.wsplit) {
+                const double x = -W[s] * Tk[s] * ar[s];
+                const double y = -0.5 * (Tk[s] * (W[s] + fabs(W[s])) + Tu[s] * (W[s] - fabs(W[s]))) * ar[s];
+                lw[s] = fct ? (first[s] ? x : (inner[s] ? y : 0.0)) : 0.0;
+            }
         }
         // HO flux minus the LO one (oce_adv_tra_ver.F90:332-434, 244-328)
         if (ver == VER_QR4C) {
@@ -842,16 +585,29 @@ __global__ void __launch_bounds__(64) kB_cols(DevMesh m, DevDyn d, DevTracers t,
                 const double ho = (-0.5 * (1.0 - pv) * Tmean - pv * (0.5 * (Tmean1 + Tmean2)) * ww) * ar[s];
                 const double top = -A[s] * ww * ar[s];
                 const double near = -0.5 * (Au[s] + A[s]) * ww * ar[s];   // next to the surface and the bottom
-                f[s] = (first[s] ? top : (deep[s] ? ho : (last[s] ? 0.0 : near))) - lk[s];
+                f[s] = (first[s] ? top : (deep[s] ? ho : (last[s] ? 0.0 : near))) - lw[s];
                 if (nzmax - nzmin == 2 && inner[s]) f[s] = near - f[s];   // both rows at once
             }
+        } else if (EXTRA && ver == VER_PPM) {
+            wave_sync();
+#pragma unroll
+            for (int s = 0; s < NV; ++s) sT[c.kb + s - 1] = A[s];
+            wave_sync();
+#pragma unroll
+            for (int s = 0; s < NV; ++s)
+                f[s] = face[s] ? ver_ppm(c.kb + s, nzmin, nzmax, sT, fct ? sW : sWe, sAr, sHn, sHo, dt, lw[s]) : 0.0;
         } else {
 #pragma unroll
             for (int s = 0; s < NV; ++s) {
                 const double ww = fct ? W[s] : We[s];
                 const double a = -ww * A[s] * ar[s];
-                const double b = -0.5 * (A[s] * (ww + fabs(ww)) + Au[s] * (ww - fabs(ww))) * ar[s];
-                f[s] = (first[s] ? a : (inner[s] ? b : 0.0)) - lk[s];
+                if (EXTRA && ver == VER_CDIFF) {   // adv_tra_ver_cdiff (oce_adv_tra_ver.F90:635-695)
+                    const double b = -(0.5 * (Au[s] + A[s])) * ww * ar[s];
+                    f[s] = first[s] ? a - lw[s] : (inner[s] ? b - lw[s] : lw[s]);
+                } else {
+                    const double b = -0.5 * (A[s] * (ww + fabs(ww)) + Au[s] * (ww - fabs(ww))) * ar[s];
+                    f[s] = (first[s] ? a : (inner[s] ? b : 0.0)) - lw[s];
+                }
             }
         }
         row_store<NV>(t.a_v + t.sNI * tb, c.ownI, f, face);
@@ -1021,311 +777,6 @@ __global__ void __launch_bounds__(64) kC_cols(DevMesh m, DevTracers t, double dt
 }
 
 // ------------------------------------------------------------------------------
-// K_D: limited fluxes, flux2dtracer, T*, implicit vertical diffusion
-// ------------------------------------------------------------------------------
-// For the steps whose last stage carries extra terms; the plain step runs K_L
-// and K_V. The Thomas sweeps of a chunk of TCH tracers run on the first wave's
-// lanes, one per tracer.
-// XF bit 0 (use_wsplit): the non-FCT tracers' implicit diffusion also takes
-// the implicit part w_i of the split W (second set of rows). XF bit 1: the
-// explicit diffusion increments (Ki, Redi, i_vert_diff off) and the Redi K33
-// terms are compiled in. Both are launched only when in use.
-template <int LB, int XF>
-__global__ void __launch_bounds__(LB) __attribute__((amdgpu_waves_per_eu(6))) kD_node(DevMesh m, DevDyn d, DevTracers t, double dt, int clamp_tracer,
-                                                    int tpb)
-{
-    constexpr int TCH = 2, CPB = 1;
-    const int w = threadIdx.x / LB;
-    const int j0 = xcd_column(m.N2) * CPB + w;
-    const bool valid = j0 < m.N2;
-    const int n = m.node_ord[valid ? j0 : m.N2 - 1];
-    // LDS reuse: Z_n lives in sAv's rows until the tracer loop starts, and the
-    // Thomas sweep's c' rows of the first two tracers of a chunk live in sRp
-    // and sRm, which are dead between a chunk's flux phase and its sweep
-    __shared__ double sRpA[CPB][LB + 2], sRmA[CPB][LB + 2], sAvA[CPB][LB + 2];
-    __shared__ double saA[CPB][LB + 2], sbA[CPB][LB + 2], scA[CPB][LB + 2];
-    __shared__ double sTsA[CPB][TCH][LB + 2], stpA[CPB][TCH][LB + 2], scpX[CPB][TCH > 2 ? TCH - 2 : 1][LB + 2];
-    __shared__ int sNz[CPB][2];
-    constexpr bool WS = (XF & 1) != 0, DX = (XF & 2) != 0;
-    constexpr int NW = WS ? LB + 2 : 1;
-    __shared__ double swaA[CPB][NW], swbA[CPB][NW], swcA[CPB][NW];
-    double *sRp = sRpA[w], *sRm = sRmA[w], *sAv = sAvA[w];
-    double *sa = saA[w], *sb = sbA[w], *sc = scA[w], *sZ = sAvA[w];
-    const int tid = threadIdx.x % LB, k = tid + 1;
-    const int L = m.L, NL = m.NL;
-    const int nzmin = valid ? m.ulevn[n] : 1, nzmax = valid ? m.nlevn[n] : 0;
-    if (tid == 0) { sNz[w][0] = nzmin; sNz[w][1] = nzmax; }
-    const bool act = (k >= nzmin && k <= nzmax - 1);
-    const size_t ci = (size_t)n * L + (k <= L ? k - 1 : L - 1);
-    const NodeEdges E = load_node_edges(m, n);
-    double hn = 1.0, hh = 0.0, av_ = 1.0, arv = 0.0;
-    if (act) {
-        hn = m.hnode_new[ci];
-        hh = m.hnode[ci];
-        av_ = m.areasvol[(size_t)n * NL + k - 1];
-        arv = m.area[(size_t)n * NL + k - 1];
-    }
-    // Z_n of the implicit diffusion, rebuilt from hnode_new when the geometry is set
-    if (act) sZ[tid] = m.zn_vd[ci];
-    __syncthreads();
-    // tridiagonal coefficients (oce_ale_tracer.F90:1098-1175): tracer independent
-    if (act) {
-        const double *kv = d.Kv + (size_t)n * NL;
-        const double zinv = 1.0 * dt;
-        double a = 0.0, b, c;
-        // Redi: K33 = Kv + Ki S3^2 at the interfaces (oce_ale_tracer.F90:1105-1108, 1138-1144, 1181-1184)
-        double tya = 0.0, tyc = 0.0;
-        const bool redi = DX && d.redi != 0;
-        if (redi) {
-            const double *zbn = m.zbn_vd + (size_t)n * NL;
-            const double *S = d.slope + (size_t)n * L * 3, *ki = d.Ki + (size_t)n * L;
-            const double s3 = S[(k - 1) * 3 + 2];
-            if (k <= nzmax - 2) {   // interface below layer k
-                const double zinv2 = 1.0 / (sZ[k - 1] - sZ[k]);
-                const double s3b = S[k * 3 + 2];
-                tyc = (zbn[k] - sZ[k]) * zinv2 * (s3 * s3) * ki[k - 1] +
-                      (sZ[k - 1] - zbn[k]) * zinv2 * (s3b * s3b) * ki[k];
-            }
-            if (k > nzmin) {   // interface above layer k
-                const double zinv1 = 1.0 / (sZ[k - 2] - sZ[k - 1]);
-                const double s3a = S[(k - 2) * 3 + 2];
-                tya = (zbn[k - 1] - sZ[k - 1]) * zinv1 * (s3a * s3a) * ki[k - 2] +
-                      (sZ[k - 2] - zbn[k - 1]) * zinv1 * (s3 * s3) * ki[k - 1];
-            }
-        }
-        if (k == nzmin) {
-            const double zinv2 = 1.0 / (sZ[k - 1] - sZ[k]);
-            c = redi ? -(kv[k] + tyc) * zinv2 * zinv * m.area[(size_t)n * NL + k] / av_
-                     : -(kv[k]) * zinv2 * zinv * m.area[(size_t)n * NL + k] / av_;
-            b = -c + hn;
-        } else if (k <= nzmax - 2) {
-            const double zinv1 = 1.0 / (sZ[k - 2] - sZ[k - 1]);
-            const double zinv2 = 1.0 / (sZ[k - 1] - sZ[k]);
-            if (redi) {
-                a = -(kv[k - 1] + tya) * zinv1 * zinv * (arv / av_);
-                c = -(kv[k] + tyc) * zinv2 * zinv * m.area[(size_t)n * NL + k] / av_;
-            } else {
-                a = -(kv[k - 1]) * zinv1 * zinv * (arv / av_);
-                c = -(kv[k]) * zinv2 * zinv * m.area[(size_t)n * NL + k] / av_;
-            }
-            b = -a - c + hn;
-        } else {
-            const double zinv1 = 1.0 / (sZ[k - 2] - sZ[k - 1]);
-            a = redi ? -(kv[k - 1] + tya) * zinv1 * zinv * (arv / av_) : -(kv[k - 1]) * zinv1 * zinv * (arv / av_);
-            c = 0.0;
-            b = -a + hn;
-        }
-        sa[tid] = a;
-        sb[tid] = b;
-        sc[tid] = c;
-        if (WS) {   // oce_ale_tracer.F90:1118-1129, 1158-1172, 1194-1202
-            const double *wi = d.w_i + (size_t)n * NL;
-            double v_adv = zinv * (arv / av_);
-            if (k == nzmin) {
-                b = b + wi[k - 1] * v_adv;
-            } else {
-                a = a + dmn(0.0, wi[k - 1]) * v_adv;
-                b = b + dmx(0.0, wi[k - 1]) * v_adv;
-            }
-            if (k <= nzmax - 2) {
-                v_adv = zinv * m.area[(size_t)n * NL + k] / av_;
-                b = b - dmn(0.0, wi[k]) * v_adv;
-                c = c - dmx(0.0, wi[k]) * v_adv;
-            }
-            swaA[w][tid] = a;
-            swbA[w][tid] = b;
-            swcA[w][tid] = c;
-        }
-    }
-    const int trb = blockIdx.y * tpb, tre = min(t.ntr, trb + tpb);
-    for (int t0 = trb; t0 < tre; t0 += TCH) {
-        const int nch = min(TCH, tre - t0);
-        for (int c = 0; c < nch; ++c) {
-            const int tr = t0 + c;
-            double *T = t.T + t.sN * tr;
-            double *Told = t.Told + t.sOld * tr;
-            const int abo = ldc(t.abo + tr);
-            const bool fct = ldc(t.lim + tr) == LIM_FCT;
-            const double *av = t.a_v + t.sNI * tr + (size_t)n * NL;
-            __syncthreads();
-            if (fct && k <= L) {
-                sRp[tid] = t.rp[t.sN * tr + ci];
-                sRm[tid] = t.rm[t.sN * tr + ci];
-            }
-            __syncthreads();
-            // limited vertical antidiffusive flux at interface k (oce_adv_tra_fct.F90:425-456)
-            if (k >= nzmin && k <= nzmax) {
-                const double flux = av[k - 1];
-                double v = flux;
-                if (fct && k <= nzmax - 1) {
-                    double ae = 1.0;
-                    if (k == nzmin) {
-                        if (flux >= 0.0) ae = dmn(ae, sRp[tid]);
-                        else ae = dmn(ae, sRm[tid]);
-                    } else {
-                        if (flux >= 0.0) {
-                            ae = dmn(ae, sRm[tid - 1]);
-                            ae = dmn(ae, sRp[tid]);
-                        } else {
-                            ae = dmn(ae, sRp[tid - 1]);
-                            ae = dmn(ae, sRm[tid]);
-                        }
-                    }
-                    v = ae * flux;
-                }
-                sAv[tid] = v;
-            }
-            __syncthreads();
-            double Tk = 0.0, v = 0.0, h = 0.0;
-            if (act) {
-                Tk = T[ci];
-                if (fct) v = v - Tk * hh + t.fct_lo[t.sN * tr + ci] * hn;
-                v = v + (sAv[tid] - sAv[tid + 1]) * dt / av_;
-            }
-            const double *ah = t.a_h + t.sE * tr;
-            const double rpn = (act && fct) ? sRp[tid] : 1.0, rmn = (act && fct) ? sRm[tid] : 1.0;
-            // 128 lanes (columns of 65-127 layers): edges in batches of two,
-            // the batch's loads (clamped to the column) issued together, then
-            // added in ascending edge order (at 1.3 M columns of up to 70
-            // layers and 10 tracers: 74 -> 66 ms per launch). At 64 lanes the
-            // extra registers cost more than the overlap gains (0.76 -> 0.79 ms
-            // at 127 k columns), so there the loop takes one edge at a time.
-            if constexpr (LB == 128) {
-                constexpr int KD_NG = 2;
-                const int kk = min(k, L) - 1;
-                for (int j0 = 0; j0 < E.deg; j0 += KD_NG) {
-                    double fl_[KD_NG], rpo_[KD_NG], rmo_[KD_NG];
-                    int q_[KD_NG];
-                    bool ok_[KD_NG];
-#pragma unroll
-                    for (int u = 0; u < KD_NG; ++u) {
-                        const bool real = j0 + u < E.deg;
-                        const int j = real ? j0 + u : 0;
-                        const int q = rl(E.q, j), mo = rl(E.other, j), a0 = rl(E.nu12, j), a1 = rl(E.nl12, j);
-                        ok_[u] = real && act && k >= a0 && k <= a1;
-                        q_[u] = q;
-                        fl_[u] = ah[(size_t)(q >> 1) * L + kk];
-                        if (fct) {
-                            const size_t oi = (size_t)mo * L + kk;
-                            rpo_[u] = t.rp[t.sN * tr + oi];
-                            rmo_[u] = t.rm[t.sN * tr + oi];
-                        }
-                    }
-#pragma unroll
-                    for (int u = 0; u < KD_NG; ++u) {
-                        if (!ok_[u]) continue;
-                        const int q = q_[u];
-                        double fl = fl_[u];
-                        if (fct) fl = limit_edge_flux(fl, q, rpn, rmn, rpo_[u], rmo_[u]);
-                        if (q & 1) h = h - fl * dt / av_;
-                        else h = h + fl * dt / av_;
-                    }
-                }
-            } else {
-                for (int j = 0; j < E.deg; ++j) {
-                    const int q = rl(E.q, j), mo = rl(E.other, j), a0 = rl(E.nu12, j), a1 = rl(E.nl12, j);
-                    if (!(act && k >= a0 && k <= a1)) continue;
-                    double fl = ah[(size_t)(q >> 1) * L + k - 1];
-                    if (fct) {
-                        const size_t oi = (size_t)mo * L + k - 1;
-                        fl = limit_edge_flux(fl, q, rpn, rmn, t.rp[t.sN * tr + oi], t.rm[t.sN * tr + oi]);
-                    }
-                    if (q & 1) h = h - fl * dt / av_;
-                    else h = h + fl * dt / av_;
-                }
-            }
-            double del = 0.0 + h + v;
-            // explicit diffusion in diff_tracers_ale's order (oce_ale_tracer.F90:595-626):
-            // edge fluxes of diff_part_hor_redi ascending, then the vertical parts
-            if (DX && d.hdiff) {
-                const double *hd = t.hd + t.sE * tr;
-                for (int j = 0; j < E.deg; ++j) {
-                    const int q = rl(E.q, j), a0 = rl(E.nu12, j), a1 = rl(E.nl12, j);
-                    if (!(act && k >= a0 && k <= a1)) continue;
-                    const double c = hd[(size_t)(q >> 1) * L + k - 1];
-                    const double r = (q & 1) ? 0.0 - c : 0.0 + c;
-                    del = del + r * dt / av_;
-                }
-            }
-            if (act) {
-                if (DX && !ldc(t.ivd + tr)) del = del + t.ve[t.sN * tr + ci];
-                if (DX && d.redi) del = del + t.vr[t.sN * tr + ci];
-                del = del + Tk * (hh - hn);
-                sTsA[w][c][tid] = Tk + del / hn;
-                // valuesold rotation (oce_tracer_mod.F90:94-123)
-                if (abo == 2) {
-                    Told[ci] = Tk;
-                } else {
-                    Told[2 * ci + 1] = Told[2 * ci];
-                    Told[2 * ci] = Tk;
-                }
-            }
-        }
-        __syncthreads();
-        // right-hand sides (oce_ale_tracer.F90:1206-1229, 1377-1383), all tracers of the chunk
-        for (int c = 0; c < nch; ++c) {
-            const int tr = t0 + c;
-            if (!ldc(t.ivd + tr) || !act) continue;
-            const double dz = hn;
-            const double *ts = sTsA[w][c];
-            const bool wim = WS && ldc(t.lim + tr) != LIM_FCT;
-            const double *ra = wim ? swaA[w] : sa, *rb = wim ? swbA[w] : sb, *rc = wim ? swcA[w] : sc;
-            double r;
-            if (k == nzmin) r = -(rb[tid] - dz) * ts[tid] - rc[tid] * ts[tid + 1];
-            else if (k <= nzmax - 2) r = -ra[tid] * ts[tid - 1] - (rb[tid] - dz) * ts[tid] - rc[tid] * ts[tid + 1];
-            else r = -ra[tid] * ts[tid - 1] - (rb[tid] - dz) * ts[tid];
-            if (bc_every_layer(ldc(t.id + tr), d)) r = r + bc_surface_dev(ldc(t.id + tr), dt, d, m.N2, L, n, k, ts[tid]);
-            else if (k == nzmin) r = r + bc_surface_dev(ldc(t.id + tr), dt, d, m.N2, L, n, nzmin, ts[tid]);
-            stpA[w][c][tid] = r;
-        }
-        __syncthreads();
-        // Thomas sweeps (oce_ale_tracer.F90:1406-1430): one lane of the first wave
-        // per (column, tracer) pair; the pivot chain (cp, m) is evaluated in the
-        // same loop as tp so that the two recurrences overlap
-        if (threadIdx.x < CPB * nch) {
-            const int wc = threadIdx.x / nch, c = threadIdx.x % nch;
-            const int z0 = sNz[wc][0], z1 = sNz[wc][1];
-            if (z1 - 1 >= z0 && ldc(t.ivd + t0 + c)) {
-                const bool wim = WS && ldc(t.lim + t0 + c) != LIM_FCT;
-                const double *a_ = wim ? swaA[wc] : saA[wc], *b_ = wim ? swbA[wc] : sbA[wc], *c_ = wim ? swcA[wc] : scA[wc];
-                double *tp_ = stpA[wc][c], *ts = sTsA[wc][c];
-                double *cp_ = c == 0 ? sRpA[wc] : (c == 1 ? sRmA[wc] : scpX[wc][c >= 2 ? c - 2 : 0]);
-                double cp = c_[z0 - 1] / b_[z0 - 1];
-                double tp = tp_[z0 - 1] / b_[z0 - 1];
-                cp_[z0 - 1] = cp;
-                tp_[z0 - 1] = tp;
-                for (int nz = z0 + 1; nz <= z1 - 1; ++nz) {
-                    const double an = a_[nz - 1];
-                    const double mm = b_[nz - 1] - cp * an;
-                    cp = c_[nz - 1] / mm;
-                    tp = (tp_[nz - 1] - tp * an) / mm;
-                    cp_[nz - 1] = cp;
-                    tp_[nz - 1] = tp;
-                }
-                double x = tp_[z1 - 2];
-                ts[z1 - 2] = ts[z1 - 2] + x;
-                for (int nz = z1 - 2; nz >= z0; --nz) {
-                    x = tp_[nz - 1] - cp_[nz - 1] * x;
-                    ts[nz - 1] = ts[nz - 1] + x;
-                }
-            }
-        }
-        __syncthreads();
-        if (act) {
-            for (int c = 0; c < nch; ++c) {
-                const int tr = t0 + c;
-                double v = sTsA[w][c][tid];
-                if (tr == clamp_tracer) {
-                    if (v > 45.0) v = 45.0;
-                    if (v < 3.0) v = 3.0;
-                }
-                t.T[t.sN * tr + ci] = v;
-            }
-        }
-    }
-}
-
-// ------------------------------------------------------------------------------
 // K_L: limited fluxes, flux2dtracer and T* (oce_adv_tra_fct.F90:425-497,
 // oce_adv_tra_driver.F90:494-646, oce_ale_tracer.F90:595-626); T* replaces T,
 // T^n goes to valuesold. The implicit vertical diffusion follows in K_V: inside
@@ -1335,8 +786,11 @@ __global__ void __launch_bounds__(LB) __attribute__((amdgpu_waves_per_eu(6))) kD
 // tracers (439, 151) and 1364 us at 40 thousand nodes, 70 layers, 10 tracers
 // (700, 328).
 // ------------------------------------------------------------------------------
-template <typename OFF, int NV, int GT>
-__global__ void __launch_bounds__(64) kL_node(DevMesh m, DevTracers t, double dt, int tpb)
+// DX compiles in the explicit diffusion increments (Ki, Redi, i_vert_diff off):
+// 20 thousand nodes, 47 layers, 4 tracers: K_L 157 us and K_V 92, 361 for one
+// kernel with a block per column.
+template <typename OFF, int NV, int GT, bool DX>
+__global__ void __launch_bounds__(64) kL_node(DevMesh m, DevDyn d, DevTracers t, double dt, int tpb)
 {
     Column<OFF, NV, GT> c;
     if (!load_column<true, OFF, NV, GT>(m, t, c)) return;
@@ -1449,12 +903,62 @@ __global__ void __launch_bounds__(64) kL_node(DevMesh m, DevTracers t, double dt
             }
             add(side, x, po, mo, a0, len);
         }
-        double ts[NV];
+        double ts[NV], del[NV];
 #pragma unroll
         for (int s = 0; s < NV; ++s) {
-            double del = 0.0 + h[s] + v[s];
-            del = del + Tk[s] * (hh[s] - hn[s]);
-            ts[s] = Tk[s] + del / hn[s];
+            del[s] = 0.0 + h[s] + v[s];
+        }
+        if constexpr (DX) {
+            // in diff_tracers_ale's order (oce_ale_tracer.F90:595-626): edge fluxes of diff_part_hor_redi
+            // ascending, then the vertical parts
+            auto diff = [&](int side, const double (&x)[NV], int a0, int len) __attribute__((always_inline)) {
+#pragma unroll
+                for (int s = 0; s < NV; ++s) {
+                    const double r = side ? 0.0 - x[s] : 0.0 + x[s];
+                    const double y = del[s] + r * dt / av[s];
+                    del[s] = edge_has(kb, s, a0, len) ? y : del[s];
+                }
+            };
+            if (d.hdiff) {
+                const double *hd = t.hd + t.sE * tb;
+#pragma unroll
+                for (int u0 = 0; u0 < CE; u0 += NB) {
+                    if (u0 < c.deg) {
+#pragma unroll
+                        for (int u = 0; u < NB; ++u) {
+                            if (u0 + u >= CE || u0 + u >= c.deg) break;
+                            row_load<NV>(hd, c.oe[u0 + u], fl[u]);
+                        }
+#pragma unroll
+                        for (int u = 0; u < NB; ++u)
+                            if (u0 + u < CE && u0 + u < c.deg) diff(c.side[u0 + u], fl[u], c.a0[u0 + u], c.len[u0 + u]);
+                    }
+                }
+                for (int u = CE; u < c.deg; ++u) {
+                    OFF on, oe;
+                    int a0, len, side;
+                    edge_offsets<OFF, NV, GT>(m, t, c, u, on, oe, a0, len, side);
+                    double x[NV];
+                    row_load<NV>(hd, oe, x);
+                    diff(side, x, a0, len);
+                }
+            }
+            double x[NV];
+            if (!t.ivd[tb + c.g]) {
+                row_load<NV>(t.ve + t.sN * tb, c.own, x);
+#pragma unroll
+                for (int s = 0; s < NV; ++s) del[s] = del[s] + x[s];
+            }
+            if (d.redi) {
+                row_load<NV>(t.vr + t.sN * tb, c.own, x);
+#pragma unroll
+                for (int s = 0; s < NV; ++s) del[s] = del[s] + x[s];
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < NV; ++s) {
+            del[s] = del[s] + Tk[s] * (hh[s] - hn[s]);
+            ts[s] = Tk[s] + del[s] / hn[s];
         }
         row_store<NV>(T, c.own, ts, c.wet);
         // valuesold rotation (oce_tracer_mod.F90:94-123)
@@ -1483,10 +987,18 @@ __global__ void __launch_bounds__(64) kL_node(DevMesh m, DevTracers t, double dt
 // lanes over the levels and leaves them in LDS; one wave sweeps with one lane
 // per row, and the waves add the result to T*. LDS rows have an odd length, so
 // that the lanes of the sweep, each on its own row, use different banks.
+// XF bit 0 (use_wsplit): the non-FCT tracers' rows also take the implicit part
+// w_i of the split W, a second set of rows; bit 1: the K33 terms of Redi and
+// tracers with i_vert_diff off, which are left as they are. KV_LO instead solves
+// the implicit upwind advection with w_i on the LO solution of the FCT tracers
+// (adv_tra_vert_impl, oce_adv_tra_ver.F90:90-240), between K_B and K_C.
+#define KV_WS 1
+#define KV_DX 2
+#define KV_LO 4
 #define KV_NW 8   // waves of a block
 #define KV_TP 2   // tracers whose rows are loaded together
-template <int NV>
-__global__ void __launch_bounds__(64 * KV_NW) __attribute__((amdgpu_waves_per_eu(8)))
+template <int NV, int XF>
+__global__ void __launch_bounds__(64 * KV_NW) __attribute__((amdgpu_waves_per_eu(XF == 0 ? 8 : 4)))
 kV_cols(DevMesh m, DevDyn d, DevTracers t, double dt, int clamp_tracer, int NC, int TB)
 {
     extern __shared__ double lds[];
@@ -1496,7 +1008,14 @@ kV_cols(DevMesh m, DevDyn d, DevTracers t, double dt, int clamp_tracer, int NC, 
     if (col0 >= m.N2) return;
     const int ncol = min(NC, m.N2 - col0);
     const int trb = blockIdx.y * TB, ntb = min(TB, t.ntr - trb);
-    double *sa = lds, *sb = sa + (size_t)NC * RS, *sc = sb + (size_t)NC * RS, *sr = sc + (size_t)NC * RS;
+    constexpr bool WS = (XF & KV_WS) != 0, LO = (XF & KV_LO) != 0;
+    const bool redi = (XF & KV_DX) != 0 && d.redi != 0;
+    const size_t set = 3 * (size_t)NC * RS;   // the rows' second set follows the first
+    double *sa = lds, *sb = sa + (size_t)NC * RS, *sc = sb + (size_t)NC * RS, *sr = lds + (WS ? 2 : 1) * set;
+    double *F = LO ? t.fct_lo : t.T;
+    // does the solve take tracer tr, and with the second set?
+    auto solved = [&](int tr) { return LO ? ldc(t.lim + tr) == LIM_FCT : (XF == 0 || ldc(t.ivd + tr) != 0); };
+    auto second = [&](int tr) { return WS && ldc(t.lim + tr) != LIM_FCT; };
     // the block's columns, one per lane
     const int nl_ = m.node_ord[col0 + min(lane, ncol - 1)];
     const int z0l = m.ulevn[nl_], z1l = m.nlevn[nl_];
@@ -1506,26 +1025,54 @@ kV_cols(DevMesh m, DevDyn d, DevTracers t, double dt, int clamp_tracer, int NC, 
         const int n = rl(nl_, c), nzmin = rl(z0l, c), nzmax = rl(z1l, c);
         const size_t nL = (size_t)n * L, nNL = (size_t)n * NL;
         double hn[NV], av[NV], zk[NV], kv[NV], ar[NV], zu[NV], zd[NV], kvd[NV], ard[NV], a_[NV], c_[NV], bd_[NV];
-        double ts[KV_TP][NV];
+        double ts[KV_TP][NV], wi[NV], wid[NV], wa[WS ? NV : 1], wb[WS ? NV : 1], wc[WS ? NV : 1], k33[NV], k33u[NV];
 #pragma unroll
-        for (int s = 0; s < NV; ++s) hn[s] = av[s] = zk[s] = kv[s] = ar[s] = 1.0;
+        for (int s = 0; s < NV; ++s) {
+            hn[s] = av[s] = zk[s] = kv[s] = ar[s] = 1.0;
+            wi[s] = k33[s] = 0.0;
+#pragma unroll
+            for (int j = 0; j < KV_TP; ++j) ts[j][s] = 0.0;
+        }
         const bool layer = kb <= nzmax - 1;
         if (kb <= nzmax) {   // interfaces to nzmax
-            row_load<NV>(d.Kv + nNL, off, kv);
+            if (!LO) row_load<NV>(d.Kv + nNL, off, kv);
+            if (WS || LO) row_load<NV>(d.w_i + nNL, off, wi);
             row_load<NV>(m.area + nNL, off, ar);
             row_load<NV>(m.areasvol + nNL, off, av);
         }
         if (layer) {
             row_load<NV>(m.hnode_new + nL, off, hn);
-            row_load<NV>(m.zn_vd + nL, off, zk);
+            if (!LO) row_load<NV>(m.zn_vd + nL, off, zk);
 #pragma unroll
             for (int j = 0; j < KV_TP; ++j)
-                if (j < ntb) row_load<NV>(t.T + t.sN * (trb + j) + nL, off, ts[j]);
+                if (j < ntb) row_load<NV>(F + t.sN * (trb + j) + nL, off, ts[j]);
         }
         col_up<NV>(zk, zu);
         col_down<NV>(zk, zd);
         col_down<NV>(kv, kvd);
         col_down<NV>(ar, ard);
+        col_down<NV>(wi, wid);
+        if (redi) {   // K33 = Kv + Ki S3^2 at the interface below a layer (oce_ale_tracer.F90:1105-1108, 1138-1144, 1181-1184)
+            double s3[NV], ki[NV], zb[NV], s3d[NV], kid[NV], zbd[NV];
+#pragma unroll
+            for (int s = 0; s < NV; ++s) s3[s] = ki[s] = zb[s] = 0.0;
+            if (kb <= nzmax) row_load<NV>(m.zbn_vd + nNL, off, zb);
+            if (layer) {
+                row_load<NV>(d.Ki + nL, off, ki);
+#pragma unroll
+                for (int s = 0; s < NV; ++s) s3[s] = d.slope[3 * (nL + kb - 1 + (kb + s <= L ? s : 0)) + 2];
+            }
+            col_down<NV>(s3, s3d);
+            col_down<NV>(ki, kid);
+            col_down<NV>(zb, zbd);
+#pragma unroll
+            for (int s = 0; s < NV; ++s) {
+                const double zinv2 = 1.0 / (zk[s] - zd[s]);
+                k33[s] = (zbd[s] - zd[s]) * zinv2 * (s3[s] * s3[s]) * ki[s] +
+                         (zk[s] - zbd[s]) * zinv2 * (s3d[s] * s3d[s]) * kid[s];
+            }
+        }
+        col_up<NV>(k33, k33u);
         // tridiagonal coefficients (oce_ale_tracer.F90:1098-1175)
 #pragma unroll
         for (int s = 0; s < NV; ++s) {
@@ -1534,17 +1081,52 @@ kV_cols(DevMesh m, DevDyn d, DevTracers t, double dt, int clamp_tracer, int NC, 
             if (k < nzmin || k > nzmax - 1) continue;
             const double zinv = 1.0 * dt;
             double a = 0.0, b, cc = 0.0;
-            if (k > nzmin) {
-                const double zinv1 = 1.0 / (zu[s] - zk[s]);
-                a = -(kv[s]) * zinv1 * zinv * (ar[s] / av[s]);
+            if constexpr (LO) {
+                double v_adv = zinv * ar[s] / av[s];
+                if (k == nzmin) {
+                    b = hn[s] + wi[s] * v_adv;
+                } else {
+                    a = dmn(0.0, wi[s]) * v_adv;
+                    b = hn[s] + dmx(0.0, wi[s]) * v_adv;
+                }
+                if (k <= nzmax - 2) {
+                    v_adv = zinv * ard[s] / av[s];
+                    b = b - dmn(0.0, wid[s]) * v_adv;
+                    cc = -dmx(0.0, wid[s]) * v_adv;
+                }
+            } else {
+                if (k > nzmin) {
+                    const double zinv1 = 1.0 / (zu[s] - zk[s]);
+                    a = -(redi ? kv[s] + k33u[s] : kv[s]) * zinv1 * zinv * (ar[s] / av[s]);
+                }
+                if (k <= nzmax - 2) {
+                    const double zinv2 = 1.0 / (zk[s] - zd[s]);
+                    cc = -(redi ? kvd[s] + k33[s] : kvd[s]) * zinv2 * zinv * ard[s] / av[s];
+                }
+                if (k == nzmin) b = -cc + hn[s];
+                else if (k <= nzmax - 2) b = -a - cc + hn[s];
+                else b = -a + hn[s];
             }
-            if (k <= nzmax - 2) {
-                const double zinv2 = 1.0 / (zk[s] - zd[s]);
-                cc = -(kvd[s]) * zinv2 * zinv * ard[s] / av[s];
+            if constexpr (WS) {   // oce_ale_tracer.F90:1118-1129, 1158-1172, 1194-1202
+                double v_adv = zinv * (ar[s] / av[s]), a2 = a, b2 = b, c2 = cc;
+                if (k == nzmin) {
+                    b2 = b2 + wi[s] * v_adv;
+                } else {
+                    a2 = a2 + dmn(0.0, wi[s]) * v_adv;
+                    b2 = b2 + dmx(0.0, wi[s]) * v_adv;
+                }
+                if (k <= nzmax - 2) {
+                    v_adv = zinv * ard[s] / av[s];
+                    b2 = b2 - dmn(0.0, wid[s]) * v_adv;
+                    c2 = c2 - dmx(0.0, wid[s]) * v_adv;
+                }
+                sa[set + c * RS + k - 1] = a2;
+                sb[set + c * RS + k - 1] = b2;
+                sc[set + c * RS + k - 1] = c2;
+                wa[s] = a2;
+                wb[s] = b2 - hn[s];
+                wc[s] = c2;
             }
-            if (k == nzmin) b = -cc + hn[s];
-            else if (k <= nzmax - 2) b = -a - cc + hn[s];
-            else b = -a + hn[s];
             sa[c * RS + k - 1] = a;
             sb[c * RS + k - 1] = b;
             sc[c * RS + k - 1] = cc;
@@ -1557,12 +1139,14 @@ kV_cols(DevMesh m, DevDyn d, DevTracers t, double dt, int clamp_tracer, int NC, 
             if (j0 > 0 && layer) {
 #pragma unroll
                 for (int j = 0; j < KV_TP; ++j)
-                    if (j0 + j < ntb) row_load<NV>(t.T + t.sN * (trb + j0 + j) + nL, off, ts[j]);
+                    if (j0 + j < ntb) row_load<NV>(F + t.sN * (trb + j0 + j) + nL, off, ts[j]);
             }
 #pragma unroll
             for (int j = 0; j < KV_TP; ++j) {
                 if (j0 + j >= ntb) break;
                 const int id = ldc(t.id + trb + j0 + j);
+                if (!solved(trb + j0 + j)) continue;
+                const bool w2 = second(trb + j0 + j);
                 double tu[NV], td[NV];
                 col_up<NV>(ts[j], tu);
                 col_down<NV>(ts[j], td);
@@ -1570,11 +1154,14 @@ kV_cols(DevMesh m, DevDyn d, DevTracers t, double dt, int clamp_tracer, int NC, 
                 for (int s = 0; s < NV; ++s) {
                     const int k = kb + s;
                     if (k < nzmin || k > nzmax - 1) continue;
+                    const double ra = WS && w2 ? wa[WS ? s : 0] : a_[s], rb = WS && w2 ? wb[WS ? s : 0] : bd_[s],
+                                 rc = WS && w2 ? wc[WS ? s : 0] : c_[s];
                     double r;
-                    if (k == nzmin) r = -bd_[s] * ts[j][s] - c_[s] * td[s];
-                    else if (k <= nzmax - 2) r = -a_[s] * tu[s] - bd_[s] * ts[j][s] - c_[s] * td[s];
-                    else r = -a_[s] * tu[s] - bd_[s] * ts[j][s];
-                    if (bc_every_layer(id, d)) r = r + bc_surface_dev(id, dt, d, m.N2, L, n, k, ts[j][s]);
+                    if (k == nzmin) r = -rb * ts[j][s] - rc * td[s];
+                    else if (k <= nzmax - 2) r = -ra * tu[s] - rb * ts[j][s] - rc * td[s];
+                    else r = -ra * tu[s] - rb * ts[j][s];
+                    if (LO) {
+                    } else if (bc_every_layer(id, d)) r = r + bc_surface_dev(id, dt, d, m.N2, L, n, k, ts[j][s]);
                     else if (k == nzmin) r = r + bc_surface_dev(id, dt, d, m.N2, L, n, nzmin, ts[j][s]);
                     sr[(c * TB + j0 + j) * RS + k - 1] = r;
                 }
@@ -1587,8 +1174,9 @@ kV_cols(DevMesh m, DevDyn d, DevTracers t, double dt, int clamp_tracer, int NC, 
     if (w == 0 && lane < ncol * ntb) {
         const int c = lane / ntb, j = lane % ntb;
         const int z0 = __shfl(z0l, c), z1 = __shfl(z1l, c);
-        const double *pa = sa + c * RS - 1, *pb = sb + c * RS - 1;
-        double *pc = sc + c * RS - 1, *pr = sr + (c * TB + j) * RS - 1;
+        const size_t o = WS && t.lim[trb + j] != LIM_FCT ? set : 0;
+        const double *pa = sa + o + c * RS - 1, *pb = sb + o + c * RS - 1;
+        double *pc = sc + o + c * RS - 1, *pr = sr + (c * TB + j) * RS - 1;
         double cp = pc[z0] / pb[z0], tp = pr[z0] / pb[z0];
         pc[z0] = cp;
         pr[z0] = tp;
@@ -1627,20 +1215,22 @@ kV_cols(DevMesh m, DevDyn d, DevTracers t, double dt, int clamp_tracer, int NC, 
             double v[2 * KV_TP][NV];
 #pragma unroll
             for (int j = 0; j < 2 * KV_TP; ++j)
-                if (j0 + j < ntb && any) row_load<NV>(t.T + t.sN * (trb + j0 + j) + nL, off, v[j]);
+                if (j0 + j < ntb && any) row_load<NV>(F + t.sN * (trb + j0 + j) + nL, off, v[j]);
 #pragma unroll
             for (int j = 0; j < 2 * KV_TP; ++j) {
                 if (j0 + j >= ntb) break;
                 const int tr = trb + j0 + j;
+                const bool add = solved(tr);
+                if (LO && !add) continue;
 #pragma unroll
                 for (int s = 0; s < NV; ++s) {
-                    if (on[s]) v[j][s] = v[j][s] + sr[(c * TB + j0 + j) * RS + kb + s - 1];
-                    if (tr == clamp_tracer) {
+                    if (on[s] && add) v[j][s] = v[j][s] + sr[(c * TB + j0 + j) * RS + kb + s - 1];
+                    if (!LO && tr == clamp_tracer) {
                         if (v[j][s] > 45.0) v[j][s] = 45.0;
                         if (v[j][s] < 3.0) v[j][s] = 3.0;
                     }
                 }
-                row_store<NV>(t.T + t.sN * tr + nL, off, v[j], on);
+                row_store<NV>(F + t.sN * tr + nL, off, v[j], on);
             }
         }
     }
@@ -1686,10 +1276,9 @@ int fgpu_compute_zn(fgpu_context *c)
     FGPU_HIP(hipStreamSynchronize(c->stream));
     return FGPU_OK;
 }
-// Extra terms compiled into K_D: bit 0 the W split (w_i rows of the implicit
-// diffusion for non-FCT tracers), bit 1 explicit diffusion increments (Ki,
-// Redi, i_vert_diff off) and the Redi K33 rows. Only the plain step (0) has
-// the one-wave-per-column variants.
+// Extra terms compiled into K_L and K_V: bit 0 the W split (w_i rows of the
+// implicit diffusion for non-FCT tracers), bit 1 explicit diffusion increments
+// (Ki, Redi, i_vert_diff off) and the Redi K33 rows.
 int fgpu_kd_extras(const fgpu_context *c)
 {
     bool dx = c->d.hdiff || c->d.redi;
@@ -1761,10 +1350,22 @@ static ColLanes col_lanes(const fgpu_context *c, int tpb)
         else hipLaunchKernelGGL((kern<unsigned, NV, GT>), grid, dim3(64), 0, c->stream, __VA_ARGS__);                \
     } while (0)
 
+#define COL_LAUNCH_X(kern, NV, GT, X, grid, ...)                                                                     \
+    do {                                                                                                             \
+        if (wide) hipLaunchKernelGGL((kern<size_t, NV, GT, X>), grid, dim3(64), 0, c->stream, __VA_ARGS__);          \
+        else hipLaunchKernelGGL((kern<unsigned, NV, GT, X>), grid, dim3(64), 0, c->stream, __VA_ARGS__);             \
+    } while (0)
+#define COL_LAUNCH_D(kern, NV, GT, dx, grid, ...)                                                                    \
+    do {                                                                                                             \
+        if (dx) COL_LAUNCH_X(kern, NV, GT, true, grid, __VA_ARGS__);                                                 \
+        else COL_LAUNCH_X(kern, NV, GT, false, grid, __VA_ARGS__);                                                   \
+    } while (0)
+
+template <int XF>
 static void launch_kv(fgpu_context *c, double dt, int clamp)
 {
     const DevMesh &m = c->m;
-    const int nt = c->t.ntr, row = 8 * (m.L | 1);
+    const int nt = c->t.ntr, row = 8 * (m.L | 1), coef = XF & KV_WS ? 6 : 3;
     // tracers in equal groups of at most ten: a column's pivots are formed once
     // per group (70 layers, 10 tracers: 328 us in one group, 682 us by fours)
     const int groups = (nt + 9) / 10, TB = (nt + groups - 1) / groups;
@@ -1772,27 +1373,12 @@ static void launch_kv(fgpu_context *c, double dt, int clamp)
     // 47 layers, 2 tracers, 126,858 nodes: 159 us, 214 us at 65,536 bytes, 191
     // us at 26,000), and 1,024 blocks on a small mesh, where the blocks' serial
     // sweeps have to run side by side
-    int NC = std::min(64 / TB, 40000 / (row * (3 + TB)));
+    int NC = std::min(64 / TB, 40000 / (row * (coef + TB)));
     NC = std::max(1, std::min(NC, (int)((size_t)m.N2 * groups / 1024)));
-    const size_t lds = (size_t)row * (3 + TB) * NC;
+    const size_t lds = (size_t)row * (coef + TB) * NC;
     const dim3 g(xcd_grid((m.N2 + NC - 1) / NC), (unsigned)groups), b(64 * KV_NW);
-    if (m.NL <= 64) hipLaunchKernelGGL(kV_cols<1>, g, b, lds, c->stream, m, c->d, c->t, dt, clamp, NC, TB);
-    else hipLaunchKernelGGL(kV_cols<2>, g, b, lds, c->stream, m, c->d, c->t, dt, clamp, NC, TB);
-}
-
-// one block of LB lanes per node column: K_B and K_D of the steps with extra schemes or terms
-template <int LB>
-static void launch_kb_node(fgpu_context *c, const dim3 &g, double dt, int tpb)
-{
-    if (c->d.wsplit) hipLaunchKernelGGL((kB_node<LB, true>), g, dim3(LB), 0, c->stream, c->m, c->d, c->t, dt, tpb);
-    else hipLaunchKernelGGL((kB_node<LB, false>), g, dim3(LB), 0, c->stream, c->m, c->d, c->t, dt, tpb);
-}
-template <int LB>
-static void launch_kd_node(fgpu_context *c, const dim3 &g, int xf, double dt, int clamp, int tpb)
-{
-    if (xf == 1) hipLaunchKernelGGL((kD_node<LB, 1>), g, dim3(LB), 0, c->stream, c->m, c->d, c->t, dt, clamp, tpb);
-    else if (xf == 2) hipLaunchKernelGGL((kD_node<LB, 2>), g, dim3(LB), 0, c->stream, c->m, c->d, c->t, dt, clamp, tpb);
-    else hipLaunchKernelGGL((kD_node<LB, 3>), g, dim3(LB), 0, c->stream, c->m, c->d, c->t, dt, clamp, tpb);
+    if (m.NL <= 64) hipLaunchKernelGGL((kV_cols<1, XF>), g, b, lds, c->stream, m, c->d, c->t, dt, clamp, NC, TB);
+    else hipLaunchKernelGGL((kV_cols<2, XF>), g, b, lds, c->stream, m, c->d, c->t, dt, clamp, NC, TB);
 }
 
 int fgpu_enqueue_fused_step(fgpu_context *c, double dt)
@@ -1828,12 +1414,16 @@ int fgpu_enqueue_fused_step(fgpu_context *c, double dt)
     }
     {
         ProfScope ps(c, "kB_node");
-        if (extra && narrow) launch_kb_node<64>(c, nodes, dt, tpb);
-        else if (extra) launch_kb_node<128>(c, nodes, dt, tpb);
-        else if (pair && m.NL > 64 && m.NL <= 96) COL_LAUNCH(kB_cols, 3, 2, nodes, m, c->d, c->t, dt, tpb);
-        else if (!narrow) COL_LAUNCH(kB_cols, 2, 1, nodes, m, c->d, c->t, dt, tpb);
-        else if (slim && pair) COL_LAUNCH(kB_cols, 1, 2, nodes, m, c->d, c->t, dt, tpb);
-        else COL_LAUNCH(kB_cols, 1, 1, nodes, m, c->d, c->t, dt, tpb);
+        if (extra && narrow) COL_LAUNCH_X(kB_cols, 1, 1, true, nodes, m, c->d, c->t, dt, tpb);
+        else if (extra) COL_LAUNCH_X(kB_cols, 2, 1, true, nodes, m, c->d, c->t, dt, tpb);
+        else if (pair && m.NL > 64 && m.NL <= 96) COL_LAUNCH_X(kB_cols, 3, 2, false, nodes, m, c->d, c->t, dt, tpb);
+        else if (!narrow) COL_LAUNCH_X(kB_cols, 2, 1, false, nodes, m, c->d, c->t, dt, tpb);
+        else if (slim && pair) COL_LAUNCH_X(kB_cols, 1, 2, false, nodes, m, c->d, c->t, dt, tpb);
+        else COL_LAUNCH_X(kB_cols, 1, 1, false, nodes, m, c->d, c->t, dt, tpb);
+    }
+    if (c->d.wsplit) {
+        ProfScope ps(c, "kV_lo");
+        launch_kv<KV_LO>(c, dt, -1);
     }
     {
         ProfScope ps(c, "kC_node");
@@ -1842,21 +1432,21 @@ int fgpu_enqueue_fused_step(fgpu_context *c, double dt)
         else if (many) COL_LAUNCH(kC_cols, 2, 2, nodes, m, c->t, dt, tpb);
         else COL_LAUNCH(kC_cols, 1, 1, nodes, m, c->t, dt, tpb);
     }
-    if (xf == 0) {
-        {
-            ProfScope ps(c, "kL_node");
-            if (pair && m.NL > 64 && m.NL <= 96) COL_LAUNCH(kL_node, 3, 2, nodes, m, c->t, dt, tpb);
-            else if (!narrow) COL_LAUNCH(kL_node, 2, 1, nodes, m, c->t, dt, tpb);
-            else if (slim && pair) COL_LAUNCH(kL_node, 1, 2, nodes, m, c->t, dt, tpb);
-            else if (pair) COL_LAUNCH(kL_node, 2, 2, nodes, m, c->t, dt, tpb);
-            else COL_LAUNCH(kL_node, 1, 1, nodes, m, c->t, dt, tpb);
-        }
+    {
+        ProfScope ps(c, "kL_node");
+        const bool dx = (xf & 2) != 0;
+        if (pair && m.NL > 64 && m.NL <= 96) COL_LAUNCH_D(kL_node, 3, 2, dx, nodes, m, c->d, c->t, dt, tpb);
+        else if (!narrow) COL_LAUNCH_D(kL_node, 2, 1, dx, nodes, m, c->d, c->t, dt, tpb);
+        else if (slim && pair) COL_LAUNCH_D(kL_node, 1, 2, dx, nodes, m, c->d, c->t, dt, tpb);
+        else if (pair) COL_LAUNCH_D(kL_node, 2, 2, dx, nodes, m, c->d, c->t, dt, tpb);
+        else COL_LAUNCH_D(kL_node, 1, 1, dx, nodes, m, c->d, c->t, dt, tpb);
+    }
+    {
         ProfScope ps(c, "kV_cols");
-        launch_kv(c, dt, clamp);
-    } else {
-        ProfScope ps(c, "kD_node");
-        if (narrow) launch_kd_node<64>(c, nodes, xf, dt, clamp, tpb);
-        else launch_kd_node<128>(c, nodes, xf, dt, clamp, tpb);
+        if (xf == 0) launch_kv<0>(c, dt, clamp);
+        else if (xf == 1) launch_kv<KV_WS>(c, dt, clamp);
+        else if (xf == 2) launch_kv<KV_DX>(c, dt, clamp);
+        else launch_kv<KV_WS | KV_DX>(c, dt, clamp);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fgpu_fail(FGPU_ERR_HIP, std::string("fused step launch: ") + hipGetErrorString(e));

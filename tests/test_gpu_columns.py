@@ -124,3 +124,26 @@ def test_explicit_diffusion_waves(monkeypatch, path, layers, ntr, redi):
         monkeypatch.setenv("FGPU_STEP", "staged")
     print(f"[gpu] explicit diffusion, {layers} layers, {ntr} tracers, {path}", flush=True)
     _check(mesh, st, schemes)
+
+
+EXTRAS = [dict(ver="PPM"), dict(ver="CDIFF", i_vert_diff=False), dict(ver="PPM", lim="NON"), dict(ver="CDIFF", hor="MUSCL", lim="NON"),
+          dict(), dict(ver="UPW1", hor="UPW1", lim="NON")]
+
+
+@pytest.mark.parametrize("split,diffusion", [(True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("layers,ntr", [(4, 6), (31, 4), (32, 6), (63, 6), (64, 3), (95, 1), (127, 6)])
+def test_extra_schemes_and_terms(layers, ntr, split, diffusion):
+    """CDIFF and PPM tracers, the split vertical velocity (implicit upwind step
+    of the low-order solution, its rows in the vertical solve), Ki with Redi and
+    tracers without implicit vertical diffusion."""
+    mesh, st = _case(layers, ntr)
+    rng = np.random.default_rng(layers)
+    schemes = EXTRAS[:ntr]
+    if split:
+        w_e = st.w * rng.uniform(0.2, 1.0, st.w.shape)
+        st = dataclasses.replace(st, w_e=w_e, w_i=st.w - w_e, use_wsplit=True)
+    if diffusion:
+        st = dataclasses.replace(st, Ki=rng.uniform(20.0, 400.0, (mesh.nod2D, layers)), redi=True,
+                                 slope_tapered=rng.normal(0.0, 0.01, (mesh.nod2D, layers, 3)))
+    print(f"[gpu] extra schemes, {layers} layers, {ntr} tracers, split {split}, diffusion {diffusion}", flush=True)
+    _check(mesh, st, schemes)
