@@ -19,6 +19,7 @@
 #include "fgpu_internal.h"
 
 #define SBLK 256
+#define CG_BLOCKS 512   // blocks of the iteration kernels: two per CU, the partial sums two per thread
 
 // Rows of a block. With a multiple of eight blocks, the blocks b with
 // b % 8 == x (one XCD) take the x-th contiguous eighth of the rows, so that the
@@ -139,10 +140,13 @@ struct CGArgs {
     // single-reduction iteration: per row the record {r, w} {s_prev, D^-1}
     // (two double2), one array per iteration parity
     double2 *rec0, *rec1;
+    int *ecol;      // its matrix: the first EW entries of the rows, entry e of row i at
+    double *eval;   // (i / 64) * 64 * EW + 64 e + i % 64, written by k_cg1_init_r
     double *part;   // 8 slots x nb: [0] b.b / p.q  [1] r.z  [2] r.r; single-reduction: [2p..2p+1], [4+p], [6]
     CGState *st;
 };
 
+#define EW 8    // row entries of the single-reduction iteration's layout; the rest of a row is read from the CSR arrays
 #define SGB 8   // row entries whose column loads and gathers are in flight together
 
 // sum over row r of v[p] * x[colind[p]] in entry order; the loads of SGB
@@ -182,17 +186,45 @@ __device__ __forceinline__ double strided_sum(const double *v, int n)
     return a;
 }
 
-// block reduction of up to three values: butterfly within each wave, then the
-// four wave sums in wave order; the result (lane 0's sums) is valid in every
+// butterfly sum over the wave (lanes 32, 16, 8, 4, 2 and 1 apart), the same in
+// every lane. By lane swaps and DPP moves, which take a register's latency where
+// a shuffle through LDS takes some 100 cycles: 0.4 us of a solver kernel's 8.
+// After the first three steps values repeat every eight lanes, so a rotation by
+// four serves as the exchange.
+template <int CTRL>
+__device__ __forceinline__ double dpp_moved(double x)
+{
+    const long long b = __double_as_longlong(x);
+    const int l = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), CTRL, 0xf, 0xf, false);
+    const int h = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)h << 32) | (unsigned int)l);
+}
+__device__ __forceinline__ double wave_sum(double x)
+{
+    long long b = __double_as_longlong(x);
+    auto l = __builtin_amdgcn_permlane32_swap((unsigned)b, (unsigned)b, false, false);
+    auto h = __builtin_amdgcn_permlane32_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+    x = __longlong_as_double(((long long)h[0] << 32) | l[0]) + __longlong_as_double(((long long)h[1] << 32) | l[1]);
+    b = __double_as_longlong(x);
+    l = __builtin_amdgcn_permlane16_swap((unsigned)b, (unsigned)b, false, false);
+    h = __builtin_amdgcn_permlane16_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+    x = __longlong_as_double(((long long)h[0] << 32) | l[0]) + __longlong_as_double(((long long)h[1] << 32) | l[1]);
+    x += dpp_moved<0x128>(x);   // row_ror:8
+    x += dpp_moved<0x124>(x);   // row_ror:4
+    x += dpp_moved<0x4e>(x);    // quad_perm 2,3,0,1
+    x += dpp_moved<0xb1>(x);    // quad_perm 1,0,3,2
+    return x;
+}
+
+// block reduction of up to three values: within each wave, then the
+// wave sums in wave order; the result is valid in every
 // thread and identical in every block for identical inputs
 __device__ void block_sum3(double &a, double &b, double &c)
 {
     __shared__ double sh[3][SBLK / 64];
-    for (int off = 32; off > 0; off >>= 1) {
-        a += __shfl_xor(a, off);
-        b += __shfl_xor(b, off);
-        c += __shfl_xor(c, off);
-    }
+    a = wave_sum(a);
+    b = wave_sum(b);
+    c = wave_sum(c);
     const int w = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0) { sh[0][w] = a; sh[1][w] = b; sh[2][w] = c; }
     __syncthreads();
@@ -402,13 +434,37 @@ __device__ __forceinline__ double cg1_slot(const CGArgs &A, int slot)
 }
 
 // r0 = b - A x0 into the parity-0 records {r0, w0 (set next)} {s_-1 = 0, D^-1};
-// partials b.b (slot 6) and r.r (slot 4); state reset
+// partials b.b (slot 6) and r.r (slot 4); the iterations' matrix layout; state reset
 __global__ void __launch_bounds__(SBLK) k_cg1_init_r(CGArgs A, double soltol, int maxiter)
 {
     double bb = 0.0, rr = 0.0, dum = 0.0;
     for (CGRows R = cg_rows(A.n, A.nb); R.row < R.end; R.row += R.step) {
         const int row = R.row;
-        const double r = A.rhs[row] - row_dot(A.rowptr, A.colind, A.val, A.x, row);
+        const int p0 = A.rowptr[row], p1 = A.rowptr[row + 1];
+        const size_t eb = (size_t)(row / 64) * (64 * EW) + row % 64;
+        double s = 0.0;
+        for (int pb = p0; pb < p1; pb += SGB) {   // row_dot's order
+            double xv[SGB], vv[SGB];
+            int jj[SGB];
+#pragma unroll
+            for (int u = 0; u < SGB; ++u) {
+                const int p = pb + u < p1 ? pb + u : p0;
+                vv[u] = A.val[p];
+                jj[u] = A.colind[p];
+                xv[u] = A.x[jj[u]];
+            }
+            if (pb == p0) {   // missing entries repeat the diagonal's column
+#pragma unroll
+                for (int u = 0; u < EW; ++u) {
+                    A.ecol[eb + 64 * u] = jj[u];
+                    A.eval[eb + 64 * u] = vv[u];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < SGB; ++u)
+                if (pb + u < p1) s = s + vv[u] * xv[u];
+        }
+        const double r = A.rhs[row] - s;
         A.rec0[2 * row] = make_double2(r, 0.0);
         A.rec0[2 * row + 1] = make_double2(0.0, A.dinv[row]);
         bb += A.rhs[row] * A.rhs[row];
@@ -470,11 +526,53 @@ __global__ void __launch_bounds__(SBLK) k_cg1_init_w(CGArgs A)
 // from an even one), and i and the previous scalars are read from the slots of
 // that parity, so a block dispatched after others have finished still reads
 // this iteration's values.
+//
+// Bound by latency where a thread has one row (126,858 rows) and by the loads'
+// bytes beyond. A row's loads do not depend on this iteration's scalars: the
+// first row's are issued before the partial sums are read. Entry e of 64
+// consecutive rows is contiguous (EW entries; the diagonal comes first and
+// needs no gather), where a CSR row per thread spreads one entry of a wave over
+// 28 cache lines. 126,858 rows: 11.0 -> 8.0 us an iteration; 400,000 rows: 22.5
+// -> 17.1 (4.5 TB/s on the 192 bytes a row takes once).
+struct CG1Row {
+    double2 o0, o1;        // {r, w}, {s_prev, D^-1}
+    double p, x, v[EW];
+    double2 a[EW], b[EW];  // the neighbours' records, [0] unused
+    int q0, q1;
+};
+__device__ __forceinline__ void cg1_load(const CGArgs &A, const double2 *rc, int row, CG1Row &q)
+{
+    const size_t eb = (size_t)(row / 64) * (64 * EW) + row % 64;
+    int j[EW];
+#pragma unroll
+    for (int u = 1; u < EW; ++u) j[u] = A.ecol[eb + 64 * u];
+    q.q0 = A.rowptr[row];
+    q.q1 = A.rowptr[row + 1];
+    q.o0 = rc[2 * row];
+    q.o1 = rc[2 * row + 1];
+#pragma unroll
+    for (int u = 0; u < EW; ++u) q.v[u] = A.eval[eb + 64 * u];
+    q.p = A.p0[row];
+    q.x = A.x[row];
+#pragma unroll
+    for (int u = 1; u < EW; ++u) {
+        q.a[u] = rc[2 * j[u]];
+        q.b[u] = rc[2 * j[u] + 1];
+    }
+}
+
 __global__ void __launch_bounds__(SBLK) k_cg1(CGArgs A, int par)
 {
     CGState *st = A.st;
-    if (st->done) return;
-    const int it = st->itp[par];
+    const double2 *rc = par ? A.rec1 : A.rec0;
+    double2 *rn = par ? A.rec0 : A.rec1;
+    const CGRows R = cg_rows(A.n, A.nb);
+    CG1Row q;
+    if (R.row < R.end) cg1_load(A, rc, R.row, q);
+    // the state's slots that this launch reads, in one go with the loads
+    const int done = st->done, it = st->itp[par], cap = st->maxiter;
+    const double gprev = st->s_oldp[2 * par], aprev = st->s_oldp[2 * par + 1], rtol_ = st->rtol, soltol = st->soltol;
+    if (done) return;
     double gam = strided_sum(A.part + (size_t)(2 * par) * A.nb, A.nb);
     double del = strided_sum(A.part + (size_t)(2 * par + 1) * A.nb, A.nb);
     double rr = strided_sum(A.part + (size_t)(4 + par) * A.nb, A.nb);
@@ -482,24 +580,23 @@ __global__ void __launch_bounds__(SBLK) k_cg1(CGArgs A, int par)
     const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
     double rtol;
     if (it == 0) {
-        rtol = st->soltol * sqrt(cg1_slot(A, 6) / (double)A.n);
+        rtol = soltol * sqrt(cg1_slot(A, 6) / (double)A.n);
         if (lead) st->rtol = rtol;
     } else {
-        rtol = st->rtol;
+        rtol = rtol_;
     }
     if (lead) st->rr_last = rr;
     if (sqrt(rr / (double)A.n) < rtol) {
         if (lead) st->done = 1;
         return;
     }
-    if (it >= st->maxiter) {
+    if (it >= cap) {
         if (lead) st->done = 3;
         return;
     }
     if (gam < 0.0 && lead) st->nneg += 1;
     double be = 0.0, den = del;
     if (it > 0) {
-        const double gprev = st->s_oldp[2 * par], aprev = st->s_oldp[2 * par + 1];
         if (gprev == 0.0) {
             if (lead) { st->nbreak += 1; st->done = 2; }
             return;
@@ -512,42 +609,33 @@ __global__ void __launch_bounds__(SBLK) k_cg1(CGArgs A, int par)
         return;
     }
     const double al = gam / den;
-    const double2 *rc = par ? A.rec1 : A.rec0;
-    double2 *rn = par ? A.rec0 : A.rec1;
     double g = 0.0, d = 0.0, r2 = 0.0;
-    const CGRows R = cg_rows(A.n, A.nb);
-    for (int row = R.row; row < R.end; row += R.step) {
-        const double2 o0 = rc[2 * row], o1 = rc[2 * row + 1];   // {r, w}, {s_prev, D^-1}
-        const double s_ = o0.y + be * o1.x;
-        const double p_ = o1.y * o0.x + be * A.p0[row];
+    for (int row = R.row; row < R.end;) {
+        const double s_ = q.o0.y + be * q.o1.x;
+        const double p_ = q.o1.y * q.o0.x + be * q.p;
         A.p0[row] = p_;
-        A.x[row] = A.x[row] + al * p_;
-        const double r_ = o0.x - al * s_;
-        // w = A z in entry order; the column, value and neighbour record loads
-        // of SGB entries are issued before any is added. Each neighbour's z
-        // comes from its record in two 16-byte loads.
+        A.x[row] = q.x + al * p_;
+        const double r_ = q.o0.x - al * s_, z_ = q.o1.y * r_;
+        // w = A z in entry order
         double w = 0.0;
-        const int q0 = A.rowptr[row], q1 = A.rowptr[row + 1];
-        for (int pb = q0; pb < q1; pb += SGB) {
-            double zv[SGB], vv[SGB];
+        w = w + q.v[0] * z_;
 #pragma unroll
-            for (int u = 0; u < SGB; ++u) {
-                const int p = pb + u < q1 ? pb + u : q0;
-                const int j = A.colind[p];
-                vv[u] = A.val[p];
-                const double2 a = rc[2 * j], b = rc[2 * j + 1];
-                zv[u] = b.y * (a.x - al * (a.y + be * b.x));
-            }
-#pragma unroll
-            for (int u = 0; u < SGB; ++u)
-                if (pb + u < q1) w = w + vv[u] * zv[u];
+        for (int u = 1; u < EW; ++u) {
+            const double z = q.b[u].y * (q.a[u].x - al * (q.a[u].y + be * q.b[u].x));
+            if (q.q0 + u < q.q1) w = w + q.v[u] * z;
+        }
+        for (int p = q.q0 + EW; p < q.q1; ++p) {
+            const int j = A.colind[p];
+            const double2 a = rc[2 * j], b = rc[2 * j + 1];
+            w = w + A.val[p] * (b.y * (a.x - al * (a.y + be * b.x)));
         }
         rn[2 * row] = make_double2(r_, w);
-        rn[2 * row + 1] = make_double2(s_, o1.y);
-        const double z_ = o1.y * r_;
+        rn[2 * row + 1] = make_double2(s_, q.o1.y);
         g += r_ * z_;
         d += w * z_;
         r2 += r_ * r_;
+        row += R.step;
+        if (row < R.end) cg1_load(A, rc, row, q);
     }
     block_sum3(g, d, r2);
     const int np = par ^ 1;
@@ -586,7 +674,7 @@ static int ssh_alloc_vectors(fgpu_context *c)
     for (double **v : {&c->ssh_rec0, &c->ssh_rec1})
         if (!*v && (rc = fgpu_alloc(c, (void **)v, 4 * n * sizeof(double)))) return rc;
     int blocks = (int)((n + SBLK - 1) / SBLK);
-    if (blocks > 512) blocks = 512;
+    if (blocks > CG_BLOCKS) blocks = CG_BLOCKS;
     c->ssh_blocks = blocks;
     if (!c->ssh_part && (rc = fgpu_alloc(c, (void **)&c->ssh_part, sizeof(double) * 8 * (size_t)blocks))) return rc;
     if (!c->ssh_out && (rc = fgpu_alloc(c, (void **)&c->ssh_out, sizeof(CGState)))) return rc;
@@ -624,6 +712,9 @@ static int ssh_alloc_matrix(fgpu_context *c, int n, int nnz)
     if (!c->ssh_colind && (rc = fgpu_alloc(c, (void **)&c->ssh_colind, sizeof(int) * nnz))) return rc;
     if (!c->ssh_val && (rc = fgpu_alloc(c, (void **)&c->ssh_val, sizeof(double) * nnz))) return rc;
     if (!c->ssh_pr && (rc = fgpu_alloc(c, (void **)&c->ssh_pr, sizeof(double) * nnz))) return rc;
+    const size_t ne = ((size_t)n + 63) / 64 * 64 * EW;
+    if (!c->ssh_ecol && (rc = fgpu_alloc(c, (void **)&c->ssh_ecol, sizeof(int) * ne))) return rc;
+    if (!c->ssh_eval && (rc = fgpu_alloc(c, (void **)&c->ssh_eval, sizeof(double) * ne))) return rc;
     return ssh_alloc_vectors(c);
 }
 
@@ -774,12 +865,14 @@ static CGArgs cg_args(fgpu_context *c)
     A.q = c->ssh_q;
     A.rec0 = (double2 *)c->ssh_rec0;
     A.rec1 = (double2 *)c->ssh_rec1;
+    A.ecol = c->ssh_ecol;
+    A.eval = c->ssh_eval;
     A.part = c->ssh_part;
     A.st = (CGState *)c->ssh_out;
     return A;
 }
 
-#define CG_GRAPH_ITERS 8
+#define CG_GRAPH_ITERS 16
 
 static int enqueue_iters(fgpu_context *c, const CGArgs &A, int iters)
 {
@@ -982,13 +1075,13 @@ extern "C" int fgpu_ssh_download(fgpu_context *c, double *x)
 // and q of the two-kernel one, sharing the area), the per-block partial sums and the CG state live in `scratch`, a static device
 // array of FGPU_NOALLOC_MAX_ROWS rows that every GPU the library runs on holds
 // until the process ends. x and rhs are the caller's device vectors. Kernels
-// are launched directly (no graph instantiation), eight iterations between
+// are launched directly (no graph instantiation), CG_GRAPH_ITERS between
 // polls of the state, with the same kernels, launch order and iteration
 // parities as fgpu_ssh_solve_cg, so both give the same x bit for bit.
 // Calls that overlap on one GPU share `scratch` and race.
 // ==============================================================================
 #define NOALLOC_VECS 9   // doubles per row: two 4-double records and p
-#define NOALLOC_PART (8 * 512)
+#define NOALLOC_PART (8 * CG_BLOCKS)
 static constexpr size_t NOALLOC_DOUBLES =
     (size_t)NOALLOC_VECS * FGPU_NOALLOC_MAX_ROWS + NOALLOC_PART + (sizeof(CGState) + 7) / 8;
 static __device__ __align__(256) double scratch[NOALLOC_DOUBLES];

@@ -1,0 +1,58 @@
+"""SSH solves on matrices of any row length (shorter and longer than the entries
+that the iteration keeps in its own layout) and of sizes around a wave, a block
+and more rows than threads."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _matrix(n, longest, seed):
+    """Symmetric, diagonally dominant; CSR with the diagonal first. Row 0 of a
+    larger matrix is coupled to ``longest`` others."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(seed)
+    i = np.arange(n)
+    pairs = [np.stack([i[:-1], i[1:]], 1)] if n > 1 else []
+    if n > 8:
+        pairs.append(rng.integers(0, n, (2 * n, 2)))
+        pairs.append(np.stack([np.zeros(min(longest, n - 1), int), 1 + rng.permutation(n - 1)[:longest]], 1))
+    a = sp.csr_matrix((n, n))
+    if pairs:
+        p = np.concatenate(pairs)
+        p = np.unique(np.sort(p[p[:, 0] != p[:, 1]], 1), axis=0)
+        off = sp.coo_matrix((-rng.uniform(0.1, 1.0, len(p)), (p[:, 0], p[:, 1])), shape=(n, n)).tocsr()
+        a = (off + off.T).tocsr()
+    a.sort_indices()
+    diag = np.asarray(abs(a).sum(1)).ravel() + rng.uniform(0.05, 0.5, n)
+    rowptr, colind, val = [1], [], []
+    for r in range(n):
+        s = slice(a.indptr[r], a.indptr[r + 1])
+        colind += [r + 1, *(a.indices[s] + 1)]
+        val += [diag[r], *a.data[s]]
+        rowptr.append(len(colind) + 1)
+    return np.array(rowptr), np.array(colind), np.array(val), a + sp.diags(diag)
+
+
+@pytest.mark.parametrize("variant", [2, 1])
+@pytest.mark.parametrize("n,longest", [(1, 0), (2, 0), (9, 7), (63, 8), (64, 40), (65, 9), (1000, 300), (4097, 8),
+                                       (140000, 20)])
+def test_solve_any_row_length(n, longest, variant):
+    from fesom2_amd import gpu
+    rowptr, colind, val, a = _matrix(n, longest, n + variant)
+    b = np.random.default_rng(n).normal(size=n)
+    print(f"[gpu] {n} rows, longest {np.diff(rowptr).max()}, preconditioner {variant}", flush=True)
+    ctx = gpu.Context()
+    try:
+        ctx.ssh_set_matrix(rowptr, colind, val)
+        ctx.ssh_solve_preconditioner(variant)
+        runs = [ctx.ssh_solve_cg(np.zeros(n), b, 1e-10) for _ in range(2)]
+    finally:
+        ctx.close()
+    x, st = runs[0]
+    assert st["converged"]
+    np.testing.assert_array_equal(x, runs[1][0])
+    # the stopping rule on the residual, plus what its recurrence and the product here can drift by
+    scale = np.sqrt(np.mean((abs(a) @ abs(x)) ** 2))
+    bound = 1e-10 * np.sqrt(np.mean(b * b)) + (2 * st["iters"] + np.diff(rowptr).max()) * 2.3e-16 * scale
+    assert np.sqrt(np.mean((b - a @ x) ** 2)) <= bound
