@@ -654,6 +654,298 @@ __global__ void __launch_bounds__(SBLK) k_cg1(CGArgs A, int par)
     }
 }
 
+// ------------------------------------------------------------------------------
+// The whole solve of a small matrix in one block. An iteration kernel on a few
+// thousand rows is all latency (about 5 us of launch, state and partial sums);
+// here the scalars stay in registers, the vectors that rows gather from in LDS,
+// and a row's entries in registers of its thread, so an iteration is two or
+// three barriers. V rows per thread. Thread t of pass v stands for thread t % 256 of
+// block 4 v + t / 256 of the iteration kernels, and sums are added in their
+// order: the iterates are theirs, bit for bit. Bound by the LDS gathers and, with
+// a sparse M^-1, by its entries from L2 (64 bytes a clock). An iteration with the
+// sparse preconditioner and with the diagonal one: 986 rows 12.9 -> 4.4 us and
+// 7.0 -> 3.0, 3,000 rows 13.4 -> 8.3 us and 6.9 -> 5.3. A fourth row per thread
+// does not fit the registers (spilling the third one cost 3 us).
+// ------------------------------------------------------------------------------
+#define CGS_THREADS 1024
+#define CGS_ROWS 3072        // V = 3: what the registers hold
+#define CGS_MAXITER 20000    // an unbounded solve stays with the kernels per iteration
+enum { CGS_SPARSE, CGS_JACOBI, CGS_SINGLE };
+
+template <int MODE, int V>
+struct CGSmall {
+    double v[V][EW];          // entries in order
+    unsigned col[V][EW / 2];  // byte offsets of their columns, two to a register
+    unsigned id[V];           // row + (number of entries, at most EW + 1) << 16; 0 without a row
+
+    __device__ __forceinline__ bool ok(int u) const { return id[u] != 0; }
+    __device__ __forceinline__ int row(int u) const { return (int)(id[u] & 0xffffu); }
+    static __device__ __forceinline__ unsigned at(int row) { return (unsigned)(row / 64 * (64 * EW) + row % 64); }
+    __device__ __forceinline__ void load(const CGArgs &A)
+    {
+#pragma unroll
+        for (int u = 0; u < V; ++u) {
+            const int b = 4 * u + (int)(threadIdx.x >> 8), t = threadIdx.x & (SBLK - 1);
+            int end = A.n, r = b * SBLK + t;
+            if (A.nb % NXCD == 0) {   // cg_rows
+                const int chunk = (A.n + NXCD - 1) / NXCD;
+                r = b % NXCD * chunk + b / NXCD * SBLK + t;
+                end = min(A.n, (b % NXCD + 1) * chunk);
+            }
+            id[u] = 0;
+#pragma unroll
+            for (int e = 0; e < EW; ++e) v[u][e] = 0.0;
+#pragma unroll
+            for (int e = 0; e < EW / 2; ++e) col[u][e] = 0;
+            if (!(b < A.nb && r < end)) continue;
+            const int q0 = A.rowptr[r], q1 = A.rowptr[r + 1];
+            id[u] = (unsigned)r | (unsigned)min(q1 - q0, EW + 1) << 16;
+#pragma unroll
+            for (int e = 0; e < EW; ++e) {
+                const int p = q0 + e < q1 ? q0 + e : q0;
+                v[u][e] = A.val[p];
+                col[u][e / 2] |= 8u * (unsigned)A.colind[p] << 16 * (e & 1);
+                if (MODE == CGS_SPARSE) A.eval[at(r) + 64 * e] = A.pr[p];   // M^-1 in k_cg1's layout, for this thread
+            }
+        }
+    }
+    // row u times the vector g in LDS, in entry order
+    template <bool PR>
+    __device__ __forceinline__ double dot(const CGArgs &A, int u, const double *g) const
+    {
+        double s = 0.0;
+        unsigned i = id[u];
+#pragma unroll
+        for (int h = 0; h < EW; h += 4) {
+            // what follows from the row's numbers is formed in place, and half a row's loads are in flight at a
+            // time: kept over the iterations they would not fit the registers
+            unsigned c0 = col[u][h / 2], c1 = col[u][h / 2 + 1];
+            asm volatile("" : "+v"(i), "+v"(c0), "+v"(c1));
+            __builtin_amdgcn_sched_barrier(0);
+            const unsigned c[4] = {c0 & 0xffffu, c0 >> 16, c1 & 0xffffu, c1 >> 16}, o = PR ? at((int)(i & 0xffffu)) : 0;
+            double x[4], m[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                x[e] = *(const double *)((const char *)g + c[e]);
+                m[e] = PR ? A.eval[o + 64 * (h + e)] : v[u][h + e];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (h + e < (int)(i >> 16)) s = s + m[e] * x[e];
+        }
+        if ((i >> 16) > EW) {
+            const int r = (int)(i & 0xffffu);
+            for (int p = A.rowptr[r] + EW; p < A.rowptr[r + 1]; ++p) s = s + (PR ? A.pr[p] : A.val[p]) * g[A.colind[p]];
+        }
+        return s;
+    }
+    // NQ sums over all rows; sh alternates between two buffers, so that one barrier per sum is enough
+    template <int NQ>
+    __device__ __forceinline__ void sum(double (*sh)[3][16 * V], int &buf, int nb, const double (&x)[NQ][V],
+                                        double (&out)[NQ]) const
+    {
+        const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+#pragma unroll
+            for (int u = 0; u < V; ++u) {
+                const double a = wave_sum(x[q][u]);
+                if (lane == 0) sh[buf][q][16 * u + w] = a;
+            }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            const double *p = sh[buf][q] + 4 * (lane < 4 * V ? lane : 0);
+            const double a = p[0] + p[1] + p[2] + p[3];
+            out[q] = wave_sum(lane < nb ? 0.0 + a : 0.0);
+        }
+        buf ^= 1;
+    }
+};
+
+template <int MODE, int V>
+__global__ void __launch_bounds__(CGS_THREADS) k_cg_small(CGArgs A, double soltol, int maxiter)
+{
+    __shared__ double gv[V * CGS_THREADS];                          // p, or z in the single-reduction iteration
+    __shared__ double gr[MODE == CGS_SPARSE ? V * CGS_THREADS : 1];   // r
+    __shared__ double sh[2][3][16 * V];
+    CGSmall<MODE, V> M;
+    int buf = 0;
+    M.load(A);
+    // what belongs to a row alone lies in LDS as well (p in gv without the single reduction, r in gr with M^-1)
+    constexpr int N1 = MODE == CGS_SINGLE ? V * CGS_THREADS : 1;
+    __shared__ double lx[V * CGS_THREADS], lw[V * CGS_THREADS], lp[N1], ls[N1], lz[MODE == CGS_SINGLE ? 1 : V * CGS_THREADS];
+    double r_[V], di[V];
+#define CGS_OWN(a, u) a[(u) * CGS_THREADS + threadIdx.x]
+#define CGS_P(u) (*(MODE == CGS_SINGLE ? &CGS_OWN(lp, u) : gv + M.row(u)))
+#define CGS_Z(u) (*(MODE == CGS_SINGLE ? gv + M.row(u) : &CGS_OWN(lz, u)))
+#define CGS_W(u) CGS_OWN(lw, u)
+#define CGS_R(u) (*(MODE == CGS_SPARSE ? gr + M.row(u) : r_ + u))
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+        const double x = A.x[M.row(u)];
+        CGS_OWN(lx, u) = x;
+        if (MODE == CGS_SINGLE) CGS_OWN(lp, u) = CGS_OWN(ls, u) = 0.0;
+        di[u] = MODE == CGS_SPARSE ? 0.0 : A.dinv[M.row(u)];
+        r_[u] = 0.0;
+        if (M.ok(u)) gv[M.row(u)] = x;
+    }
+    __syncthreads();
+    double a0[3][V], o0[3];   // b.b, then what the mode needs of the initial residual
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+        a0[0][u] = a0[1][u] = a0[2][u] = 0.0;
+        if (!M.ok(u)) continue;
+        const double b = A.rhs[M.row(u)];
+        CGS_R(u) = b - M.template dot<false>(A, u, gv);
+        a0[0][u] = 0.0 + b * b;
+    }
+    __syncthreads();
+    double rr = 0.0, gam = 0.0, del = 0.0;
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+        if (!M.ok(u)) continue;
+        if constexpr (MODE == CGS_SINGLE) {
+            a0[1][u] = 0.0 + CGS_R(u) * CGS_R(u);
+            CGS_Z(u) = di[u] * r_[u];
+        } else {
+            const double z = MODE == CGS_SPARSE ? M.template dot<true>(A, u, gr) : di[u] * r_[u];
+            CGS_Z(u) = z;
+            a0[1][u] = 0.0 + CGS_R(u) * z;
+        }
+    }
+    M.template sum<3>(sh, buf, A.nb, a0, o0);
+    const double rtol = soltol * sqrt(o0[0] / (double)A.n);
+    int it = 0, done = 0, nbreak = 0, nneg = 0;
+    double rr_last = 0.0, s_old = 0.0, alp = 0.0;
+    if constexpr (MODE == CGS_SINGLE) {
+        rr = o0[1];
+        double a[2][V], o[2];
+#pragma unroll
+        for (int u = 0; u < V; ++u) {
+            a[0][u] = a[1][u] = 0.0;
+            if (!M.ok(u)) continue;
+            const double w = M.template dot<false>(A, u, gv), z = CGS_Z(u);
+            CGS_W(u) = w;
+            a[0][u] = 0.0 + CGS_R(u) * z;
+            a[1][u] = 0.0 + w * z;
+        }
+        M.template sum<2>(sh, buf, A.nb, a, o);
+        gam = o[0];
+        del = o[1];
+    } else {
+        gam = o0[1];   // r.z
+    }
+    while (true) {
+        if constexpr (MODE == CGS_SINGLE) {   // k_cg1
+            rr_last = rr;
+            if (sqrt(rr / (double)A.n) < rtol) { done = 1; break; }
+            if (it >= maxiter) { done = 3; break; }
+            if (gam < 0.0) nneg += 1;
+            double be = 0.0, den = del;
+            if (it > 0) {
+                if (s_old == 0.0) { nbreak += 1; done = 2; break; }
+                be = gam / s_old;
+                den = del - be * gam / alp;
+            }
+            if (!(den > 0.0)) { nbreak += 1; done = 2; break; }
+            const double al = gam / den;
+#pragma unroll
+            for (int u = 0; u < V; ++u) {
+                if (!M.ok(u)) continue;
+                const double s = CGS_W(u) + be * CGS_OWN(ls, u), p = di[u] * r_[u] + be * CGS_P(u);
+                CGS_OWN(ls, u) = s;
+                CGS_P(u) = p;
+                CGS_OWN(lx, u) = CGS_OWN(lx, u) + al * p;
+                r_[u] = r_[u] - al * s;
+                CGS_Z(u) = di[u] * r_[u];
+            }
+            __syncthreads();
+            double a[3][V], o[3];
+#pragma unroll
+            for (int u = 0; u < V; ++u) {
+                a[0][u] = a[1][u] = a[2][u] = 0.0;
+                if (!M.ok(u)) continue;
+                const double w = M.template dot<false>(A, u, gv), z = CGS_Z(u);
+                CGS_W(u) = w;
+                a[0][u] = 0.0 + CGS_R(u) * z;
+                a[1][u] = 0.0 + w * z;
+                a[2][u] = 0.0 + CGS_R(u) * CGS_R(u);
+            }
+            M.template sum<3>(sh, buf, A.nb, a, o);
+            s_old = gam;
+            alp = al;
+            gam = o[0];
+            del = o[1];
+            rr = o[2];
+        } else {   // k_cg_a, k_cg_b, k_cg_c
+            double be = 0.0;
+            if (it > 0) {
+                rr_last = rr;
+                if (sqrt(rr / (double)A.n) < rtol) { done = 1; break; }
+                if (gam < 0.0) nneg += 1;
+                if (s_old == 0.0) { nbreak += 1; done = 2; break; }
+                be = gam / s_old;
+            }
+            if (it >= maxiter) { done = 3; break; }
+            s_old = gam;
+#pragma unroll
+            for (int u = 0; u < V; ++u) {
+                if (M.ok(u)) CGS_P(u) = it == 0 ? CGS_Z(u) : CGS_Z(u) + be * CGS_P(u);
+            }
+            __syncthreads();
+            double a[1][V], o[1];
+#pragma unroll
+            for (int u = 0; u < V; ++u) {
+                a[0][u] = 0.0;
+                if (!M.ok(u)) continue;
+                const double w = M.template dot<false>(A, u, gv);
+                CGS_W(u) = w;
+                a[0][u] = 0.0 + CGS_P(u) * w;
+            }
+            M.template sum<1>(sh, buf, A.nb, a, o);
+            if (o[0] <= 0.0 || o[0] != o[0]) { nbreak += 1; done = 2; it += 1; break; }
+            const double al = s_old / o[0];
+#pragma unroll
+            for (int u = 0; u < V; ++u) {
+                if (!M.ok(u)) continue;
+                CGS_OWN(lx, u) = CGS_OWN(lx, u) + al * CGS_P(u);
+                CGS_R(u) = CGS_R(u) - al * CGS_W(u);
+            }
+            if (MODE == CGS_SPARSE) __syncthreads();
+            double a2[2][V], o2[2];
+#pragma unroll
+            for (int u = 0; u < V; ++u) {
+                a2[0][u] = a2[1][u] = 0.0;
+                if (!M.ok(u)) continue;
+                const double z = MODE == CGS_SPARSE ? M.template dot<true>(A, u, gr) : di[u] * r_[u];
+                CGS_Z(u) = z;
+                a2[0][u] = 0.0 + CGS_R(u) * z;
+                a2[1][u] = 0.0 + CGS_R(u) * CGS_R(u);
+            }
+            M.template sum<2>(sh, buf, A.nb, a2, o2);
+            gam = o2[0];
+            rr = o2[1];
+        }
+        it += 1;
+    }
+#pragma unroll
+    for (int u = 0; u < V; ++u)
+        if (M.ok(u)) A.x[M.row(u)] = CGS_OWN(lx, u);
+    if (threadIdx.x == 0) {
+        CGState q{};
+        q.soltol = soltol;
+        q.maxiter = maxiter;
+        q.iter = it;
+        q.done = done;
+        q.nbreak = nbreak;
+        q.nneg = nneg;
+        q.rtol = rtol;
+        q.rr_last = rr_last;
+        *A.st = q;
+    }
+}
+
 __global__ void k_copy(double *dst, const double *src, int n)
 {
     const int i = blockIdx.x * SBLK + threadIdx.x;
@@ -872,6 +1164,27 @@ static CGArgs cg_args(fgpu_context *c)
     return A;
 }
 
+template <int V>
+static void launch_cg_small(fgpu_context *c, const CGArgs &A, double soltol, int maxiter)
+{
+    const dim3 g(1), b(CGS_THREADS);
+    if (A.variant != 2) hipLaunchKernelGGL((k_cg_small<CGS_SPARSE, V>), g, b, 0, c->stream, A, soltol, maxiter);
+    else if (!c->ssh_single_reduction) hipLaunchKernelGGL((k_cg_small<CGS_JACOBI, V>), g, b, 0, c->stream, A, soltol, maxiter);
+    else hipLaunchKernelGGL((k_cg_small<CGS_SINGLE, V>), g, b, 0, c->stream, A, soltol, maxiter);
+}
+
+// one solve in one kernel where the rows fit one block, and on average the
+// registers (a mesh's rows have seven entries; the entries of longer ones pass
+// through one CU); false: not taken
+static bool enqueue_cg_small(fgpu_context *c, const CGArgs &A, double soltol, int maxiter)
+{
+    if (A.n > CGS_ROWS || (size_t)c->ssh_nnz > (size_t)EW * A.n || maxiter > CGS_MAXITER) return false;
+    if (A.n <= CGS_THREADS) launch_cg_small<1>(c, A, soltol, maxiter);
+    else if (A.n <= 2 * CGS_THREADS) launch_cg_small<2>(c, A, soltol, maxiter);
+    else launch_cg_small<3>(c, A, soltol, maxiter);
+    return true;
+}
+
 #define CG_GRAPH_ITERS 16
 
 static int enqueue_iters(fgpu_context *c, const CGArgs &A, int iters)
@@ -924,6 +1237,14 @@ static int launch_cg(fgpu_context *c, double soltol, int maxiter, int variant)
 {
     CGArgs A = cg_args(c);
     A.variant = variant;
+    CGState hs;
+    if (enqueue_cg_small(c, A, soltol, maxiter)) {
+        FGPU_HIP(hipGetLastError());
+        FGPU_HIP(hipMemcpyAsync(&hs, c->ssh_out, sizeof(CGState), hipMemcpyDeviceToHost, c->stream));
+        FGPU_HIP(hipStreamSynchronize(c->stream));
+        c->ssh_last_iters = hs.iter;
+        return FGPU_OK;
+    }
     int rc = cg_graph(c, A);
     if (rc) return rc;
     const dim3 g(A.nb), b(SBLK);
@@ -939,7 +1260,6 @@ static int launch_cg(fgpu_context *c, double soltol, int maxiter, int variant)
     int expect = c->ssh_last_iters > 0 ? c->ssh_last_iters : 4 * CG_GRAPH_ITERS;
     int launched = 0;
     int batch = (expect + CG_GRAPH_ITERS - 1) / CG_GRAPH_ITERS;
-    CGState hs;
     while (true) {
         for (int i = 0; i < batch && launched < max_graphs; ++i, ++launched)
             FGPU_HIP(hipGraphLaunch(c->ssh_graph, c->stream));
@@ -1135,7 +1455,9 @@ extern "C" int fgpu_ssh_solve_cg_noalloc(fgpu_context *c, double *x_dev, const d
     A.part = s + NOALLOC_VECS * M;
     A.st = (CGState *)(s + NOALLOC_VECS * M + NOALLOC_PART);
     const dim3 g(A.nb), b(SBLK);
-    if (A.variant == 2 && c->ssh_single_reduction) {
+    const bool small = enqueue_cg_small(c, A, soltol, maxiter);
+    if (small) {
+    } else if (A.variant == 2 && c->ssh_single_reduction) {
         hipLaunchKernelGGL(k_cg1_init_r, g, b, 0, c->stream, A, soltol, maxiter);
         hipLaunchKernelGGL(k_cg1_init_w, g, b, 0, c->stream, A);
     } else {
@@ -1147,7 +1469,7 @@ extern "C" int fgpu_ssh_solve_cg_noalloc(fgpu_context *c, double *x_dev, const d
     CGState hs;
     hs.done = 0;
     for (int batch = 0; batch < max_batches && !hs.done; ++batch) {
-        if ((rc = enqueue_iters(c, A, CG_GRAPH_ITERS))) return rc;
+        if (!small && (rc = enqueue_iters(c, A, CG_GRAPH_ITERS))) return rc;
         FGPU_HIP(hipMemcpyAsync(&hs, A.st, sizeof(CGState), hipMemcpyDeviceToHost, c->stream));
         FGPU_HIP(hipStreamSynchronize(c->stream));
     }

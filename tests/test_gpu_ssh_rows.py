@@ -1,6 +1,7 @@
 """SSH solves on matrices of any row length (shorter and longer than the entries
 that the iteration keeps in its own layout) and of sizes around a wave, a block
-and more rows than threads."""
+and more rows than threads; and small matrices, solved in one kernel, against
+the kernels per iteration."""
 import numpy as np
 import pytest
 
@@ -56,3 +57,30 @@ def test_solve_any_row_length(n, longest, variant):
     scale = np.sqrt(np.mean((abs(a) @ abs(x)) ** 2))
     bound = 1e-10 * np.sqrt(np.mean(b * b)) + (2 * st["iters"] + np.diff(rowptr).max()) * 2.3e-16 * scale
     assert np.sqrt(np.mean((b - a @ x) ** 2)) <= bound
+
+
+@pytest.mark.parametrize("loop", ["classic", "single", "sparse"])
+@pytest.mark.parametrize("n", [1, 64, 1000, 1024, 1025, 1793, 2048, 2049, 3072, 3073])
+def test_one_kernel_solve_bitwise(monkeypatch, n, loop):
+    """The same iterates whether the solve runs in one kernel or, from an
+    iteration cap above 20,000 on, in one or more kernels per iteration."""
+    from fesom2_amd import gpu
+    if loop == "classic":
+        monkeypatch.setenv("FGPU_SSH_CG", "classic")
+    rowptr, colind, val, _ = _matrix(n, 30, n)
+    rng = np.random.default_rng(n)
+    b, x0 = rng.normal(size=n), 0.1 * rng.normal(size=n)
+    print(f"[gpu] {n} rows, {loop}", flush=True)
+    ctx = gpu.Context()
+    try:
+        ctx.ssh_set_matrix(rowptr, colind, val)
+        ctx.ssh_solve_preconditioner(1 if loop == "sparse" else 2)
+        for tol, cap in ((1e-10, 2000), (1e-10, 3), (1e-2, 2000)):
+            x, st = ctx.ssh_solve_cg(x0, b, tol, cap)
+            if cap < 2000 and not st["converged"]:
+                continue
+            y, su = ctx.ssh_solve_cg(x0, b, tol, 20001)
+            np.testing.assert_array_equal(x, y)
+            assert {k: st[k] for k in st if k != "ms"} == {k: su[k] for k in su if k != "ms"}
+    finally:
+        ctx.close()
