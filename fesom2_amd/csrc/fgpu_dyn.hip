@@ -540,12 +540,14 @@ extern "C" int fgpu_vert_vel_download(fgpu_context *c, double *w, double *w_e, d
     struct { double *dst; const double *src; size_t n; } cp[] = {
         {w, c->d.w, N2 * NL}, {w_e, c->d.w_e, N2 * NL}, {w_i, c->d.w_i, N2 * NL}, {cfl_z, c->vv_cfl, N2 * NL},
         {hnode_new, c->m.hnode_new, N2 * (NL - 1)}};
+    FgpuPart parts[5];
+    int np = 0;
     for (auto &x : cp) {
         if (!x.dst) continue;
         if (!x.src) return fgpu_fail(FGPU_ERR_STATE, "nothing computed yet (fgpu_vert_vel_ale)");
-        FGPU_HIP(hipMemcpy(x.dst, x.src, sizeof(double) * x.n, hipMemcpyDeviceToHost));
+        parts[np++] = {x.dst, x.src, sizeof(double) * x.n};
     }
-    return FGPU_OK;
+    return fgpu_fetch(c, parts, np);
 }
 
 extern "C" int fgpu_compute_ssh_rhs_ale(fgpu_context *c, const double *uv_rhs, const double *ssh_rhs_old,

@@ -195,6 +195,8 @@ struct ProfEntry {
 #define KD_WAVELOCAL 2
 #define KDP_SHORT_NL 72   // columns to this many interfaces take three or four per block in fgpu_step_shape's report
 
+struct FgpuFetcher;
+
 struct fgpu_context {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -206,6 +208,8 @@ struct fgpu_context {
     int N2 = 0, F2 = 0, E2 = 0, nl = 0, kmax = 0;
     double cyclic_length = 0.0;
     bool edge_gap = false;             // some edge's elements share no level and leave a gap between their ranges
+    FgpuFetcher *fetcher = nullptr;    // threads and pinned slots of large downloads (fgpu_runtime.hip)
+    bool fetch_plain = false;          // they could not be had
     std::vector<void *> allocs;        // everything hipMalloc'ed by the context
     std::vector<void *> tracer_allocs; // released on fgpu_tracers_init
     // tracer configuration (host mirror)
@@ -270,6 +274,10 @@ struct fgpu_context {
     double *vv_colmax = nullptr;    // per-column max of CFL_z (nod2D)
     void *vv_flags = nullptr;       // max CFL_z bits, NaN column count
 };
+
+// downloads into pageable memory (fgpu_runtime.hip)
+struct FgpuPart { void *dst; const void *src; size_t bytes; };
+int fgpu_fetch(fgpu_context *c, const FgpuPart *parts, int nparts);
 
 // error helpers (fgpu_runtime.hip)
 int fgpu_fail(int code, const std::string &msg);
