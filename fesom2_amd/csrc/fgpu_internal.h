@@ -309,6 +309,8 @@ int fgpu_enqueue_fused_step(fgpu_context *c, double dt);
 void fgpu_kd_shape(const fgpu_context *c, int *tch, int *cpb);
 int fgpu_kd_extras(const fgpu_context *c);
 int fgpu_compute_zn(fgpu_context *c);
+void fgpu_launch_kv(fgpu_context *c, int tr0, int ntr, double dt, int all, int clamp);
+void fgpu_launch_kv_lo(fgpu_context *c, int tr0, int ntr, double dt);
 int fgpu_ensure_staged(fgpu_context *c, int slots);
 // explicit diffusion terms (fgpu_diff.hip)
 int fgpu_ensure_diff(fgpu_context *c);

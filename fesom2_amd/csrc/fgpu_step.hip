@@ -999,7 +999,7 @@ __global__ void __launch_bounds__(64) kL_node(DevMesh m, DevDyn d, DevTracers t,
 #define KV_TP 2   // tracers whose rows are loaded together
 template <int NV, int XF>
 __global__ void __launch_bounds__(64 * KV_NW) __attribute__((amdgpu_waves_per_eu(XF == 0 ? 8 : 4)))
-kV_cols(DevMesh m, DevDyn d, DevTracers t, double dt, int clamp_tracer, int NC, int TB)
+kV_cols(DevMesh m, DevDyn d, DevTracers t, int tr0, int ntr, double dt, int all, int clamp_tracer, int NC, int TB)
 {
     extern __shared__ double lds[];
     const int L = m.L, NL = m.NL, RS = L | 1;
@@ -1007,14 +1007,14 @@ kV_cols(DevMesh m, DevDyn d, DevTracers t, double dt, int clamp_tracer, int NC, 
     const int col0 = xcd_unit() * NC;
     if (col0 >= m.N2) return;
     const int ncol = min(NC, m.N2 - col0);
-    const int trb = blockIdx.y * TB, ntb = min(TB, t.ntr - trb);
+    const int trb = tr0 + blockIdx.y * TB, ntb = min(TB, tr0 + ntr - trb);
     constexpr bool WS = (XF & KV_WS) != 0, LO = (XF & KV_LO) != 0;
     const bool redi = (XF & KV_DX) != 0 && d.redi != 0;
     const size_t set = 3 * (size_t)NC * RS;   // the rows' second set follows the first
     double *sa = lds, *sb = sa + (size_t)NC * RS, *sc = sb + (size_t)NC * RS, *sr = lds + (WS ? 2 : 1) * set;
     double *F = LO ? t.fct_lo : t.T;
     // does the solve take tracer tr, and with the second set?
-    auto solved = [&](int tr) { return LO ? ldc(t.lim + tr) == LIM_FCT : (XF == 0 || ldc(t.ivd + tr) != 0); };
+    auto solved = [&](int tr) { return LO ? ldc(t.lim + tr) == LIM_FCT : (XF == 0 || all || ldc(t.ivd + tr) != 0); };
     auto second = [&](int tr) { return WS && ldc(t.lim + tr) != LIM_FCT; };
     // the block's columns, one per lane
     const int nl_ = m.node_ord[col0 + min(lane, ncol - 1)];
@@ -1362,10 +1362,10 @@ static ColLanes col_lanes(const fgpu_context *c, int tpb)
     } while (0)
 
 template <int XF>
-static void launch_kv(fgpu_context *c, double dt, int clamp)
+static void launch_kv(fgpu_context *c, int tr0, int nt, double dt, int all, int clamp)
 {
     const DevMesh &m = c->m;
-    const int nt = c->t.ntr, row = 8 * (m.L | 1), coef = XF & KV_WS ? 6 : 3;
+    const int row = 8 * (m.L | 1), coef = XF & KV_WS ? 6 : 3;
     // tracers in equal groups of at most ten: a column's pivots are formed once
     // per group (70 layers, 10 tracers: 328 us in one group, 682 us by fours)
     const int groups = (nt + 9) / 10, TB = (nt + groups - 1) / groups;
@@ -1377,9 +1377,21 @@ static void launch_kv(fgpu_context *c, double dt, int clamp)
     NC = std::max(1, std::min(NC, (int)((size_t)m.N2 * groups / 1024)));
     const size_t lds = (size_t)row * (coef + TB) * NC;
     const dim3 g(xcd_grid((m.N2 + NC - 1) / NC), (unsigned)groups), b(64 * KV_NW);
-    if (m.NL <= 64) hipLaunchKernelGGL((kV_cols<1, XF>), g, b, lds, c->stream, m, c->d, c->t, dt, clamp, NC, TB);
-    else hipLaunchKernelGGL((kV_cols<2, XF>), g, b, lds, c->stream, m, c->d, c->t, dt, clamp, NC, TB);
+    if (m.NL <= 64) hipLaunchKernelGGL((kV_cols<1, XF>), g, b, lds, c->stream, m, c->d, c->t, tr0, nt, dt, all, clamp, NC, TB);
+    else hipLaunchKernelGGL((kV_cols<2, XF>), g, b, lds, c->stream, m, c->d, c->t, tr0, nt, dt, all, clamp, NC, TB);
 }
+
+// K_V of tracers tr0..tr0+ntr-1; all: also of those with i_vert_diff off
+void fgpu_launch_kv(fgpu_context *c, int tr0, int ntr, double dt, int all, int clamp)
+{
+    bool dx = c->d.redi != 0;
+    for (int i = tr0; i < tr0 + ntr; ++i) dx = dx || (!all && !c->h_ivd[i]);
+    if (c->d.wsplit && dx) launch_kv<KV_WS | KV_DX>(c, tr0, ntr, dt, all, clamp);
+    else if (c->d.wsplit) launch_kv<KV_WS>(c, tr0, ntr, dt, all, clamp);
+    else if (dx) launch_kv<KV_DX>(c, tr0, ntr, dt, all, clamp);
+    else launch_kv<0>(c, tr0, ntr, dt, all, clamp);
+}
+void fgpu_launch_kv_lo(fgpu_context *c, int tr0, int ntr, double dt) { launch_kv<KV_LO>(c, tr0, ntr, dt, 0, -1); }
 
 int fgpu_enqueue_fused_step(fgpu_context *c, double dt)
 {
@@ -1423,7 +1435,7 @@ int fgpu_enqueue_fused_step(fgpu_context *c, double dt)
     }
     if (c->d.wsplit) {
         ProfScope ps(c, "kV_lo");
-        launch_kv<KV_LO>(c, dt, -1);
+        fgpu_launch_kv_lo(c, 0, nt, dt);
     }
     {
         ProfScope ps(c, "kC_node");
@@ -1443,10 +1455,7 @@ int fgpu_enqueue_fused_step(fgpu_context *c, double dt)
     }
     {
         ProfScope ps(c, "kV_cols");
-        if (xf == 0) launch_kv<0>(c, dt, clamp);
-        else if (xf == 1) launch_kv<KV_WS>(c, dt, clamp);
-        else if (xf == 2) launch_kv<KV_DX>(c, dt, clamp);
-        else launch_kv<KV_WS | KV_DX>(c, dt, clamp);
+        fgpu_launch_kv(c, 0, nt, dt, 0, clamp);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fgpu_fail(FGPU_ERR_HIP, std::string("fused step launch: ") + hipGetErrorString(e));

@@ -31,6 +31,33 @@ __device__ __forceinline__ double upw1_h(double t1, double t2, double vflux, dou
     return -0.5 * (t1 * (vflux + fabs(vflux)) + t2 * (vflux - fabs(vflux))) - fin;
 }
 
+// The (row, level) of a thread in the kernels over the levels of all nodes, edges
+// or elements. ROW: a wave takes 64 levels of one row, so the row's topology and
+// geometry are scalar loads; else threads take consecutive (row, level) pairs,
+// all lanes in use whatever the number of levels.
+template <bool ROW>
+__device__ __forceinline__ bool cell(int rows, int L, int &row, int &k)
+{
+    if (ROW) {
+        row = __builtin_amdgcn_readfirstlane(xcd_unit() * (BLK / 64) + (int)(threadIdx.x >> 6));
+        k = (int)(blockIdx.z * 64 + (threadIdx.x & 63)) + 1;
+        return row < rows && k <= L;
+    }
+    const size_t i = (size_t)blockIdx.x * BLK + threadIdx.x, n = (size_t)rows * L;
+    if (i >= n) return false;
+    row = n <= 0xffffffffu ? (int)((unsigned)i / (unsigned)L) : (int)(i / L);
+    k = (int)(i - (size_t)row * L) + 1;
+    return true;
+}
+
+// a mesh or tracer record: wave-uniform, and so a scalar load, with ROW
+template <bool ROW, typename T>
+__device__ __forceinline__ T ld(const T *p)
+{
+    if constexpr (ROW) return ldc(p);
+    else return *p;
+}
+
 // ------------------------------------------------------------------------------
 // K1: init_tracers_AB (oce_tracer_mod.F90:44-123): valuesAB and the valuesold
 // rotation, every level of every column.
@@ -62,10 +89,9 @@ __global__ void __launch_bounds__(BLK) k_init_ab(DevMesh m, DevTracers t, int tr
 __global__ void __launch_bounds__(BLK) k_tr_xy(DevMesh m, DevTracers t, int tr0)
 {
     const int tr = tr0 + blockIdx.y;
-    const size_t i = (size_t)blockIdx.x * BLK + threadIdx.x;
-    if (i >= (size_t)m.F2 * m.L) return;
-    const int el = (int)(i / m.L);
-    const int k = (int)(i - (size_t)el * m.L) + 1;
+    int el, k;
+    if (!cell<false>(m.F2, m.L, el, k)) return;
+    const size_t i = (size_t)el * m.L + k - 1;
     if (k < m.ulev[el] || k > m.nlev[el] - 1) return;
     const double *T = t.T + t.sN * tr;
     const int n0 = m.elem_nodes[3 * el], n1 = m.elem_nodes[3 * el + 1], n2 = m.elem_nodes[3 * el + 2];
@@ -81,15 +107,16 @@ __global__ void __launch_bounds__(BLK) k_tr_xy(DevMesh m, DevTracers t, int tr0)
 // fill_up_dn_grad for one (edge, level) (oce_muscl_adv.F90:356-525), evaluated
 // where the MFCT flux needs it instead of materialising edge_up_dn_grad.
 // ------------------------------------------------------------------------------
+template <bool ROW>
 __device__ __forceinline__ void node_mean_grad(const DevMesh &m, const double *trxy, int node, int k,
                                                double &gx, double &gy)
 {
     double tvol = 0.0, tx = 0.0, ty = 0.0;
-    const int num = m.nie_num[node];
+    const int num = ld<ROW>(m.nie_num + node);
     for (int j = 0; j < num; ++j) {
-        const int el = m.nie[(size_t)node * m.kmax + j];
-        if (m.nlev[el] - 1 < k || k < m.ulev[el]) continue;
-        const double a = m.elem_area[el];
+        const int el = ld<ROW>(m.nie + ((size_t)node * m.kmax + j));
+        if (ld<ROW>(m.nlev + el) - 1 < k || k < ld<ROW>(m.ulev + el)) continue;
+        const double a = ld<ROW>(m.elem_area + el);
         const double *g = trxy + ((size_t)el * m.L + k - 1) * 2;
         tvol = tvol + a;
         tx = tx + g[0] * a;
@@ -99,42 +126,43 @@ __device__ __forceinline__ void node_mean_grad(const DevMesh &m, const double *t
     gy = ty / tvol;
 }
 
+template <bool ROW>
 __device__ __forceinline__ void up_dn_grad(const DevMesh &m, const double *trxy, int e, int n1, int n2, int k,
                                            double g[4])
 {
     g[0] = g[1] = g[2] = g[3] = 0.0;
-    const int up = m.updn[2 * e], dn = m.updn[2 * e + 1];
+    const int up = ld<ROW>(m.updn + (2 * e)), dn = ld<ROW>(m.updn + (2 * e + 1));
     double gx, gy;
     if (up >= 0 && dn >= 0) {
-        const int nzmin = max(m.ulevn_max[n1], m.ulevn_max[n2]);
-        const int nzmax = min(m.nlevn_min[n1], m.nlevn_min[n2]);
+        const int nzmin = max(ld<ROW>(m.ulevn_max + n1), ld<ROW>(m.ulevn_max + n2));
+        const int nzmax = min(ld<ROW>(m.nlevn_min + n1), ld<ROW>(m.nlevn_min + n2));
         // writes in the reference's order; a later write wins
-        if (k >= m.ulevn[n1] && k <= nzmin - 1) { node_mean_grad(m, trxy, n1, k, gx, gy); g[0] = gx; g[2] = gy; }
-        if (k >= m.ulevn[n2] && k <= nzmin - 1) { node_mean_grad(m, trxy, n2, k, gx, gy); g[1] = gx; g[3] = gy; }
+        if (k >= ld<ROW>(m.ulevn + n1) && k <= nzmin - 1) { node_mean_grad<ROW>(m, trxy, n1, k, gx, gy); g[0] = gx; g[2] = gy; }
+        if (k >= ld<ROW>(m.ulevn + n2) && k <= nzmin - 1) { node_mean_grad<ROW>(m, trxy, n2, k, gx, gy); g[1] = gx; g[3] = gy; }
         if (k >= nzmin && k <= nzmax - 1) {
             const double *gu = trxy + ((size_t)up * m.L + k - 1) * 2;
             const double *gd = trxy + ((size_t)dn * m.L + k - 1) * 2;
             g[0] = gu[0]; g[1] = gd[0]; g[2] = gu[1]; g[3] = gd[1];
         }
-        if (k >= nzmax && k <= m.nlevn[n1] - 1) { node_mean_grad(m, trxy, n1, k, gx, gy); g[0] = gx; g[2] = gy; }
-        if (k >= nzmax && k <= m.nlevn[n2] - 1) { node_mean_grad(m, trxy, n2, k, gx, gy); g[1] = gx; g[3] = gy; }
+        if (k >= nzmax && k <= ld<ROW>(m.nlevn + n1) - 1) { node_mean_grad<ROW>(m, trxy, n1, k, gx, gy); g[0] = gx; g[2] = gy; }
+        if (k >= nzmax && k <= ld<ROW>(m.nlevn + n2) - 1) { node_mean_grad<ROW>(m, trxy, n2, k, gx, gy); g[1] = gx; g[3] = gy; }
     } else {
-        if (k >= m.ulevn[n1] && k <= m.nlevn[n1] - 1) { node_mean_grad(m, trxy, n1, k, gx, gy); g[0] = gx; g[2] = gy; }
-        if (k >= m.ulevn[n2] && k <= m.nlevn[n2] - 1) { node_mean_grad(m, trxy, n2, k, gx, gy); g[1] = gx; g[3] = gy; }
+        if (k >= ld<ROW>(m.ulevn + n1) && k <= ld<ROW>(m.nlevn + n1) - 1) { node_mean_grad<ROW>(m, trxy, n1, k, gx, gy); g[0] = gx; g[2] = gy; }
+        if (k >= ld<ROW>(m.ulevn + n2) && k <= ld<ROW>(m.nlevn + n2) - 1) { node_mean_grad<ROW>(m, trxy, n2, k, gx, gy); g[1] = gx; g[3] = gy; }
     }
 }
 
 // debug: materialise edge_up_dn_grad of one tracer (per-function parity)
+template <bool ROW>
 __global__ void __launch_bounds__(BLK) k_fill_up_dn_grad(DevMesh m, DevTracers t, int tr)
 {
-    const size_t i = (size_t)blockIdx.x * BLK + threadIdx.x;
-    if (i >= (size_t)m.E2 * m.L) return;
-    const int e = (int)(i / m.L);
-    const int k = (int)(i - (size_t)e * m.L) + 1;
-    const int n1 = m.edges[2 * e], n2 = m.edges[2 * e + 1];
-    if (k > max(m.nlevn[n1], m.nlevn[n2]) - 1) return;
+    int e, k;
+    if (!cell<ROW>(m.E2, m.L, e, k)) return;
+    const size_t i = (size_t)e * m.L + k - 1;
+    const int n1 = ld<ROW>(m.edges + (2 * e)), n2 = ld<ROW>(m.edges + (2 * e + 1));
+    if (k > max(ld<ROW>(m.nlevn + n1), ld<ROW>(m.nlevn + n2)) - 1) return;
     double g[4];
-    up_dn_grad(m, t.tr_xy + t.sStg * tr, e, n1, n2, k, g);
+    up_dn_grad<ROW>(m, t.tr_xy + t.sStg * tr, e, n1, n2, k, g);
     double *o = t.dbg_grad + 4 * i;
     // levels a node does not reach keep zero in components it would write
     o[0] = g[0]; o[1] = g[1]; o[2] = g[2]; o[3] = g[3];
@@ -154,14 +182,14 @@ __device__ __forceinline__ double seg_vflux(int seg, const double *uv1, const do
     return (-uv1[1] * dX1 + uv1[0] * dY1) * h1 + (uv2[1] * dX2 - uv2[0] * dY2) * h2;
 }
 
+template <bool ROW>
 __global__ void __launch_bounds__(BLK) k_edge_flux(DevMesh m, DevDyn d, DevTracers t, int tr0)
 {
     const int tr = tr0 + blockIdx.y;
-    const size_t i = (size_t)blockIdx.x * BLK + threadIdx.x;
-    if (i >= (size_t)m.E2 * m.L) return;
-    const int e = (int)(i / m.L);
-    const int k = (int)(i - (size_t)e * m.L) + 1;
-    const int nl1 = m.einfo[4 * e], nu1 = m.einfo[4 * e + 1], nl2 = m.einfo[4 * e + 2], nu2 = m.einfo[4 * e + 3];
+    int e, k;
+    if (!cell<ROW>(m.E2, m.L, e, k)) return;
+    const size_t i = (size_t)e * m.L + k - 1;
+    const int nl1 = ld<ROW>(m.einfo + (4 * e)), nu1 = ld<ROW>(m.einfo + (4 * e + 1)), nl2 = ld<ROW>(m.einfo + (4 * e + 2)), nu2 = ld<ROW>(m.einfo + (4 * e + 3));
     const int nl12 = min(nl1, nl2), nu12 = max(nu1, nu2);
     bool in[5];
     in[0] = (k >= nu1 && k <= nu12 - 1);
@@ -170,21 +198,21 @@ __global__ void __launch_bounds__(BLK) k_edge_flux(DevMesh m, DevDyn d, DevTrace
     in[3] = (k >= nl12 + 1 && k <= nl1);
     in[4] = (k >= nl12 + 1 && k <= nl2);
     if (!(in[0] || in[1] || in[2] || in[3] || in[4])) return;
-    const int n1 = m.edges[2 * e], n2 = m.edges[2 * e + 1];
-    const int el1 = m.edge_tri[2 * e], el2 = m.edge_tri[2 * e + 1];
-    const double dX1 = m.ecd[4 * e], dY1 = m.ecd[4 * e + 1];
+    const int n1 = ld<ROW>(m.edges + (2 * e)), n2 = ld<ROW>(m.edges + (2 * e + 1));
+    const int el1 = ld<ROW>(m.edge_tri + (2 * e)), el2 = ld<ROW>(m.edge_tri + (2 * e + 1));
+    const double dX1 = ld<ROW>(m.ecd + (4 * e)), dY1 = ld<ROW>(m.ecd + (4 * e + 1));
     double dX2 = 0.0, dY2 = 0.0;
-    double a = FGPU_R_EARTH * m.elem_cos[el1];
+    double a = FGPU_R_EARTH * ld<ROW>(m.elem_cos + el1);
     if (el2 >= 0) {
-        dX2 = m.ecd[4 * e + 2];
-        dY2 = m.ecd[4 * e + 3];
-        a = 0.5 * (a + FGPU_R_EARTH * m.elem_cos[el2]);
+        dX2 = ld<ROW>(m.ecd + (4 * e + 2));
+        dY2 = ld<ROW>(m.ecd + (4 * e + 3));
+        a = 0.5 * (a + FGPU_R_EARTH * ld<ROW>(m.elem_cos + el2));
     }
     const double *uv1 = d.uv + ((size_t)el1 * m.L + k - 1) * 2;
     const double *uv2 = el2 >= 0 ? d.uv + ((size_t)el2 * m.L + k - 1) * 2 : uv1;
     const double h1 = m.helem[(size_t)el1 * m.L + k - 1];
     const double h2 = el2 >= 0 ? m.helem[(size_t)el2 * m.L + k - 1] : 0.0;
-    const int lim = t.lim[tr], hor = t.hor[tr];
+    const int lim = ld<ROW>(t.lim + tr), hor = ld<ROW>(t.hor + tr);
     const double *T = t.T + t.sN * tr;
     const double *TAB = t.TAB + t.sN * tr;
     const size_t o1 = (size_t)n1 * m.L + k - 1, o2 = (size_t)n2 * m.L + k - 1;
@@ -199,13 +227,13 @@ __global__ void __launch_bounds__(BLK) k_edge_flux(DevMesh m, DevDyn d, DevTrace
     const double A1 = TAB[o1], A2 = TAB[o2];
     double f = flo;   // o_init_zero=.false. with FCT, zero otherwise
     if (hor != HOR_UPW1) {   // MFCT, MUSCL
-        const double no = t.ph[tr];
+        const double no = ld<ROW>(t.ph + tr);
         double g[4];
-        up_dn_grad(m, t.tr_xy + t.sStg * tr, e, n1, n2, k, g);
-        const double edx = m.edge_dxdy[2 * e], edy = m.edge_dxdy[2 * e + 1];
+        up_dn_grad<ROW>(m, t.tr_xy + t.sStg * tr, e, n1, n2, k, g);
+        const double edx = ld<ROW>(m.edge_dxdy + (2 * e)), edy = ld<ROW>(m.edge_dxdy + (2 * e + 1));
         double Tmean2, Tmean1;
         if (hor == HOR_MUSCL) {   // reconstruction only down to nboundary_lay (oce_adv_tra_hor.F90:356-367)
-            const double c1 = k <= m.nblay[n1] ? 1.0 : 0.0, c2 = k <= m.nblay[n2] ? 1.0 : 0.0;
+            const double c1 = k <= ld<ROW>(m.nblay + n1) ? 1.0 : 0.0, c2 = k <= ld<ROW>(m.nblay + n2) ? 1.0 : 0.0;
             Tmean2 = A2 - (2.0 * (A2 - A1) + edx * a * g[1] + edy * FGPU_R_EARTH * g[3]) / 6.0 * c2;
             Tmean1 = A1 + (2.0 * (A2 - A1) + edx * a * g[0] + edy * FGPU_R_EARTH * g[2]) / 6.0 * c1;
         } else {
@@ -282,14 +310,14 @@ __device__ __forceinline__ double ver_ho(int ver, int j, int nzmin, int nzmax, c
 // antidiffusive vertical flux at the top interface of the cell (and at the
 // bottom interface for the deepest cell).
 // ------------------------------------------------------------------------------
+template <bool ROW>
 __global__ void __launch_bounds__(BLK) k_node_lo(DevMesh m, DevDyn d, DevTracers t, int tr0, double dt)
 {
     const int tr = tr0 + blockIdx.y;
-    const size_t i = (size_t)blockIdx.x * BLK + threadIdx.x;
-    if (i >= t.sN) return;
-    const int n = (int)(i / m.L);
-    const int k = (int)(i - (size_t)n * m.L) + 1;
-    const int nzmin = m.ulevn[n], nzmax = m.nlevn[n];
+    int n, k;
+    if (!cell<ROW>(m.N2, m.L, n, k)) return;
+    const size_t i = (size_t)n * m.L + k - 1;
+    const int nzmin = ld<ROW>(m.ulevn + n), nzmax = ld<ROW>(m.nlevn + n);
     if (k < nzmin || k > nzmax - 1) return;
     const int L = m.L, NL = m.NL;
     const double *T = t.T + t.sN * tr + (size_t)n * L;
@@ -298,18 +326,18 @@ __global__ void __launch_bounds__(BLK) k_node_lo(DevMesh m, DevDyn d, DevTracers
     const double *Zn = m.Z3d + (size_t)n * L;
     const double *zb = m.zbar3d + (size_t)n * NL;
     double *av = t.a_v + t.sNI * tr + (size_t)n * NL;
-    const int lim = t.lim[tr], ver = t.ver[tr];
-    const double pv = t.pv[tr];
+    const int lim = ld<ROW>(t.lim + tr), ver = ld<ROW>(t.ver + tr);
+    const double pv = ld<ROW>(t.pv + tr);
     const double *hn = m.hnode_new + (size_t)n * L, *ho = m.hnode + (size_t)n * L;
     if (lim == LIM_FCT) {
         const double *We = d.w_e + (size_t)n * NL;
         const double *W = d.w + (size_t)n * NL;
         const double *lo_h = t.lo_h + t.sE * tr;
         double acc = 0.0;
-        for (int p = m.ne_ptr[n]; p < m.ne_ptr[n + 1]; ++p) {
-            const int q = m.ne_idx[p];
+        for (int p = ld<ROW>(m.ne_ptr + n); p < ld<ROW>(m.ne_ptr + (n + 1)); ++p) {
+            const int q = ld<ROW>(m.ne_idx + p);
             const int e = q >> 1;
-            if (k < m.erange[2 * e] || k > m.erange[2 * e + 1]) continue;
+            if (k < ld<ROW>(m.erange + (2 * e)) || k > ld<ROW>(m.erange + (2 * e + 1))) continue;
             const double fl = lo_h[(size_t)e * L + k - 1];
             acc = (q & 1) ? acc - fl : acc + fl;
         }
@@ -319,7 +347,7 @@ __global__ void __launch_bounds__(BLK) k_node_lo(DevMesh m, DevDyn d, DevTracers
         t.fct_lo[i + t.sN * tr] = (T[k - 1] * m.hnode[i] + (acc + (lk - lk1)) * dt / av_) / m.hnode_new[i];
         // with the W split the LO flux handed to the HO scheme is upwind with
         // the full W (oce_adv_tra_driver.F90:323-331); the implicit part enters
-        // the LO solution in k_vert_impl
+        // the LO solution afterwards
         const double fk = d.wsplit ? ver_upw1(k, nzmin, nzmax, T, W, ar, 0.0) : lk;
         av[k - 1] = ver_ho(ver, k, nzmin, nzmax, TAB, W, ar, Zn, zb, pv, hn, ho, dt, fk);
         if (k == nzmax - 1) {
@@ -334,79 +362,15 @@ __global__ void __launch_bounds__(BLK) k_node_lo(DevMesh m, DevDyn d, DevTracers
 }
 
 // ------------------------------------------------------------------------------
-// K4b (use_wsplit only): adv_tra_vert_impl (oce_adv_tra_ver.F90:90-240) on the
-// LO solution of the FCT tracers: implicit first-order upwind advection with
-// w_i, one tridiagonal solve per column, thread per column. Coefficients are
-// formed on the fly in the forward sweep (each depends only on its own level).
-// ------------------------------------------------------------------------------
-template <int MAXL>
-__global__ void __launch_bounds__(64) k_vert_impl(DevMesh m, DevDyn d, DevTracers t, int tr0, double dt)
-{
-    const int tr = tr0 + blockIdx.y;
-    if (t.lim[tr] != LIM_FCT) return;
-    const int n = blockIdx.x * 64 + threadIdx.x;
-    if (n >= m.N2) return;
-    const int L = m.L, NL = m.NL;
-    const int nzmin = m.ulevn[n], nzmax = m.nlevn[n];
-    double *TF = t.fct_lo + t.sN * tr + (size_t)n * L;
-    const double *wi = d.w_i + (size_t)n * NL;
-    const double *ar = m.area + (size_t)n * NL;
-    const double *avl = m.areasvol + (size_t)n * NL;
-    const double *hn = m.hnode_new + (size_t)n * L;
-    double cp[MAXL + 1], tp[MAXL + 1];
-#define I(kk) ((kk) - 1)
-    const double zinv = 1.0 * dt;
-    int nz = nzmin;
-    double v_adv = zinv * ar[I(nz)] / avl[I(nz)];
-    double a = 0.0;
-    double b = hn[I(nz)] + wi[I(nz)] * v_adv;
-    v_adv = zinv * ar[I(nz + 1)] / avl[I(nz)];
-    b = b - dmn(0.0, wi[I(nz + 1)]) * v_adv;
-    double c = -dmx(0.0, wi[I(nz + 1)]) * v_adv;
-    double Tm, Tk = TF[I(nz)], Tp = TF[I(nz + 1)];
-    double r = -(b - hn[I(nz)]) * Tk - c * Tp;
-    cp[I(nz)] = c / b;
-    tp[I(nz)] = r / b;
-    for (nz = nzmin + 1; nz <= nzmax - 1; ++nz) {
-        Tm = Tk;
-        Tk = Tp;
-        v_adv = zinv * ar[I(nz)] / avl[I(nz)];
-        a = dmn(0.0, wi[I(nz)]) * v_adv;
-        b = hn[I(nz)] + dmx(0.0, wi[I(nz)]) * v_adv;
-        if (nz <= nzmax - 2) {
-            v_adv = zinv * ar[I(nz + 1)] / avl[I(nz)];
-            b = b - dmn(0.0, wi[I(nz + 1)]) * v_adv;
-            c = -dmx(0.0, wi[I(nz + 1)]) * v_adv;
-            Tp = TF[I(nz + 1)];
-            r = -a * Tm - (b - hn[I(nz)]) * Tk - c * Tp;
-        } else {
-            c = 0.0;
-            r = -a * Tm - (b - hn[I(nz)]) * Tk;
-        }
-        const double mm = b - cp[I(nz - 1)] * a;
-        cp[I(nz)] = c / mm;
-        tp[I(nz)] = (r - tp[I(nz - 1)] * a) / mm;
-    }
-    double x = tp[I(nzmax - 1)];
-    TF[I(nzmax - 1)] = TF[I(nzmax - 1)] + x;
-    for (nz = nzmax - 2; nz >= nzmin; --nz) {
-        x = tp[I(nz)] - cp[I(nz)] * x;
-        TF[I(nz)] = TF[I(nz)] + x;
-    }
-#undef I
-}
-
-// ------------------------------------------------------------------------------
 // K5: FCT a1+a2 (oce_adv_tra_fct.F90:119-178): element bounds with +-1e3 padding
 // ------------------------------------------------------------------------------
 __global__ void __launch_bounds__(BLK) k_elem_aux(DevMesh m, DevTracers t, int tr0)
 {
     const int tr = tr0 + blockIdx.y;
     if (t.lim[tr] != LIM_FCT) return;
-    const size_t i = (size_t)blockIdx.x * BLK + threadIdx.x;
-    if (i >= (size_t)m.F2 * m.L) return;
-    const int el = (int)(i / m.L);
-    const int k = (int)(i - (size_t)el * m.L) + 1;
+    int el, k;
+    if (!cell<false>(m.F2, m.L, el, k)) return;
+    const size_t i = (size_t)el * m.L + k - 1;
     double *o = t.aux + t.sStg * tr + 2 * i;
     if (k <= m.ulev[el] - 1 || k >= m.nlev[el]) {
         o[0] = -1e3;
@@ -430,43 +394,44 @@ __global__ void __launch_bounds__(BLK) k_elem_aux(DevMesh m, DevTracers t, int t
 // K6: FCT a3 + b1 + b2 per (node, level) (oce_adv_tra_fct.F90:195-405):
 // admissible increments, P+/P- from the vertical and the edge gather, R+/R-.
 // ------------------------------------------------------------------------------
+template <bool ROW>
 __device__ __forceinline__ void tvert(const DevMesh &m, const double *aux, int n, int k, double &vmax, double &vmin)
 {
     const int *ne = m.nie + (size_t)n * m.kmax;
-    const double *a0 = aux + ((size_t)ne[0] * m.L + k - 1) * 2;
+    const double *a0 = aux + ((size_t)ld<ROW>(ne) * m.L + k - 1) * 2;
     vmax = a0[0];
     vmin = a0[1];
-    const int num = m.nie_num[n];
+    const int num = ld<ROW>(m.nie_num + n);
     for (int j = 1; j < num; ++j) {
-        const double *a = aux + ((size_t)ne[j] * m.L + k - 1) * 2;
+        const double *a = aux + ((size_t)ld<ROW>(ne + j) * m.L + k - 1) * 2;
         vmax = dmx(vmax, a[0]);
         vmin = dmn(vmin, a[1]);
     }
 }
 
+template <bool ROW>
 __global__ void __launch_bounds__(BLK) k_node_limit(DevMesh m, DevTracers t, int tr0, double dt)
 {
     const int tr = tr0 + blockIdx.y;
-    if (t.lim[tr] != LIM_FCT) return;
-    const size_t i = (size_t)blockIdx.x * BLK + threadIdx.x;
-    if (i >= t.sN) return;
-    const int n = (int)(i / m.L);
-    const int k = (int)(i - (size_t)n * m.L) + 1;
-    const int nzmin = m.ulevn[n], nzmax = m.nlevn[n];
+    if (ld<ROW>(t.lim + tr) != LIM_FCT) return;
+    int n, k;
+    if (!cell<ROW>(m.N2, m.L, n, k)) return;
+    const size_t i = (size_t)n * m.L + k - 1;
+    const int nzmin = ld<ROW>(m.ulevn + n), nzmax = ld<ROW>(m.nlevn + n);
     if (k < nzmin || k > nzmax - 1) return;
     const int L = m.L, NL = m.NL;
     const double *aux = t.aux + t.sStg * tr;
     const double lo = t.fct_lo[t.sN * tr + i];
     double bmax, bmin, vmax, vmin;
     if (k == nzmax - 1 || k == nzmin) {
-        tvert(m, aux, n, k, vmax, vmin);
+        tvert<ROW>(m, aux, n, k, vmax, vmin);
         bmax = vmax - lo;
         bmin = vmin - lo;
     } else {
         double x0, y0, x1, y1, x2, y2;
-        tvert(m, aux, n, k - 1, x0, y0);
-        tvert(m, aux, n, k, x1, y1);
-        tvert(m, aux, n, k + 1, x2, y2);
+        tvert<ROW>(m, aux, n, k - 1, x0, y0);
+        tvert<ROW>(m, aux, n, k, x1, y1);
+        tvert<ROW>(m, aux, n, k + 1, x2, y2);
         bmax = dmx(dmx(x0, x1), x2) - lo;
         bmin = dmn(dmn(y0, y1), y2) - lo;
     }
@@ -475,10 +440,10 @@ __global__ void __launch_bounds__(BLK) k_node_limit(DevMesh m, DevTracers t, int
     p = p + (dmx(0.0, av[k - 1]) + dmx(0.0, -av[k]));
     q = q + (dmn(0.0, av[k - 1]) + dmn(0.0, -av[k]));
     const double *ah = t.a_h + t.sE * tr;
-    for (int pp = m.ne_ptr[n]; pp < m.ne_ptr[n + 1]; ++pp) {
-        const int qq = m.ne_idx[pp];
+    for (int pp = ld<ROW>(m.ne_ptr + n); pp < ld<ROW>(m.ne_ptr + (n + 1)); ++pp) {
+        const int qq = ld<ROW>(m.ne_idx + pp);
         const int e = qq >> 1;
-        if (k < m.erange[2 * e] || k > m.erange[2 * e + 1]) continue;
+        if (k < ld<ROW>(m.erange + (2 * e)) || k > ld<ROW>(m.erange + (2 * e + 1))) continue;
         const double fl = ah[(size_t)e * L + k - 1];
         if (qq & 1) {
             p = p + dmx(0.0, -fl);
@@ -503,10 +468,9 @@ __global__ void __launch_bounds__(BLK) k_edge_limit(DevMesh m, DevTracers t, int
 {
     const int tr = tr0 + blockIdx.y;
     if (t.lim[tr] != LIM_FCT) return;
-    const size_t i = (size_t)blockIdx.x * BLK + threadIdx.x;
-    if (i >= (size_t)m.E2 * m.L) return;
-    const int e = (int)(i / m.L);
-    const int k = (int)(i - (size_t)e * m.L) + 1;
+    int e, k;
+    if (!cell<false>(m.E2, m.L, e, k)) return;
+    const size_t i = (size_t)e * m.L + k - 1;
     if (k < m.erange[2 * e] || k > m.erange[2 * e + 1]) return;
     const int n1 = m.edges[2 * e], n2 = m.edges[2 * e + 1];
     const double *rp = t.rp + t.sN * tr, *rm = t.rm + t.sN * tr;
@@ -556,36 +520,37 @@ __device__ __forceinline__ double av_limited(int j, int nzmin, int nzmax, const 
 // precomputed increments (fgpu_diff.hip), in the order of diff_tracers_ale:
 // edges of diff_part_hor_redi ascending, diff_ver_part_expl_ale,
 // diff_ver_part_redi_expl
+template <bool ROW>
 __device__ __forceinline__ double add_explicit_diffusion(const DevMesh &m, const DevDyn &d, const DevTracers &t, int tr,
                                                          int n, int k, size_t i, double avol, double dt, double del)
 {
     if (d.hdiff) {
         const double *hd = t.hd + t.sE * tr;
-        for (int p = m.ne_ptr[n]; p < m.ne_ptr[n + 1]; ++p) {
-            const int q = m.ne_idx[p];
+        for (int p = ld<ROW>(m.ne_ptr + n); p < ld<ROW>(m.ne_ptr + (n + 1)); ++p) {
+            const int q = ld<ROW>(m.ne_idx + p);
             const int e = q >> 1;
-            if (k < m.erange[2 * e] || k > m.erange[2 * e + 1]) continue;
+            if (k < ld<ROW>(m.erange + (2 * e)) || k > ld<ROW>(m.erange + (2 * e + 1))) continue;
             const double c = hd[(size_t)e * m.L + k - 1];
             const double r = (q & 1) ? 0.0 - c : 0.0 + c;
             del = del + r * dt / avol;
         }
     }
-    if (!t.ivd[tr]) del = del + t.ve[t.sN * tr + i];
+    if (!ld<ROW>(t.ivd + tr)) del = del + t.ve[t.sN * tr + i];
     if (d.redi) del = del + t.vr[t.sN * tr + i];
     return del;
 }
 
+template <bool ROW>
 __global__ void __launch_bounds__(BLK) k_node_update(DevMesh m, DevDyn d, DevTracers t, int tr0, double dt, int mode)
 {
     const int tr = tr0 + blockIdx.y;
-    const size_t i = (size_t)blockIdx.x * BLK + threadIdx.x;
-    if (i >= t.sN) return;
-    const int n = (int)(i / m.L);
-    const int k = (int)(i - (size_t)n * m.L) + 1;
-    const int nzmin = m.ulevn[n], nzmax = m.nlevn[n];
+    int n, k;
+    if (!cell<ROW>(m.N2, m.L, n, k)) return;
+    const size_t i = (size_t)n * m.L + k - 1;
+    const int nzmin = ld<ROW>(m.ulevn + n), nzmax = ld<ROW>(m.nlevn + n);
     if (k < nzmin || k > nzmax - 1) return;
     const int L = m.L, NL = m.NL;
-    const bool fct = t.lim[tr] == LIM_FCT;
+    const bool fct = ld<ROW>(t.lim + tr) == LIM_FCT;
     const double *av = t.a_v + t.sNI * tr + (size_t)n * NL;
     double fk, fk1;
     if (fct) {
@@ -605,17 +570,17 @@ __global__ void __launch_bounds__(BLK) k_node_update(DevMesh m, DevDyn d, DevTra
     v = v + (fk - fk1) * dt / avol;
     double h = 0.0;
     const double *ah = t.a_h + t.sE * tr;
-    for (int p = m.ne_ptr[n]; p < m.ne_ptr[n + 1]; ++p) {
-        const int q = m.ne_idx[p];
+    for (int p = ld<ROW>(m.ne_ptr + n); p < ld<ROW>(m.ne_ptr + (n + 1)); ++p) {
+        const int q = ld<ROW>(m.ne_idx + p);
         const int e = q >> 1;
-        if (k < m.erange[2 * e] || k > m.erange[2 * e + 1]) continue;
+        if (k < ld<ROW>(m.erange + (2 * e)) || k > ld<ROW>(m.erange + (2 * e + 1))) continue;
         const double fl = ah[(size_t)e * L + k - 1];
         if (q & 1) h = h - fl * dt / avol;
         else h = h + fl * dt / avol;
     }
     if (mode == 0) {
         double del = 0.0 + h + v;
-        del = add_explicit_diffusion(m, d, t, tr, n, k, i, avol, dt, del);
+        del = add_explicit_diffusion<ROW>(m, d, t, tr, n, k, i, avol, dt, del);
         del = del + Tk * (m.hnode[i] - m.hnode_new[i]);
         T[i] = Tk + del / m.hnode_new[i];
     } else {
@@ -630,149 +595,15 @@ __global__ void __launch_bounds__(BLK) k_node_update(DevMesh m, DevDyn d, DevTra
 // T* update from stored del_ttf_adv* (per-tracer diff_tracers_ale entry)
 __global__ void __launch_bounds__(BLK) k_tstar(DevMesh m, DevDyn d, DevTracers t, int tr, double dt)
 {
-    const size_t i = (size_t)blockIdx.x * BLK + threadIdx.x;
-    if (i >= t.sN) return;
-    const int n = (int)(i / m.L);
-    const int k = (int)(i - (size_t)n * m.L) + 1;
+    int n, k;
+    if (!cell<false>(m.N2, m.L, n, k)) return;
+    const size_t i = (size_t)n * m.L + k - 1;
     if (k < m.ulevn[n] || k > m.nlevn[n] - 1) return;
     double *T = t.T + t.sN * tr;
     double del = 0.0 + t.dttf_h[i] + t.dttf_v[i];
-    del = add_explicit_diffusion(m, d, t, tr, n, k, i, m.areasvol[(size_t)n * m.NL + k - 1], dt, del);
+    del = add_explicit_diffusion<false>(m, d, t, tr, n, k, i, m.areasvol[(size_t)n * m.NL + k - 1], dt, del);
     del = del + T[i] * (m.hnode[i] - m.hnode_new[i]);
     T[i] = T[i] + del / m.hnode_new[i];
-}
-
-// ------------------------------------------------------------------------------
-// K9: diff_ver_part_impl_ale (oce_ale_tracer.F90:907-1435) per column: Thomas
-// solve of the implicit vertical diffusion, bc_surface at the top
-// (:1828-2108), then the salinity clamp of solve_tracers_ale (:502-514) for
-// the second tracer. Redi off (isredi = 0), no w-split implicit advection.
-// ------------------------------------------------------------------------------
-template <int MAXL>
-__global__ void __launch_bounds__(64) k_vdiff(DevMesh m, DevDyn d, DevTracers t, int tr0, double dt, int do_diff,
-                                              int clamp_tracer)
-{
-    const int tr = tr0 + blockIdx.y;
-    const int n = blockIdx.x * 64 + threadIdx.x;
-    if (n >= m.N2) return;
-    const int L = m.L, NL = m.NL;
-    const int nzmin = m.ulevn[n], nzmax = m.nlevn[n];
-    double *T = t.T + t.sN * tr + (size_t)n * L;
-    if (do_diff == 2 || (do_diff == 1 && t.ivd[tr])) {
-        const double *hn = m.hnode_new + (size_t)n * L;
-        const double *ar = m.area + (size_t)n * NL;
-        const double *avl = m.areasvol + (size_t)n * NL;
-        const double *kv = d.Kv + (size_t)n * NL;
-        double Z_n[MAXL + 1], cp[MAXL + 1], tp[MAXL + 1], zbn[MAXL + 2];
-#define I(kk) ((kk) - 1)
-        // zbar_n/Z_n rebuilt bottom-up from hnode_new (oce_ale_tracer.F90:1088-1096)
-        double zb = m.zbar_n_bot[n];
-        zbn[I(nzmax)] = zb;
-        Z_n[I(nzmax - 1)] = zb + hn[I(nzmax - 1)] / 2.0;
-        for (int nz = nzmax - 1; nz >= nzmin + 1; --nz) {
-            zb = zb + hn[I(nz)];
-            zbn[I(nz)] = zb;
-            Z_n[I(nz - 1)] = zb + hn[I(nz - 1)] / 2.0;
-        }
-        // Redi: K33 = Kv + Ki S3^2 interpolated to the interfaces
-        // (oce_ale_tracer.F90:1105-1108, 1138-1144, 1181-1184)
-        const bool redi = d.redi != 0;
-        const double *S = d.slope + (size_t)n * L * 3, *ki = d.Ki + (size_t)n * L;
-#define S3(kk) S[((kk) - 1) * 3 + 2]
-#define KI(kk) ki[(kk) - 1]
-#define TY_BELOW(nz, zi) ((zbn[I((nz) + 1)] - Z_n[I((nz) + 1)]) * (zi) * (S3(nz) * S3(nz)) * KI(nz) + \
-                          (Z_n[I(nz)] - zbn[I((nz) + 1)]) * (zi) * (S3((nz) + 1) * S3((nz) + 1)) * KI((nz) + 1))
-#define TY_ABOVE(nz, zi) ((zbn[I(nz)] - Z_n[I(nz)]) * (zi) * (S3((nz) - 1) * S3((nz) - 1)) * KI((nz) - 1) + \
-                          (Z_n[I((nz) - 1)] - zbn[I(nz)]) * (zi) * (S3(nz) * S3(nz)) * KI(nz))
-        // forward sweep: coefficients on the fly, cp/tp kept
-        const double zinv = 1.0 * dt;
-        int nz = nzmin;
-        double zinv2 = 1.0 / (Z_n[I(nz)] - Z_n[I(nz + 1)]);
-        double a = 0.0;
-        double c = redi ? -(kv[I(nz + 1)] + TY_BELOW(nz, zinv2)) * zinv2 * zinv * ar[I(nz + 1)] / avl[I(nz)]
-                        : -(kv[I(nz + 1)]) * zinv2 * zinv * ar[I(nz + 1)] / avl[I(nz)];
-        double b = -c + hn[I(nz)];
-        // implicit part of the split W (oce_ale_tracer.F90:1118-1129, 1158-1172,
-        // 1194-1202); FCT tracers took it in their LO solution
-        const bool wimpl = d.wsplit && t.lim[tr] != LIM_FCT;
-        const double *wi = d.w_i + (size_t)n * NL;
-        if (wimpl) {
-            double v_adv = zinv * (ar[I(nz)] / avl[I(nz)]);
-            b = b + wi[I(nz)] * v_adv;
-            v_adv = zinv * ar[I(nz + 1)] / avl[I(nz)];
-            b = b - dmn(0.0, wi[I(nz + 1)]) * v_adv;
-            c = c - dmx(0.0, wi[I(nz + 1)]) * v_adv;
-        }
-        double zinv1 = zinv2;
-        double Tm = 0.0, Tk = T[I(nz)], Tp = T[I(nz + 1)];
-        double tr_ = -(b - hn[I(nz)]) * Tk - c * Tp;
-        const bool hall = bc_every_layer(t.id[tr], d);
-        tr_ = tr_ + bc_surface_dev(t.id[tr], dt, d, m.N2, m.L, n, nzmin, Tk);
-        cp[I(nz)] = c / b;
-        tp[I(nz)] = tr_ / b;
-        for (nz = nzmin + 1; nz <= nzmax - 1; ++nz) {
-            Tm = Tk;
-            Tk = Tp;
-            if (nz <= nzmax - 2) {
-                zinv2 = 1.0 / (Z_n[I(nz)] - Z_n[I(nz + 1)]);
-                if (redi) {
-                    a = -(kv[I(nz)] + TY_ABOVE(nz, zinv1)) * zinv1 * zinv * (ar[I(nz)] / avl[I(nz)]);
-                    c = -(kv[I(nz + 1)] + TY_BELOW(nz, zinv2)) * zinv2 * zinv * ar[I(nz + 1)] / avl[I(nz)];
-                } else {
-                    a = -(kv[I(nz)]) * zinv1 * zinv * (ar[I(nz)] / avl[I(nz)]);
-                    c = -(kv[I(nz + 1)]) * zinv2 * zinv * ar[I(nz + 1)] / avl[I(nz)];
-                }
-                b = -a - c + hn[I(nz)];
-                zinv1 = zinv2;
-                if (wimpl) {
-                    double v_adv = zinv * (ar[I(nz)] / avl[I(nz)]);
-                    a = a + dmn(0.0, wi[I(nz)]) * v_adv;
-                    b = b + dmx(0.0, wi[I(nz)]) * v_adv;
-                    v_adv = zinv * ar[I(nz + 1)] / avl[I(nz)];
-                    b = b - dmn(0.0, wi[I(nz + 1)]) * v_adv;
-                    c = c - dmx(0.0, wi[I(nz + 1)]) * v_adv;
-                }
-                Tp = T[I(nz + 1)];
-                tr_ = -a * Tm - (b - hn[I(nz)]) * Tk - c * Tp;
-                if (hall) tr_ = tr_ + bc_surface_dev(t.id[tr], dt, d, m.N2, m.L, n, nz, Tk);
-            } else {
-                a = redi ? -(kv[I(nz)] + TY_ABOVE(nz, zinv1)) * zinv1 * zinv * (ar[I(nz)] / avl[I(nz)])
-                         : -(kv[I(nz)]) * zinv1 * zinv * (ar[I(nz)] / avl[I(nz)]);
-                c = 0.0;
-                b = -a + hn[I(nz)];
-                if (wimpl) {
-                    const double v_adv = zinv * (ar[I(nz)] / avl[I(nz)]);
-                    a = a + dmn(0.0, wi[I(nz)]) * v_adv;
-                    b = b + dmx(0.0, wi[I(nz)]) * v_adv;
-                }
-                tr_ = -a * Tm - (b - hn[I(nz)]) * Tk;
-                if (hall) tr_ = tr_ + bc_surface_dev(t.id[tr], dt, d, m.N2, m.L, n, nz, Tk);
-            }
-            const double mm = b - cp[I(nz - 1)] * a;
-            cp[I(nz)] = c / mm;
-            tp[I(nz)] = (tr_ - tp[I(nz - 1)] * a) / mm;
-        }
-#undef TY_BELOW
-#undef TY_ABOVE
-#undef S3
-#undef KI
-        // back substitution and update
-        double x = tp[I(nzmax - 1)];
-        T[I(nzmax - 1)] = T[I(nzmax - 1)] + x;
-        for (nz = nzmax - 2; nz >= nzmin; --nz) {
-            x = tp[I(nz)] - cp[I(nz)] * x;
-            T[I(nz)] = T[I(nz)] + x;
-        }
-#undef I
-    }
-    if (tr == clamp_tracer) {
-        for (int nz = nzmin; nz <= nzmax - 1; ++nz) {
-            double s = T[nz - 1];
-            if (s > 45.0) s = 45.0;
-            if (s < 3.0) s = 3.0;
-            T[nz - 1] = s;
-        }
-    }
 }
 
 // ------------------------------------------------------------------------------
@@ -836,15 +667,30 @@ static int check_tracer(fgpu_context *c, int tr_num)
         if (_e != hipSuccess) return fgpu_fail(FGPU_ERR_HIP, std::string(name) + ": " + hipGetErrorString(_e)); \
     } while (0)
 
+// A wave per row from 33 levels on, where more than half of the lanes have one.
+// One step of one tracer (k_edge_flux, k_node_lo, k_node_limit, k_node_update), us
+// by rows and by pairs: 40 thousand nodes, 47 layers 185, 96, 98, 59 and 205, 130,
+// 131, 70; 20 thousand nodes, 70 layers 122, 66, 72, 44 and 170, 98, 98, 52; 33
+// layers 77, 44, 46, 29 and 83, 49, 54, 32; 24 layers 63, 40, 44, 29 and 59, 37,
+// 37, 23. The kernels with a few loads per level are bound by those and take pairs.
+static bool cell_rows(const fgpu_context *c) { return c->m.L > 32; }
+// a kernel over the levels of `rows` rows, for ntr tracers
+#define CELL_LAUNCH(kern, rows, ntr, ...)                                                                         \
+    do {                                                                                                          \
+        const DevMesh &m_ = c->m;                                                                                 \
+        if (cell_rows(c))                                                                                         \
+            hipLaunchKernelGGL(kern<true>, dim3(xcd_grid((rows + BLK / 64 - 1) / (BLK / 64)), ntr, (m_.L + 63) / 64), \
+                               dim3(BLK), 0, c->stream, __VA_ARGS__);                                             \
+        else hipLaunchKernelGGL(kern<false>, dim3(nblk((size_t)rows * m_.L), ntr), dim3(BLK), 0, c->stream, __VA_ARGS__); \
+        LAUNCH_CHECK(#kern);                                                                                      \
+    } while (0)
+
+// K9: implicit vertical diffusion and salinity clamp, K_V of the fused step; do_diff 1: of the tracers with
+// i_vert_diff, 2: of all
 static int launch_vdiff(fgpu_context *c, int tr0, int ntr, double dt, int do_diff, int clamp_tracer)
 {
-    dim3 g(nblk(c->N2, 64), ntr);
-    const int L = c->nl - 1;
     ProfScope ps(c, "k_vdiff");
-    if (L <= 32) hipLaunchKernelGGL(k_vdiff<32>, g, dim3(64), 0, c->stream, c->m, c->d, c->t, tr0, dt, do_diff, clamp_tracer);
-    else if (L <= 48) hipLaunchKernelGGL(k_vdiff<48>, g, dim3(64), 0, c->stream, c->m, c->d, c->t, tr0, dt, do_diff, clamp_tracer);
-    else if (L <= 72) hipLaunchKernelGGL(k_vdiff<72>, g, dim3(64), 0, c->stream, c->m, c->d, c->t, tr0, dt, do_diff, clamp_tracer);
-    else hipLaunchKernelGGL(k_vdiff<FGPU_MAX_NL>, g, dim3(64), 0, c->stream, c->m, c->d, c->t, tr0, dt, do_diff, clamp_tracer);
+    fgpu_launch_kv(c, tr0, ntr, dt, do_diff == 2, clamp_tracer);
     LAUNCH_CHECK("k_vdiff");
     return FGPU_OK;
 }
@@ -859,7 +705,7 @@ static int launch_init_ab(fgpu_context *c, int tr0, int ntr)
     }
     {
         ProfScope ps(c, "k_tr_xy");
-        hipLaunchKernelGGL(k_tr_xy, dim3(nblk((size_t)m.F2 * m.L), ntr), dim3(BLK), 0, c->stream, m, c->t, tr0);
+        hipLaunchKernelGGL(k_tr_xy, dim3(nblk((size_t)c->m.F2 * c->m.L), ntr), dim3(BLK), 0, c->stream, m, c->t, tr0);
         LAUNCH_CHECK("k_tr_xy");
     }
     return FGPU_OK;
@@ -871,37 +717,29 @@ static int launch_adv(fgpu_context *c, int tr0, int ntr, double dt, int mode)
     const size_t nE = (size_t)m.E2 * m.L, nF = (size_t)m.F2 * m.L, nN = c->t.sN;
     {
         ProfScope ps(c, "k_edge_flux");
-        hipLaunchKernelGGL(k_edge_flux, dim3(nblk(nE), ntr), dim3(BLK), 0, c->stream, m, c->d, c->t, tr0);
-        LAUNCH_CHECK("k_edge_flux");
+        CELL_LAUNCH(k_edge_flux, c->m.E2, ntr, m, c->d, c->t, tr0);
     }
     {
         ProfScope ps(c, "k_node_lo");
-        hipLaunchKernelGGL(k_node_lo, dim3(nblk(nN), ntr), dim3(BLK), 0, c->stream, m, c->d, c->t, tr0, dt);
-        LAUNCH_CHECK("k_node_lo");
+        CELL_LAUNCH(k_node_lo, c->m.N2, ntr, m, c->d, c->t, tr0, dt);
     }
     if (c->d.wsplit) {
-        ProfScope ps(c, "k_vert_impl");
-        const dim3 g(nblk(c->N2, 64), ntr);
-        const int L = c->nl - 1;
-        if (L <= 32) hipLaunchKernelGGL(k_vert_impl<32>, g, dim3(64), 0, c->stream, m, c->d, c->t, tr0, dt);
-        else if (L <= 48) hipLaunchKernelGGL(k_vert_impl<48>, g, dim3(64), 0, c->stream, m, c->d, c->t, tr0, dt);
-        else if (L <= 72) hipLaunchKernelGGL(k_vert_impl<72>, g, dim3(64), 0, c->stream, m, c->d, c->t, tr0, dt);
-        else hipLaunchKernelGGL(k_vert_impl<FGPU_MAX_NL>, g, dim3(64), 0, c->stream, m, c->d, c->t, tr0, dt);
+        ProfScope ps(c, "k_vert_impl");   // adv_tra_vert_impl on the LO solution of the FCT tracers
+        fgpu_launch_kv_lo(c, tr0, ntr, dt);
         LAUNCH_CHECK("k_vert_impl");
     }
     {
         ProfScope ps(c, "k_elem_aux");
-        hipLaunchKernelGGL(k_elem_aux, dim3(nblk(nF), ntr), dim3(BLK), 0, c->stream, m, c->t, tr0);
+        hipLaunchKernelGGL(k_elem_aux, dim3(nblk((size_t)c->m.F2 * c->m.L), ntr), dim3(BLK), 0, c->stream, m, c->t, tr0);
         LAUNCH_CHECK("k_elem_aux");
     }
     {
         ProfScope ps(c, "k_node_limit");
-        hipLaunchKernelGGL(k_node_limit, dim3(nblk(nN), ntr), dim3(BLK), 0, c->stream, m, c->t, tr0, dt);
-        LAUNCH_CHECK("k_node_limit");
+        CELL_LAUNCH(k_node_limit, c->m.N2, ntr, m, c->t, tr0, dt);
     }
     {
         ProfScope ps(c, "k_edge_limit");
-        hipLaunchKernelGGL(k_edge_limit, dim3(nblk(nE), ntr), dim3(BLK), 0, c->stream, m, c->t, tr0);
+        hipLaunchKernelGGL(k_edge_limit, dim3(nblk((size_t)c->m.E2 * c->m.L), ntr), dim3(BLK), 0, c->stream, m, c->t, tr0);
         LAUNCH_CHECK("k_edge_limit");
     }
     if (mode == 0) {   // the explicit diffusion terms read T^n, which k_node_update overwrites
@@ -910,8 +748,7 @@ static int launch_adv(fgpu_context *c, int tr0, int ntr, double dt, int mode)
     }
     {
         ProfScope ps(c, "k_node_update");
-        hipLaunchKernelGGL(k_node_update, dim3(nblk(nN), ntr), dim3(BLK), 0, c->stream, m, c->d, c->t, tr0, dt, mode);
-        LAUNCH_CHECK("k_node_update");
+        CELL_LAUNCH(k_node_update, c->m.N2, ntr, m, c->d, c->t, tr0, dt, mode);
     }
     return FGPU_OK;
 }
@@ -924,8 +761,7 @@ extern "C" int fgpu_init_tracers_AB(fgpu_context *c, int tr_num)
     if ((rc = fgpu_ensure_staged(c, 1))) return rc;
     const int tr = tr_num - 1;
     if ((rc = launch_init_ab(c, tr, 1))) return rc;
-    hipLaunchKernelGGL(k_fill_up_dn_grad, dim3(nblk((size_t)c->m.E2 * c->m.L)), dim3(BLK), 0, c->stream, c->m, c->t, tr);
-    LAUNCH_CHECK("k_fill_up_dn_grad");
+    CELL_LAUNCH(k_fill_up_dn_grad, c->m.E2, 1, c->m, c->t, tr);
     FGPU_HIP(hipStreamSynchronize(c->stream));
     return FGPU_OK;
 }
@@ -946,7 +782,7 @@ extern "C" int fgpu_tracer_set_valuesAB(fgpu_context *c, int tr_num, const doubl
     FGPU_HIP(hipMemcpyAsync(c->t.TAB + c->t.sN * tr, valuesAB, c->t.sN * sizeof(double), hipMemcpyHostToDevice,
                             c->stream));
     hipLaunchKernelGGL(k_tr_xy, dim3(nblk((size_t)c->m.F2 * c->m.L), 1), dim3(BLK), 0, c->stream, c->m, c->t, tr);
-    LAUNCH_CHECK("k_tr_xy");
+        LAUNCH_CHECK("k_tr_xy");
     FGPU_HIP(hipStreamSynchronize(c->stream));
     return FGPU_OK;
 }
@@ -979,8 +815,8 @@ extern "C" int fgpu_diff_tracers_ale(fgpu_context *c, double dt, int tr_num)
     if ((rc = fgpu_check_bc_inputs(c, tr, 1))) return rc;
     if ((rc = fgpu_ensure_diff(c))) return rc;
     if ((rc = fgpu_launch_diff(c, tr, 1, dt))) return rc;
-    hipLaunchKernelGGL(k_tstar, dim3(nblk(c->t.sN)), dim3(BLK), 0, c->stream, c->m, c->d, c->t, tr, dt);
-    LAUNCH_CHECK("k_tstar");
+    hipLaunchKernelGGL(k_tstar, dim3(nblk((size_t)c->m.N2 * c->m.L), 1), dim3(BLK), 0, c->stream, c->m, c->d, c->t, tr, dt);
+        LAUNCH_CHECK("k_tstar");
     if (c->h_ivd[tr])
         if ((rc = launch_vdiff(c, tr, 1, dt, 1, -1))) return rc;
     FGPU_HIP(hipStreamSynchronize(c->stream));

@@ -147,3 +147,46 @@ def test_extra_schemes_and_terms(layers, ntr, split, diffusion):
                                  slope_tapered=rng.normal(0.0, 0.01, (mesh.nod2D, layers, 3)))
     print(f"[gpu] extra schemes, {layers} layers, {ntr} tracers, split {split}, diffusion {diffusion}", flush=True)
     _check(mesh, st, schemes)
+
+
+@pytest.mark.parametrize("ivd,split", [(True, False), (False, False), (True, True)])
+@pytest.mark.parametrize("layers", [32, 33, 64, 65, 127])
+def test_per_tracer_calls(layers, ivd, split):
+    """The per-tracer calls, by (row, level) pairs up to 32 levels and by rows of
+    up to 64 levels per wave beyond, with the diffusion terms and the W split."""
+    from fesom2_amd import gpu
+    from oracle.oracle import Oracle
+    mesh, st = _case(layers, 2)
+    rng = np.random.default_rng(layers)
+    st = dataclasses.replace(st, Ki=rng.uniform(20.0, 400.0, (mesh.nod2D, layers)), redi=True,
+                             slope_tapered=rng.normal(0.0, 0.01, (mesh.nod2D, layers, 3)))
+    if split:
+        w_e = st.w * rng.uniform(0.2, 1.0, st.w.shape)
+        st = dataclasses.replace(st, w_e=w_e, w_i=st.w - w_e, use_wsplit=True)
+    schemes = dict(i_vert_diff=ivd)
+    print(f"[gpu] per-tracer calls, {layers} layers, ivd {ivd}, split {split}", flush=True)
+    ctx = gpu.context_for(mesh, st, schemes=schemes)
+    o = Oracle(mesh)
+    k = np.arange(1, mesh.nl)
+    w = (k[None, :] >= mesh.ulevels_nod2D[:, None]) & (k[None, :] < mesh.nlevels_nod2D[:, None])
+    e = mesh.edge_tri
+    no2 = e[:, 1] < 0
+    lo = np.where(no2, mesh.ulevels[e[:, 0]], np.minimum(mesh.ulevels[e[:, 0]], mesh.ulevels[e[:, 1]]))
+    hi = np.where(no2, mesh.nlevels[e[:, 0]], np.maximum(mesh.nlevels[e[:, 0]], mesh.nlevels[e[:, 1]]))
+    em = (k[None, :] >= lo[:, None]) & (k[None, :] < hi[:, None])
+    try:
+        ctx.init_tracers_AB(2)
+        grad = ctx.work(2, "edge_up_dn_grad", (mesh.edge2D, layers, 4))
+        ctx.do_oce_adv_tra(st.dt, 2)
+        hor = ctx.work(2, "del_ttf_advhoriz", (mesh.nod2D, layers))
+        ctx.diff_tracers_ale(st.dt, 2)
+        gv, gvo = ctx.tracer_download(2)
+    finally:
+        ctx.close()
+    v, vo = st.values[1].copy(), st.valuesold[1].copy()
+    out = o.adv_stage(st, v, vo, ID=int(st.ids[1]), i_vert_diff=ivd)
+    o.diff_stage(st)
+    np.testing.assert_array_equal(grad[em], out["edge_up_dn_grad"][em])
+    np.testing.assert_array_equal(hor[w], out["del_ttf_advhoriz"][w])
+    np.testing.assert_array_equal(gv[w], v[w])
+    np.testing.assert_array_equal(gvo[w], vo[w])
