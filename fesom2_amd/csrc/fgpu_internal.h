@@ -172,6 +172,7 @@ struct DevTracers {
     // buffers of the per-stage kernels only, allocated on first use (fgpu_ensure_staged)
     double *TAB;              // N2*L per tracer (valuesAB)
     double *tr_xy, *aux;      // F2*L*2 per slot (tracers%work: one slot shared by the per-tracer calls)
+    double *ngrad;            // N2*L*2 per slot: node means of tr_xy (fill_up_dn_grad)
     double *dttf_h, *dttf_v;  // N2*L, one tracer's worth
     double *dbg_av;           // N2*NL limited vertical flux of the last per-tracer call
     double *dbg_grad;         // E2*L*4 materialised edge_up_dn_grad of the last per-tracer call

@@ -350,7 +350,7 @@ int fgpu_ensure_staged(fgpu_context *c, int slots)
     if (!t.TAB) {
         struct A { double **p; size_t n; } arrs[] = {
             {&t.TAB, t.sN * (size_t)t.ntr}, {&t.lo_h, t.sE * (size_t)t.ntr}, {&t.dttf_h, t.sN}, {&t.dttf_v, t.sN},
-            {&t.dbg_av, t.sNI}, {&t.dbg_grad, t.sE * 4}};
+            {&t.dbg_av, t.sNI}, {&t.dbg_grad, t.sE * 4}, {&t.ngrad, t.sG}};
         for (auto &a : arrs) {
             if ((rc = fgpu_alloc(c, (void **)a.p, a.n * sizeof(double), true))) return rc;
             FGPU_HIP(hipMemset(*a.p, 0, a.n * sizeof(double)));
@@ -365,6 +365,10 @@ int fgpu_ensure_staged(fgpu_context *c, int slots)
         }
         c->stage_slots = slots;
         t.sStg = slots > 1 ? t.sF2 : 0;
+        if (slots > 1) {   // such a context's steps are staged: the fused step's array is free
+            FGPU_HIP(hipMemset(t.gmean, 0, t.sG * (size_t)t.ntr * sizeof(double)));
+            t.ngrad = t.gmean;
+        }
     }
     c->graph_valid = false;
     return FGPU_OK;
@@ -967,7 +971,7 @@ extern "C" int fgpu_tracers_init(fgpu_context *c, int num_tracers)
     t.sG = N2 * L * 2;
     t.sStg = 0;
     int rc;
-    t.lo_h = t.TAB = t.tr_xy = t.aux = t.dttf_h = t.dttf_v = t.dbg_av = t.dbg_grad = nullptr;
+    t.lo_h = t.TAB = t.tr_xy = t.aux = t.dttf_h = t.dttf_v = t.dbg_av = t.dbg_grad = t.ngrad = nullptr;
     t.hd = t.ve = t.vr = t.zbh = nullptr;
     c->stage_slots = 0;
     // the fused batched step needs only these; the per-stage buffers come with

@@ -104,65 +104,80 @@ __global__ void __launch_bounds__(BLK) k_tr_xy(DevMesh m, DevTracers t, int tr0)
 }
 
 // ------------------------------------------------------------------------------
+// K2b: area-weighted mean of the element gradients around a node
+// (oce_muscl_adv.F90:388-401, 443-520) at its wet levels. An edge takes it at the
+// levels that its up- or downwind triangle lacks; formed per edge there, each wave
+// went through both nodes' elements for the lanes of a few levels (40 thousand
+// nodes, 47 layers: k_edge_flux 186 -> 132 us and about 60 of k_fill_up_dn_grad's,
+// for 38 us here).
+// ------------------------------------------------------------------------------
+template <bool ROW>
+__global__ void __launch_bounds__(BLK) k_node_grad(DevMesh m, DevTracers t, int tr0)
+{
+    const int tr = tr0 + blockIdx.y;
+    int n, k;
+    if (!cell<ROW>(m.N2, m.L, n, k)) return;
+    if (k < ld<ROW>(m.ulevn + n) || k > ld<ROW>(m.nlevn + n) - 1) return;
+    const double *trxy = t.tr_xy + t.sStg * tr;
+    double tvol = 0.0, tx = 0.0, ty = 0.0;
+    const int num = ld<ROW>(m.nie_num + n);
+    for (int j = 0; j < num; ++j) {
+        const int el = ld<ROW>(m.nie + ((size_t)n * m.kmax + j));
+        if (ld<ROW>(m.nlev + el) - 1 < k || k < ld<ROW>(m.ulev + el)) continue;
+        const double a = ld<ROW>(m.elem_area + el);
+        const double2 g = *(const double2 *)(trxy + ((size_t)el * m.L + k - 1) * 2);
+        tvol = tvol + a;
+        tx = tx + g.x * a;
+        ty = ty + g.y * a;
+    }
+    *(double2 *)(t.ngrad + (t.sStg ? t.sG * tr : 0) + ((size_t)n * m.L + k - 1) * 2) = make_double2(tx / tvol, ty / tvol);
+}
+
+// ------------------------------------------------------------------------------
 // fill_up_dn_grad for one (edge, level) (oce_muscl_adv.F90:356-525), evaluated
 // where the MFCT flux needs it instead of materialising edge_up_dn_grad.
 // ------------------------------------------------------------------------------
 template <bool ROW>
-__device__ __forceinline__ void node_mean_grad(const DevMesh &m, const double *trxy, int node, int k,
-                                               double &gx, double &gy)
-{
-    double tvol = 0.0, tx = 0.0, ty = 0.0;
-    const int num = ld<ROW>(m.nie_num + node);
-    for (int j = 0; j < num; ++j) {
-        const int el = ld<ROW>(m.nie + ((size_t)node * m.kmax + j));
-        if (ld<ROW>(m.nlev + el) - 1 < k || k < ld<ROW>(m.ulev + el)) continue;
-        const double a = ld<ROW>(m.elem_area + el);
-        const double *g = trxy + ((size_t)el * m.L + k - 1) * 2;
-        tvol = tvol + a;
-        tx = tx + g[0] * a;
-        ty = ty + g[1] * a;
-    }
-    gx = tx / tvol;
-    gy = ty / tvol;
-}
-
-template <bool ROW>
-__device__ __forceinline__ void up_dn_grad(const DevMesh &m, const double *trxy, int e, int n1, int n2, int k,
+__device__ __forceinline__ void up_dn_grad(const DevMesh &m, const DevTracers &t, int tr, int e, int n1, int n2, int k,
                                            double g[4])
 {
+    const double *trxy = t.tr_xy + t.sStg * tr, *mean = t.ngrad + (t.sStg ? t.sG * tr : 0);
     g[0] = g[1] = g[2] = g[3] = 0.0;
-    const int up = ld<ROW>(m.updn + (2 * e)), dn = ld<ROW>(m.updn + (2 * e + 1));
-    double gx, gy;
+    const int up = ld<ROW>(m.updn + 2 * e), dn = ld<ROW>(m.updn + (2 * e + 1));
+    const int top1 = ld<ROW>(m.ulevn + n1), bot1 = ld<ROW>(m.nlevn + n1) - 1;
+    const int top2 = ld<ROW>(m.ulevn + n2), bot2 = ld<ROW>(m.nlevn + n2) - 1;
+    int nzmin = 0x7fffffff, nzmax = 0x7fffffff;   // without both triangles: the means throughout
     if (up >= 0 && dn >= 0) {
-        const int nzmin = max(ld<ROW>(m.ulevn_max + n1), ld<ROW>(m.ulevn_max + n2));
-        const int nzmax = min(ld<ROW>(m.nlevn_min + n1), ld<ROW>(m.nlevn_min + n2));
-        // writes in the reference's order; a later write wins
-        if (k >= ld<ROW>(m.ulevn + n1) && k <= nzmin - 1) { node_mean_grad<ROW>(m, trxy, n1, k, gx, gy); g[0] = gx; g[2] = gy; }
-        if (k >= ld<ROW>(m.ulevn + n2) && k <= nzmin - 1) { node_mean_grad<ROW>(m, trxy, n2, k, gx, gy); g[1] = gx; g[3] = gy; }
-        if (k >= nzmin && k <= nzmax - 1) {
-            const double *gu = trxy + ((size_t)up * m.L + k - 1) * 2;
-            const double *gd = trxy + ((size_t)dn * m.L + k - 1) * 2;
-            g[0] = gu[0]; g[1] = gd[0]; g[2] = gu[1]; g[3] = gd[1];
-        }
-        if (k >= nzmax && k <= ld<ROW>(m.nlevn + n1) - 1) { node_mean_grad<ROW>(m, trxy, n1, k, gx, gy); g[0] = gx; g[2] = gy; }
-        if (k >= nzmax && k <= ld<ROW>(m.nlevn + n2) - 1) { node_mean_grad<ROW>(m, trxy, n2, k, gx, gy); g[1] = gx; g[3] = gy; }
-    } else {
-        if (k >= ld<ROW>(m.ulevn + n1) && k <= ld<ROW>(m.nlevn + n1) - 1) { node_mean_grad<ROW>(m, trxy, n1, k, gx, gy); g[0] = gx; g[2] = gy; }
-        if (k >= ld<ROW>(m.ulevn + n2) && k <= ld<ROW>(m.nlevn + n2) - 1) { node_mean_grad<ROW>(m, trxy, n2, k, gx, gy); g[1] = gx; g[3] = gy; }
+        nzmin = max(ld<ROW>(m.ulevn_max + n1), ld<ROW>(m.ulevn_max + n2));
+        nzmax = min(ld<ROW>(m.nlevn_min + n1), ld<ROW>(m.nlevn_min + n2));
+    }
+    // in the reference's order of writes: the means above, the triangles, the means below
+    if (k >= nzmin && k <= nzmax - 1) {
+        const double2 u = *(const double2 *)(trxy + ((size_t)up * m.L + k - 1) * 2);
+        const double2 d = *(const double2 *)(trxy + ((size_t)dn * m.L + k - 1) * 2);
+        g[0] = u.x; g[1] = d.x; g[2] = u.y; g[3] = d.y;
+    }
+    const bool mean_here = k <= nzmin - 1 || k >= nzmax;
+    if (mean_here && k >= top1 && k <= bot1) {
+        const double2 a = *(const double2 *)(mean + ((size_t)n1 * m.L + k - 1) * 2);
+        g[0] = a.x; g[2] = a.y;
+    }
+    if (mean_here && k >= top2 && k <= bot2) {
+        const double2 a = *(const double2 *)(mean + ((size_t)n2 * m.L + k - 1) * 2);
+        g[1] = a.x; g[3] = a.y;
     }
 }
 
 // debug: materialise edge_up_dn_grad of one tracer (per-function parity)
-template <bool ROW>
 __global__ void __launch_bounds__(BLK) k_fill_up_dn_grad(DevMesh m, DevTracers t, int tr)
 {
     int e, k;
-    if (!cell<ROW>(m.E2, m.L, e, k)) return;
+    if (!cell<false>(m.E2, m.L, e, k)) return;
     const size_t i = (size_t)e * m.L + k - 1;
-    const int n1 = ld<ROW>(m.edges + (2 * e)), n2 = ld<ROW>(m.edges + (2 * e + 1));
-    if (k > max(ld<ROW>(m.nlevn + n1), ld<ROW>(m.nlevn + n2)) - 1) return;
+    const int n1 = m.edges[2 * e], n2 = m.edges[2 * e + 1];
+    if (k > max(m.nlevn[n1], m.nlevn[n2]) - 1) return;
     double g[4];
-    up_dn_grad<ROW>(m, t.tr_xy + t.sStg * tr, e, n1, n2, k, g);
+    up_dn_grad<false>(m, t, tr, e, n1, n2, k, g);
     double *o = t.dbg_grad + 4 * i;
     // levels a node does not reach keep zero in components it would write
     o[0] = g[0]; o[1] = g[1]; o[2] = g[2]; o[3] = g[3];
@@ -229,7 +244,7 @@ __global__ void __launch_bounds__(BLK) k_edge_flux(DevMesh m, DevDyn d, DevTrace
     if (hor != HOR_UPW1) {   // MFCT, MUSCL
         const double no = ld<ROW>(t.ph + tr);
         double g[4];
-        up_dn_grad<ROW>(m, t.tr_xy + t.sStg * tr, e, n1, n2, k, g);
+        up_dn_grad<ROW>(m, t, tr, e, n1, n2, k, g);
         const double edx = ld<ROW>(m.edge_dxdy + (2 * e)), edy = ld<ROW>(m.edge_dxdy + (2 * e + 1));
         double Tmean2, Tmean1;
         if (hor == HOR_MUSCL) {   // reconstruction only down to nboundary_lay (oce_adv_tra_hor.F90:356-367)
@@ -667,18 +682,20 @@ static int check_tracer(fgpu_context *c, int tr_num)
         if (_e != hipSuccess) return fgpu_fail(FGPU_ERR_HIP, std::string(name) + ": " + hipGetErrorString(_e)); \
     } while (0)
 
-// A wave per row from 33 levels on, where more than half of the lanes have one.
-// One step of one tracer (k_edge_flux, k_node_lo, k_node_limit, k_node_update), us
-// by rows and by pairs: 40 thousand nodes, 47 layers 185, 96, 98, 59 and 205, 130,
-// 131, 70; 20 thousand nodes, 70 layers 122, 66, 72, 44 and 170, 98, 98, 52; 33
-// layers 77, 44, 46, 29 and 83, 49, 54, 32; 24 layers 63, 40, 44, 29 and 59, 37,
-// 37, 23. The kernels with a few loads per level are bound by those and take pairs.
-static bool cell_rows(const fgpu_context *c) { return c->m.L > 32; }
+// A wave per row from 33 levels on, where more than half of the lanes have one,
+// for the edge flux from 41. One step of one tracer, us by rows and by pairs
+// (k_node_grad, k_node_lo, k_node_limit, k_node_update; k_edge_flux): 40 thousand
+// nodes, 47 layers 38, 97, 97, 59; 132 and 55, 128, 129, 70; 136. 20 thousand
+// nodes, 70 layers 29, 69, 72, 44; 89 and 43, 98, 96, 52; 96. 33 layers 20, 45, 45,
+// 29; 57 and 26, 48, 54, 33; 46. 24 layers 19, 39, 43, 29; 47 and 17, 35, 36, 23;
+// 33. The kernels with a few loads per level are bound by those and take pairs.
+#define ROW_LEVELS 33
+#define ROW_LEVELS_EDGE 41
 // a kernel over the levels of `rows` rows, for ntr tracers
-#define CELL_LAUNCH(kern, rows, ntr, ...)                                                                         \
+#define CELL_LAUNCH(kern, levels, rows, ntr, ...)                                                                         \
     do {                                                                                                          \
         const DevMesh &m_ = c->m;                                                                                 \
-        if (cell_rows(c))                                                                                         \
+        if (m_.L >= levels)                                                                                       \
             hipLaunchKernelGGL(kern<true>, dim3(xcd_grid((rows + BLK / 64 - 1) / (BLK / 64)), ntr, (m_.L + 63) / 64), \
                                dim3(BLK), 0, c->stream, __VA_ARGS__);                                             \
         else hipLaunchKernelGGL(kern<false>, dim3(nblk((size_t)rows * m_.L), ntr), dim3(BLK), 0, c->stream, __VA_ARGS__); \
@@ -708,6 +725,10 @@ static int launch_init_ab(fgpu_context *c, int tr0, int ntr)
         hipLaunchKernelGGL(k_tr_xy, dim3(nblk((size_t)c->m.F2 * c->m.L), ntr), dim3(BLK), 0, c->stream, m, c->t, tr0);
         LAUNCH_CHECK("k_tr_xy");
     }
+    {
+        ProfScope ps(c, "k_node_grad");
+        CELL_LAUNCH(k_node_grad, ROW_LEVELS, c->m.N2, ntr, m, c->t, tr0);
+    }
     return FGPU_OK;
 }
 
@@ -717,11 +738,11 @@ static int launch_adv(fgpu_context *c, int tr0, int ntr, double dt, int mode)
     const size_t nE = (size_t)m.E2 * m.L, nF = (size_t)m.F2 * m.L, nN = c->t.sN;
     {
         ProfScope ps(c, "k_edge_flux");
-        CELL_LAUNCH(k_edge_flux, c->m.E2, ntr, m, c->d, c->t, tr0);
+        CELL_LAUNCH(k_edge_flux, ROW_LEVELS_EDGE, c->m.E2, ntr, m, c->d, c->t, tr0);
     }
     {
         ProfScope ps(c, "k_node_lo");
-        CELL_LAUNCH(k_node_lo, c->m.N2, ntr, m, c->d, c->t, tr0, dt);
+        CELL_LAUNCH(k_node_lo, ROW_LEVELS, c->m.N2, ntr, m, c->d, c->t, tr0, dt);
     }
     if (c->d.wsplit) {
         ProfScope ps(c, "k_vert_impl");   // adv_tra_vert_impl on the LO solution of the FCT tracers
@@ -735,7 +756,7 @@ static int launch_adv(fgpu_context *c, int tr0, int ntr, double dt, int mode)
     }
     {
         ProfScope ps(c, "k_node_limit");
-        CELL_LAUNCH(k_node_limit, c->m.N2, ntr, m, c->t, tr0, dt);
+        CELL_LAUNCH(k_node_limit, ROW_LEVELS, c->m.N2, ntr, m, c->t, tr0, dt);
     }
     {
         ProfScope ps(c, "k_edge_limit");
@@ -748,7 +769,7 @@ static int launch_adv(fgpu_context *c, int tr0, int ntr, double dt, int mode)
     }
     {
         ProfScope ps(c, "k_node_update");
-        CELL_LAUNCH(k_node_update, c->m.N2, ntr, m, c->d, c->t, tr0, dt, mode);
+        CELL_LAUNCH(k_node_update, ROW_LEVELS, c->m.N2, ntr, m, c->d, c->t, tr0, dt, mode);
     }
     return FGPU_OK;
 }
@@ -761,7 +782,11 @@ extern "C" int fgpu_init_tracers_AB(fgpu_context *c, int tr_num)
     if ((rc = fgpu_ensure_staged(c, 1))) return rc;
     const int tr = tr_num - 1;
     if ((rc = launch_init_ab(c, tr, 1))) return rc;
-    CELL_LAUNCH(k_fill_up_dn_grad, c->m.E2, 1, c->m, c->t, tr);
+    {
+        ProfScope ps(c, "k_fill_up_dn_grad");
+        hipLaunchKernelGGL(k_fill_up_dn_grad, dim3(nblk((size_t)c->m.E2 * c->m.L)), dim3(BLK), 0, c->stream, c->m, c->t, tr);
+        LAUNCH_CHECK("k_fill_up_dn_grad");
+    }
     FGPU_HIP(hipStreamSynchronize(c->stream));
     return FGPU_OK;
 }
@@ -783,6 +808,7 @@ extern "C" int fgpu_tracer_set_valuesAB(fgpu_context *c, int tr_num, const doubl
                             c->stream));
     hipLaunchKernelGGL(k_tr_xy, dim3(nblk((size_t)c->m.F2 * c->m.L), 1), dim3(BLK), 0, c->stream, c->m, c->t, tr);
         LAUNCH_CHECK("k_tr_xy");
+    CELL_LAUNCH(k_node_grad, ROW_LEVELS, c->m.N2, 1, c->m, c->t, tr);
     FGPU_HIP(hipStreamSynchronize(c->stream));
     return FGPU_OK;
 }

@@ -150,7 +150,7 @@ def test_extra_schemes_and_terms(layers, ntr, split, diffusion):
 
 
 @pytest.mark.parametrize("ivd,split", [(True, False), (False, False), (True, True)])
-@pytest.mark.parametrize("layers", [32, 33, 64, 65, 127])
+@pytest.mark.parametrize("layers", [32, 33, 40, 41, 64, 65, 127])
 def test_per_tracer_calls(layers, ivd, split):
     """The per-tracer calls, by (row, level) pairs up to 32 levels and by rows of
     up to 64 levels per wave beyond, with the diffusion terms and the W split."""
