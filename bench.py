@@ -46,14 +46,16 @@ def kernel_bytes(name, mesh, ntr):
     N3, E3, F3 = mesh.n3, mesh.e3, mesh.f3
     NI = N3 + N2
     lists = 4 * (N2 + 1) + 8 * E2           # node -> edge gather lists
-    if name == "kA_edge":                    # T^n, T^n-1 ; LO_h, A_h | uv, helem, edge/elem geometry
-        return ntr * (16 * N3 + 16 * E3) + 24 * F3 + 88 * E2 + 76 * F2 + 24 * N2
-    if name == "kB_node":                    # LO_h, T^n, T^n-1 ; LO, A_v | w, w_e, area, zbar, Z, h, h_new, areasvol
-        return ntr * (8 * E3 + 16 * N3 + 8 * N3 + 8 * NI) + 32 * NI + 32 * N3 + lists + 8 * E2 + 8 * N2
+    if name == "kA_edge":                    # T^n, T^n-1 ; A_h | volume flux, uv, helem, edge/elem geometry
+        return ntr * (16 * N3 + 8 * E3) + 8 * E3 + 24 * F3 + 88 * E2 + 76 * F2 + 24 * N2
+    if name == "kB_node":                    # T^n, T^n-1 ; LO, A_v | volume flux, w, w_e, area, zbar, Z, h, h_new, areasvol
+        return ntr * (16 * N3 + 8 * N3 + 8 * NI) + 8 * E3 + 32 * NI + 32 * N3 + lists + 8 * E2 + 8 * N2
     if name == "kC_node":                    # LO, T^n, A_v, A_h ; R+, R- | h_new, areasvol, edge info
         return ntr * (16 * N3 + 8 * NI + 8 * E3 + 16 * N3) + 16 * N3 + lists + 32 * E2 + 8 * N2
-    if name == "kD_node":                    # R+-, A_v, A_h, LO, T^n ; T^n+1, T^n -> valuesold | h, h_new, areasvol, area, Kv
-        return ntr * (16 * N3 + 8 * NI + 8 * E3 + 16 * N3 + 16 * N3) + 32 * N3 + 8 * NI + lists + 16 * E2 + 16 * N2
+    if name == "kL_node":                    # R+-, A_v, A_h, LO, T^n ; T*, T^n -> valuesold | h, h_new, areasvol
+        return ntr * (16 * N3 + 8 * NI + 8 * E3 + 16 * N3 + 16 * N3) + 24 * N3 + lists + 16 * E2 + 16 * N2
+    if name == "kV_cols":                    # T* ; T^n+1 | h_new, areasvol, area, Kv
+        return ntr * 16 * N3 + 16 * N3 + 16 * NI + 16 * N2
     # staged per-stage kernels (FGPU_STEP=staged)
     if name == "k_init_ab":
         return ntr * 32 * N2 * L

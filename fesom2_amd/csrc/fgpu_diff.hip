@@ -21,7 +21,7 @@
 // against one thread per column, whose neighbours in a wave read rows apart.
 //
 // They write the increments' parts (t.hd, t.ve, t.vr); the node update of
-// either step (k_node_update / k_tstar, kD_node) adds them to del_ttf in the
+// either step (k_node_update / k_tstar, kL_node) adds them to del_ttf in the
 // reference's order: advection, edges in ascending order, explicit vertical,
 // explicit Redi, then the T* update. Arithmetic keeps the reference's
 // evaluation order, so the sums are bit-identical to a serial run.
