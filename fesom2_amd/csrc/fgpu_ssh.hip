@@ -186,36 +186,6 @@ __device__ __forceinline__ double strided_sum(const double *v, int n)
     return a;
 }
 
-// butterfly sum over the wave (lanes 32, 16, 8, 4, 2 and 1 apart), the same in
-// every lane. By lane swaps and DPP moves, which take a register's latency where
-// a shuffle through LDS takes some 100 cycles: 0.4 us of a solver kernel's 8.
-// After the first three steps values repeat every eight lanes, so a rotation by
-// four serves as the exchange.
-template <int CTRL>
-__device__ __forceinline__ double dpp_moved(double x)
-{
-    const long long b = __double_as_longlong(x);
-    const int l = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), CTRL, 0xf, 0xf, false);
-    const int h = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, false);
-    return __longlong_as_double(((long long)h << 32) | (unsigned int)l);
-}
-__device__ __forceinline__ double wave_sum(double x)
-{
-    long long b = __double_as_longlong(x);
-    auto l = __builtin_amdgcn_permlane32_swap((unsigned)b, (unsigned)b, false, false);
-    auto h = __builtin_amdgcn_permlane32_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
-    x = __longlong_as_double(((long long)h[0] << 32) | l[0]) + __longlong_as_double(((long long)h[1] << 32) | l[1]);
-    b = __double_as_longlong(x);
-    l = __builtin_amdgcn_permlane16_swap((unsigned)b, (unsigned)b, false, false);
-    h = __builtin_amdgcn_permlane16_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
-    x = __longlong_as_double(((long long)h[0] << 32) | l[0]) + __longlong_as_double(((long long)h[1] << 32) | l[1]);
-    x += dpp_moved<0x128>(x);   // row_ror:8
-    x += dpp_moved<0x124>(x);   // row_ror:4
-    x += dpp_moved<0x4e>(x);    // quad_perm 2,3,0,1
-    x += dpp_moved<0xb1>(x);    // quad_perm 1,0,3,2
-    return x;
-}
-
 // block reduction of up to three values: within each wave, then the
 // wave sums in wave order; the result is valid in every
 // thread and identical in every block for identical inputs
