@@ -84,3 +84,36 @@ def test_one_kernel_solve_bitwise(monkeypatch, n, loop):
             assert {k: st[k] for k in st if k != "ms"} == {k: su[k] for k in su if k != "ms"}
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("n,longest", [(2, 0), (63, 8), (64, 40), (65, 9), (1000, 300), (140000, 20)])
+def test_learned_any_row_length(n, longest):
+    """The network on full and partial tiles and rows of any length against its
+    CPU reference, to that reference's bf16 tolerance, and the flexible CG with
+    the untrained network, also on more rows than threads."""
+    from fesom2_amd import gpu
+    from oracle import mpnn_ref as nn
+    rowptr, colind, val, a = _matrix(n, longest, n)
+    rng = np.random.default_rng(n)
+    b = rng.normal(size=n)
+    print(f"[gpu] learned, {n} rows, longest {np.diff(rowptr).max()}", flush=True)
+    ctx = gpu.Context()
+    try:
+        ctx.ssh_set_matrix(rowptr, colind, val)
+        ctx.ssh_solve_preconditioner(2)
+        ctx.nn_init(0)
+        x, st = ctx.ssh_solve_learned(np.zeros(n), b, 1e-10)
+        if n <= 1000:
+            p = nn.init_params(4)
+            p["w_out"] = rng.normal(0, 0.2, nn.C).astype(np.float32)
+            ctx.nn_set_weights(nn.flatten(p))
+            ctx.N2 = n   # as mesh_init sets it: the wrapper's output size
+            z = ctx.nn_apply(b)
+            ref, _ = nn.forward(nn.Graph(rowptr - 1, colind - 1, val), p, b)
+            assert np.linalg.norm(z - ref) < 2e-2 * np.linalg.norm(ref)
+    finally:
+        ctx.close()
+    assert st["converged"]
+    scale = np.sqrt(np.mean((abs(a) @ abs(x)) ** 2))
+    bound = 1e-10 * np.sqrt(np.mean(b * b)) + (2 * st["iters"] + np.diff(rowptr).max()) * 2.3e-16 * scale
+    assert np.sqrt(np.mean((b - a @ x) ** 2)) <= bound
