@@ -1316,8 +1316,10 @@ void fgpu_kd_shape(const fgpu_context *c, int *tch_out, int *cpb_out)
 // The lanes of the column waves: NV levels per lane and GT tracers per wave, so
 // that a lane group holds every interface of a column (NV x 64 / GT >= NL). Two
 // tracers share a wave where they share its scheme branches and both rows lie
-// within a 32-bit offset of the wave's base. The lines between the mappings were
-// measured per kernel, in us, at 47 layers with 2 tracers (126,858 nodes) and 32
+// within a 32-bit offset of the wave's base; from 65 to 96 interfaces on also
+// beyond, with 64-bit offsets: at 1.3 million nodes, 70 layers, 10 tracers K_B
+// takes 16.4 ms by <3,2> and 22.6 by <2,1> with 32-bit ones, K_L 21.9 and 22.1.
+// The lines between the mappings were measured per kernel, in us, at 47 layers with 2 tracers (126,858 nodes) and 32
 // tracers (12 thousand), and at 70 layers with 10 tracers (40 thousand):
 //   K_A  <1,1> 473, 567; <2,2> 502, 430 | <2,1> 728, <3,2> 744
 //   K_B  <1,1> 298, 270; <2,2> 349, 297 | <2,1> 591, <3,2> 520
@@ -1331,6 +1333,7 @@ void fgpu_kd_shape(const fgpu_context *c, int *tch_out, int *cpb_out)
 struct ColLanes {
     bool pair;    // tracers two to a wave
     bool wide;    // row offsets need 64 bits
+    bool wide2;   // those of a pair do
 };
 static ColLanes col_lanes(const fgpu_context *c, int tpb)
 {
@@ -1341,18 +1344,19 @@ static ColLanes col_lanes(const fgpu_context *c, int tpb)
         same = same && c->h_lim[i] == c->h_lim[0] && c->h_abo[i] == c->h_abo[0] && c->h_hor[i] == c->h_hor[0] &&
                c->h_ver[i] == c->h_ver[0] && c->h_ph[i] == c->h_ph[0] && c->h_pv[i] == c->h_pv[0];
     const size_t reach = c->step_wide ? 0 : 0xffffffffu;
-    return {same && std::min(tpb, t.ntr) >= 2 && 2 * field < (size_t)0xffffffffu, field >= reach};
+    const bool far = 2 * field >= (size_t)0xffffffffu, deep = c->m.NL > 64 && c->m.NL <= 96;
+    return {same && std::min(tpb, t.ntr) >= 2 && (!far || deep), field >= reach, far || field >= reach};
 }
 
 #define COL_LAUNCH(kern, NV, GT, grid, ...)                                                                          \
     do {                                                                                                             \
-        if (wide) hipLaunchKernelGGL((kern<size_t, NV, GT>), grid, dim3(64), 0, c->stream, __VA_ARGS__);             \
+        if (GT > 1 ? cl.wide2 : cl.wide) hipLaunchKernelGGL((kern<size_t, NV, GT>), grid, dim3(64), 0, c->stream, __VA_ARGS__);             \
         else hipLaunchKernelGGL((kern<unsigned, NV, GT>), grid, dim3(64), 0, c->stream, __VA_ARGS__);                \
     } while (0)
 
 #define COL_LAUNCH_X(kern, NV, GT, X, grid, ...)                                                                     \
     do {                                                                                                             \
-        if (wide) hipLaunchKernelGGL((kern<size_t, NV, GT, X>), grid, dim3(64), 0, c->stream, __VA_ARGS__);          \
+        if (GT > 1 ? cl.wide2 : cl.wide) hipLaunchKernelGGL((kern<size_t, NV, GT, X>), grid, dim3(64), 0, c->stream, __VA_ARGS__);          \
         else hipLaunchKernelGGL((kern<unsigned, NV, GT, X>), grid, dim3(64), 0, c->stream, __VA_ARGS__);             \
     } while (0)
 #define COL_LAUNCH_D(kern, NV, GT, dx, grid, ...)                                                                    \
@@ -1412,7 +1416,7 @@ int fgpu_enqueue_fused_step(fgpu_context *c, double dt)
     const bool narrow = m.NL <= 64, slim = m.NL <= 32;
     const dim3 nodes(xcd_grid(m.N2), ny), edges(xcd_grid(m.E2), ny);
     const ColLanes cl = col_lanes(c, tpb);
-    const bool pair = cl.pair, wide = cl.wide, many = pair && std::min(tpb, nt) >= 4;
+    const bool pair = cl.pair, many = pair && std::min(tpb, nt) >= 4;
     {
         ProfScope ps(c, "kG_node");
         hipLaunchKernelGGL(kG_node, nodes, dim3(64), 0, c->stream, m, c->t, c->d_kneed, tpb);
