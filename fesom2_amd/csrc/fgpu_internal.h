@@ -194,6 +194,7 @@ struct DevTracers {
     double *T, *Told;
     double *a_h;              // E2*L
     double *vf;               // E2*L, all tracers': volume flux through an edge per level
+    double *vf2;              // E2*L, on a mesh with a level gap across an edge: the lower element's flux in the gaps
     double *lo_h;             // E2*L, per-stage kernels
     double *fct_lo;           // N2*L
     double *a_v;              // N2*NL

@@ -972,15 +972,16 @@ extern "C" int fgpu_tracers_init(fgpu_context *c, int num_tracers)
     t.sStg = 0;
     int rc;
     t.lo_h = t.TAB = t.tr_xy = t.aux = t.dttf_h = t.dttf_v = t.dbg_av = t.dbg_grad = t.ngrad = nullptr;
-    t.hd = t.ve = t.vr = t.zbh = nullptr;
+    t.hd = t.ve = t.vr = t.zbh = t.vf2 = nullptr;
     c->stage_slots = 0;
     // the fused batched step needs only these; the per-stage buffers come with
     // the first per-tracer call (fgpu_ensure_staged)
     struct A { double **p; size_t n; } arrs[] = {
         {&t.T, t.sN * nt}, {&t.Told, t.sOld * nt}, {&t.a_h, t.sE * nt}, {&t.vf, t.sE},
         {&t.fct_lo, t.sN * nt}, {&t.a_v, t.sNI * nt}, {&t.rp, t.sN * nt}, {&t.rm, t.sN * nt},
-        {&t.gmean, t.sG * nt}};
+        {&t.gmean, t.sG * nt}, {&t.vf2, c->edge_gap ? t.sE : 0}};
     for (auto &a : arrs) {
+        if (a.n == 0) continue;
         if ((rc = fgpu_alloc(c, (void **)a.p, a.n * sizeof(double), true))) return rc;
         FGPU_HIP(hipMemset(*a.p, 0, a.n * sizeof(double)));
     }

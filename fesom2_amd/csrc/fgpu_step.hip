@@ -239,6 +239,14 @@ __device__ __forceinline__ void edge_offsets(const DevMesh &m, const DevTracers 
     oe = lev + 8 * (OFF)c.g * (OFF)t.sE + 8 * (OFF)(r[0] >> 1) * (OFF)m.L;
 }
 
+// the levels g0..g1 between the elements of a column's edge where those share none: none on most edges (g0 > g1)
+__device__ __forceinline__ void edge_gap(const DevMesh &m, int p, int &g0, int &g1)
+{
+    const i32x8 r = ldc((const i32x8 *)m.col_ne + p);   // [4..7]: nl1, nu1, nl2, nu2
+    g0 = min(r[4], r[6]) + 1;
+    g1 = r[7] > 0 ? max(r[5], r[7]) - 1 : 0;
+}
+
 template <bool LANES_OFF, typename OFF, int NV, int GT>
 __device__ __forceinline__ bool load_column(const DevMesh &m, const DevTracers &t, Column<OFF, NV, GT> &c)
 {
@@ -285,7 +293,11 @@ __device__ __forceinline__ bool load_column(const DevMesh &m, const DevTracers &
 // a LO flux per tracer. 126,858 nodes, 47 layers, 2 tracers: 544 -> 473 us; 12
 // thousand nodes, 32 tracers: 689 -> 430; 40 thousand nodes, 70 layers, 10
 // tracers: 1067 -> 730.
-template <typename OFF, int NV, int GT>
+// GAP is the form for a mesh with a level gap across some edge: the reference's
+// segments of both elements reach into the gap (oce_adv_tra_hor.F90:166-249),
+// the upper element's first, so two fluxes follow each other there. K_B and K_C
+// have the form too; other meshes do not carry its registers.
+template <typename OFF, int NV, int GT, bool GAP>
 __global__ void __launch_bounds__(64) kA_edge(DevMesh m, DevDyn d, DevTracers t, int tpb)
 {
     const int lane = threadIdx.x;
@@ -310,8 +322,8 @@ __global__ void __launch_bounds__(64) kA_edge(DevMesh m, DevDyn d, DevTracers t,
         ow[j] = gN + 8 * (OFF)ldc(ri + ER_DA0 + j) * (OFF)L;
     }
     // volume flux per level: the elements with that level add up
-    double vf[NV];
-    bool act[NV], mean[NV], any_mean = false;
+    double vf[NV], vl[GAP ? NV : 1];   // vl: the lower element's at a gap's levels, vf the upper one's
+    bool act[NV], mean[NV], gap[GAP ? NV : 1], any_mean = false;
     {
         const double dX1 = ldc(rd + ER_DX1), dY1 = ldc(rd + ER_DY1), dX2 = ldc(rd + ER_DX2), dY2 = ldc(rd + ER_DY2);
         double uv1[2 * NV], h1[NV], uv2[2 * NV], h2[NV];
@@ -329,6 +341,13 @@ __global__ void __launch_bounds__(64) kA_edge(DevMesh m, DevDyn d, DevTracers t,
             const double f2 = (uv2[2 * s + 1] * dX2 - uv2[2 * s] * dY2) * h2[s];
             vf[s] = in1 ? (in2 ? f1 + f2 : f1) : f2;
             act[s] = in1 || in2;
+            if constexpr (GAP) {
+                const bool under1 = nu2 > 0 && k > nl1 && k < nu2, under2 = nu2 > 0 && k > nl2 && k < nu1;
+                gap[s] = under1 || under2;
+                vf[s] = under1 ? f1 : vf[s];
+                vl[s] = under1 ? f2 : f1;
+                act[s] = act[s] || gap[s];
+            }
             // fill_up_dn_grad (oce_muscl_adv.F90:375-520): the triangles' gradients at the levels their
             // nodes share (an empty range without both triangles), else the node means
             mean[s] = act[s] && !(k >= s0 && k <= s1 - 1);
@@ -344,7 +363,10 @@ __global__ void __launch_bounds__(64) kA_edge(DevMesh m, DevDyn d, DevTracers t,
     const double edxa = ldc(rd + ER_EDX) * ldc(rd + ER_A), edyr = ldc(rd + ER_EDY) * FGPU_R_EARTH;
     const OFF oE = lev + 8 * (OFF)g * (OFF)t.sE;
     const int trb = blockIdx.y * tpb, tre = min(t.ntr, trb + tpb);
-    if (trb == 0 && g == 0) row_store<NV>(t.vf + (size_t)e * L, lev, vf, act);   // K_B forms the LO fluxes again from it
+    if (trb == 0 && g == 0) {   // K_B forms the LO fluxes again from it
+        row_store<NV>(t.vf + (size_t)e * L, lev, vf, act);
+        if constexpr (GAP) row_store<NV>(t.vf2 + (size_t)e * L, lev, vl, gap);
+    }
     for (int tb = trb; tb < tre; tb += GT) {
         if (GT > 1 && tb + g >= tre) return;   // the last group's missing tracers
         const double *T = t.T + t.sN * tb, *Told = t.Told + t.sOld * tb;
@@ -381,7 +403,11 @@ __global__ void __launch_bounds__(64) kA_edge(DevMesh m, DevDyn d, DevTracers t,
         double f[NV];
         if (lim == LIM_FCT) {
 #pragma unroll
-            for (int s = 0; s < NV; ++s) f[s] = -0.5 * (T1[s] * vp[s] + T2[s] * vm[s]) - 0.0;
+            for (int s = 0; s < NV; ++s) {
+                f[s] = -0.5 * (T1[s] * vp[s] + T2[s] * vm[s]) - 0.0;
+                if constexpr (GAP)
+                    if (gap[s]) f[s] = -0.5 * (T1[s] * (vl[s] + fabs(vl[s])) + T2[s] * (vl[s] - fabs(vl[s]))) - f[s];
+            }
         } else {
 #pragma unroll
             for (int s = 0; s < NV; ++s) f[s] = 0.0;
@@ -440,10 +466,19 @@ __global__ void __launch_bounds__(64) kA_edge(DevMesh m, DevDyn d, DevTracers t,
                 const double Tmean2 = A2[s] - c2[s], Tmean1 = A1[s] + c1[s];
                 const double cHO = vp[s] * Tmean1 + vm[s] * Tmean2;
                 f[s] = -0.5 * (1.0 - no) * cHO - vf[s] * no * 0.5 * (Tmean1 + Tmean2) - f[s];
+                if constexpr (GAP)
+                    if (gap[s]) {
+                        const double c = (vl[s] + fabs(vl[s])) * Tmean1 + (vl[s] - fabs(vl[s])) * Tmean2;
+                        f[s] = -0.5 * (1.0 - no) * c - vl[s] * no * 0.5 * (Tmean1 + Tmean2) - f[s];
+                    }
             }
         } else {
 #pragma unroll
-            for (int s = 0; s < NV; ++s) f[s] = -0.5 * (A1[s] * vp[s] + A2[s] * vm[s]) - f[s];
+            for (int s = 0; s < NV; ++s) {
+                f[s] = -0.5 * (A1[s] * vp[s] + A2[s] * vm[s]) - f[s];
+                if constexpr (GAP)
+                    if (gap[s]) f[s] = -0.5 * (A1[s] * (vl[s] + fabs(vl[s])) + A2[s] * (vl[s] - fabs(vl[s]))) - f[s];
+            }
         }
         row_store<NV>(t.a_h + t.sE * tb + (size_t)e * L, oE, f, act);
     }
@@ -464,9 +499,12 @@ __global__ void __launch_bounds__(64) kA_edge(DevMesh m, DevDyn d, DevTracers t,
 // it). PPM reads up to four layers around an interface, from LDS. 20 thousand
 // nodes, 47 layers, 4 tracers, W split: 140 us and 45 for the implicit step, 367
 // with a block per column, its sweeps on one lane.
-template <typename OFF, int NV, int GT, bool EXTRA>
+#define KB_EXTRA 1
+#define KB_GAP 2
+template <typename OFF, int NV, int GT, int FORM>
 __global__ void __launch_bounds__(64) kB_cols(DevMesh m, DevDyn d, DevTracers t, double dt, int tpb)
 {
+    constexpr bool EXTRA = (FORM & KB_EXTRA) != 0, GAP = (FORM & KB_GAP) != 0;
     Column<OFF, NV, GT> c;
     if (!load_column<(NV > 1), OFF, NV, GT>(m, t, c)) return;
     static_assert(!EXTRA || GT == 1, "one column's rows in LDS");
@@ -618,8 +656,26 @@ __global__ void __launch_bounds__(64) kB_cols(DevMesh m, DevDyn d, DevTracers t,
         for (int s = 0; s < NV; ++s) acc[s] = 0.0;
         int kb = c.kb;
         if constexpr (NV > 1) asm volatile("" : "+v"(kb));   // the level masks are formed in place: they would not fit the scalar registers
-        auto add = [&](int side, const double (&v)[NV], const double (&to)[NV], int a0, int len)
+        auto add = [&](int u, OFF oe, int side, const double (&v)[NV], const double (&to)[NV], int a0, int len)
             __attribute__((always_inline)) {
+            if constexpr (GAP) {
+                int g0, g1;
+                edge_gap(m, c.p0 + u, g0, g1);
+                if (g0 <= g1) {   // the edge's levels one by one, both fluxes in the gap
+                    double w[NV];
+                    row_load<NV>(t.vf2, oe - 8 * (OFF)c.g * (OFF)t.sE, w);
+#pragma unroll
+                    for (int s = 0; s < NV; ++s) {
+                        const double x1 = side ? to[s] : Tk[s], x2 = side ? Tk[s] : to[s];
+                        double z = -0.5 * (x1 * (v[s] + fabs(v[s])) + x2 * (v[s] - fabs(v[s]))) - 0.0;
+                        const double zl = -0.5 * (x1 * (w[s] + fabs(w[s])) + x2 * (w[s] - fabs(w[s]))) - z;
+                        z = kb + s >= g0 && kb + s <= g1 ? zl : z;
+                        const double x = side ? acc[s] - z : acc[s] + z;
+                        acc[s] = edge_has(kb, s, a0, len) ? x : acc[s];
+                    }
+                    return;
+                }
+            }
             // side 0: acc + -0.5 (Tk (v + |v|) + to (v - |v|)); side 1: acc - -0.5 (to (v + |v|) + Tk (v - |v|))
             const long long sgn = (long long)side << 63;
             const double half = side ? 0.5 : -0.5;
@@ -641,7 +697,7 @@ __global__ void __launch_bounds__(64) kB_cols(DevMesh m, DevDyn d, DevTracers t,
                 }
 #pragma unroll
                 for (int u = 0; u < NB; ++u)
-                    if (u0 + u < CE && u0 + u < c.deg) add(c.side[u0 + u], vf[VREG ? u0 + u : u], tm[u], c.a0[u0 + u], c.len[u0 + u]);
+                    if (u0 + u < CE && u0 + u < c.deg) add(u0 + u, c.oe[u0 + u], c.side[u0 + u], vf[VREG ? u0 + u : u], tm[u], c.a0[u0 + u], c.len[u0 + u]);
             }
         }
         for (int u = CE; u < c.deg; ++u) {
@@ -651,7 +707,7 @@ __global__ void __launch_bounds__(64) kB_cols(DevMesh m, DevDyn d, DevTracers t,
             double v[NV], to[NV];
             row_load<NV>(t.vf, oe - 8 * (OFF)c.g * (OFF)t.sE, v);
             row_load<NV>(T, on, to);
-            add(side, v, to, a0, len);
+            add(u, oe, side, v, to, a0, len);
         }
         double ld[NV], o[NV];
         col_down<NV>(lk, ld);
@@ -671,7 +727,9 @@ __global__ void __launch_bounds__(64) kB_cols(DevMesh m, DevDyn d, DevTracers t,
 // ------------------------------------------------------------------------------
 // 126,858 nodes, 47 layers, 2 tracers: 344 -> 295 us; 12 thousand nodes, 32
 // tracers: 520 -> 395; 40 thousand nodes, 70 layers, 10 tracers: 744 -> 610.
-template <typename OFF, int NV, int GT>
+// GAP: in a level gap neither element has the level, and the other node is no
+// part of its bounds.
+template <typename OFF, int NV, int GT, bool GAP>
 __global__ void __launch_bounds__(64) kC_cols(DevMesh m, DevTracers t, double dt, int tpb)
 {
     Column<OFF, NV, GT> c;
@@ -710,19 +768,22 @@ __global__ void __launch_bounds__(64) kC_cols(DevMesh m, DevTracers t, double dt
         };
         int kb = c.kb;
         if constexpr (NV > 1) asm volatile("" : "+v"(kb));   // see K_B
-        auto add = [&](int side, const double (&a)[NV], const double (&b)[NV], const double (&x)[NV], int a0, int len)
+        auto add = [&](int u, int side, const double (&a)[NV], const double (&b)[NV], const double (&x)[NV], int a0, int len)
             __attribute__((always_inline)) {
             const long long sgn = (long long)side << 63;
+            int g0 = 1, g1 = 0;
+            if constexpr (GAP) edge_gap(m, c.p0 + u, g0, g1);
 #pragma unroll
             for (int s = 0; s < NV; ++s) {
                 const bool has = edge_has(kb, s, a0, len);
-                if constexpr (NV == 1) {   // outside the edge's levels a and b are the column's own values
+                if constexpr (NV == 1 && !GAP) {   // outside the edge's levels a and b are the column's own values
                     vmax[s] = dmx(vmax[s], dmx(a[s], b[s]));
                     vmin[s] = dmn(vmin[s], dmn(a[s], b[s]));
                 } else {
                     const double hi = dmx(vmax[s], dmx(a[s], b[s])), lw = dmn(vmin[s], dmn(a[s], b[s]));
-                    vmax[s] = has ? hi : vmax[s];
-                    vmin[s] = has ? lw : vmin[s];
+                    const bool in = has && !(GAP && kb + s >= g0 && kb + s <= g1);
+                    vmax[s] = in ? hi : vmax[s];
+                    vmin[s] = in ? lw : vmin[s];
                 }
                 const double y = has ? signed_by(x[s], sgn) : 0.0;
                 p[s] = p[s] + dmx(0.0, y);
@@ -746,7 +807,7 @@ __global__ void __launch_bounds__(64) kC_cols(DevMesh m, DevTracers t, double dt
                 if (u0 > 0) load(u0);
 #pragma unroll
                 for (int u = 0; u < NB; ++u)
-                    if (u0 + u < CE && u0 + u < c.deg) add(c.side[u0 + u], lm[u], tm[u], fl[u], c.a0[u0 + u], c.len[u0 + u]);
+                    if (u0 + u < CE && u0 + u < c.deg) add(u0 + u, c.side[u0 + u], lm[u], tm[u], fl[u], c.a0[u0 + u], c.len[u0 + u]);
             }
         }
         for (int u = CE; u < c.deg; ++u) {
@@ -757,7 +818,7 @@ __global__ void __launch_bounds__(64) kC_cols(DevMesh m, DevTracers t, double dt
             row_load<NV>(LO, on, a);
             row_load<NV>(T, on, b);
             row_load<NV>(ah, oe, x);
-            add(side, a, b, x, a0, len);
+            add(u, side, a, b, x, a0, len);
         }
         double mxu[NV], mxd[NV], mnu[NV], mnd[NV], rp[NV], rm[NV];
         col_up<NV>(vmax, mxu);
@@ -1348,21 +1409,15 @@ static ColLanes col_lanes(const fgpu_context *c, int tpb)
     return {same && std::min(tpb, t.ntr) >= 2 && (!far || deep), field >= reach, far || field >= reach};
 }
 
-#define COL_LAUNCH(kern, NV, GT, grid, ...)                                                                          \
-    do {                                                                                                             \
-        if (GT > 1 ? cl.wide2 : cl.wide) hipLaunchKernelGGL((kern<size_t, NV, GT>), grid, dim3(64), 0, c->stream, __VA_ARGS__);             \
-        else hipLaunchKernelGGL((kern<unsigned, NV, GT>), grid, dim3(64), 0, c->stream, __VA_ARGS__);                \
-    } while (0)
-
-#define COL_LAUNCH_X(kern, NV, GT, X, grid, ...)                                                                     \
+#define COL_LAUNCH(kern, NV, GT, X, grid, ...)                                                                       \
     do {                                                                                                             \
         if (GT > 1 ? cl.wide2 : cl.wide) hipLaunchKernelGGL((kern<size_t, NV, GT, X>), grid, dim3(64), 0, c->stream, __VA_ARGS__);          \
         else hipLaunchKernelGGL((kern<unsigned, NV, GT, X>), grid, dim3(64), 0, c->stream, __VA_ARGS__);             \
     } while (0)
 #define COL_LAUNCH_D(kern, NV, GT, dx, grid, ...)                                                                    \
     do {                                                                                                             \
-        if (dx) COL_LAUNCH_X(kern, NV, GT, true, grid, __VA_ARGS__);                                                 \
-        else COL_LAUNCH_X(kern, NV, GT, false, grid, __VA_ARGS__);                                                   \
+        if (dx) COL_LAUNCH(kern, NV, GT, true, grid, __VA_ARGS__);                                                 \
+        else COL_LAUNCH(kern, NV, GT, false, grid, __VA_ARGS__);                                                   \
     } while (0)
 
 template <int XF>
@@ -1423,19 +1478,23 @@ int fgpu_enqueue_fused_step(fgpu_context *c, double dt)
     }
     {
         ProfScope ps(c, "kA_edge");
-        if (!narrow) COL_LAUNCH(kA_edge, 2, 1, edges, m, c->d, c->t, tpb);
-        else if (slim && pair) COL_LAUNCH(kA_edge, 1, 2, edges, m, c->d, c->t, tpb);
-        else if (many) COL_LAUNCH(kA_edge, 2, 2, edges, m, c->d, c->t, tpb);
-        else COL_LAUNCH(kA_edge, 1, 1, edges, m, c->d, c->t, tpb);
+        if (c->edge_gap && narrow) COL_LAUNCH(kA_edge, 1, 1, true, edges, m, c->d, c->t, tpb);
+        else if (c->edge_gap) COL_LAUNCH(kA_edge, 2, 1, true, edges, m, c->d, c->t, tpb);
+        else if (!narrow) COL_LAUNCH(kA_edge, 2, 1, false, edges, m, c->d, c->t, tpb);
+        else if (slim && pair) COL_LAUNCH(kA_edge, 1, 2, false, edges, m, c->d, c->t, tpb);
+        else if (many) COL_LAUNCH(kA_edge, 2, 2, false, edges, m, c->d, c->t, tpb);
+        else COL_LAUNCH(kA_edge, 1, 1, false, edges, m, c->d, c->t, tpb);
     }
     {
         ProfScope ps(c, "kB_node");
-        if (extra && narrow) COL_LAUNCH_X(kB_cols, 1, 1, true, nodes, m, c->d, c->t, dt, tpb);
-        else if (extra) COL_LAUNCH_X(kB_cols, 2, 1, true, nodes, m, c->d, c->t, dt, tpb);
-        else if (pair && m.NL > 64 && m.NL <= 96) COL_LAUNCH_X(kB_cols, 3, 2, false, nodes, m, c->d, c->t, dt, tpb);
-        else if (!narrow) COL_LAUNCH_X(kB_cols, 2, 1, false, nodes, m, c->d, c->t, dt, tpb);
-        else if (slim && pair) COL_LAUNCH_X(kB_cols, 1, 2, false, nodes, m, c->d, c->t, dt, tpb);
-        else COL_LAUNCH_X(kB_cols, 1, 1, false, nodes, m, c->d, c->t, dt, tpb);
+        if (c->edge_gap && narrow) COL_LAUNCH(kB_cols, 1, 1, KB_EXTRA | KB_GAP, nodes, m, c->d, c->t, dt, tpb);
+        else if (c->edge_gap) COL_LAUNCH(kB_cols, 2, 1, KB_EXTRA | KB_GAP, nodes, m, c->d, c->t, dt, tpb);
+        else if (extra && narrow) COL_LAUNCH(kB_cols, 1, 1, KB_EXTRA, nodes, m, c->d, c->t, dt, tpb);
+        else if (extra) COL_LAUNCH(kB_cols, 2, 1, KB_EXTRA, nodes, m, c->d, c->t, dt, tpb);
+        else if (pair && m.NL > 64 && m.NL <= 96) COL_LAUNCH(kB_cols, 3, 2, 0, nodes, m, c->d, c->t, dt, tpb);
+        else if (!narrow) COL_LAUNCH(kB_cols, 2, 1, 0, nodes, m, c->d, c->t, dt, tpb);
+        else if (slim && pair) COL_LAUNCH(kB_cols, 1, 2, 0, nodes, m, c->d, c->t, dt, tpb);
+        else COL_LAUNCH(kB_cols, 1, 1, 0, nodes, m, c->d, c->t, dt, tpb);
     }
     if (c->d.wsplit) {
         ProfScope ps(c, "kV_lo");
@@ -1443,10 +1502,12 @@ int fgpu_enqueue_fused_step(fgpu_context *c, double dt)
     }
     {
         ProfScope ps(c, "kC_node");
-        if (!narrow) COL_LAUNCH(kC_cols, 2, 1, nodes, m, c->t, dt, tpb);
-        else if (slim && pair) COL_LAUNCH(kC_cols, 1, 2, nodes, m, c->t, dt, tpb);
-        else if (many) COL_LAUNCH(kC_cols, 2, 2, nodes, m, c->t, dt, tpb);
-        else COL_LAUNCH(kC_cols, 1, 1, nodes, m, c->t, dt, tpb);
+        if (c->edge_gap && narrow) COL_LAUNCH(kC_cols, 1, 1, true, nodes, m, c->t, dt, tpb);
+        else if (c->edge_gap) COL_LAUNCH(kC_cols, 2, 1, true, nodes, m, c->t, dt, tpb);
+        else if (!narrow) COL_LAUNCH(kC_cols, 2, 1, false, nodes, m, c->t, dt, tpb);
+        else if (slim && pair) COL_LAUNCH(kC_cols, 1, 2, false, nodes, m, c->t, dt, tpb);
+        else if (many) COL_LAUNCH(kC_cols, 2, 2, false, nodes, m, c->t, dt, tpb);
+        else COL_LAUNCH(kC_cols, 1, 1, false, nodes, m, c->t, dt, tpb);
     }
     {
         ProfScope ps(c, "kL_node");

@@ -865,16 +865,10 @@ extern "C" int fgpu_diff_ver_part_impl_ale(fgpu_context *c, double dt, int tr_nu
     return FGPU_OK;
 }
 
-// The fused step takes a level of an edge as belonging to its first element,
-// its second or both. Where the elements' level ranges leave a gap between
-// them, the reference's segments reach into it (oce_adv_tra_hor.F90:166-249)
-// and two of them meet: such a mesh steps through the per-stage kernels.
-static bool step_fused(const fgpu_context *c) { return c->fused && !c->edge_gap; }
-
 // one batched step of every tracer, enqueued on the context stream
 static int enqueue_step(fgpu_context *c, double dt)
 {
-    if (step_fused(c)) return fgpu_enqueue_fused_step(c, dt);
+    if (c->fused) return fgpu_enqueue_fused_step(c, dt);
     const int nt = c->t.ntr;
     int rc;
     if ((rc = launch_init_ab(c, 0, nt))) return rc;
@@ -896,7 +890,7 @@ static int check_step(fgpu_context *c)
 static int run_steps(fgpu_context *c, double dt, int nsteps)
 {
     int rc;
-    if (!step_fused(c) && (rc = fgpu_ensure_staged(c, c->t.ntr))) return rc;
+    if (!c->fused && (rc = fgpu_ensure_staged(c, c->t.ntr))) return rc;
     if ((rc = fgpu_ensure_diff(c))) return rc;   // before any capture
     if (c->prof) {
         for (int s = 0; s < nsteps; ++s)
