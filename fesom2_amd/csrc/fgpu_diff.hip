@@ -239,7 +239,7 @@ int fgpu_ensure_diff(fgpu_context *c)
         if (!a.need || *a.p) continue;
         int rc = fgpu_alloc(c, (void **)a.p, a.n * sizeof(double), true);
         if (rc) return rc;
-        FGPU_HIP(hipMemset(*a.p, 0, a.n * sizeof(double)));
+        if ((rc = fgpu_zero(c, *a.p, a.n * sizeof(double)))) return rc;
         c->graph_valid = false;
     }
     return FGPU_OK;

@@ -410,7 +410,7 @@ int ensure_const_buf(fgpu_context *c, const double **p, size_t n)
     double *q = nullptr;
     int rc = fgpu_alloc(c, (void **)&q, sizeof(double) * n);
     if (rc) return rc;
-    FGPU_HIP(hipMemset(q, 0, sizeof(double) * n));
+    if ((rc = fgpu_zero(c, q, sizeof(double) * n))) return rc;
     *p = q;
     return FGPU_OK;
 }

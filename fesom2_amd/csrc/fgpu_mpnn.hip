@@ -963,8 +963,8 @@ static int nn_setup(fgpu_context *c)
         {(void **)&d.loss, sizeof(double)}, {(void **)&d.st, sizeof(FCGState)}};
     for (auto &b : bufs)
         if ((rc = fgpu_alloc(c, b.p, b.bytes))) return rc;
-    FGPU_HIP(hipMemset(d.dpart, 0, sizeof(double) * NSLOT * d.nbd));
-    FGPU_HIP(hipMemset(d.st, 0, sizeof(FCGState)));
+    if ((rc = fgpu_zero(c, d.dpart, sizeof(double) * NSLOT * d.nbd))) return rc;
+    if ((rc = fgpu_zero(c, d.st, sizeof(FCGState)))) return rc;
     // Ahat and its transpose per CSR entry
     std::vector<double> val(nnz);
     FGPU_HIP(hipStreamSynchronize(c->stream));
@@ -1077,8 +1077,8 @@ extern "C" int fgpu_ssh_nn_init(fgpu_context *c, unsigned long long seed)
         for (int k = 0; k < 128 * NNC; ++k) th[OFF_W(l) + k] = (float)(sd * nd(gen));
     NNDev &d = *c->nn;
     FGPU_HIP(hipMemcpy(d.theta, th.data(), sizeof(float) * NNP, hipMemcpyHostToDevice));
-    FGPU_HIP(hipMemset(d.am, 0, sizeof(float) * NNP));
-    FGPU_HIP(hipMemset(d.av, 0, sizeof(float) * NNP));
+    if ((rc = fgpu_zero(c, d.am, sizeof(float) * NNP))) return rc;
+    if ((rc = fgpu_zero(c, d.av, sizeof(float) * NNP))) return rc;
     d.adam_t = 0;
     d.weights = true;
     rc = nn_pack(c);
@@ -1096,8 +1096,8 @@ extern "C" int fgpu_ssh_nn_set_weights(fgpu_context *c, const float *theta, int 
     if (rc) return rc;
     NNDev &d = *c->nn;
     FGPU_HIP(hipMemcpy(d.theta, theta, sizeof(float) * NNP, hipMemcpyHostToDevice));
-    FGPU_HIP(hipMemset(d.am, 0, sizeof(float) * NNP));
-    FGPU_HIP(hipMemset(d.av, 0, sizeof(float) * NNP));
+    if ((rc = fgpu_zero(c, d.am, sizeof(float) * NNP))) return rc;
+    if ((rc = fgpu_zero(c, d.av, sizeof(float) * NNP))) return rc;
     d.adam_t = 0;
     d.weights = true;
     rc = nn_pack(c);

@@ -1325,10 +1325,10 @@ int fgpu_compute_zn(fgpu_context *c)
         double *p;
         int rc = fgpu_alloc(c, (void **)&p, sizeof(double) * (size_t)c->N2 * (c->nl - 1));
         if (rc) return rc;
-        FGPU_HIP(hipMemset(p, 0, sizeof(double) * (size_t)c->N2 * (c->nl - 1)));
+        if ((rc = fgpu_zero(c, p, sizeof(double) * (size_t)c->N2 * (c->nl - 1)))) return rc;
         c->m.zn_vd = p;
         if ((rc = fgpu_alloc(c, (void **)&p, sizeof(double) * (size_t)c->N2 * c->nl))) return rc;
-        FGPU_HIP(hipMemset(p, 0, sizeof(double) * (size_t)c->N2 * c->nl));
+        if ((rc = fgpu_zero(c, p, sizeof(double) * (size_t)c->N2 * c->nl))) return rc;
         c->m.zbn_vd = p;
     }
     hipLaunchKernelGGL(k_zn_vdiff, dim3((c->N2 + 255) / 256), dim3(256), 0, c->stream, c->m, (double *)c->m.zn_vd,

@@ -1,0 +1,71 @@
+"""The library's host code on a stand-in of the HIP runtime (host_runtime.c):
+device memory is host memory and no kernel runs, so these tests see the order
+of calls and the handling of failed allocations, without a GPU. Each runs in a
+process of its own, the stand-in loaded first."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+SETUP = """
+import ctypes, os, sys
+rt = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+rt.host_live_bytes.restype = ctypes.c_size_t
+import numpy as np
+from fesom2_amd import gpu, meshgen as mg
+mesh = mg.build_mesh(nx=12, ny=10, dx=20e3, jitter=0.2, seed=0, cartesian=True, nlayers=8, hmax=4000.0, min_layers=4,
+                     max_layers=8, topo="bumps", bump_height=1500.0)
+st = mg.build_state(mesh, seed=0, ntr=2, dt=600.0, dx=20e3)
+"""
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("hip") / "libhost_runtime.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-o", so, os.path.join(HERE, "host_runtime.c")], check=True)
+    return so
+
+
+def _run(runtime, code, **env):
+    r = subprocess.run([sys.executable, "-c", SETUP + textwrap.dedent(code), runtime], cwd=os.path.dirname(HERE),
+                       env={**os.environ, **env}, capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+    return r.stdout
+
+
+@pytest.mark.parametrize("step", ["fused", "staged"])
+def test_fills_are_done_before_the_stream_uses_them(runtime, step):
+    """Buffers that start at zero are filled before anything of the context's
+    stream can read or write them."""
+    _run(runtime, """
+        ctx = gpu.context_for(mesh, st, schemes=dict(i_vert_diff=False))
+        assert rt.host_hazards() == 0, "set-up"
+        n, L = mesh.nod2D, mesh.nl - 1
+        ctx.set_ki(np.ones((n, L)), np.zeros((n, L, 3)), True)
+        ctx.solve_tracers_ale(st.dt, 2)
+        assert rt.host_hazards() == 0, "step"
+        ctx.init_tracers_AB(1)
+        ctx.do_oce_adv_tra(st.dt, 1)
+        ctx.diff_tracers_ale(st.dt, 1)
+        assert rt.host_hazards() == 0, "per-tracer calls"
+        ctx.tracer_config(2, 2, AB_order=3)
+        ctx.solve_tracers_ale(st.dt, 1)
+        assert rt.host_hazards() == 0, "AB3"
+        ctx.close()
+        ctx = gpu.Context()
+        ctx.mesh_init(mesh)
+        ctx.set_uv(st.uv)
+        ctx.vert_vel_ale(st.dt)
+        assert rt.host_hazards() == 0, "vertical velocity"
+        i = np.arange(100)
+        ctx.ssh_set_matrix(1 + np.arange(101), 1 + i, 1.0 + i)
+        ctx.ssh_solve_preconditioner(2)
+        ctx.nn_init(0)
+        ctx.nn_loss_grad(np.ones((1, 100)), np.ones((1, 100)))
+        assert rt.host_hazards() == 0, "learned preconditioner"
+        ctx.close()
+        """, FGPU_STEP=step)
