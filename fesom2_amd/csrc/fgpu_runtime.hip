@@ -354,33 +354,31 @@ static void free_tracer_buf(fgpu_context *c, double *&p)
 int fgpu_ensure_staged(fgpu_context *c, int slots)
 {
     DevTracers &t = c->t;
-    if (t.TAB && c->stage_slots >= slots) return FGPU_OK;
+    if (c->stage_slots >= slots) return FGPU_OK;   // set once everything is there
     FGPU_HIP(hipSetDevice(c->device));
     FGPU_HIP(hipStreamSynchronize(c->stream));
     int rc;
-    if (!t.TAB) {
-        struct A { double **p; size_t n; } arrs[] = {
-            {&t.TAB, t.sN * (size_t)t.ntr}, {&t.lo_h, t.sE * (size_t)t.ntr}, {&t.dttf_h, t.sN}, {&t.dttf_v, t.sN},
-            {&t.dbg_av, t.sNI}, {&t.dbg_grad, t.sE * 4}, {&t.ngrad, t.sG}};
-        for (auto &a : arrs) {
-            if ((rc = fgpu_alloc(c, (void **)a.p, a.n * sizeof(double), true))) return rc;
-            if ((rc = fgpu_zero(c, *a.p, a.n * sizeof(double)))) return rc;
-        }
+    struct A { double **p; size_t n; } arrs[] = {
+        {&t.TAB, t.sN * (size_t)t.ntr}, {&t.lo_h, t.sE * (size_t)t.ntr}, {&t.dttf_h, t.sN}, {&t.dttf_v, t.sN},
+        {&t.dbg_av, t.sNI}, {&t.dbg_grad, t.sE * 4}, {&t.ngrad, t.sG}};
+    for (auto &a : arrs) {
+        if (*a.p) continue;
+        if ((rc = fgpu_alloc(c, (void **)a.p, a.n * sizeof(double), true))) return rc;
+        if ((rc = fgpu_zero(c, *a.p, a.n * sizeof(double)))) return rc;
     }
-    if (c->stage_slots < slots) {
-        free_tracer_buf(c, t.tr_xy);
-        free_tracer_buf(c, t.aux);
-        for (double **p : {&t.tr_xy, &t.aux}) {
-            if ((rc = fgpu_alloc(c, (void **)p, t.sF2 * (size_t)slots * sizeof(double), true))) return rc;
-            if ((rc = fgpu_zero(c, *p, t.sF2 * (size_t)slots * sizeof(double)))) return rc;
-        }
-        c->stage_slots = slots;
-        t.sStg = slots > 1 ? t.sF2 : 0;
-        if (slots > 1) {   // such a context's steps are staged: the fused step's array is free
-            if ((rc = fgpu_zero(c, t.gmean, t.sG * (size_t)t.ntr * sizeof(double)))) return rc;
-            t.ngrad = t.gmean;
-        }
+    c->stage_slots = 0;
+    free_tracer_buf(c, t.tr_xy);
+    free_tracer_buf(c, t.aux);
+    for (double **p : {&t.tr_xy, &t.aux}) {
+        if ((rc = fgpu_alloc(c, (void **)p, t.sF2 * (size_t)slots * sizeof(double), true))) return rc;
+        if ((rc = fgpu_zero(c, *p, t.sF2 * (size_t)slots * sizeof(double)))) return rc;
     }
+    if (slots > 1) {   // such a context's steps are staged: the fused step's array is free
+        if ((rc = fgpu_zero(c, t.gmean, t.sG * (size_t)t.ntr * sizeof(double)))) return rc;
+        t.ngrad = t.gmean;
+    }
+    t.sStg = slots > 1 ? t.sF2 : 0;
+    c->stage_slots = slots;
     c->graph_valid = false;
     return FGPU_OK;
 }

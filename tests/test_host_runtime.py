@@ -69,3 +69,40 @@ def test_fills_are_done_before_the_stream_uses_them(runtime, step):
         assert rt.host_hazards() == 0, "learned preconditioner"
         ctx.close()
         """, FGPU_STEP=step)
+
+
+@pytest.mark.parametrize("slots", ["one", "all"])
+def test_staged_buffers_after_a_failed_allocation(runtime, slots):
+    """A call repeated after FGPU_ERR_NOMEM allocates what the failed one could
+    not, whichever allocation failed, also where the buffers of the per-tracer
+    calls are replaced by those of the batched per-stage step."""
+    _run(runtime, f"""
+        def calls(ctx):
+            ctx.init_tracers_AB(1)
+            if {slots == "all"}:
+                ctx.solve_tracers_ale(st.dt, 1)
+        ctx = gpu.context_for(mesh, st)
+        base = rt.host_live_bytes()
+        calls(ctx)
+        want = rt.host_live_bytes() - base
+        ctx.close()
+        failed = 0
+        for k in range(100):
+            ctx = gpu.context_for(mesh, st)
+            base = rt.host_live_bytes()
+            rt.host_fail_in(k)
+            try:
+                calls(ctx)
+            except gpu.FesomGpuError as e:
+                assert "hipMalloc" in str(e)
+                failed += 1
+            else:
+                assert rt.host_fail_left() >= 0
+                rt.host_fail_in(-1)
+                break
+            ctx.init_tracers_AB(1)
+            calls(ctx)
+            assert rt.host_live_bytes() - base == want, k
+            ctx.close()
+        assert failed == {9 if slots == "one" else 11}
+        """, FGPU_STEP="staged")
