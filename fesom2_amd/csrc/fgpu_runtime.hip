@@ -965,6 +965,7 @@ extern "C" int fgpu_tracers_init(fgpu_context *c, int num_tracers)
     if (num_tracers < 1 || num_tracers > 4096) return fgpu_fail(FGPU_ERR_ARG, "num_tracers out of range");
     FGPU_HIP(hipSetDevice(c->device));
     FGPU_HIP(hipStreamSynchronize(c->stream));
+    c->tracers_ready = false;   // until every array below is there
     free_list(c->tracer_allocs);
     if (c->graph) { (void)hipGraphExecDestroy(c->graph); c->graph = nullptr; }
     c->graph_valid = false;

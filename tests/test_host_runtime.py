@@ -106,3 +106,32 @@ def test_staged_buffers_after_a_failed_allocation(runtime, slots):
             ctx.close()
         assert failed == {9 if slots == "one" else 11}
         """, FGPU_STEP="staged")
+
+
+def test_tracers_after_a_failed_allocation(runtime):
+    """fgpu_tracers_init releases the former tracers first: after it has failed
+    there are none, and a repeated call sets them up."""
+    _run(runtime, """
+        ctx = gpu.context_for(mesh, st)
+        for k in range(11):
+            rt.host_fail_in(k)
+            try:
+                ctx.tracers_init(3)
+                raise AssertionError(k)
+            except gpu.FesomGpuError as e:
+                assert "hipMalloc" in str(e)
+            for call in (lambda: ctx.solve_tracers_ale(st.dt, 1), lambda: ctx.init_tracers_AB(1),
+                         lambda: ctx.tracer_config(1, 1), lambda: ctx.tracer_content(1),
+                         lambda: ctx.tracer_upload(1, st.values[0], st.valuesold[0])):
+                try:
+                    call()
+                    raise AssertionError(k)
+                except gpu.FesomGpuError as e:
+                    assert "tracers not initialised" in str(e), (k, e)
+        ctx.tracers_init(2)
+        for i in range(2):
+            ctx.tracer_config(i + 1, i + 1)
+            ctx.tracer_upload(i + 1, st.values[i], st.valuesold[i])
+        ctx.solve_tracers_ale(st.dt, 1)
+        ctx.close()
+        """)
