@@ -322,6 +322,7 @@ int fgpu_fail(int code, const std::string &msg);
 
 int fgpu_alloc(fgpu_context *c, void **p, size_t bytes, bool tracer_scope = false);
 int fgpu_zero(fgpu_context *c, void *p, size_t bytes);
+void fgpu_free(fgpu_context *c, void **p);   // of a context-scope allocation
 // FGPU_ERR_STATE unless every flux array that the IDs of tracers tr0..tr0+ntr-1 read is set
 int fgpu_check_bc_inputs(fgpu_context *c, int tr0, int ntr);
 

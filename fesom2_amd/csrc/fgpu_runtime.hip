@@ -335,16 +335,17 @@ static void free_list(std::vector<void *> &v)
     v.clear();
 }
 
-// free one tracer-scope allocation (the stream must be idle)
-static void free_tracer_buf(fgpu_context *c, double *&p)
+// free one allocation (the stream must be idle)
+static void free_one(std::vector<void *> &v, void *&p)
 {
     if (!p) return;
-    auto &v = c->tracer_allocs;
     for (size_t i = 0; i < v.size(); ++i)
-        if (v[i] == (void *)p) { v.erase(v.begin() + (long)i); break; }
+        if (v[i] == p) { v.erase(v.begin() + (long)i); break; }
     (void)hipFree(p);
     p = nullptr;
 }
+static void free_tracer_buf(fgpu_context *c, double *&p) { free_one(c->tracer_allocs, (void *&)p); }
+void fgpu_free(fgpu_context *c, void **p) { free_one(c->allocs, *p); }
 
 // Per-stage buffers: valuesAB for every tracer, the del_ttf/limited-flux/edge
 // gradient work arrays of one tracer, and `slots` copies of tr_xy and the FCT

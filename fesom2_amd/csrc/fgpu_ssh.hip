@@ -968,6 +968,14 @@ static int ssh_alloc_matrix(fgpu_context *c, int n, int nnz)
     int rc;
     if (c->ssh_ready && (c->ssh_n != n || c->ssh_nnz != nnz))
         return fgpu_fail(FGPU_ERR_STATE, "SSH matrix shape changed");
+    if (c->ssh_n != n || c->ssh_nnz != nnz) {   // what a failed call of another size has left
+        void **left[] = {(void **)&c->ssh_rowptr, (void **)&c->ssh_colind, (void **)&c->ssh_val, (void **)&c->ssh_pr,
+                         (void **)&c->ssh_ecol, (void **)&c->ssh_eval, (void **)&c->ssh_x, (void **)&c->ssh_x0,
+                         (void **)&c->ssh_rhs, (void **)&c->ssh_r, (void **)&c->ssh_z, (void **)&c->ssh_p,
+                         (void **)&c->ssh_p1, (void **)&c->ssh_q, (void **)&c->ssh_diag_inv, (void **)&c->ssh_rec0,
+                         (void **)&c->ssh_rec1, (void **)&c->ssh_part, (void **)&c->ssh_out};
+        for (void **p : left) fgpu_free(c, p);
+    }
     c->ssh_n = n;
     c->ssh_nnz = nnz;
     if (!c->ssh_rowptr && (rc = fgpu_alloc(c, (void **)&c->ssh_rowptr, sizeof(int) * (n + 1)))) return rc;

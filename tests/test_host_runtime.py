@@ -135,3 +135,29 @@ def test_tracers_after_a_failed_allocation(runtime):
         ctx.solve_tracers_ale(st.dt, 1)
         ctx.close()
         """)
+
+
+def test_ssh_matrix_after_a_failed_allocation(runtime):
+    """A matrix of another size after one that could not be allocated gets
+    arrays of its own size."""
+    _run(runtime, """
+        def diagonal(ctx, n):
+            ctx.ssh_set_matrix(1 + np.arange(n + 1), 1 + np.arange(n), np.ones(n))
+        ctx = gpu.Context()
+        base = rt.host_live_bytes()
+        diagonal(ctx, 2000)
+        want = rt.host_live_bytes() - base
+        ctx.close()
+        for k in range(19):
+            ctx = gpu.Context()
+            base = rt.host_live_bytes()
+            rt.host_fail_in(k)
+            try:
+                diagonal(ctx, 50)
+                raise AssertionError(k)
+            except gpu.FesomGpuError as e:
+                assert "hipMalloc" in str(e)
+            diagonal(ctx, 2000)
+            assert rt.host_live_bytes() - base == want, k
+            ctx.close()
+        """)
