@@ -240,7 +240,7 @@ struct fgpu_context {
     int N2 = 0, F2 = 0, E2 = 0, nl = 0, kmax = 0;
     double cyclic_length = 0.0;
     bool edge_gap = false;             // some edge's elements share no level and leave a gap between their ranges
-    FgpuFetcher *fetcher = nullptr;    // threads and pinned slots of large downloads (fgpu_runtime.hip)
+    FgpuFetcher *fetcher = nullptr;    // its device's threads and pinned slots of large downloads (fgpu_runtime.hip)
     bool fetch_plain = false;          // they could not be had
     std::vector<void *> allocs;        // everything hipMalloc'ed by the context
     std::vector<void *> tracer_allocs; // released on fgpu_tracers_init

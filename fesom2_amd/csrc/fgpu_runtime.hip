@@ -70,21 +70,28 @@ static int upload(fgpu_context *c, T **dst, const T *src, size_t n)
 
 // ---------------------------------------------------------------- downloads
 // A copy from the device into pageable memory is bound by the host: one thread
-// moves it out of the runtime's staging buffer at about 10 GB/s, and into pages
-// that are being touched for the first time. Large downloads go through pinned
-// slots in pieces, each taken by one of FETCH_THREADS threads that waits for its
-// own piece and moves it on. The threads and slots belong to the context, come
-// with its first large download and end with it. A tracer and its old level of
-// 60 MB: 4.2 -> 2.6 ms (23 GB/s), of 191 MB: 19 -> 6.0 ms (32 GB/s), of 9 MB:
-// 1.2 -> 0.65 ms; below 4 MB the threads' start costs what they save.
+// moves it out of the runtime's staging buffer at about 17 GB/s, and at 4 GB/s
+// into pages that are being touched for the first time. Large downloads go
+// through pinned slots in pieces, each taken by one of FETCH_THREADS threads that
+// waits for its own piece and moves it on. In ms, one copy and by pieces: 4 MB
+// 0.25 and 0.23, 8 MB 0.48 and 0.41, 24 MB 1.43 and 0.74, 96 MB 5.8 and 2.6; into
+// fresh pages 4 MB 1.05 and 0.37, 24 MB 6.2 and 1.6, 96 MB 24 and 5.3. A piece
+// costs some 20 us one after the other besides its bytes, so none is made smaller
+// than FETCH_PIECE (4 MB in 16 pieces: 0.33 ms).
+// The threads and slots come with the first large download from a device, serve
+// all its contexts and end with the last one that has used them: starting them
+// and touching the slots takes 0.6 to 1.2 ms. The pieces go through the null
+// stream, like hipMemcpy: the first large copy of a process through a further
+// stream takes 6.5 ms.
 #define FETCH_THREADS 8
-#define FETCH_SLOT ((size_t)2 << 20)   // bytes per thread
-#define FETCH_MIN ((size_t)4 << 20)    // smaller downloads stay with one copy
+#define FETCH_SLOT ((size_t)2 << 20)      // bytes per thread
+#define FETCH_PIECE ((size_t)512 << 10)
+#define FETCH_MIN ((size_t)4 << 20)       // smaller downloads stay with one copy
 
 struct FgpuFetcher {
-    int device = 0;
+    int device = 0, users = 0;      // contexts that have used it
+    FgpuFetcher *other = nullptr;   // another device's
     char *slots = nullptr;
-    hipStream_t stream = nullptr;   // the context's: a process's first further streams cost 3 ms each
     hipEvent_t arrived[FETCH_THREADS] = {};
     std::vector<std::thread> threads;
     std::mutex use, m;   // one download at a time; the job below
@@ -106,8 +113,8 @@ struct FgpuFetcher {
             if (p == nparts || err.load()) return;
             const size_t o = i * piece, n = std::min(piece, parts[p].bytes - o);
             char *slot = slots + FETCH_SLOT * w;
-            hipError_t e = hipMemcpyAsync(slot, (const char *)parts[p].src + o, n, hipMemcpyDeviceToHost, stream);
-            if (e == hipSuccess) e = hipEventRecord(arrived[w], stream);
+            hipError_t e = hipMemcpyAsync(slot, (const char *)parts[p].src + o, n, hipMemcpyDeviceToHost, nullptr);
+            if (e == hipSuccess) e = hipEventRecord(arrived[w], nullptr);
             if (e == hipSuccess) e = hipEventSynchronize(arrived[w]);
             if (e != hipSuccess) {
                 err.store((int)e);
@@ -131,10 +138,9 @@ struct FgpuFetcher {
             if (--running == 0) end.notify_one();
         }
     }
-    bool open(int dev, hipStream_t st)
+    bool open(int dev)
     {
         device = dev;
-        stream = st;
         if (hipHostMalloc((void **)&slots, FETCH_SLOT * FETCH_THREADS, hipHostMallocDefault) != hipSuccess) return false;
         for (hipEvent_t &e : arrived)
             if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
@@ -152,7 +158,7 @@ struct FgpuFetcher {
             std::lock_guard<std::mutex> lk(m);
             parts = list;
             nparts = n;
-            piece = std::min(FETCH_SLOT, (total / (2 * FETCH_THREADS) + 65535) / 65536 * 65536);
+            piece = std::min(FETCH_SLOT, std::max(FETCH_PIECE, (total / (2 * FETCH_THREADS) + 65535) / 65536 * 65536));
             next.store(0);
             err.store(0);
             running = (int)threads.size();
@@ -178,29 +184,48 @@ struct FgpuFetcher {
     }
 };
 
+static std::mutex fetchers_m;   // the devices' threads and their users
+static FgpuFetcher *fetchers = nullptr;
+
+// the threads of the context's device; null without pinned memory or threads
+static FgpuFetcher *fetcher_of(fgpu_context *c)
+{
+    std::lock_guard<std::mutex> lk(fetchers_m);
+    if (c->fetcher || c->fetch_plain) return c->fetcher;
+    FgpuFetcher *f = fetchers;
+    while (f && f->device != c->device) f = f->other;
+    if (!f) {
+        f = new (std::nothrow) FgpuFetcher;
+        if (!f || !f->open(c->device)) {   // one copy, as for a small download
+            (void)hipGetLastError();
+            delete f;
+            c->fetch_plain = true;
+            return nullptr;
+        }
+        f->other = fetchers;
+        fetchers = f;
+    }
+    ++f->users;
+    return c->fetcher = f;
+}
+
+static void fetcher_leave(fgpu_context *c)
+{
+    std::lock_guard<std::mutex> lk(fetchers_m);
+    if (!c->fetcher || --c->fetcher->users > 0) return;
+    FgpuFetcher **at = &fetchers;
+    while (*at != c->fetcher) at = &(*at)->other;
+    *at = c->fetcher->other;
+    delete c->fetcher;
+}
+
 // copies from the device whose contents are complete (the context's stream has been waited for)
 int fgpu_fetch(fgpu_context *c, const FgpuPart *parts, int nparts)
 {
     size_t total = 0;
     for (int i = 0; i < nparts; ++i) total += parts[i].bytes;
     if (total >= FETCH_MIN) {
-        FgpuFetcher *f = nullptr;
-        {
-            static std::mutex first;
-            std::lock_guard<std::mutex> lk(first);
-            if (!c->fetcher && !c->fetch_plain) {
-                f = new (std::nothrow) FgpuFetcher;
-                if (f && f->open(c->device, c->stream)) {
-                    c->fetcher = f;
-                } else {   // without pinned memory or threads: one copy, as for a small download
-                    (void)hipGetLastError();
-                    delete f;
-                    c->fetch_plain = true;
-                }
-            }
-            f = c->fetcher;
-        }
-        if (f) {
+        if (FgpuFetcher *f = fetcher_of(c)) {
             const hipError_t e = f->run(parts, nparts, total);
             if (e != hipSuccess) return fgpu_fail(FGPU_ERR_HIP, std::string("download: ") + hipGetErrorString(e));
             return FGPU_OK;
@@ -394,7 +419,7 @@ extern "C" int fgpu_destroy(fgpu_context *c)
     if (c->graph) (void)hipGraphExecDestroy(c->graph);
     if (c->ssh_graph) (void)hipGraphExecDestroy(c->ssh_graph);
     fgpu_nn_release(c);
-    delete c->fetcher;
+    fetcher_leave(c);
     free_list(c->tracer_allocs);
     free_list(c->allocs);
     (void)hipStreamDestroy(c->stream);

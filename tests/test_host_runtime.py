@@ -161,3 +161,34 @@ def test_ssh_matrix_after_a_failed_allocation(runtime):
             assert rt.host_live_bytes() - base == want, k
             ctx.close()
         """)
+
+
+def test_contexts_share_the_download_threads(runtime):
+    """The threads of large downloads come once, whatever the number of
+    contexts, and end with the last context that has used them."""
+    _run(runtime, """
+        def threads():
+            return len(os.listdir("/proc/self/task"))
+        big = mg.build_mesh(nx=93, ny=60, dx=20e3, jitter=0.2, seed=0, cartesian=True, nlayers=47, hmax=4000.0,
+                            min_layers=4, max_layers=47, topo="bumps", bump_height=1500.0)
+        bst = mg.build_state(big, seed=0, ntr=1, dt=600.0, dx=20e3)
+        base = threads()
+        ctx = [gpu.context_for(big, bst) for _ in range(3)]
+        assert threads() == base
+        n = []
+        for c in ctx:
+            v, vo = c.tracer_download(1)
+            assert np.array_equal(v, bst.values[0]) and np.array_equal(vo, bst.valuesold[0])
+            n.append(threads() - base)
+        assert n[0] > 0 and n == [n[0]] * 3, n
+        ctx[1].close()
+        ctx[0].close()
+        assert threads() - base == n[0]
+        assert np.array_equal(ctx[2].tracer_download(1)[0], bst.values[0])
+        ctx[2].close()
+        assert threads() == base
+        c = gpu.context_for(big, bst)
+        assert np.array_equal(c.tracer_download(1)[0], bst.values[0])
+        c.close()
+        assert threads() == base
+        """)
