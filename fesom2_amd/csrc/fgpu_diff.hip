@@ -87,7 +87,10 @@ __global__ void __launch_bounds__(64) k_hdiff_edge(DevMesh m, DevDyn d, DevTrace
         // cases (A)/(D): el1 alone, (B)/(E): el2 alone, (C): both. The levels without either keep the zeros
         // that the buffer starts with
         const bool p1 = k >= nu1 && k <= nl1, p2 = two && k >= nu2 && k <= nl2;
-        const bool out = (p1 || p2) && idx < (1 << sh) - 1;
+        // in a level gap between the elements both segments reach into it, where the reference's element
+        // gradients are zero: the slope terms of both
+        const bool gap = REDI && two && ((k > nl1 && k < nu2) || (k > nl2 && k < nu1));
+        const bool out = (p1 || p2 || gap) && idx < (1 << sh) - 1;
         const size_t c1 = (size_t)n1 * L + kc - 1, c2 = (size_t)n2 * L + kc - 1;
         const double Kh = (d.Ki[c1] + d.Ki[c2]) / 2.0;
         const double h1 = m.helem[(size_t)el1 * L + kc - 1], h2 = m.helem[(size_t)q2 * L + kc - 1];
@@ -116,7 +119,12 @@ __global__ void __launch_bounds__(64) k_hdiff_edge(DevMesh m, DevDyn d, DevTrace
             grad_el(E2, T + kc - 1, gx2, gy2);
             const double Tx = p1 ? (p2 ? 0.5 * (gx1 + gx2) : gx1) : gx2, Ty = p1 ? (p2 ? 0.5 * (gy1 + gy2) : gy1) : gy2;
             const double Fx = Kh * (Tx + sx), Fy = Kh * (Ty + sy);
-            if (out) hd[t.sE * (tr0 + tb) + k - 1] = (a * Fy - b * Fx) * dz;
+            double c = (a * Fy - b * Fx) * dz;
+            if (REDI && gap) {
+                const double gx = Kh * sx, gy = Kh * sy;
+                c = (-dX1 * gy + dY1 * gx) * h1 + (dX2 * gy - dY2 * gx) * h2;
+            }
+            if (out) hd[t.sE * (tr0 + tb) + k - 1] = c;
         }
     }
 }

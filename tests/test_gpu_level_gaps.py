@@ -69,7 +69,7 @@ def _check(mesh, st, schemes, nsteps=2):
 
 
 @pytest.mark.parametrize("rows", ["", "wide"])
-@pytest.mark.parametrize("terms", [False, True])
+@pytest.mark.parametrize("terms", ["", "diffusion", "redi"])
 @pytest.mark.parametrize("layers,ntr", [(24, 2), (31, 6), (63, 6), (70, 6), (127, 3)])
 def test_level_gaps(monkeypatch, layers, ntr, terms, rows):
     monkeypatch.setenv("FGPU_STEP_ROWS", rows)
@@ -80,5 +80,7 @@ def test_level_gaps(monkeypatch, layers, ntr, terms, rows):
         w_e = st.w * rng.uniform(0.2, 1.0, st.w.shape)
         st = dataclasses.replace(st, w_e=w_e, w_i=st.w - w_e, use_wsplit=True,
                                  Ki=rng.uniform(20.0, 400.0, (mesh.nod2D, layers)))
-    print(f"[gpu] level gaps, {layers} layers, {ntr} tracers, terms {terms}, rows {rows or 'as chosen'}", flush=True)
+    if terms == "redi":
+        st = dataclasses.replace(st, redi=True, slope_tapered=rng.normal(0.0, 0.01, (mesh.nod2D, layers, 3)))
+    print(f"[gpu] level gaps, {layers} layers, {ntr} tracers, terms {terms or 'none'}, rows {rows or 'as chosen'}", flush=True)
     _check(mesh, st, SCHEMES[:ntr] if ntr > 2 else None)
