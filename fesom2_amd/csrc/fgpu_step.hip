@@ -24,6 +24,7 @@
 // edges in ascending edge order. Results are bit-identical to a serial run of
 // the reference's loops.
 #include <algorithm>
+#include <type_traits>
 
 #include "fgpu_internal.h"
 #include "fgpu_vert.h"
@@ -1392,33 +1393,31 @@ void fgpu_kd_shape(const fgpu_context *c, int *tch_out, int *cpb_out)
 // tracer-independent work. Rows of up to 32 interfaces leave half a wave free,
 // which a second tracer takes at no cost.
 struct ColLanes {
-    bool pair;    // tracers two to a wave
-    bool wide;    // row offsets need 64 bits
-    bool wide2;   // those of a pair do
+    bool pair;   // tracers two to a wave
+    bool wide;   // row offsets need 64 bits
+    bool far;    // those of a pair do
 };
 static ColLanes col_lanes(const fgpu_context *c, int tpb)
 {
     const DevTracers &t = c->t;
-    const size_t field = 8 * std::max(std::max(t.sE, t.sNI), std::max(t.sOld, t.sG)) + 4096;
+    const size_t field = 8 * std::max(std::max(t.sE, t.sNI), std::max(t.sOld, t.sG)) + 4096, reach = 0xffffffffu;
     bool same = true;
     for (int i = 1; i < t.ntr; ++i)
         same = same && c->h_lim[i] == c->h_lim[0] && c->h_abo[i] == c->h_abo[0] && c->h_hor[i] == c->h_hor[0] &&
                c->h_ver[i] == c->h_ver[0] && c->h_ph[i] == c->h_ph[0] && c->h_pv[i] == c->h_pv[0];
-    const size_t reach = c->step_wide ? 0 : 0xffffffffu;
-    const bool far = 2 * field >= (size_t)0xffffffffu, deep = c->m.NL > 64 && c->m.NL <= 96;
-    return {same && std::min(tpb, t.ntr) >= 2 && (!far || deep), field >= reach, far || field >= reach};
+    const bool wide = c->step_wide || field >= reach, far = wide || 2 * field >= reach;
+    const bool deep = c->m.NL > 64 && c->m.NL <= 96;
+    return {same && std::min(tpb, t.ntr) >= 2 && (!far || deep), wide, far};
 }
 
 #define COL_LAUNCH(kern, NV, GT, X, grid, ...)                                                                       \
     do {                                                                                                             \
-        if (GT > 1 ? cl.wide2 : cl.wide) hipLaunchKernelGGL((kern<size_t, NV, GT, X>), grid, dim3(64), 0, c->stream, __VA_ARGS__);          \
+        if (GT > 1 ? cl.far : cl.wide) hipLaunchKernelGGL((kern<size_t, NV, GT, X>), grid, dim3(64), 0, c->stream, __VA_ARGS__);            \
         else hipLaunchKernelGGL((kern<unsigned, NV, GT, X>), grid, dim3(64), 0, c->stream, __VA_ARGS__);             \
     } while (0)
-#define COL_LAUNCH_D(kern, NV, GT, dx, grid, ...)                                                                    \
-    do {                                                                                                             \
-        if (dx) COL_LAUNCH(kern, NV, GT, true, grid, __VA_ARGS__);                                                 \
-        else COL_LAUNCH(kern, NV, GT, false, grid, __VA_ARGS__);                                                   \
-    } while (0)
+// pairs of up to 64 interfaces, within 32-bit offsets
+#define COL_NEAR(kern, NV, X, grid, ...)                                                                             \
+    hipLaunchKernelGGL((kern<unsigned, NV, 2, X>), grid, dim3(64), 0, c->stream, __VA_ARGS__)
 
 template <int XF>
 static void launch_kv(fgpu_context *c, int tr0, int nt, double dt, int all, int clamp)
@@ -1481,8 +1480,8 @@ int fgpu_enqueue_fused_step(fgpu_context *c, double dt)
         if (c->edge_gap && narrow) COL_LAUNCH(kA_edge, 1, 1, true, edges, m, c->d, c->t, tpb);
         else if (c->edge_gap) COL_LAUNCH(kA_edge, 2, 1, true, edges, m, c->d, c->t, tpb);
         else if (!narrow) COL_LAUNCH(kA_edge, 2, 1, false, edges, m, c->d, c->t, tpb);
-        else if (slim && pair) COL_LAUNCH(kA_edge, 1, 2, false, edges, m, c->d, c->t, tpb);
-        else if (many) COL_LAUNCH(kA_edge, 2, 2, false, edges, m, c->d, c->t, tpb);
+        else if (slim && pair) COL_NEAR(kA_edge, 1, false, edges, m, c->d, c->t, tpb);
+        else if (many) COL_NEAR(kA_edge, 2, false, edges, m, c->d, c->t, tpb);
         else COL_LAUNCH(kA_edge, 1, 1, false, edges, m, c->d, c->t, tpb);
     }
     {
@@ -1493,7 +1492,7 @@ int fgpu_enqueue_fused_step(fgpu_context *c, double dt)
         else if (extra) COL_LAUNCH(kB_cols, 2, 1, KB_EXTRA, nodes, m, c->d, c->t, dt, tpb);
         else if (pair && m.NL > 64 && m.NL <= 96) COL_LAUNCH(kB_cols, 3, 2, 0, nodes, m, c->d, c->t, dt, tpb);
         else if (!narrow) COL_LAUNCH(kB_cols, 2, 1, 0, nodes, m, c->d, c->t, dt, tpb);
-        else if (slim && pair) COL_LAUNCH(kB_cols, 1, 2, 0, nodes, m, c->d, c->t, dt, tpb);
+        else if (slim && pair) COL_NEAR(kB_cols, 1, 0, nodes, m, c->d, c->t, dt, tpb);
         else COL_LAUNCH(kB_cols, 1, 1, 0, nodes, m, c->d, c->t, dt, tpb);
     }
     if (c->d.wsplit) {
@@ -1505,18 +1504,23 @@ int fgpu_enqueue_fused_step(fgpu_context *c, double dt)
         if (c->edge_gap && narrow) COL_LAUNCH(kC_cols, 1, 1, true, nodes, m, c->t, dt, tpb);
         else if (c->edge_gap) COL_LAUNCH(kC_cols, 2, 1, true, nodes, m, c->t, dt, tpb);
         else if (!narrow) COL_LAUNCH(kC_cols, 2, 1, false, nodes, m, c->t, dt, tpb);
-        else if (slim && pair) COL_LAUNCH(kC_cols, 1, 2, false, nodes, m, c->t, dt, tpb);
-        else if (many) COL_LAUNCH(kC_cols, 2, 2, false, nodes, m, c->t, dt, tpb);
+        else if (slim && pair) COL_NEAR(kC_cols, 1, false, nodes, m, c->t, dt, tpb);
+        else if (many) COL_NEAR(kC_cols, 2, false, nodes, m, c->t, dt, tpb);
         else COL_LAUNCH(kC_cols, 1, 1, false, nodes, m, c->t, dt, tpb);
     }
     {
         ProfScope ps(c, "kL_node");
         const bool dx = (xf & 2) != 0;
-        if (pair && m.NL > 64 && m.NL <= 96) COL_LAUNCH_D(kL_node, 3, 2, dx, nodes, m, c->d, c->t, dt, tpb);
-        else if (!narrow) COL_LAUNCH_D(kL_node, 2, 1, dx, nodes, m, c->d, c->t, dt, tpb);
-        else if (slim && pair) COL_LAUNCH_D(kL_node, 1, 2, dx, nodes, m, c->d, c->t, dt, tpb);
-        else if (pair) COL_LAUNCH_D(kL_node, 2, 2, dx, nodes, m, c->d, c->t, dt, tpb);
-        else COL_LAUNCH_D(kL_node, 1, 1, dx, nodes, m, c->d, c->t, dt, tpb);
+        auto launch = [&](auto DX) {
+            constexpr bool X = decltype(DX)::value;
+            if (pair && m.NL > 64 && m.NL <= 96) COL_LAUNCH(kL_node, 3, 2, X, nodes, m, c->d, c->t, dt, tpb);
+            else if (!narrow) COL_LAUNCH(kL_node, 2, 1, X, nodes, m, c->d, c->t, dt, tpb);
+            else if (slim && pair) COL_NEAR(kL_node, 1, X, nodes, m, c->d, c->t, dt, tpb);
+            else if (pair) COL_NEAR(kL_node, 2, X, nodes, m, c->d, c->t, dt, tpb);
+            else COL_LAUNCH(kL_node, 1, 1, X, nodes, m, c->d, c->t, dt, tpb);
+        };
+        if (dx) launch(std::true_type{});
+        else launch(std::false_type{});
     }
     {
         ProfScope ps(c, "kV_cols");
