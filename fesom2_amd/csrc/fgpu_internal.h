@@ -220,8 +220,8 @@ struct ProfEntry {
     int launches = 0;
 };
 
-// last-kernel settings of fgpu_set_step_shape, kept as fgpu_step_variant
-// reports them; the step's kernels no longer differ by them
+// last-kernel settings of fgpu_set_step_shape: checked, kept and reported for
+// callers that set them; no kernel differs by them
 #define KD_LOCKSTEP 0
 #define KD_SWEEPWAVE 1
 #define KD_WAVELOCAL 2
@@ -338,7 +338,7 @@ struct ProfScope {
 };
 int fgpu_prof_flush(fgpu_context *c);
 
-// fused batched step (fgpu_step.hip): four launches per step for all tracers
+// fused batched step (fgpu_step.hip): six launches per step for all tracers
 int fgpu_enqueue_fused_step(fgpu_context *c, double dt);
 void fgpu_kd_shape(const fgpu_context *c, int *tch, int *cpb);
 int fgpu_kd_extras(const fgpu_context *c);

@@ -37,8 +37,9 @@ extern "C" int fgpu_version(void) { return 1; }
 
 int fgpu_alloc(fgpu_context *c, void **p, size_t bytes, bool tracer_scope)
 {
-    // the fused step reads rows of levels two or three at a time, so a row's last
-    // read may run up to 16 bytes past its end (the values are not used)
+    // the fused step reads rows NV = two or three levels at a time, so a row's last
+    // read may run 8 (NV - 1) bytes past its end, and 16 (NV - 1) where a level has
+    // two values: 32 on the old levels of an AB3 tracer (the values are not used)
     bytes += 64;
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess)

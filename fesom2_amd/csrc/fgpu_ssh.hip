@@ -635,10 +635,10 @@ __global__ void __launch_bounds__(SBLK) k_cg1(CGArgs A, int par)
 // a sparse M^-1, by its entries from L2 (64 bytes a clock). An iteration with the
 // sparse preconditioner and with the diagonal one: 986 rows 12.9 -> 4.4 us and
 // 7.0 -> 3.0, 3,000 rows 13.4 -> 8.3 us and 6.9 -> 5.3. A fourth row per thread
-// does not fit the registers (spilling the third one cost 3 us).
+// does not fit the registers.
 // ------------------------------------------------------------------------------
 #define CGS_THREADS 1024
-#define CGS_ROWS 3072        // V = 3: what the registers hold
+#define CGS_ROWS 3072        // V = 3, which spills 6 to 8 registers (28 to 36 bytes a lane)
 #define CGS_MAXITER 20000    // an unbounded solve stays with the kernels per iteration
 enum { CGS_SPARSE, CGS_JACOBI, CGS_SINGLE };
 

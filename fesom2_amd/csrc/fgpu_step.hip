@@ -124,13 +124,16 @@ __global__ void __launch_bounds__(64) kG_node(DevMesh m, DevTracers t, const int
 // Column waves: one wave per node column (or edge), NV adjacent levels per lane
 // and GT tracers per wave, 64 / GT lanes each.
 //
-// These kernels are bound by instruction issue: a SIMD issues one instruction
-// every four cycles whatever its kind, and with 64-bit row addresses formed in
-// scalar registers and branches around masked lanes the scalar instructions
-// outnumbered the vector ones. So the rows' byte offsets are formed once per
-// column in vector registers (the tracers of a block only change the scalar
-// base), loads are not masked (lanes without a wet level read a valid row
-// entry), and the level ranges of the edges are lane masks that select results.
+// These kernels are bound by the vector memory pipeline: at 1.3 million nodes,
+// 70 layers, 10 tracers a CU's texture data unit is busy 97 to 99 % of the time
+// in K_A to K_L, 46 to 63 % of that waiting for L2. Instruction issue is not far
+// behind: a SIMD issues some instruction in 64 to 87 % of its cycles, VALU work in
+// 46 to 69 %, and with 64-bit row addresses formed in scalar registers and
+// branches around masked lanes the scalar instructions outnumbered the vector
+// ones. So the rows' byte offsets are formed once per column in vector registers
+// (the tracers of a block only change the scalar base), loads are not masked
+// (lanes without a wet level read a valid row entry), and the level ranges of the
+// edges are lane masks that select results.
 // One wave per block: with four, a block's slots stay taken until its slowest
 // wave is done (70 layers, 10 tracers: K_L 3 % slower).
 // ------------------------------------------------------------------------------
@@ -288,12 +291,11 @@ __device__ __forceinline__ bool load_column(const DevMesh &m, const DevTracers &
 // K_A: edge pass
 // ------------------------------------------------------------------------------
 // Per tracer it gathers T and the old level at the edge's nodes and T at the
-// nodes of the upwind and downwind triangles. Bound by the vector memory
-// pipeline (ten row loads and a store per tracer) and the latency of a wave's
-// dependent loads. The volume fluxes are stored once for all tracers instead of
-// a LO flux per tracer. 126,858 nodes, 47 layers, 2 tracers: 544 -> 473 us; 12
-// thousand nodes, 32 tracers: 689 -> 430; 40 thousand nodes, 70 layers, 10
-// tracers: 1067 -> 730.
+// nodes of the upwind and downwind triangles: ten row loads and a store per
+// tracer. The volume fluxes are stored once for all tracers instead of a LO flux
+// per tracer. Against a block per edge, 126,858 nodes, 47 layers, 2 tracers: 670
+// -> 506 us; 12 thousand nodes, 32 tracers: 886 -> 445; 40 thousand nodes, 70
+// layers, 10 tracers: 1390 -> 730.
 // GAP is the form for a mesh with a level gap across some edge: the reference's
 // segments of both elements reach into the gap (oce_adv_tra_hor.F90:166-249),
 // the upper element's first, so two fluxes follow each other there. K_B and K_C
@@ -491,9 +493,9 @@ __global__ void __launch_bounds__(64) kA_edge(DevMesh m, DevDyn d, DevTracers t,
 // The edges' LO fluxes are formed again from the volume fluxes and the T of the
 // neighbours, whose rows a node's edges share, where a stored LO flux is a row
 // per edge and tracer, three times as many. Levels exchange values by wave
-// shifts. 12 thousand nodes, 47 layers, 32 tracers: 350 -> 270 us; 40 thousand
-// nodes, 70 layers, 10 tracers: 551 -> 520; 126,858 nodes, 47 layers, 2 tracers:
-// 287 -> 298, against K_A's gain.
+// shifts. Against a block per column, 12 thousand nodes, 47 layers, 32 tracers:
+// 352 -> 281 us; 40 thousand nodes, 70 layers, 10 tracers: 537 -> 518; 126,858
+// nodes, 47 layers, 2 tracers: 291 -> 298, against K_A's gain.
 // EXTRA compiles in the CDIFF and PPM tracers and the W split (use_wsplit), where
 // the HO scheme is handed the upwind flux with the full W and the LO solution of
 // FCT tracers takes the implicit upwind advection with w_i afterwards (K_V on
@@ -726,8 +728,9 @@ __global__ void __launch_bounds__(64) kB_cols(DevMesh m, DevDyn d, DevTracers t,
 // together with the padding -1e3 (max) / +1e3 (min) of every element around
 // the node that lacks the level (oce_adv_tra_fct.F90:148-178).
 // ------------------------------------------------------------------------------
-// 126,858 nodes, 47 layers, 2 tracers: 344 -> 295 us; 12 thousand nodes, 32
-// tracers: 520 -> 395; 40 thousand nodes, 70 layers, 10 tracers: 744 -> 610.
+// Against a block per column, 126,858 nodes, 47 layers, 2 tracers: 347 -> 315 us;
+// 12 thousand nodes, 32 tracers: 482 -> 382; 40 thousand nodes, 70 layers, 10
+// tracers: 745 -> 647.
 // GAP: in a level gap neither element has the level, and the other node is no
 // part of its bounds.
 template <typename OFF, int NV, int GT, bool GAP>
@@ -843,10 +846,10 @@ __global__ void __launch_bounds__(64) kC_cols(DevMesh m, DevTracers t, double dt
 // oce_adv_tra_driver.F90:494-646, oce_ale_tracer.F90:595-626); T* replaces T,
 // T^n goes to valuesold. The implicit vertical diffusion follows in K_V: inside
 // the column's wave its sweeps kept 2 to 10 of 64 lanes busy for most of the
-// kernel's instructions. One kernel for both took 757 us at 126,858 nodes, 47
-// layers, 2 tracers (K_L 349 us, K_V 159), 1179 us at 12 thousand nodes, 32
-// tracers (439, 151) and 1364 us at 40 thousand nodes, 70 layers, 10 tracers
-// (700, 328).
+// kernel's instructions. One kernel for both, a block per column, took 775 us at
+// 126,858 nodes, 47 layers, 2 tracers (K_L 350 us, K_V 160), 988 us at 12 thousand
+// nodes, 32 tracers (420, 150) and 1429 us at 40 thousand nodes, 70 layers, 10
+// tracers (688, 325).
 // ------------------------------------------------------------------------------
 // DX compiles in the explicit diffusion increments (Ki, Redi, i_vert_diff off):
 // 20 thousand nodes, 47 layers, 4 tracers: K_L 157 us and K_V 92, 361 for one
@@ -1048,7 +1051,9 @@ __global__ void __launch_bounds__(64) kL_node(DevMesh m, DevDyn d, DevTracers t,
 // wave forms the tridiagonal rows and right-hand sides of its columns with
 // lanes over the levels and leaves them in LDS; one wave sweeps with one lane
 // per row, and the waves add the result to T*. LDS rows have an odd length, so
-// that the lanes of the sweep, each on its own row, use different banks.
+// that the lanes of the sweep, each on its own row, use different banks. Eight
+// waves per SIMD leave the plain form 64 registers, of which two levels per lane
+// spill 7 (32 bytes a lane).
 // XF bit 0 (use_wsplit): the non-FCT tracers' rows also take the implicit part
 // w_i of the split W, a second set of rows; bit 1: the K33 terms of Redi and
 // tracers with i_vert_diff off, which are left as they are. KV_LO instead solves
@@ -1383,10 +1388,10 @@ void fgpu_kd_shape(const fgpu_context *c, int *tch_out, int *cpb_out)
 // takes 16.4 ms by <3,2> and 22.6 by <2,1> with 32-bit ones, K_L 21.9 and 22.1.
 // The lines between the mappings were measured per kernel, in us, at 47 layers with 2 tracers (126,858 nodes) and 32
 // tracers (12 thousand), and at 70 layers with 10 tracers (40 thousand):
-//   K_A  <1,1> 473, 567; <2,2> 502, 430 | <2,1> 728, <3,2> 744
-//   K_B  <1,1> 298, 270; <2,2> 349, 297 | <2,1> 591, <3,2> 520
-//   K_C  <1,1> 295, 459; <2,2> 330, 395 | <2,1> 610, <3,2> 638
-//   K_L  <1,1> 362, 494; <2,2> 349, 439 | <2,1> 732, <3,2> 686
+//   K_A  <1,1> 507, 576; <2,2> 506, 440 | <2,1> 730, <3,2> 740
+//   K_B  <1,1> 298, 271; <2,2> 469, 366 | <2,1> 710, <3,2> 518
+//   K_C  <1,1> 315, 462; <2,2> 329, 396 | <2,1> 648, <3,2> 637
+//   K_L  <1,1> 363, 491; <2,2> 351, 441 | <2,1> 700, <3,2> 687
 // Two levels per lane halve a row's vector memory instructions, two tracers per
 // wave form the offsets once for both; against that stand the registers (fewer
 // waves per SIMD) and what a second tracer's lanes repeat of the first one's

@@ -807,7 +807,7 @@ extern "C" int fgpu_tracer_set_valuesAB(fgpu_context *c, int tr_num, const doubl
     FGPU_HIP(hipMemcpyAsync(c->t.TAB + c->t.sN * tr, valuesAB, c->t.sN * sizeof(double), hipMemcpyHostToDevice,
                             c->stream));
     hipLaunchKernelGGL(k_tr_xy, dim3(nblk((size_t)c->m.F2 * c->m.L), 1), dim3(BLK), 0, c->stream, c->m, c->t, tr);
-        LAUNCH_CHECK("k_tr_xy");
+    LAUNCH_CHECK("k_tr_xy");
     CELL_LAUNCH(k_node_grad, ROW_LEVELS, c->m.N2, 1, c->m, c->t, tr);
     FGPU_HIP(hipStreamSynchronize(c->stream));
     return FGPU_OK;
@@ -842,7 +842,7 @@ extern "C" int fgpu_diff_tracers_ale(fgpu_context *c, double dt, int tr_num)
     if ((rc = fgpu_ensure_diff(c))) return rc;
     if ((rc = fgpu_launch_diff(c, tr, 1, dt))) return rc;
     hipLaunchKernelGGL(k_tstar, dim3(nblk((size_t)c->m.N2 * c->m.L), 1), dim3(BLK), 0, c->stream, c->m, c->d, c->t, tr, dt);
-        LAUNCH_CHECK("k_tstar");
+    LAUNCH_CHECK("k_tstar");
     if (c->h_ivd[tr])
         if ((rc = launch_vdiff(c, tr, 1, dt, 1, -1))) return rc;
     FGPU_HIP(hipStreamSynchronize(c->stream));

@@ -383,31 +383,30 @@ class Context:
         return out
 
     def autotune_step(self, dt, nsteps=5):
-        """Pick the fastest launch shape of the fused step; returns (tracers per block, ms/step)."""
+        """Pick the fastest number of tracers per block of the fused step; returns (tracers per block, ms/step)."""
         tpb = C.c_int()
         ms = C.c_double()
         _check(self.L.fgpu_autotune_step(self.h, float(dt), int(nsteps), C.byref(tpb), C.byref(ms)))
         return tpb.value, ms.value
 
     def step_shape(self):
-        """(tracers per block, tracers per Thomas chunk, columns per block) of the fused step."""
+        """(tracers per block, Thomas chunk, columns per block): the first as launched, the others settings that
+        no kernel reads (fgpu_step_shape)."""
         a, b, c = C.c_int(), C.c_int(), C.c_int()
         _check(self.L.fgpu_step_shape(self.h, C.byref(a), C.byref(b), C.byref(c)))
         return a.value, b.value, c.value
 
     def set_step_shape(self, tpb, tch, cpb, kd=0, kc=0, ka=1, kb=1):
-        """Fix (tracers per block, Thomas chunk, columns per block, last-kernel variant,
-        tracers per block of the (tracer, level) bound kernel, 0 for the per-column one,
-        levels per lane of the edge-flux and of the LO kernel, 1 or 2)."""
+        """Fix the tracers per block. The other settings told former kernels apart: they are kept and
+        reported, and select nothing (fgpu_set_step_shape)."""
         _check(self.L.fgpu_set_step_shape(self.h, int(tpb), int(tch), int(cpb), int(kd), int(kc), int(ka), int(kb)))
 
     def step_variant(self):
-        """Last kernel of the plain step: 0 lock-step, 1 with a sweep wave, 2 one wave per column."""
+        """The kept last-kernel setting, which no kernel reads."""
         return self.step_variants()[0]
 
     def step_variants(self):
-        """(last-kernel variant, tracers per block of the (tracer, level) bound kernel or 0,
-        levels per lane of the edge-flux kernel, levels per lane of the LO kernel)."""
+        """The kept settings (kd, kc, ka, kb), which no kernel reads (fgpu_step_variant)."""
         v, kc, ka, kb = C.c_int(), C.c_int(), C.c_int(), C.c_int()
         _check(self.L.fgpu_step_variant(self.h, C.byref(v), C.byref(kc), C.byref(ka), C.byref(kb)))
         return v.value, kc.value, ka.value, kb.value

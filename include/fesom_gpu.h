@@ -223,40 +223,28 @@ int fgpu_solve_tracers_ale_timed(fgpu_context *ctx, double dt, int nsteps, doubl
 int fgpu_profile_enable(fgpu_context *ctx, int on);
 int fgpu_profile_count(fgpu_context *ctx);
 int fgpu_profile_read(fgpu_context *ctx, int idx, char *name, int name_len, double *total_ms, int *launches);
-/* Autotuner of the fused step (no counterpart in the reference): times the
- * candidate launch shapes (tracers per block 1, 2, 4, ..., all, crossed with 2,
- * 4, 5 or 8 tracers per Thomas chunk and 1, 4 or 8 columns per block of the last
- * kernel for columns of up to 64 levels, 1 to 4 for columns of up to 72
- * interfaces, 1 or 2 for deeper ones) over nsteps
- * replayed steps, keeps the fastest
- * for this context and reports its tracers per block and time. The tracer
- * state is restored afterwards; results do not depend on the choice. */
+/* Autotuner of the fused step (no counterpart in the reference): times 1, 2, 4,
+ * ... and all tracers per block over nsteps replayed steps each, keeps the
+ * fastest for this context and reports it and its time. The tracer state is
+ * restored afterwards; results do not depend on the choice. */
 int fgpu_autotune_step(fgpu_context *ctx, double dt, int nsteps, int *best_tpb, double *best_ms_per_step);
-/* The fused step's current launch shape (no counterpart in the reference):
- * tracers per block, tracers per Thomas chunk, columns per block of the last
- * kernel as launched (a shape that needs another chunk size reports the one used). */
+/* The fused step's launch shape (no counterpart in the reference):
+ * tracers_per_block as launched. thomas_chunk and columns_per_block are the
+ * settings of fgpu_set_step_shape, brought into the sets that the former last
+ * kernel had; no kernel reads them. */
 int fgpu_step_shape(fgpu_context *ctx, int *tracers_per_block, int *thomas_chunk, int *columns_per_block);
-/* Kernel variants of the step (no counterpart in the reference). kd_variant,
- * the last kernel of the plain step:
- * 0 the block's waves in lock-step, the sweeps on the first wave's lanes;
- * 1 one wave per column plus a wave per block that sweeps the previous chunk
- *   while the column waves compute the next;
- * 2 one wave per column that sweeps its own column.
- * kc_tracers, the bound kernel: 0 one column's levels over the lanes, 1, 2 or 4
- * tracers per block with (tracer, level) items over the lanes.
- * ka_levels_per_lane, the edge-flux kernel: 1 one level per lane (64 or 128
- * lanes per edge), 2 two adjacent levels per lane with 16-byte accesses (one
- * wave per edge; meshes with an even number of layers only).
- * kb_levels_per_lane, the LO kernel, likewise (also not with the W split or
- * CDIFF/PPM tracers).
- * The autotuner picks all four with the shape; FGPU_STEP_KD=lockstep|sweepwave|
- * wavelocal, FGPU_STEP_KC=0|1|2|4, FGPU_STEP_KA=1|2 and FGPU_STEP_KB=1|2 set
- * them when a context is created. Results are the same bit for bit. */
+/* The other settings of fgpu_set_step_shape, as a former step's kernels would
+ * have taken them (kd_variant 0 on a step with extra terms, levels per lane 1 for
+ * an odd number of layers). No kernel reads them: how many levels a lane and how
+ * many tracers a wave takes follows from the column depth, the tracers' schemes
+ * and the field size. */
 int fgpu_step_variant(fgpu_context *ctx, int *kd_variant, int *kc_tracers, int *ka_levels_per_lane,
                       int *kb_levels_per_lane);
-/* Sets the launch shape and the kernel variants instead of the autotuner (no
- * counterpart in the reference); values outside the sets above fall back as
- * fgpu_step_shape reports. */
+/* Sets tracers_per_block instead of the autotuner (no counterpart in the
+ * reference). The other arguments, and FGPU_STEP_TCH, FGPU_STEP_CPB,
+ * FGPU_STEP_KD, FGPU_STEP_KC, FGPU_STEP_KA and FGPU_STEP_KB at the context's
+ * creation, told former kernels apart: they are checked, kept and reported by the
+ * two calls above, and select nothing. */
 int fgpu_set_step_shape(fgpu_context *ctx, int tracers_per_block, int thomas_chunk, int columns_per_block,
                         int kd_variant, int kc_tracers, int ka_levels_per_lane, int kb_levels_per_lane);
 /* Tracer content sum_n sum_k areasvol*hnode_new*T (deterministic device sum). */
