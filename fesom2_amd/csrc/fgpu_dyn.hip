@@ -411,6 +411,7 @@ int ensure_const_buf(fgpu_context *c, const double **p, size_t n)
     int rc = fgpu_alloc(c, (void **)&q, sizeof(double) * n);
     if (rc) return rc;
     if ((rc = fgpu_zero(c, q, sizeof(double) * n))) return rc;
+    FGPU_HIP(hipStreamSynchronize(c->stream));   // fgpu_set_velocity uploads into it
     *p = q;
     return FGPU_OK;
 }

@@ -3,7 +3,9 @@
  * that the library's calls resolve to it. It counts what is enqueued on
  * another stream while a fill of the null stream may still run (hipMemset
  * returns before the fill has ended, and a non-blocking stream does not wait
- * for the null stream), and it can let the n-th allocation from now fail. */
+ * for the null stream), and what the null stream reads or writes while a fill of
+ * another stream may still run there. It can let the n-th allocation from now
+ * fail. */
 #include <stddef.h>
 #include <stdlib.h>
 #include <string.h>
@@ -14,6 +16,8 @@ enum { NOMEM = 2, D2D = 3 };
 
 static int pending, hazards, fail_in = -1;
 static size_t live;
+static struct { char *p; size_t n; } fill[64];   /* fills of the other streams that may still run */
+static int fills;
 
 EXPORT int host_hazards(void) { return hazards; }
 EXPORT void host_fail_in(int n) { fail_in = n; }   /* 0: the next allocation; < 0: none */
@@ -29,6 +33,11 @@ static int waited(void)
 {
     pending = 0;
     return 0;
+}
+static void touched(const void *q, size_t n)
+{
+    for (int i = 0; i < fills; ++i)
+        if ((const char *)q < fill[i].p + fill[i].n && fill[i].p < (const char *)q + n) ++hazards;
 }
 
 EXPORT int hipMalloc(void **p, size_t n)
@@ -51,27 +60,57 @@ EXPORT int hipFree(void *p)
         live -= q[0];
         free(q);
     }
+    fills = 0;   /* waits for the device */
     return waited();
 }
 EXPORT int hipHostMalloc(void **p, size_t n, unsigned flags) { (void)flags; *p = calloc(1, n); return 0; }
 EXPORT int hipHostFree(void *p) { free(p); return waited(); }
-EXPORT int hipMemset(void *p, int v, size_t n) { memset(p, v, n); pending = 1; return 0; }
-EXPORT int hipMemsetAsync(void *p, int v, size_t n, void *s) { memset(p, v, n); if (!s) pending = 1; return used(s); }
+EXPORT int hipMemset(void *p, int v, size_t n) { touched(p, n); memset(p, v, n); pending = 1; return 0; }
+EXPORT int hipMemsetAsync(void *p, int v, size_t n, void *s)
+{
+    memset(p, v, n);
+    if (!s) {
+        touched(p, n);
+        pending = 1;
+    } else if (fills < 64) {
+        fill[fills].p = p;
+        fill[fills++].n = n;
+    } else {
+        abort();
+    }
+    return used(s);
+}
 EXPORT int hipMemcpy(void *d, const void *s, size_t n, int kind)
 {
+    touched(d, n);
+    touched(s, n);
     memmove(d, s, n);
     if (kind == D2D) pending = 1;
     else waited();
     return 0;
 }
-EXPORT int hipMemcpyAsync(void *d, const void *s, size_t n, int kind, void *st) { (void)kind; memmove(d, s, n); return used(st); }
+EXPORT int hipMemcpyAsync(void *d, const void *s, size_t n, int kind, void *st)
+{
+    (void)kind;
+    if (!st) {
+        touched(d, n);
+        touched(s, n);
+    }
+    memmove(d, s, n);
+    return used(st);
+}
 EXPORT int hipLaunchKernel(const void *f, dim3_t g, dim3_t b, void **a, size_t l, void *s)
 {
     (void)f; (void)g; (void)b; (void)a; (void)l;
     return used(s);
 }
 EXPORT int hipGraphLaunch(void *g, void *s) { (void)g; return used(s); }
-EXPORT int hipStreamSynchronize(void *s) { return s ? 0 : waited(); }
+EXPORT int hipStreamSynchronize(void *s)
+{
+    if (!s) return waited();
+    fills = 0;   /* one stream a context, one context at a time in the tests that fill */
+    return 0;
+}
 
 EXPORT int hipGetDeviceCount(int *n) { *n = 1; return 0; }
 EXPORT int hipSetDevice(int d) { (void)d; return 0; }
