@@ -1327,15 +1327,15 @@ __global__ void k_zn_vdiff(DevMesh m, double *zn, double *zbn)
 // ==============================================================================
 int fgpu_compute_zn(fgpu_context *c)
 {
-    if (!c->m.zn_vd) {
-        double *p;
-        int rc = fgpu_alloc(c, (void **)&p, sizeof(double) * (size_t)c->N2 * (c->nl - 1));
+    struct A { const double **p; size_t n; } arrs[] = {
+        {&c->m.zn_vd, (size_t)c->N2 * (c->nl - 1)}, {&c->m.zbn_vd, (size_t)c->N2 * c->nl}};
+    for (auto &a : arrs) {
+        if (*a.p) continue;
+        double *q = nullptr;
+        int rc = fgpu_alloc(c, (void **)&q, sizeof(double) * a.n);
         if (rc) return rc;
-        if ((rc = fgpu_zero(c, p, sizeof(double) * (size_t)c->N2 * (c->nl - 1)))) return rc;
-        c->m.zn_vd = p;
-        if ((rc = fgpu_alloc(c, (void **)&p, sizeof(double) * (size_t)c->N2 * c->nl))) return rc;
-        if ((rc = fgpu_zero(c, p, sizeof(double) * (size_t)c->N2 * c->nl))) return rc;
-        c->m.zbn_vd = p;
+        if ((rc = fgpu_zero(c, q, sizeof(double) * a.n))) return rc;
+        *a.p = q;
     }
     hipLaunchKernelGGL(k_zn_vdiff, dim3((c->N2 + 255) / 256), dim3(256), 0, c->stream, c->m, (double *)c->m.zn_vd,
                        (double *)c->m.zbn_vd);

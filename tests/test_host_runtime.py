@@ -192,3 +192,31 @@ def test_contexts_share_the_download_threads(runtime):
         c.close()
         assert threads() == base
         """)
+
+
+def test_vertical_after_a_failed_allocation(runtime):
+    """fgpu_set_vertical repeated after FGPU_ERR_NOMEM has every array, those of
+    the implicit diffusion's levels among them."""
+    _run(runtime, """
+        ctx = gpu.Context()
+        ctx.mesh_init(mesh)
+        want = rt.host_live_bytes()
+        ctx.close()
+        failed = 0
+        for k in range(200):
+            ctx = gpu.Context()
+            rt.host_fail_in(k)
+            try:
+                ctx.mesh_init(mesh)
+            except gpu.FesomGpuError as e:
+                assert "hipMalloc" in str(e)
+                if ctx.nl:   # the mesh is there, its vertical geometry is not
+                    failed += 1
+                    ctx.set_vertical(mesh)
+                    assert rt.host_live_bytes() == want, k
+            else:
+                rt.host_fail_in(-1)
+                break
+            ctx.close()
+        assert failed == 12
+        """)
