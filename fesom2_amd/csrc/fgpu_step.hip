@@ -1047,9 +1047,9 @@ __global__ void __launch_bounds__(64) kL_node(DevMesh m, DevDyn d, DevTracers t,
 // a block: three dependent loads, the rows, and two serial passes over the
 // levels (about 200 cycles a level for the two dependent divisions).
 // ------------------------------------------------------------------------------
-// A block of eight waves takes NC columns x TB tracers, NC x TB <= 64 rows. Each
-// wave forms the tridiagonal rows and right-hand sides of its columns with
-// lanes over the levels and leaves them in LDS; one wave sweeps with one lane
+// A block of up to eight waves takes NC columns x TB tracers, NC x TB <= 64 rows.
+// Each wave forms the tridiagonal rows and right-hand sides of its columns with
+// lanes over the levels, of 64 >> lsh columns at once (SH), and leaves them in LDS; one wave sweeps with one lane
 // per row, and the waves add the result to T*. LDS rows have an odd length, so
 // that the lanes of the sweep, each on its own row, use different banks. Eight
 // waves per SIMD leave the plain form 64 registers, of which two levels per lane
@@ -1062,15 +1062,16 @@ __global__ void __launch_bounds__(64) kL_node(DevMesh m, DevDyn d, DevTracers t,
 #define KV_WS 1
 #define KV_DX 2
 #define KV_LO 4
-#define KV_NW 8   // waves of a block
+#define KV_NW 8   // waves of a block at most
 #define KV_TP 2   // tracers whose rows are loaded together
-template <int NV, int XF>
-__global__ void __launch_bounds__(64 * KV_NW) __attribute__((amdgpu_waves_per_eu(XF == 0 ? 8 : 4)))
-kV_cols(DevMesh m, DevDyn d, DevTracers t, int tr0, int ntr, double dt, int all, int clamp_tracer, int NC, int TB)
+template <int NV, int XF, bool SH>
+__global__ void __launch_bounds__(64 * KV_NW) __attribute__((amdgpu_waves_per_eu(XF == 0 ? (SH ? 6 : 8) : 4)))
+kV_cols(DevMesh m, DevDyn d, DevTracers t, int tr0, int ntr, double dt, int all, int clamp_tracer, int NC, int TB, int lsh)
 {
     extern __shared__ double lds[];
     const int L = m.L, NL = m.NL, RS = L | 1;
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int part = SH ? lane >> lsh : 0, step = (int)(blockDim.x >> 6) << (SH ? 6 - lsh : 0);
     const int col0 = xcd_unit() * NC;
     if (col0 >= m.N2) return;
     const int ncol = min(NC, m.N2 - col0);
@@ -1084,12 +1085,28 @@ kV_cols(DevMesh m, DevDyn d, DevTracers t, int tr0, int ntr, double dt, int all,
     auto solved = [&](int tr) { return LO ? ldc(t.lim + tr) == LIM_FCT : (XF == 0 || all || ldc(t.ivd + tr) != 0); };
     auto second = [&](int tr) { return WS && ldc(t.lim + tr) != LIM_FCT; };
     // the block's columns, one per lane
-    const int nl_ = m.node_ord[col0 + min(lane, ncol - 1)];
-    const int z0l = m.ulevn[nl_], z1l = m.nlevn[nl_];
-    const int kb = lane * NV + 1;
+    const int *rec = m.col_rec + 8 * (size_t)(col0 + min(lane, ncol - 1));
+    const int nl_ = rec[0], z0l = rec[3], z1l = rec[4];
+    const int kb = (SH ? lane & ((1 << lsh) - 1) : lane) * NV + 1;
     const unsigned off = 8u * (unsigned)(kb - 1);
-    for (int c = w; c < ncol; c += KV_NW) {
-        const int n = rl(nl_, c), nzmin = rl(z0l, c), nzmax = rl(z1l, c);
+    // the lane's column of the block, the wave's one without SH; past the last one a lane has no level
+    auto column = [&](int c, int &n, int &nzmin, int &nzmax) __attribute__((always_inline)) {
+        if constexpr (SH) {
+            const int at = min(c, ncol - 1);
+            n = __shfl(nl_, at);
+            nzmin = __shfl(z0l, at);
+            nzmax = __shfl(z1l, at);
+            if (c >= ncol) nzmax = 0;
+        } else {
+            n = rl(nl_, c);
+            nzmin = rl(z0l, c);
+            nzmax = rl(z1l, c);
+        }
+    };
+    for (int c0 = SH ? w << (6 - lsh) : w; c0 < ncol; c0 += step) {
+        const int c = c0 + part;
+        int n, nzmin, nzmax;
+        column(c, n, nzmin, nzmax);
         const size_t nL = (size_t)n * L, nNL = (size_t)n * NL;
         double hn[NV], av[NV], zk[NV], kv[NV], ar[NV], zu[NV], zd[NV], kvd[NV], ard[NV], a_[NV], c_[NV], bd_[NV];
         double ts[KV_TP][NV], wi[NV], wid[NV], wa[WS ? NV : 1], wb[WS ? NV : 1], wc[WS ? NV : 1], k33[NV], k33u[NV];
@@ -1269,8 +1286,10 @@ kV_cols(DevMesh m, DevDyn d, DevTracers t, int tr0, int ntr, double dt, int all,
         }
     }
     __syncthreads();
-    for (int c = w; c < ncol; c += KV_NW) {
-        const int n = rl(nl_, c), nzmin = rl(z0l, c), nzmax = rl(z1l, c);
+    for (int c0 = SH ? w << (6 - lsh) : w; c0 < ncol; c0 += step) {
+        const int c = c0 + part;
+        int n, nzmin, nzmax;
+        column(c, n, nzmin, nzmax);
         const size_t nL = (size_t)n * L;
         bool on[NV], any = false;
 #pragma unroll
@@ -1438,10 +1457,19 @@ static void launch_kv(fgpu_context *c, int tr0, int nt, double dt, int all, int 
     // sweeps have to run side by side
     int NC = std::min(64 / TB, 40000 / (row * (coef + TB)));
     NC = std::max(1, std::min(NC, (int)((size_t)m.N2 * groups / 1024)));
+    // up to 32 layers leave half a wave free, which further columns take: with one
+    // column to a wave 120 thousand nodes, 4 layers, 1 tracer took 67 us (13), 60
+    // thousand nodes, 16 layers 48 us (24)
+    int lsh = 6;
+    while (lsh > 1 && (1 << (lsh - 1)) >= m.L) --lsh;
+    // no waves without a column: they held the slots of further blocks (3,000
+    // nodes, 24 layers, 1 tracer: 22 us with eight waves, 15 with one)
+    const int waves = std::min(KV_NW, (NC + (64 >> lsh) - 1) >> (6 - lsh));
     const size_t lds = (size_t)row * (coef + TB) * NC;
-    const dim3 g(xcd_grid((m.N2 + NC - 1) / NC), (unsigned)groups), b(64 * KV_NW);
-    if (m.NL <= 64) hipLaunchKernelGGL((kV_cols<1, XF>), g, b, lds, c->stream, m, c->d, c->t, tr0, nt, dt, all, clamp, NC, TB);
-    else hipLaunchKernelGGL((kV_cols<2, XF>), g, b, lds, c->stream, m, c->d, c->t, tr0, nt, dt, all, clamp, NC, TB);
+    const dim3 g(xcd_grid((m.N2 + NC - 1) / NC), (unsigned)groups), b(64 * waves);
+    if (lsh < 6) hipLaunchKernelGGL((kV_cols<1, XF, true>), g, b, lds, c->stream, m, c->d, c->t, tr0, nt, dt, all, clamp, NC, TB, lsh);
+    else if (m.NL <= 64) hipLaunchKernelGGL((kV_cols<1, XF, false>), g, b, lds, c->stream, m, c->d, c->t, tr0, nt, dt, all, clamp, NC, TB, lsh);
+    else hipLaunchKernelGGL((kV_cols<2, XF, false>), g, b, lds, c->stream, m, c->d, c->t, tr0, nt, dt, all, clamp, NC, TB, lsh);
 }
 
 // K_V of tracers tr0..tr0+ntr-1; all: also of those with i_vert_diff off
