@@ -12,13 +12,17 @@
 //                 (:1439-1522) under Redi.
 //
 // k_hdiff_edge and k_vextra give an edge or column to one wave: 2^sh lanes take
-// its levels, 2^sh the smallest power of two above the number of layers and at
-// most 64, and the wave's 64 / 2^sh lane groups take a tracer each. What does
-// not depend on the tracer is loaded once per level. Both are bound by the
-// gathers of T. 20 thousand nodes, 47 layers, 4 tracers: k_hdiff_edge 232 ->
-// 124 us against one thread per (edge, level, tracer), which divided its index
-// and loaded the edge's geometry for itself; k_zbar and k_vextra 1124 -> 113 us
-// against one thread per column, whose neighbours in a wave read rows apart.
+// its levels, 2^sh the smallest power of two above the number of layers (without
+// Redi k_hdiff_edge's not below it) and at most 64, and the wave's 64 / 2^sh lane
+// groups take a tracer each. What does not depend on the tracer is loaded once
+// per level. Fewer tracers than groups leave the others to further edges or
+// columns. Both are bound by the gathers of T. 20 thousand nodes, 47 layers, 4
+// tracers: k_hdiff_edge 232 -> 124 us against one thread per (edge, level,
+// tracer), which divided its index and loaded the edge's geometry for itself;
+// k_zbar and k_vextra 1124 -> 113 us against one thread per column, whose
+// neighbours in a wave read rows apart. 120 thousand nodes, 4 layers, 1 tracer,
+// one edge or column to a wave and as many as fit: k_hdiff_edge with Redi 226 and
+// 62 us, without 159 and 29, k_vextra 174 and 43.
 //
 // They write the increments' parts (t.hd, t.ve, t.vr); the node update of
 // either step (k_node_update / k_tstar, kL_node) adds them to del_ttf in the
@@ -64,12 +68,15 @@ __device__ __forceinline__ void grad_el(const Elem &E, const double *T, double &
     gy = E.g[3] * t0 + E.g[4] * t1 + E.g[5] * t2;
 }
 
-template <bool REDI>
-__global__ void __launch_bounds__(64) k_hdiff_edge(DevMesh m, DevDyn d, DevTracers t, int tr0, int ntr, int sh)
+// MULTI: with fewer tracers than lane groups the groups go round 2^eg edges
+// or columns, whose records the lanes then load for themselves
+template <bool REDI, bool MULTI>
+__global__ void __launch_bounds__(64) k_hdiff_edge(DevMesh m, DevDyn d, DevTracers t, int tr0, int ntr, int sh, int eg)
 {
-    const int je = xcd_unit();
+    const int L = m.L, idx = threadIdx.x & ((1 << sh) - 1), gt = 64 >> sh >> (MULTI ? eg : 0);
+    const int g = (int)(threadIdx.x >> sh) & (gt - 1);
+    const int je = MULTI ? (xcd_unit() << eg) + (int)(threadIdx.x >> sh) / gt : xcd_unit();
     if (je >= m.E2) return;
-    const int L = m.L, idx = threadIdx.x & ((1 << sh) - 1), g = threadIdx.x >> sh, gt = 64 >> sh;
     const int *ri = m.erec_i + (size_t)je * ERI;
     const double *rd = m.erec_d + (size_t)je * ERD;
     const int n1 = ldc(ri + ER_N1), n2 = ldc(ri + ER_N2), el1 = ldc(ri + ER_EL1), el2 = ldc(ri + ER_EL2);
@@ -81,8 +88,8 @@ __global__ void __launch_bounds__(64) k_hdiff_edge(DevMesh m, DevDyn d, DevTrace
     const Elem E1 = load_elem(m, el1), E2 = load_elem(m, q2);
     double *hd = t.hd + (size_t)ldc(ri + ER_E) * L;
     const int zt1 = ldc(m.ulevn + n1), zb1 = ldc(m.nlevn + n1), zt2 = ldc(m.ulevn + n2), zb2 = ldc(m.nlevn + n2);
-    // the last lane only supplies T_z at its upper interface to the lane before
-    for (int kb = lo; kb <= hi; kb += (1 << sh) - 1) {
+    // with the slope terms the last lane only supplies T_z at its upper interface to the lane before
+    for (int kb = lo; kb <= hi; kb += (1 << sh) - (REDI ? 1 : 0)) {
         const int k = kb + idx, kc = min(k, L), ku = max(kc - 1, 1);
         // cases (A)/(D): el1 alone, (B)/(E): el2 alone, (C): both. The levels without either keep the zeros
         // that the buffer starts with
@@ -90,7 +97,7 @@ __global__ void __launch_bounds__(64) k_hdiff_edge(DevMesh m, DevDyn d, DevTrace
         // in a level gap between the elements both segments reach into it, where the reference's element
         // gradients are zero: the slope terms of both
         const bool gap = REDI && two && ((k > nl1 && k < nu2) || (k > nl2 && k < nu1));
-        const bool out = (p1 || p2 || gap) && idx < (1 << sh) - 1;
+        const bool out = (p1 || p2 || gap) && (!REDI || idx < (1 << sh) - 1);
         const size_t c1 = (size_t)n1 * L + kc - 1, c2 = (size_t)n2 * L + kc - 1;
         const double Kh = (d.Ki[c1] + d.Ki[c2]) / 2.0;
         const double h1 = m.helem[(size_t)el1 * L + kc - 1], h2 = m.helem[(size_t)q2 * L + kc - 1];
@@ -161,11 +168,13 @@ __global__ void __launch_bounds__(64) k_zbar(DevMesh m, double *zb)
         for (int k = threadIdx.x; k < NL; k += 64) zb[(size_t)(n0 + c) * NL + k] = zs[c * P + k];
 }
 
-__global__ void __launch_bounds__(64) k_vextra(DevMesh m, DevDyn d, DevTracers t, int tr0, int ntr, int sh, double dt)
+template <bool MULTI>
+__global__ void __launch_bounds__(64) k_vextra(DevMesh m, DevDyn d, DevTracers t, int tr0, int ntr, int sh, int eg, double dt)
 {
-    const int jn = xcd_unit();
+    const int L = m.L, NL = m.NL, lp = 1 << sh, idx = threadIdx.x & (lp - 1), gt = 64 >> sh >> (MULTI ? eg : 0);
+    const int g = (int)(threadIdx.x >> sh) & (gt - 1);
+    const int jn = MULTI ? (xcd_unit() << eg) + (int)(threadIdx.x >> sh) / gt : xcd_unit();
     if (jn >= m.N2) return;
-    const int L = m.L, NL = m.NL, lp = 1 << sh, idx = threadIdx.x & (lp - 1), g = threadIdx.x >> sh, gt = 64 >> sh;
     const int n = ldc(m.node_ord + jn), ul1 = ldc(m.ulevn + n), nl1 = ldc(m.nlevn + n) - 1;
     const int num = ldc(m.nie_num + n);
     const bool redi = d.redi != 0;
@@ -259,14 +268,27 @@ int fgpu_launch_diff(fgpu_context *c, int tr0, int ntr, double dt)
     const DevMesh &m = c->m;
     bool ve = false;
     for (int i = tr0; i < tr0 + ntr; ++i) ve = ve || !c->h_ivd[i];
-    int sh = 3;   // lanes per column: above the layer count, so that the lane below the deepest layer exists
+    // lanes per column: above the layer count where levels exchange values, so that the lane below the deepest
+    // layer exists, else (1 << se) no fewer than it
+    int sh = 3, se = 2;
     while (sh < 6 && (1 << sh) <= m.L) ++sh;
+    while (se < 6 && (1 << se) < m.L) ++se;
+    if (c->d.redi) se = sh;
+    // 2^eg edges and 2^cg columns per wave, as many as leave a lane group to each tracer
+    auto per_wave = [&](int s) {
+        int g = 6 - s;
+        while (g > 0 && (64 >> s >> g) < ntr) --g;
+        return g;
+    };
+    const int eg = per_wave(se), cg = per_wave(sh);
     if (c->d.hdiff) {
         if (!c->t.hd) return fgpu_fail(FGPU_ERR_STATE, "diffusion buffers not allocated");
         ProfScope ps(c, "k_hdiff_edge");
-        const dim3 g(xcd_grid(m.E2));
-        if (c->d.redi) hipLaunchKernelGGL(k_hdiff_edge<true>, g, dim3(64), 0, c->stream, m, c->d, c->t, tr0, ntr, sh);
-        else hipLaunchKernelGGL(k_hdiff_edge<false>, g, dim3(64), 0, c->stream, m, c->d, c->t, tr0, ntr, sh);
+        const dim3 g(xcd_grid((m.E2 + (1 << eg) - 1) >> eg)), b(64);
+        if (c->d.redi && eg) hipLaunchKernelGGL((k_hdiff_edge<true, true>), g, b, 0, c->stream, m, c->d, c->t, tr0, ntr, se, eg);
+        else if (c->d.redi) hipLaunchKernelGGL((k_hdiff_edge<true, false>), g, b, 0, c->stream, m, c->d, c->t, tr0, ntr, se, eg);
+        else if (eg) hipLaunchKernelGGL((k_hdiff_edge<false, true>), g, b, 0, c->stream, m, c->d, c->t, tr0, ntr, se, eg);
+        else hipLaunchKernelGGL((k_hdiff_edge<false, false>), g, b, 0, c->stream, m, c->d, c->t, tr0, ntr, se, eg);
         FGPU_HIP(hipGetLastError());
     }
     if (ve || c->d.redi) {
@@ -279,7 +301,9 @@ int fgpu_launch_diff(fgpu_context *c, int tr0, int ntr, double dt)
             FGPU_HIP(hipGetLastError());
         }
         ProfScope ps(c, "k_vextra");
-        hipLaunchKernelGGL(k_vextra, dim3(xcd_grid(m.N2)), dim3(64), 0, c->stream, m, c->d, c->t, tr0, ntr, sh, dt);
+        const dim3 g(xcd_grid((m.N2 + (1 << cg) - 1) >> cg)), b(64);
+        if (cg) hipLaunchKernelGGL(k_vextra<true>, g, b, 0, c->stream, m, c->d, c->t, tr0, ntr, sh, cg, dt);
+        else hipLaunchKernelGGL(k_vextra<false>, g, b, 0, c->stream, m, c->d, c->t, tr0, ntr, sh, cg, dt);
         FGPU_HIP(hipGetLastError());
     }
     return FGPU_OK;

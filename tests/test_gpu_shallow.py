@@ -55,6 +55,16 @@ def test_shallow_columns(layers, ntr, nx, ny, terms):
     _check(mesh, st, schemes)
 
 
+@pytest.mark.parametrize("layers,ntr,nx,ny", [(3, 1, 20, 14), (4, 2, 61, 50), (8, 1, 60, 50), (12, 3, 60, 50), (16, 1, 61, 50),
+                                              (17, 2, 60, 50), (32, 1, 60, 50), (33, 1, 60, 50)])
+def test_shallow_horizontal_diffusion(layers, ntr, nx, ny):
+    """Ki without Redi, whose levels exchange nothing: rows of exactly a lane group too."""
+    mesh, st = _case(layers, ntr, nx, ny)
+    st = dataclasses.replace(st, Ki=np.random.default_rng(layers).uniform(20.0, 400.0, (mesh.nod2D, layers)))
+    print(f"[gpu] Ki, {layers} layers, {ntr} tracers, {nx} x {ny} nodes", flush=True)
+    _check(mesh, st, [dict(i_vert_diff=i % 2 == 1) for i in range(ntr)])
+
+
 @pytest.mark.parametrize("layers,nx,ny", [(4, 120, 100), (12, 120, 101), (32, 60, 50), (33, 60, 50)])
 def test_shallow_per_tracer_calls(layers, nx, ny):
     from fesom2_amd import gpu
