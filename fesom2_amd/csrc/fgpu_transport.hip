@@ -105,19 +105,19 @@ __global__ void __launch_bounds__(BLK) k_tr_xy(DevMesh m, DevTracers t, int tr0)
 
 // ------------------------------------------------------------------------------
 // K2b: area-weighted mean of the element gradients around a node
-// (oce_muscl_adv.F90:388-401, 443-520) at its wet levels. An edge takes it at the
-// levels that its up- or downwind triangle lacks; formed per edge there, each wave
-// went through both nodes' elements for the lanes of a few levels (40 thousand
-// nodes, 47 layers: k_edge_flux 186 -> 132 us and about 60 of k_fill_up_dn_grad's,
-// for 38 us here).
+// (oce_muscl_adv.F90:388-401, 443-520) at its wet levels from kneed on, the first
+// one where an edge takes it: where its up- or downwind triangle lacks the level.
+// Formed per edge there, each wave went through both nodes' elements for the lanes
+// of a few levels (40 thousand nodes, 47 layers: k_edge_flux 186 -> 132 us and
+// about 60 of k_fill_up_dn_grad's, for 25 us here, 38 at every wet level).
 // ------------------------------------------------------------------------------
 template <bool ROW>
-__global__ void __launch_bounds__(BLK) k_node_grad(DevMesh m, DevTracers t, int tr0)
+__global__ void __launch_bounds__(BLK) k_node_grad(DevMesh m, DevTracers t, const int *kneed, int tr0)
 {
     const int tr = tr0 + blockIdx.y;
     int n, k;
     if (!cell<ROW>(m.N2, m.L, n, k)) return;
-    if (k < ld<ROW>(m.ulevn + n) || k > ld<ROW>(m.nlevn + n) - 1) return;
+    if (k < max(ld<ROW>(kneed + n), ld<ROW>(m.ulevn + n)) || k > ld<ROW>(m.nlevn + n) - 1) return;
     const double *trxy = t.tr_xy + t.sStg * tr;
     double tvol = 0.0, tx = 0.0, ty = 0.0;
     const int num = ld<ROW>(m.nie_num + n);
@@ -727,7 +727,7 @@ static int launch_init_ab(fgpu_context *c, int tr0, int ntr)
     }
     {
         ProfScope ps(c, "k_node_grad");
-        CELL_LAUNCH(k_node_grad, ROW_LEVELS, c->m.N2, ntr, m, c->t, tr0);
+        CELL_LAUNCH(k_node_grad, ROW_LEVELS, c->m.N2, ntr, m, c->t, c->d_kneed, tr0);
     }
     return FGPU_OK;
 }
@@ -808,7 +808,7 @@ extern "C" int fgpu_tracer_set_valuesAB(fgpu_context *c, int tr_num, const doubl
                             c->stream));
     hipLaunchKernelGGL(k_tr_xy, dim3(nblk((size_t)c->m.F2 * c->m.L), 1), dim3(BLK), 0, c->stream, c->m, c->t, tr);
     LAUNCH_CHECK("k_tr_xy");
-    CELL_LAUNCH(k_node_grad, ROW_LEVELS, c->m.N2, 1, c->m, c->t, tr);
+    CELL_LAUNCH(k_node_grad, ROW_LEVELS, c->m.N2, 1, c->m, c->t, c->d_kneed, tr);
     FGPU_HIP(hipStreamSynchronize(c->stream));
     return FGPU_OK;
 }
