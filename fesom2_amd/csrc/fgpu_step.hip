@@ -496,23 +496,27 @@ __global__ void __launch_bounds__(64) kA_edge(DevMesh m, DevDyn d, DevTracers t,
 // shifts. Against a block per column, 12 thousand nodes, 47 layers, 32 tracers:
 // 352 -> 281 us; 40 thousand nodes, 70 layers, 10 tracers: 537 -> 518; 126,858
 // nodes, 47 layers, 2 tracers: 291 -> 298, against K_A's gain.
-// EXTRA compiles in the CDIFF and PPM tracers and the W split (use_wsplit), where
-// the HO scheme is handed the upwind flux with the full W and the LO solution of
-// FCT tracers takes the implicit upwind advection with w_i afterwards (K_V on
-// it). PPM reads up to four layers around an interface, from LDS. 20 thousand
-// nodes, 47 layers, 4 tracers, W split: 140 us and 45 for the implicit step, 367
-// with a block per column, its sweeps on one lane.
-#define KB_EXTRA 1
+// KB_XV compiles in the CDIFF and PPM tracers; PPM reads up to four layers around
+// an interface, from LDS. KB_WS compiles in the W split (use_wsplit), where the HO
+// scheme is handed the upwind flux with the full W and the LO solution of FCT
+// tracers takes the implicit upwind advection with w_i afterwards (K_V on it). Each
+// has its own registers: 120 thousand nodes, 12 layers, 1 tracer 169 us with the W
+// split and 305 with PPM (168 without either), 299 and 414 where one form carried
+// both and ran two waves per SIMD. So one level per lane is held to the registers
+// of four waves, three with PPM.
+#define KB_XV 1    // CDIFF and PPM
 #define KB_GAP 2
+#define KB_WS 4    // the W split
 template <typename OFF, int NV, int GT, int FORM>
-__global__ void __launch_bounds__(64) kB_cols(DevMesh m, DevDyn d, DevTracers t, double dt, int tpb)
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NV > 1 || (FORM & KB_GAP) ? 1 : (FORM & KB_XV ? 3 : 4))))
+kB_cols(DevMesh m, DevDyn d, DevTracers t, double dt, int tpb)
 {
-    constexpr bool EXTRA = (FORM & KB_EXTRA) != 0, GAP = (FORM & KB_GAP) != 0;
+    constexpr bool XV = (FORM & KB_XV) != 0, GAP = (FORM & KB_GAP) != 0, WS = (FORM & KB_WS) != 0;
     Column<OFF, NV, GT> c;
     if (!load_column<(NV > 1), OFF, NV, GT>(m, t, c)) return;
-    static_assert(!EXTRA || GT == 1, "one column's rows in LDS");
-    __shared__ double sT[EXTRA ? 64 * NV : 1], sHn[EXTRA ? 64 * NV : 1], sHo[EXTRA ? 64 * NV : 1];
-    __shared__ double sW[EXTRA ? 64 * NV : 1], sWe[EXTRA ? 64 * NV : 1], sAr[EXTRA ? 64 * NV : 1];
+    static_assert(!XV || GT == 1, "one column's rows in LDS");
+    __shared__ double sT[XV ? 64 * NV : 1], sHn[XV ? 64 * NV : 1], sHo[XV ? 64 * NV : 1];
+    __shared__ double sW[XV ? 64 * NV : 1], sWe[XV ? 64 * NV : 1], sAr[XV ? 64 * NV : 1];
     const int nzmin = c.nzmin, nzmax = c.nzmax;
     const int L = m.L;
     bool first[NV], inner[NV], deep[NV], last[NV], face[NV];
@@ -549,7 +553,7 @@ __global__ void __launch_bounds__(64) kB_cols(DevMesh m, DevDyn d, DevTracers t,
             dz[s] = zu[s] - z[s];
             d1[s] = zb[s] - z[s];
             d2[s] = zb[s] - zu[s];
-            if constexpr (EXTRA) {
+            if constexpr (XV) {
                 const int i = c.kb + s - 1;
                 sHn[i] = hn[s];
                 sHo[i] = hh[s];
@@ -589,7 +593,7 @@ __global__ void __launch_bounds__(64) kB_cols(DevMesh m, DevDyn d, DevTracers t,
             const double b = -0.5 * (Tk[s] * (We[s] + fabs(We[s])) + Tu[s] * (We[s] - fabs(We[s]))) * ar[s];
             lk[s] = fct ? (first[s] ? a : (inner[s] ? b : 0.0)) : 0.0;
             lw[s] = lk[s];
-            if (EXTRA && d.wsplit) {
+            if (WS && d.wsplit) {
                 const double x = -W[s] * Tk[s] * ar[s];
                 const double y = -0.5 * (Tk[s] * (W[s] + fabs(W[s])) + Tu[s] * (W[s] - fabs(W[s]))) * ar[s];
                 lw[s] = fct ? (first[s] ? x : (inner[s] ? y : 0.0)) : 0.0;
@@ -629,7 +633,7 @@ __global__ void __launch_bounds__(64) kB_cols(DevMesh m, DevDyn d, DevTracers t,
                 f[s] = (first[s] ? top : (deep[s] ? ho : (last[s] ? 0.0 : near))) - lw[s];
                 if (nzmax - nzmin == 2 && inner[s]) f[s] = near - f[s];   // both rows at once
             }
-        } else if (EXTRA && ver == VER_PPM) {
+        } else if (XV && ver == VER_PPM) {
             wave_sync();
 #pragma unroll
             for (int s = 0; s < NV; ++s) sT[c.kb + s - 1] = A[s];
@@ -642,7 +646,7 @@ __global__ void __launch_bounds__(64) kB_cols(DevMesh m, DevDyn d, DevTracers t,
             for (int s = 0; s < NV; ++s) {
                 const double ww = fct ? W[s] : We[s];
                 const double a = -ww * A[s] * ar[s];
-                if (EXTRA && ver == VER_CDIFF) {   // adv_tra_ver_cdiff (oce_adv_tra_ver.F90:635-695)
+                if (XV && ver == VER_CDIFF) {   // adv_tra_ver_cdiff (oce_adv_tra_ver.F90:635-695)
                     const double b = -(0.5 * (Au[s] + A[s])) * ww * ar[s];
                     f[s] = first[s] ? a - lw[s] : (inner[s] ? b - lw[s] : lw[s]);
                 } else {
@@ -849,7 +853,7 @@ __global__ void __launch_bounds__(64) kC_cols(DevMesh m, DevTracers t, double dt
 // kernel's instructions. One kernel for both, a block per column, took 775 us at
 // 126,858 nodes, 47 layers, 2 tracers (K_L 350 us, K_V 160), 988 us at 12 thousand
 // nodes, 32 tracers (420, 150) and 1429 us at 40 thousand nodes, 70 layers, 10
-// tracers (688, 325).
+// tracers (688, 309).
 // ------------------------------------------------------------------------------
 // DX compiles in the explicit diffusion increments (Ki, Redi, i_vert_diff off):
 // 20 thousand nodes, 47 layers, 4 tracers: K_L 157 us and K_V 92, 361 for one
@@ -1053,7 +1057,7 @@ __global__ void __launch_bounds__(64) kL_node(DevMesh m, DevDyn d, DevTracers t,
 // per row, and the waves add the result to T*. LDS rows have an odd length, so
 // that the lanes of the sweep, each on its own row, use different banks. Eight
 // waves per SIMD leave the plain form 64 registers, of which two levels per lane
-// spill 7 (32 bytes a lane).
+// spill 7 (32 bytes a lane); several columns per wave need more, and six waves do.
 // XF bit 0 (use_wsplit): the non-FCT tracers' rows also take the implicit part
 // w_i of the split W, a second set of rows; bit 1: the K33 terms of Redi and
 // tracers with i_vert_diff off, which are left as they are. KV_LO instead solves
@@ -1493,8 +1497,8 @@ int fgpu_enqueue_fused_step(fgpu_context *c, double dt)
     // tracers per block: 1 runs every tracer's chain in its own waves
     const int tpb = std::max(1, std::min(c->step_tpb, nt));
     const unsigned ny = (unsigned)((nt + tpb - 1) / tpb);
-    bool extra = c->d.wsplit != 0;   // the W split (implicit upwind LO step) or a CDIFF or PPM tracer
-    for (int v : c->h_ver) extra = extra || v == VER_CDIFF || v == VER_PPM;
+    bool xv = false;   // a CDIFF or PPM tracer
+    for (int v : c->h_ver) xv = xv || v == VER_CDIFF || v == VER_PPM;
     const int xf = fgpu_kd_extras(c);
     {   // explicit diffusion terms from T^n (no-op without Ki, Redi or explicit vertical diffusion)
         int rc = fgpu_launch_diff(c, 0, nt, dt);
@@ -1519,10 +1523,15 @@ int fgpu_enqueue_fused_step(fgpu_context *c, double dt)
     }
     {
         ProfScope ps(c, "kB_node");
-        if (c->edge_gap && narrow) COL_LAUNCH(kB_cols, 1, 1, KB_EXTRA | KB_GAP, nodes, m, c->d, c->t, dt, tpb);
-        else if (c->edge_gap) COL_LAUNCH(kB_cols, 2, 1, KB_EXTRA | KB_GAP, nodes, m, c->d, c->t, dt, tpb);
-        else if (extra && narrow) COL_LAUNCH(kB_cols, 1, 1, KB_EXTRA, nodes, m, c->d, c->t, dt, tpb);
-        else if (extra) COL_LAUNCH(kB_cols, 2, 1, KB_EXTRA, nodes, m, c->d, c->t, dt, tpb);
+        const bool ws = c->d.wsplit != 0;
+        if (c->edge_gap && narrow) COL_LAUNCH(kB_cols, 1, 1, KB_XV | KB_WS | KB_GAP, nodes, m, c->d, c->t, dt, tpb);
+        else if (c->edge_gap) COL_LAUNCH(kB_cols, 2, 1, KB_XV | KB_WS | KB_GAP, nodes, m, c->d, c->t, dt, tpb);
+        else if (xv && ws && narrow) COL_LAUNCH(kB_cols, 1, 1, KB_XV | KB_WS, nodes, m, c->d, c->t, dt, tpb);
+        else if (xv && ws) COL_LAUNCH(kB_cols, 2, 1, KB_XV | KB_WS, nodes, m, c->d, c->t, dt, tpb);
+        else if (xv && narrow) COL_LAUNCH(kB_cols, 1, 1, KB_XV, nodes, m, c->d, c->t, dt, tpb);
+        else if (xv) COL_LAUNCH(kB_cols, 2, 1, KB_XV, nodes, m, c->d, c->t, dt, tpb);
+        else if (ws && narrow) COL_LAUNCH(kB_cols, 1, 1, KB_WS, nodes, m, c->d, c->t, dt, tpb);
+        else if (ws) COL_LAUNCH(kB_cols, 2, 1, KB_WS, nodes, m, c->d, c->t, dt, tpb);
         else if (pair && m.NL > 64 && m.NL <= 96) COL_LAUNCH(kB_cols, 3, 2, 0, nodes, m, c->d, c->t, dt, tpb);
         else if (!narrow) COL_LAUNCH(kB_cols, 2, 1, 0, nodes, m, c->d, c->t, dt, tpb);
         else if (slim && pair) COL_NEAR(kB_cols, 1, 0, nodes, m, c->d, c->t, dt, tpb);
