@@ -76,8 +76,10 @@ static int upload(fgpu_context *c, T **dst, const T *src, size_t n)
 // waits for its own piece and moves it on. In ms, one copy and by pieces: 4 MB
 // 0.25 and 0.23, 8 MB 0.48 and 0.41, 24 MB 1.43 and 0.74, 96 MB 5.8 and 2.6; into
 // fresh pages 4 MB 1.05 and 0.37, 24 MB 6.2 and 1.6, 96 MB 24 and 5.3. A piece
-// costs some 20 us one after the other besides its bytes, so none is made smaller
-// than FETCH_PIECE (4 MB in 16 pieces: 0.33 ms).
+// costs some 20 us one after the other besides its bytes, so a piece is about
+// FETCH_PIECE at least (4 MB in 16 pieces: 0.33 ms), and a part is cut evenly, with
+// no short last piece (5 parts of 1.1 MB: 0.43 ms at once, 0.49 in 3 pieces each,
+// the last of them short, 0.39 in 2).
 // The threads and slots come with the first large download from a device, serve
 // all its contexts and end with the last one that has used them: starting them
 // and touching the slots takes 0.6 to 1.2 ms. The pieces go through the null
@@ -104,14 +106,22 @@ struct FgpuFetcher {
     std::atomic<size_t> next{0};
     std::atomic<int> err{0};
 
+    // the pieces of a part: of about `piece` bytes, none beyond a slot
+    size_t count(const FgpuPart &q) const
+    {
+        return std::max((q.bytes + FETCH_SLOT - 1) / FETCH_SLOT, std::max((q.bytes + piece / 2) / piece, (size_t)1));
+    }
     void pieces(int w)
     {
         for (;;) {
             size_t i = next.fetch_add(1);
             int p = 0;
-            while (p < nparts && i >= (parts[p].bytes + piece - 1) / piece) i -= (parts[p++].bytes + piece - 1) / piece;
+            while (p < nparts && i >= count(parts[p])) i -= count(parts[p++]);
             if (p == nparts || err.load()) return;
-            const size_t o = i * piece, n = std::min(piece, parts[p].bytes - o);
+            const size_t bytes = parts[p].bytes, k = count(parts[p]);
+            const size_t chunk = ((bytes + k - 1) / k + 63) / 64 * 64, o = i * chunk;   // at most a slot
+            if (o >= bytes) continue;
+            const size_t n = std::min(chunk, bytes - o);
             char *slot = slots + FETCH_SLOT * w;
             hipError_t e = hipMemcpyAsync(slot, (const char *)parts[p].src + o, n, hipMemcpyDeviceToHost, nullptr);
             if (e == hipSuccess) e = hipEventRecord(arrived[w], nullptr);

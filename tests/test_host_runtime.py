@@ -220,3 +220,24 @@ def test_vertical_after_a_failed_allocation(runtime):
             ctx.close()
         assert failed == 12
         """)
+
+
+@pytest.mark.parametrize("nx,ny,layers", [(64, 64, 64), (65, 63, 64), (64, 66, 64), (87, 100, 63), (128, 96, 127), (70, 50, 121)])
+def test_download_in_pieces(runtime, nx, ny, layers):
+    """Fields around a whole number of slots and pieces come back whole, several at once too."""
+    _run(runtime, f"""
+        m = mg.build_mesh(nx={nx}, ny={ny}, dx=20e3, jitter=0.2, seed=0, cartesian=True, nlayers={layers}, hmax=4000.0,
+                          min_layers=4, max_layers={layers}, topo="bumps", bump_height=1500.0)
+        s = mg.build_state(m, seed=0, ntr=1, dt=600.0, dx=20e3)
+        rng = np.random.default_rng(0)
+        v, vo = rng.normal(size=(2, m.nod2D, {layers}))
+        c = gpu.context_for(m, s)
+        c.tracer_upload(1, v, vo)
+        for _ in range(3):
+            gv, gvo = c.tracer_download(1)
+            assert np.array_equal(gv, v) and np.array_equal(gvo, vo)
+        c.vert_vel_ale(s.dt)
+        w = c.vert_vel_download()
+        assert np.array_equal(w["w"], s.w) and np.array_equal(w["w_i"], s.w_i) and np.array_equal(w["hnode_new"], m.hnode_new)
+        c.close()
+        """)
