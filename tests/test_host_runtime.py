@@ -241,3 +241,17 @@ def test_download_in_pieces(runtime, nx, ny, layers):
         assert np.array_equal(w["w"], s.w) and np.array_equal(w["w_i"], s.w_i) and np.array_equal(w["hnode_new"], m.hnode_new)
         c.close()
         """)
+
+
+@pytest.mark.parametrize("nx,ny", [(8, 6), (38, 36), (53, 27), (67, 61), (151, 113)])
+def test_mesh_set_up_in_parts(runtime, nx, ny):
+    """The up- and downwind triangles are the oracle's, whatever number of parts the edges are searched in."""
+    _run(runtime, f"""
+        from oracle.oracle import Oracle
+        m = mg.build_mesh(nx={nx}, ny={ny}, dx=20e3, jitter=0.2, seed=1, cartesian=True, nlayers=4, hmax=4000.0,
+                          min_layers=3, max_layers=4, topo="bumps", bump_height=1500.0)
+        s = mg.build_state(m, seed=0, ntr=1, dt=600.0, dx=20e3)
+        c = gpu.context_for(m, s)
+        assert np.array_equal(c.edge_up_dn_tri(m.edge2D) - 1, Oracle(m).edge_up_dn_tri)   # 0: no such triangle
+        c.close()
+        """)
